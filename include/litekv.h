@@ -29,12 +29,12 @@
  * 16, 32, 64, 128 or 256 (the reference's --page_size,
  * lite_llama/server.py:1038-1161, "typically 16-256",
  * lite_llama/executor/paged_attention.py:27): the attention kernels walk a
- * larger page as 2 .. 16 consecutive 16-token pieces; head_dim 128 and 64 on the MFMA-tiled kernels, and 32, 64 or 256
- * (the reference kernels take the head dim as a block size,
- * lite_llama/kernels/flashdecoding.py:305, 393-396) through the same entry
- * points on one general kernel with fp32 arithmetic where no tiled kernel
- * exists (32 and 256): it writes the final rows in a single launch whatever
- * schedule was asked for, and uses no workspace.
+ * larger page as 2 .. 16 consecutive 16-token pieces; head_dim 128 and 64 (and 256 in
+ * prefill) on the MFMA-tiled kernels (the reference kernels take the head dim as
+ * a block size, lite_llama/kernels/flashdecoding.py:305, 393-396), 32 and a
+ * decode step at 256 through the same entry points on one general kernel with
+ * fp32 arithmetic: it writes the final rows in a single launch whatever schedule
+ * was asked for, and uses no workspace.
  */
 #ifndef LITEKV_H
 #define LITEKV_H

@@ -30,6 +30,7 @@ SOURCES = (
     "decode_advance.hip",
     "paged_prefill.hip",
     "paged_prefill_hd64.hip",
+    "paged_prefill_hd256.hip",
     "generic_attention.hip",
 )
 
@@ -55,6 +56,7 @@ HIPCC_FLAGS = (
 PER_FILE_FLAGS = {
     "paged_prefill.hip": ("-fno-honor-nans", "-Wno-inline-asm"),
     "paged_prefill_hd64.hip": ("-fno-honor-nans", "-Wno-inline-asm"),
+    "paged_prefill_hd256.hip": ("-fno-honor-nans", "-Wno-inline-asm"),
     # the decode step behind a shared prefix runs the same tile kernel as one role of its launch
     "paged_decode.hip": ("-Wno-inline-asm",),
     "paged_decode_hd64.hip": ("-Wno-inline-asm",),

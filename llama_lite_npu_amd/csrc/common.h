@@ -138,22 +138,26 @@ struct PrefillKeySplit {
 };
 constexpr int kMaxPrefillKeySlices = 8;
 
-// The launchers of the head dim 64 build of paged_prefill.hip (paged_prefill_hd64.hip).
-int hd64_paged_prefill(const char *what, const void *q, int64_t q_token_stride, const void *kv_pool,
-                       const float *kv_scales, int format, const int32_t *block_table,
-                       int32_t block_table_stride,
-                       const int32_t *cu_q_lens, const int32_t *context_lens, void *out,
-                       int64_t out_token_stride, int32_t batch, int32_t num_q_heads,
-                       int32_t num_kv_heads, int32_t page_size, int64_t num_pages,
-                       int32_t max_q_len, float softmax_scale, void *stream,
-                       const PrefillKeySplit &split);
-int32_t hd64_prefill_key_slices(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads,
-                                int32_t max_q_len, int64_t max_kv_len);
-int hd64_varlen_prefill(const void *q, int64_t q_token_stride, const void *k, int64_t k_token_stride,
-                        const void *v, int64_t v_token_stride, const int32_t *seq_starts,
-                        const int32_t *seq_lens, void *out, int64_t out_token_stride, int32_t batch,
-                        int32_t num_q_heads, int32_t num_kv_heads, int32_t max_seq_len,
-                        int64_t num_tokens, float softmax_scale, void *stream);
+// The launchers of one head dim's build of paged_prefill.hip (paged_prefill_hd64.hip,
+// paged_prefill_hd256.hip), to which the head dim 128 build, which owns the C ABI, hands calls of
+// that width. `kv_scales` and `format` (kv_fp8.h) describe a pool of 8-bit codes.
+struct PrefillBuild {
+  int (*paged)(const char *what, const void *q, int64_t q_token_stride, const void *kv_pool,
+               const float *kv_scales, const int32_t *block_table, int32_t block_table_stride,
+               const int32_t *cu_q_lens, const int32_t *context_lens, void *out,
+               int64_t out_token_stride, int32_t batch, int32_t num_q_heads, int32_t num_kv_heads,
+               int32_t head_dim, int32_t page_size, int64_t num_pages, int32_t max_q_len,
+               float softmax_scale, void *stream, int format, const PrefillKeySplit &split);
+  int (*varlen)(const void *q, int64_t q_token_stride, const void *k, int64_t k_token_stride,
+                const void *v, int64_t v_token_stride, const int32_t *seq_starts,
+                const int32_t *seq_lens, void *out, int64_t out_token_stride, int32_t batch,
+                int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t max_seq_len,
+                int64_t num_tokens, float softmax_scale, void *stream);
+  int32_t (*key_slices)(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t max_q_len,
+                        int64_t max_kv_len);
+};
+const PrefillBuild &hd64_prefill();
+const PrefillBuild &hd256_prefill();
 
 // The launchers of the head dim 64 build of paged_decode.hip (paged_decode_hd64.hip), to which the
 // head dim 128 build, which owns the C ABI, hands calls with head_dim == 64. `scales` marks a pool
@@ -170,8 +174,8 @@ int hd64_balanced(const char *what, const void *q, int64_t q_batch_stride, void 
                   int32_t block_table_stride, int32_t chunks, float softmax_scale, void *stream,
                   int format);
 
-// Attention for the head dims the tuned kernels (128) do not take: 32, 64 and 256
-// (generic_attention.hip). A launch is a decode step (seq_lens), a paged prefill (cu_q_lens,
+// Attention for what the tuned kernels do not take: head dim 32, decode at 256, and 256-wide
+// prefill with strides the tiled kernel cannot address (generic_attention.hip). A launch is a decode step (seq_lens), a paged prefill (cu_q_lens,
 // context_lens) or a packed prefill (kv_pool null; k, v, seq_starts, q_lens); `rows_per_seq` is
 // 1 for decode and the longest prompt or chunk otherwise. `format` is the pool's storage format
 // (kv_fp8.h); k_new / v_new fuse a decode step's append.

@@ -1,5 +1,5 @@
-// Attention for head dims other than 128 (32, 64, 256): one kernel behind the decode and prefill
-// entry points, whose tuned kernels are built around 128-wide rows. The reference kernels take
+// Attention for the head dims without a tuned kernel (32; 256 in a decode step, and in prefill where
+// the tiled kernel cannot address the rows): one kernel behind the decode and prefill entry points. The reference kernels take
 // the head dim as a compile-time block size (lite_llama/kernels/flashdecoding.py:305, 393-396;
 // flashattention2_nopad.py:39-163) and serve every model config through the same call
 // (lite_llama/models/model_config.py:200); this is that generality, with plain fp32 arithmetic

@@ -29,17 +29,24 @@ static int validate_prefill(const char *what, const void *q, int64_t q_stride, c
   return LITEKV_OK;
 }
 
-// How a GQA group of `group` heads is cut into workgroups of `col_tiles` column tiles (two per
-// wavefront).
+// Whether a 256-wide prefill goes to the tiled kernel: all of them but rows it cannot address
+// (16-byte stores of the output, 32-bit offsets into q), which stay with the general kernel. Four
+// prompts of 300 to 2048 tokens, 16 / 4 heads: 9198 us there, without matrix instructions and with
+// every K row read by one lane at a time, 81 us here.
+[[maybe_unused]] static bool tiled_256(int64_t q_stride, int64_t out_stride, int32_t num_kv_heads) {
+  return q_stride < (1 << 25) && out_stride % 8 == 0 && num_kv_heads <= 1024;
+}
+
+// How a GQA group of `group` heads is cut into workgroups.
 struct PrefillShape {
   int head_splits, heads_per_wg, row_tiles;
   unsigned row_blocks;
 };
-static PrefillShape prefill_shape(int group, int max_q_len, int col_tiles = kWgColTiles) {
+static PrefillShape prefill_shape(int group, int max_q_len) {
   PrefillShape s;
-  s.head_splits = (group + col_tiles - 1) / col_tiles;
+  s.head_splits = (group + kWgColTiles - 1) / kWgColTiles;
   s.heads_per_wg = (group + s.head_splits - 1) / s.head_splits;
-  s.row_tiles = col_tiles / s.heads_per_wg;
+  s.row_tiles = kWgColTiles / s.heads_per_wg;
   s.row_blocks = (unsigned)((max_q_len + 16 * s.row_tiles - 1) / (16 * s.row_tiles));
   return s;
 }
@@ -101,7 +108,7 @@ static int32_t prefill_key_slices(int32_t batch, int32_t num_q_heads, int32_t nu
       max_q_len <= 0 || max_kv_len <= 0 || num_q_heads / num_kv_heads > kMaxGroup) {
     return 1;
   }
-  const PrefillShape s = prefill_shape(num_q_heads / num_kv_heads, max_q_len, kColTiles * kTiledWaves);
+  const PrefillShape s = prefill_shape(num_q_heads / num_kv_heads, max_q_len);
   const int64_t wgs = (int64_t)num_kv_heads * s.head_splits * s.row_blocks * batch;
   static thread_local int cached_device = -1, cached_cus = 0;  // compute units of the current device
   int dev = 0;
@@ -116,7 +123,7 @@ static int32_t prefill_key_slices(int32_t batch, int32_t num_q_heads, int32_t nu
     cached_cus = cus;
   }
   const int64_t cus = cached_cus;
-  const int64_t slots = cus * (kHD == 64 ? 3 : 2);
+  const int64_t slots = cus * kWgPerCu;
   if (2 * wgs > slots) return 1;
   const double tile_us = kHD == 64 ? 0.6 : 1.0;
   const double tiles = (double)((max_kv_len + kKvTile - 1) / kKvTile);
@@ -147,18 +154,21 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
                                 int64_t out_token_stride, int32_t batch, int32_t num_q_heads,
                                 int32_t num_kv_heads, int32_t head_dim, int32_t page_size,
                                 int64_t num_pages, int32_t max_q_len, float softmax_scale,
-                                void *stream, int format,
-                                const PrefillKeySplit &split = PrefillKeySplit{}) {
+                                void *stream, int format, const PrefillKeySplit &split) {
   const bool fp8 = format != kKvF16;  // a pool of 8-bit codes
   LITEKV_REQUIRE(split.key_slices >= 1 && split.key_slices <= kMaxPrefillKeySlices,
                  "%s: key_slices %d out of [1, %d]", what, split.key_slices, kMaxPrefillKeySlices);
   LITEKV_REQUIRE(split.key_slices == 1 || head_dim == 128 || head_dim == 64,
                  "%s: key slices take head_dim 64 or 128", what);
 #if LITEKV_HD == 128
-  if (head_dim == 64) {  // the head dim 64 build of this file
-    return hd64_paged_prefill(what, q, q_token_stride, kv_pool, kv_scales, format, block_table, block_table_stride,
-                              cu_q_lens, context_lens, out, out_token_stride, batch, num_q_heads,
-                              num_kv_heads, page_size, num_pages, max_q_len, softmax_scale, stream, split);
+  const PrefillBuild *build = head_dim == 64 ? &hd64_prefill()
+                              : head_dim == 256 && tiled_256(q_token_stride, out_token_stride, num_kv_heads)
+                                  ? &hd256_prefill()
+                                  : nullptr;
+  if (build != nullptr) {  // another head dim's build of this file
+    return build->paged(what, q, q_token_stride, kv_pool, kv_scales, block_table, block_table_stride, cu_q_lens,
+                        context_lens, out, out_token_stride, batch, num_q_heads, num_kv_heads, head_dim,
+                        page_size, num_pages, max_q_len, softmax_scale, stream, format, split);
   }
 #endif
   if (head_dim != kHD && generic_head_dim(head_dim)) {  // see generic_attention.hip
@@ -209,6 +219,7 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
                     num_kv_heads, (int32_t)num_pages, kv_scales, page_shift};
   PackedSource packed{nullptr, nullptr, 0, 0, nullptr};
   const int group = num_q_heads / num_kv_heads;
+#if LITEKV_HD != 256
   if (split.key_slices > 1) {
     // every block's keys in key_slices runs of tiles, one workgroup each, then the merge
     const int slices = split.key_slices;
@@ -219,7 +230,7 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
     LITEKV_REQUIRE(split.workspace != nullptr && aligned16(split.workspace) && split.workspace_bytes >= need,
                    "%s: workspace of %zu bytes needed for %d key slices, got %zu", what, need, slices,
                    split.workspace_bytes);
-    const PrefillShape s = prefill_shape(group, max_q_len, kColTiles * kTiledWaves);
+    const PrefillShape s = prefill_shape(group, max_q_len);
     LITEKV_REQUIRE((uint64_t)s.row_blocks * slices <= 65535u, "%s: max_q_len %d too large for %d key slices",
                    what, max_q_len, slices);
     float *part_o = static_cast<float *>(split.workspace);
@@ -248,12 +259,12 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
                        out_token_stride, rows, num_q_heads, slices);
     return check_launch(what);
   }
-  const int waves = (format == kKvF16 && LITEKV_PREFILL_WAVES == kWideWaves) ? kWideWaves : kTiledWaves;
-  const PrefillShape s = prefill_shape(group, max_q_len, kColTiles * waves);
+#endif  // LITEKV_HD != 256
+  const PrefillShape s = prefill_shape(group, max_q_len);
   LITEKV_REQUIRE(s.row_blocks <= 65535u, "%s: max_q_len %d too large", what, max_q_len);
   const dim3 grid((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch);
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(waves * kWave), 0, static_cast<hipStream_t>(stream),
+    hipLaunchKernelGGL(kernel, grid, dim3(kTiledWaves * kWave), 0, static_cast<hipStream_t>(stream),
                        static_cast<const half_t *>(q), q_token_stride, static_cast<half_t *>(out),
                        out_token_stride, paged, packed, PrefixTask{}, cu_q_lens,
                        (const int32_t *)nullptr, context_lens, group, s.head_splits, s.heads_per_wg,
@@ -263,8 +274,6 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
     launch(varlen_prefill_tiled_kernel<kPagedPrefillInt8>);
   } else if (format == kKvFp8) {
     launch(varlen_prefill_tiled_kernel<kPagedPrefillFp8>);
-  } else if (waves == kWideWaves) {
-    launch(varlen_prefill_tiled_kernel<kPagedPrefill, kWideWaves>);
   } else {
     launch(varlen_prefill_tiled_kernel<kPagedPrefill>);
   }
@@ -279,10 +288,16 @@ static int launch_varlen_prefill(const void *q, int64_t q_token_stride, const vo
                                  int32_t num_kv_heads, int32_t head_dim, int32_t max_seq_len,
                                  int64_t num_tokens, float softmax_scale, void *stream) {
 #if LITEKV_HD == 128
-  if (head_dim == 64) {  // the head dim 64 build of this file
-    return hd64_varlen_prefill(q, q_token_stride, k, k_token_stride, v, v_token_stride, seq_starts,
-                               seq_lens, out, out_token_stride, batch, num_q_heads, num_kv_heads,
-                               max_seq_len, num_tokens, softmax_scale, stream);
+  const PrefillBuild *build =
+      head_dim == 64 ? &hd64_prefill()
+      : head_dim == 256 && tiled_256(q_token_stride, out_token_stride, num_kv_heads) &&
+              k_token_stride < (1 << 25) && v_token_stride < (1 << 25)
+          ? &hd256_prefill()
+          : nullptr;
+  if (build != nullptr) {  // another head dim's build of this file
+    return build->varlen(q, q_token_stride, k, k_token_stride, v, v_token_stride, seq_starts, seq_lens, out,
+                         out_token_stride, batch, num_q_heads, num_kv_heads, head_dim, max_seq_len,
+                         num_tokens, softmax_scale, stream);
   }
 #endif
   if (head_dim != kHD && generic_head_dim(head_dim)) {  // see generic_attention.hip
@@ -328,55 +343,33 @@ static int launch_varlen_prefill(const void *q, int64_t q_token_stride, const vo
   PackedSource packed{static_cast<const half_t *>(k), static_cast<const half_t *>(v),
                       k_token_stride, v_token_stride, seq_starts};
   const int group = num_q_heads / num_kv_heads;
-  const int waves = LITEKV_PREFILL_WAVES == kWideWaves ? kWideWaves : kTiledWaves;
-  const PrefillShape s = prefill_shape(group, max_seq_len, kColTiles * waves);
+  const PrefillShape s = prefill_shape(group, max_seq_len);
   LITEKV_REQUIRE(s.row_blocks <= 65535u, "varlen_prefill: max_seq_len %d too large", max_seq_len);
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel,
                        dim3((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch),
-                       dim3(waves * kWave), 0, static_cast<hipStream_t>(stream),
+                       dim3(kTiledWaves * kWave), 0, static_cast<hipStream_t>(stream),
                        static_cast<const half_t *>(q), q_token_stride, static_cast<half_t *>(out),
                        out_token_stride, paged, packed, PrefixTask{}, seq_starts, seq_lens,
                        (const int32_t *)nullptr, group, s.head_splits, s.heads_per_wg, s.row_tiles,
                        softmax_scale * kLog2eP, 1);
   };
-  if (waves == kWideWaves) {
-    launch(varlen_prefill_tiled_kernel<kPackedPrefill, kWideWaves>);
-  } else {
-    launch(varlen_prefill_tiled_kernel<kPackedPrefill>);
-  }
+  launch(varlen_prefill_tiled_kernel<kPackedPrefill>);
   return check_launch("varlen_prefill");
 }
 }  // namespace LITEKV_HD_NS
 
 #if LITEKV_HD == 64
-int hd64_paged_prefill(const char *what, const void *q, int64_t q_token_stride, const void *kv_pool,
-                       const float *kv_scales, int format, const int32_t *block_table,
-                       int32_t block_table_stride,
-                       const int32_t *cu_q_lens, const int32_t *context_lens, void *out,
-                       int64_t out_token_stride, int32_t batch, int32_t num_q_heads,
-                       int32_t num_kv_heads, int32_t page_size, int64_t num_pages,
-                       int32_t max_q_len, float softmax_scale, void *stream,
-                       const PrefillKeySplit &split) {
-  return launch_paged_prefill(what, q, q_token_stride, kv_pool, kv_scales, block_table,
-                              block_table_stride, cu_q_lens, context_lens, out, out_token_stride,
-                              batch, num_q_heads, num_kv_heads, 64, page_size, num_pages, max_q_len,
-                              softmax_scale, stream, format, split);
+const PrefillBuild &hd64_prefill() {
+  static const PrefillBuild build{launch_paged_prefill, launch_varlen_prefill, prefill_key_slices};
+  return build;
 }
-int32_t hd64_prefill_key_slices(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads,
-                                int32_t max_q_len, int64_t max_kv_len) {
-  return prefill_key_slices(batch, num_q_heads, num_kv_heads, max_q_len, max_kv_len);
+#elif LITEKV_HD == 256
+const PrefillBuild &hd256_prefill() {
+  static const PrefillBuild build{launch_paged_prefill, launch_varlen_prefill, nullptr};
+  return build;
 }
-int hd64_varlen_prefill(const void *q, int64_t q_token_stride, const void *k, int64_t k_token_stride,
-                        const void *v, int64_t v_token_stride, const int32_t *seq_starts,
-                        const int32_t *seq_lens, void *out, int64_t out_token_stride, int32_t batch,
-                        int32_t num_q_heads, int32_t num_kv_heads, int32_t max_seq_len,
-                        int64_t num_tokens, float softmax_scale, void *stream) {
-  return launch_varlen_prefill(q, q_token_stride, k, k_token_stride, v, v_token_stride, seq_starts,
-                               seq_lens, out, out_token_stride, batch, num_q_heads, num_kv_heads, 64,
-                               max_seq_len, num_tokens, softmax_scale, stream);
-}
-#endif  // LITEKV_HD == 64
+#endif
 }  // namespace litekv
 
 #if LITEKV_HD == 128  // the C ABI lives in the head dim 128 build of this file
@@ -392,7 +385,7 @@ extern "C" int litekv_paged_prefill(const void *q, int64_t q_token_stride, const
                                       block_table_stride, cu_q_lens, context_lens, out,
                                       out_token_stride, batch, num_q_heads, num_kv_heads, head_dim,
                                       page_size, num_pages, max_q_len, softmax_scale, stream,
-                                      litekv::kKvF16);
+                                      litekv::kKvF16, litekv::PrefillKeySplit{});
 }
 
 extern "C" size_t litekv_paged_prefill_split_workspace_bytes(int64_t num_tokens, int32_t num_q_heads,
@@ -406,7 +399,7 @@ extern "C" int32_t litekv_paged_prefill_key_slices(int32_t batch, int32_t num_q_
                                                    int32_t num_kv_heads, int32_t head_dim,
                                                    int32_t max_q_len, int64_t max_kv_len) {
   if (head_dim == 64) {
-    return litekv::hd64_prefill_key_slices(batch, num_q_heads, num_kv_heads, max_q_len, max_kv_len);
+    return litekv::hd64_prefill().key_slices(batch, num_q_heads, num_kv_heads, max_q_len, max_kv_len);
   }
   if (head_dim != 128) return 1;
   return litekv::prefill_key_slices(batch, num_q_heads, num_kv_heads, max_q_len, max_kv_len);
@@ -466,7 +459,7 @@ extern "C" int litekv_paged_prefill_fp8(const void *q, int64_t q_token_stride, c
                                       block_table, block_table_stride, cu_q_lens, context_lens, out,
                                       out_token_stride, batch, num_q_heads, num_kv_heads, head_dim,
                                       page_size, num_pages, max_q_len, softmax_scale, stream,
-                                      litekv::kKvFp8);
+                                      litekv::kKvFp8, litekv::PrefillKeySplit{});
 }
 
 extern "C" int litekv_paged_prefill_int8(const void *q, int64_t q_token_stride, const void *kv_pool,
@@ -481,7 +474,7 @@ extern "C" int litekv_paged_prefill_int8(const void *q, int64_t q_token_stride, 
                                       block_table, block_table_stride, cu_q_lens, context_lens, out,
                                       out_token_stride, batch, num_q_heads, num_kv_heads, head_dim,
                                       page_size, num_pages, max_q_len, softmax_scale, stream,
-                                      litekv::kKvInt8);
+                                      litekv::kKvInt8, litekv::PrefillKeySplit{});
 }
 
 extern "C" int litekv_varlen_prefill(const void *q, int64_t q_token_stride, const void *k,

@@ -63,13 +63,6 @@
 #include "head_dim.h"
 #include "kv_fp8.h"
 
-// Wavefronts per workgroup of the fp16 prefill launches: 4, or 8 (twice the query rows on every
-// staged K/V tile, one workgroup per compute unit instead of two; measured 2 to 5 % slower on
-// ragged prompts of 128 to 2048 tokens, 1 % faster on 8192-token ones).
-#ifndef LITEKV_PREFILL_WAVES
-#define LITEKV_PREFILL_WAVES 4
-#endif
-
 namespace litekv {
 inline namespace LITEKV_HD_NS {
 namespace prefill_tile {
@@ -84,8 +77,20 @@ constexpr int kLoadsPerWave = 16 / kRowsPerLoad;  // such instructions per wavef
 // XOR applied to the 16-byte chunk index of staged row r, for K (and q) and for V. A row of 256
 // bytes covers all 64 banks, so consecutive rows must differ in the chunk; rows of 128 bytes
 // alternate between the bank halves, so it is every second row that must.
-__device__ __forceinline__ int k_swz(int r) { return kHD == 128 ? (r & 15) : ((r >> 1) & 7); }
-__device__ __forceinline__ int v_swz(int r) { return kHD == 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); }
+// (Rows of 512 bytes cover the banks twice over: the map of 256-byte rows inside each half.)
+__device__ __forceinline__ int k_swz(int r) { return kHD >= 128 ? (r & 15) : ((r >> 1) & 7); }
+__device__ __forceinline__ int v_swz(int r) { return kHD >= 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); }
+
+// At head dim 256 a probability reaches the second product as two fp16 numbers, its rounding and
+// what the rounding left (22 bits together), each with an MFMA of its own: prompts of that width
+// have always been attended with fp32 probabilities. It costs half as many MFMAs again (the V
+// fragments and their LDS reads are shared).
+constexpr bool kTwoPartP = kHD == 256;
+// Workgroups per compute unit: bounded by registers at 64 and 128 (about 150 and 235 per lane), by
+// LDS at 256 (two tiles of K and of V are 128 KiB), where a lane may then use all 512 registers.
+constexpr int kWgPerCu = kHD == 64 ? 3 : kHD == 128 ? 2 : 1;
+// Immediate of s_waitcnt that waits for all but the n youngest vector memory requests.
+constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 
 constexpr float kLog2eP = 1.4426950408889634f;
 
@@ -122,8 +127,8 @@ struct PackedSource {
 
 constexpr int kKvTile = 64;
 constexpr int kColTiles = 2;      // 16-column tiles per wavefront
-constexpr int kTiledWaves = 4;    // wavefronts of a workgroup, unless the kernel is built for kWideWaves
-constexpr int kWideWaves = 8;     // fp16 prefill only: twice the columns on every staged K/V tile
+constexpr int kTiledWaves = 4;    // wavefronts of a prefill workgroup
+constexpr int kWideWaves = 8;     // a shared prefix: twice the columns on every staged K/V tile (prefill: 2 to 5 % slower)
 constexpr int kWgColTiles = kColTiles * kTiledWaves;
 constexpr int kTileHalfs = kKvTile * kHD;  // one staged tile: 64 rows of 2 * kHD bytes
 
@@ -181,14 +186,14 @@ __device__ __forceinline__ void prefill_tile_body(
   // (rows of 64 codes staged by 8 wavefronts would leave a lane 8 codes, half a 16-byte load)
   static_assert(W == kTiledWaves || (W == kWideWaves && (!FP8 || kHD == 128)),
                 "eight wavefronts: fp16 K/V, or 8-bit codes at head dim 128");
+  static_assert(kHD != 256 || (W == kTiledWaves && !KSPLIT && !SHARED), "256: plain prefill only");
   // Rows of a 64-key tile one wavefront stages (a page, or half of one), and the direct-load
   // instructions that takes per operand.
   constexpr int kRowsPerWave = kKvTile / W;
   constexpr int kLoads = kRowsPerWave / kRowsPerLoad;
-  // Two tiles of K, then two of V: tile t sits in half t % 2. Eight wavefronts have a third
-  // region of the same size behind them: q of wavefronts 4..7, and room for the output rows.
+  // Two tiles of K, then two of V: tile t sits in half t % 2. (Eight wavefronts have a third
+  // region of the same size behind them: room for their partial rows.)
   const uint32_t v_lds = k_lds + 4u * kTileHalfs;  // LDS byte addresses
-  const uint32_t x_lds = v_lds + 4u * kTileHalfs;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -392,8 +397,8 @@ __device__ __forceinline__ void prefill_tile_body(
   // the fragments are read back from there. Requested before tile 0: vmcnt counts in order.
   uint32_t q_lds = 0;
   if constexpr (!SHARED) {
-    q_lds = wave < 4 ? ((wave & 2) ? v_lds : k_lds) + (uint32_t)(kTileHalfs * 2 + (wave & 1) * (64 * kHD))
-                     : x_lds + (uint32_t)((wave - 4) * (64 * kHD));
+    static_assert(SHARED || W == kTiledWaves, "the q rows of four wavefronts fit a tile half of K and of V");
+    q_lds = ((wave & 2) ? v_lds : k_lds) + (uint32_t)(kTileHalfs * 2 + (wave & 1) * (64 * kHD));
 #pragma unroll
     for (int u = 0; u < kColTiles; ++u) {
       const int t = wave * kColTiles + u;
@@ -456,9 +461,9 @@ __device__ __forceinline__ void prefill_tile_body(
   if constexpr (!SHARED) {
     // the loads of tile 0 (K and V) were requested after q's
     if constexpr (FP8) {
-      __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * kRawVecs));
+      __builtin_amdgcn_s_waitcnt(wait_vm(2 * kRawVecs));
     } else {
-      __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * kLoads));
+      __builtin_amdgcn_s_waitcnt(wait_vm(2 * kLoads));
     }
 #pragma unroll
     for (int u = 0; u < kColTiles; ++u) {
@@ -512,6 +517,7 @@ __device__ __forceinline__ void prefill_tile_body(
 
   float4_t st[2][kColTiles];
   half8_t pk[kColTiles];
+  half8_t pk_lo[kColTiles];  // kTwoPartP: what the rounding of pk left
 
   // S^T of 32 keys (rows 32 s2 .. +31 of the staged K tile) against this wavefront's columns.
   auto scores_into = [&](float4_t (&st)[2][kColTiles], int s2, auto seeded_tag) {
@@ -552,32 +558,46 @@ __device__ __forceinline__ void prefill_tile_body(
   typedef float float2_t __attribute__((ext_vector_type(2)));
   typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
   // General path: p = 2^(s * k_mul - m) from unseeded scores.
-  auto exponentials_of = [&](const float4_t (&st)[2][kColTiles], half8_t (&pk)[kColTiles], int u) {
+  auto put_pair = [&](float2_t p, half8_t &hi, half8_t &lo, int at) {
+    const half2_t ph = __builtin_convertvector(p, half2_t);
+    hi[at] = ph[0];
+    hi[at + 1] = ph[1];
+    if constexpr (kTwoPartP) {
+      const half2_t pl = __builtin_convertvector(p - __builtin_convertvector(ph, float2_t), half2_t);
+      lo[at] = pl[0];
+      lo[at + 1] = pl[1];
+    }
+  };
+  auto exponentials_of = [&](const float4_t (&st)[2][kColTiles], half8_t (&pk)[kColTiles],
+                             half8_t (&pk_lo)[kColTiles], int u) {
     const float neg_m = -m_run[u];
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
 #pragma unroll
       for (int i = 0; i < 4; i += 2) {
-        const float2_t p = float2_t{fast_exp2(__builtin_fmaf(st[m][u][i], k_mul, neg_m)),
-                                    fast_exp2(__builtin_fmaf(st[m][u][i + 1], k_mul, neg_m))};
-        const half2_t ph = __builtin_convertvector(p, half2_t);
-        pk[u][4 * m + i] = ph[0];
-        pk[u][4 * m + i + 1] = ph[1];
+        put_pair(float2_t{fast_exp2(__builtin_fmaf(st[m][u][i], k_mul, neg_m)),
+                          fast_exp2(__builtin_fmaf(st[m][u][i + 1], k_mul, neg_m))},
+                 pk[u], pk_lo[u], 4 * m + i);
       }
     }
   };
   // Fast path: the scores were seeded with -m / k_mul, so they are the exponents up to that factor.
-  auto exponentials_seeded = [&](const float4_t (&st)[2][kColTiles], half8_t (&pk)[kColTiles], int u) {
+  auto exponentials_seeded = [&](const float4_t (&st)[2][kColTiles], half8_t (&pk)[kColTiles],
+                                 half8_t (&pk_lo)[kColTiles], int u) {
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
 #pragma unroll
       for (int i = 0; i < 4; i += 2) {
-        const float2_t p = float2_t{fast_exp2(st[m][u][i] * k_mul), fast_exp2(st[m][u][i + 1] * k_mul)};
-        const half2_t ph = __builtin_convertvector(p, half2_t);
-        pk[u][4 * m + i] = ph[0];
-        pk[u][4 * m + i + 1] = ph[1];
+        put_pair(float2_t{fast_exp2(st[m][u][i] * k_mul), fast_exp2(st[m][u][i + 1] * k_mul)}, pk[u],
+                 pk_lo[u], 4 * m + i);
       }
     }
+  };
+  // One MFMA with the probabilities of a column tile (two where they come in two parts).
+  auto mfma_p = [&](half8_t a, half8_t hi, half8_t lo, float4_t c) -> float4_t {
+    c = mfma_16x16x32(a, hi, c);
+    if constexpr (kTwoPartP) c = mfma_16x16x32(a, lo, c);
+    return c;
   };
   // True if any probability of the sub-tile exceeds 2^8 (or is not finite): the running maximum
   // is then too low for these keys and the sub-tile has to be redone with a rescale. Probabilities
@@ -596,9 +616,9 @@ __device__ __forceinline__ void prefill_tile_body(
     return __builtin_amdgcn_ballot_w64(top > 0x5C00u) != 0;  // 0x5C00 = 256.0
   };
   // O^T += V^T . P^T,  l += 1^T . P^T for keys 32 s2 .. +31 of the staged V tile.
-  auto accumulate_with = [&](const half8_t (&pk)[kColTiles], int s2) {
+  auto accumulate_sub = [&](int s2) {
 #pragma unroll
-    for (int u = 0; u < kColTiles; ++u) dsum[u] = mfma_16x16x32(ones, pk[u], dsum[u]);
+    for (int u = 0; u < kColTiles; ++u) dsum[u] = mfma_p(ones, pk[u], pk_lo[u], dsum[u]);
 #pragma unroll
     for (int j = 0; j < kJTiles; ++j) {
       const uint32_t at = v_addr[j] + 2u * 32 * s2 * kHD;
@@ -608,7 +628,7 @@ __device__ __forceinline__ void prefill_tile_body(
       const short8_t both = short8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       const half8_t a = __builtin_bit_cast(half8_t, both);
 #pragma unroll
-      for (int u = 0; u < kColTiles; ++u) acc[j][u] = mfma_16x16x32(a, pk[u], acc[j][u]);
+      for (int u = 0; u < kColTiles; ++u) acc[j][u] = mfma_p(a, pk[u], pk_lo[u], acc[j][u]);
     }
   };
   // V^T fragment j (A operand: d rows 16j.., keys 32 s2 + {4g..4g+3, 16+4g..}) of the staged tile.
@@ -622,10 +642,9 @@ __device__ __forceinline__ void prefill_tile_body(
   };
   auto scores_sub = [&](int s2) { scores_into(st, s2, std::false_type{}); };
   auto column_max = [&](int u) { return column_max_of(st, u); };
-  auto exponentials = [&](int u) { exponentials_of(st, pk, u); };
-  auto accumulate_sub = [&](int s2) { accumulate_with(pk, s2); };
+  auto exponentials = [&](int u) { exponentials_of(st, pk, pk_lo, u); };
   float4_t st1[2][kColTiles];  // scores of the second half of a fast tile
-  half8_t pk1[kColTiles];
+  half8_t pk1[kColTiles], pk1_lo[kColTiles];
 
   // Publishes tile kt (already requested) and requests tile kt + 1 into the other half.
   auto sync_and_prefetch = [&](int kt, bool issue_next = true) {
@@ -645,7 +664,7 @@ __device__ __forceinline__ void prefill_tile_body(
         *(lds_half8_t *)(uintptr_t)(v_lds + row_at + 16u * (uint32_t)(chunk ^ v_swz(r))) = vh;
       }
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's part of tile kt is in LDS
+    __builtin_amdgcn_s_waitcnt(wait_vm(0));  // this wavefront's part of tile kt is in LDS
     __syncthreads();                     // ... and everyone's; everyone is done with tile kt-1
     if (issue_next && kt + 1 < n_tiles) issue_tile(kt + 1);
   };
@@ -734,8 +753,8 @@ __device__ __forceinline__ void prefill_tile_body(
           mask_sub(0, key0);
           mask_sub(1, key0);
         }
-        exponentials_seeded(st, pk, 0);
-        exponentials_seeded(st, pk, 1);
+        exponentials_seeded(st, pk, pk_lo, 0);
+        exponentials_seeded(st, pk, pk_lo, 1);
         if (overflowed(pk)) return 1 + s2;
         accumulate_sub(s2);
       }
@@ -803,46 +822,46 @@ __device__ __forceinline__ void prefill_tile_body(
         for (int u = 0; u < kColTiles; ++u) st1[i & 1][u] = mfma_16x16x32(kf1[i], qf[u][i >> 1], st1[i & 1][u]);
         vf[i] = load_vfrag(i, 0);
       }
-      exponentials_seeded(st, pk, 0);
-      exponentials_seeded(st, pk, 1);
+      exponentials_seeded(st, pk, pk_lo, 0);
+      exponentials_seeded(st, pk, pk_lo, 1);
       const bool over_a = overflowed(pk);
 #pragma unroll
       for (int i = 0; i < kJTiles; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, kTwoPartP ? 6 : 5, 0);
       }
       if (over_a) return 1;
       // Block 2: second product of the first half beside the second half's exponentials; each
       // fragment register takes the second half's fragment as soon as its MFMAs are issued.
       half8_t vf2[kJTiles];
 #pragma unroll
-      for (int u = 0; u < kColTiles; ++u) dsum[u] = mfma_16x16x32(ones, pk[u], dsum[u]);
+      for (int u = 0; u < kColTiles; ++u) dsum[u] = mfma_p(ones, pk[u], pk_lo[u], dsum[u]);
 #pragma unroll
       for (int j = 0; j < kJTiles; ++j) {
 #pragma unroll
-        for (int u = 0; u < kColTiles; ++u) acc[j][u] = mfma_16x16x32(vf[j], pk[u], acc[j][u]);
+        for (int u = 0; u < kColTiles; ++u) acc[j][u] = mfma_p(vf[j], pk[u], pk_lo[u], acc[j][u]);
         vf2[j] = load_vfrag(j, 1);
       }
-      exponentials_seeded(st1, pk1, 0);
-      exponentials_seeded(st1, pk1, 1);
+      exponentials_seeded(st1, pk1, pk1_lo, 0);
+      exponentials_seeded(st1, pk1, pk1_lo, 1);
       const bool over_b = overflowed(pk1);
 #pragma unroll
       for (int i = 0; i < kJTiles; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, kTwoPartP ? 4 : 2, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, kTwoPartP ? 6 : 5, 0);
       }
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, kTwoPartP ? 4 : 2, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
       if (over_b) return 2;
       // Block 3: second product of the second half.
 #pragma unroll
-      for (int u = 0; u < kColTiles; ++u) dsum[u] = mfma_16x16x32(ones, pk1[u], dsum[u]);
+      for (int u = 0; u < kColTiles; ++u) dsum[u] = mfma_p(ones, pk1[u], pk1_lo[u], dsum[u]);
 #pragma unroll
       for (int j = 0; j < kJTiles; ++j) {
 #pragma unroll
-        for (int u = 0; u < kColTiles; ++u) acc[j][u] = mfma_16x16x32(vf2[j], pk1[u], acc[j][u]);
+        for (int u = 0; u < kColTiles; ++u) acc[j][u] = mfma_p(vf2[j], pk1[u], pk1_lo[u], acc[j][u]);
       }
     }
     return 0;
@@ -873,9 +892,7 @@ __device__ __forceinline__ void prefill_tile_body(
     // (the K/V tiles are done with) and leave as whole 256-byte rows, 4 rows per instruction.
     constexpr int kOutPitch = 2 * kHD + 16;  // bytes; at 128: 68 dwords, a half-wave's 8-byte writes hit 64 banks
     __syncthreads();                              // every wavefront is done reading the last tile
-    const uint32_t mine = W == kWideWaves
-                              ? k_lds + (uint32_t)(wave * kColTiles * 16 * kOutPitch)
-                              : ((wave & 2) ? v_lds : k_lds) + (uint32_t)((wave & 1) * kColTiles * 16 * kOutPitch);
+    const uint32_t mine = ((wave & 2) ? v_lds : k_lds) + (uint32_t)((wave & 1) * kColTiles * 16 * kOutPitch);
 #pragma unroll
     for (int u = 0; u < kColTiles; ++u) {
       const float inv = v_scale / dsum[u][0];
@@ -969,25 +986,25 @@ __device__ __forceinline__ void prefill_tile_body(
   }
 }
 
-template <int MODE, int W = kTiledWaves>
-__global__ __launch_bounds__(W *kWave, W == kWideWaves ? 1 : (kHD == 64 ? 3 : 2)) void varlen_prefill_tiled_kernel(
+template <int MODE>
+__global__ __launch_bounds__(kTiledWaves *kWave, kWgPerCu) void varlen_prefill_tiled_kernel(
     const half_t *__restrict__ q, int64_t q_stride, half_t *__restrict__ out, int64_t out_stride,
     PagedSource paged, PackedSource packed, PrefixTask prefix,
     const int32_t *__restrict__ q_starts_or_cu, const int32_t *__restrict__ q_lens_or_null,
     const int32_t *__restrict__ context_lens, int32_t group, int32_t head_splits,
     int32_t heads_per_wg, int32_t row_tiles, float scale_log2, int32_t key_slices) {
-  __shared__ __attribute__((aligned(1024))) half_t lds_all[tile_lds_bytes<W>() / 2];
+  __shared__ __attribute__((aligned(1024))) half_t lds_all[tile_lds_bytes<kTiledWaves>() / 2];
   if constexpr (MODE == kPagedPrefillSplit || MODE == kPagedPrefillSplitFp8 ||
                 MODE == kPagedPrefillSplitInt8) {
     // blockIdx.y = row block * key_slices + slice: the slices of a block are neighbours
     const int by = (int)blockIdx.y / key_slices;
-    prefill_tile_body<MODE, W>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, by,
+    prefill_tile_body<MODE, kTiledWaves>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, by,
                                (int)blockIdx.z, (int)gridDim.y / key_slices, q, q_stride, out, out_stride,
                                paged, packed, prefix, q_starts_or_cu, q_lens_or_null, context_lens, group,
                                head_splits, heads_per_wg, row_tiles, scale_log2,
                                (int)blockIdx.y - by * key_slices, key_slices);
   } else {
-    prefill_tile_body<MODE, W>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, (int)blockIdx.y,
+    prefill_tile_body<MODE, kTiledWaves>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, (int)blockIdx.y,
                                (int)blockIdx.z, (int)gridDim.y, q, q_stride, out, out_stride, paged, packed,
                                prefix, q_starts_or_cu, q_lens_or_null, context_lens, group, head_splits,
                                heads_per_wg, row_tiles, scale_log2);
