@@ -469,6 +469,22 @@ int litekv_paged_decode_prefix_fp8(const void *q, int64_t q_batch_stride, void *
                                    int32_t shared_pages, float softmax_scale, void *stream);
 
 /*
+ * Up to 8 small device arrays copied in one launch: the inputs of a decode step
+ * that is replayed from a graph, moved into the graph's fixed tensors (the copies
+ * of NpuGraphRunner.replay, lite_llama/executor/npu_graph.py:183-197):
+ *     dst[r * dst_pitch + c] = src[r * src_pitch + c]   r in [0, rows), c in [0, row_bytes)
+ * `segments` is a HOST array, read during the call. Addresses, sizes and pitches
+ * are multiples of 4 bytes; sources and destinations must not overlap; a segment
+ * without bytes is skipped; at most 1 GiB each.
+ */
+typedef struct {
+  const void *src;
+  void *dst;
+  int64_t rows, row_bytes, src_pitch, dst_pitch;
+} litekv_copy_segment;
+int litekv_copy_segments(const litekv_copy_segment *segments, int32_t count, void *stream);
+
+/*
  * Advances the metadata of a decode batch by one token on the device, so that
  * a captured graph of a decode step replays without host work. Replaces, per
  * step, PagedReqTokensManager.extend_req + batch_metadata

@@ -183,6 +183,7 @@ SIGNATURES = {
         [c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
          c_int64, c_int32, c_void_p, c_int32, c_int32, c_int64, c_int32, c_void_p],
     ),
+    "litekv_copy_segments": (c_int32, [c_void_p, c_int32, c_void_p]),
     "litekv_profile_next_decode": (c_int32, [c_void_p, c_void_p]),
     "litekv_paged_prefill": (
         c_int32,

@@ -28,6 +28,7 @@ SOURCES = (
     "paged_decode.hip",
     "paged_decode_hd64.hip",
     "decode_advance.hip",
+    "copy_segments.hip",
     "paged_prefill.hip",
     "paged_prefill_hd64.hip",
     "paged_prefill_hd256.hip",

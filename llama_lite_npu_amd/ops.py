@@ -7,6 +7,7 @@ enqueue work on ``torch.cuda.current_stream()``.
 
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Optional, Sequence
 
@@ -487,6 +488,43 @@ def decode_advance(request_tables: torch.Tensor, request_ids: torch.Tensor, seq_
         _ptr(seq_lens), _ptr(seq_lens_i64), _ptr(slot_mapping), _ptr(position_ids), _ptr(block_table),
         block_table.stride(0) if b > 1 else max(block_table.stride(0), width), width, _ptr(overflow), b,
         int(page_size), int(num_pages), int(increment), _stream()))
+
+
+def _segment(dst: torch.Tensor, src: torch.Tensor) -> Optional[tuple]:
+    """(src, dst, rows, row bytes, src pitch, dst pitch) of a copy litekv_copy_segments can take, or None."""
+    if not (src.is_cuda and src.dtype == dst.dtype and src.shape == dst.shape and src.device == dst.device):
+        return None
+    size = dst.element_size()
+    if src.is_contiguous() and dst.is_contiguous():
+        rows, row_bytes = 1, dst.numel() * size
+        src_pitch = dst_pitch = row_bytes
+    elif dst.dim() == 2 and dst.stride(1) == 1 and src.stride(1) == 1:
+        rows, row_bytes = dst.shape[0], dst.shape[1] * size
+        src_pitch, dst_pitch = src.stride(0) * size, dst.stride(0) * size
+        if rows > 1 and (src_pitch < row_bytes or dst_pitch < row_bytes):    # a broadcast row
+            return None
+    else:
+        return None
+    entry = (src.data_ptr(), dst.data_ptr(), rows, row_bytes, src_pitch, dst_pitch)
+    aligned = (entry[0] | entry[1] | row_bytes | src_pitch | dst_pitch) % 4 == 0
+    return entry if aligned and rows * row_bytes <= 1 << 30 else None
+
+
+def copy_tensors(pairs: Sequence[tuple]) -> None:
+    """dst.copy_(src) for every (dst, src): small device tensors of equal type and shape go eight to a
+    launch, whatever else there is one by one."""
+    segments: list = []
+    count = 0
+    for dst, src in pairs:
+        entry = _segment(dst, src) if dst.is_cuda else None
+        if entry is None:
+            dst.copy_(src)
+            continue
+        segments += entry
+        count += 1
+    for i in range(0, count, 8):
+        part = segments[6 * i:6 * (i + 8)]
+        _lib.check(_lib.load().litekv_copy_segments((ctypes.c_int64 * len(part))(*part), len(part) // 6, _stream()))
 
 
 def decode_step(q: torch.Tensor, kv_pool: torch.Tensor, plan: DecodePlan,
