@@ -24,27 +24,35 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device as the C ABI takes it (torch.cuda.current_stream() builds
+    a Stream object around the same number, which takes longer than the rest of a wrapper's checks)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
+# The wrappers run once per layer and step: checks on their path are plain conditions, and the message
+# of one is only put together when it fails.
 def _need(cond: bool, msg: str) -> None:
     if not cond:
         raise ValueError(msg)
 
 
 def _dev_half(name: str, t: torch.Tensor) -> None:
-    _need(t.is_cuda, f"{name} must live on the GPU")
-    _need(t.dtype == torch.float16, f"{name} must be float16, got {t.dtype}")
+    if not t.is_cuda:
+        raise ValueError(f"{name} must live on the GPU")
+    if t.dtype is not torch.float16:
+        raise ValueError(f"{name} must be float16, got {t.dtype}")
 
 
 FP8_DTYPES = (torch.uint8, torch.float8_e4m3fn)
 INT8_DTYPES = (torch.int8,)
+_Q8_DTYPES = FP8_DTYPES + INT8_DTYPES
 
 
 def _dev_pool(name: str, t: torch.Tensor) -> None:
-    _need(t.is_cuda, f"{name} must live on the GPU")
-    _need(t.dtype == torch.float16 or t.dtype in FP8_DTYPES + INT8_DTYPES,
-          f"{name} must be float16, fp8 or int8, got {t.dtype}")
+    if not t.is_cuda:
+        raise ValueError(f"{name} must live on the GPU")
+    if t.dtype is not torch.float16 and t.dtype not in _Q8_DTYPES:
+        raise ValueError(f"{name} must be float16, fp8 or int8, got {t.dtype}")
 
 
 def is_fp8_pool(kv_pool: torch.Tensor) -> bool:
@@ -59,7 +67,7 @@ def is_int8_pool(kv_pool: torch.Tensor) -> bool:
 
 def is_quantised_pool(kv_pool: torch.Tensor) -> bool:
     """A pool of 8-bit codes (fp8 or int8) with one fp32 scale per kv head: value = code * scale."""
-    return is_fp8_pool(kv_pool) or is_int8_pool(kv_pool)
+    return kv_pool.dtype in _Q8_DTYPES
 
 
 def _q8_entry(lib, stem: str, kv_pool: torch.Tensor):
@@ -68,33 +76,43 @@ def _q8_entry(lib, stem: str, kv_pool: torch.Tensor):
 
 
 def _dev_fp8_pool(kv_pool: torch.Tensor, scales: Optional[torch.Tensor], num_kv_heads: int) -> None:
-    _need(kv_pool.is_cuda and is_quantised_pool(kv_pool),
-          f"kv_pool must be an fp8 (uint8 / float8_e4m3fn) or int8 GPU tensor, got {kv_pool.dtype}")
-    _need(scales is not None, "a pool of 8-bit codes needs its per-head scales")
-    _need(scales.is_cuda and scales.dtype == torch.float32 and scales.is_contiguous()
-          and scales.numel() == 2 * num_kv_heads, "scales must be float32 [2 * Hkv] on the GPU (K heads, then V heads)")
+    if not (kv_pool.is_cuda and kv_pool.dtype in _Q8_DTYPES):
+        raise ValueError(f"kv_pool must be an fp8 (uint8 / float8_e4m3fn) or int8 GPU tensor, got {kv_pool.dtype}")
+    if scales is None:
+        raise ValueError("a pool of 8-bit codes needs its per-head scales")
+    if not (scales.is_cuda and scales.dtype is torch.float32 and scales.is_contiguous()
+            and scales.numel() == 2 * num_kv_heads):
+        raise ValueError("scales must be float32 [2 * Hkv] on the GPU (K heads, then V heads)")
 
 
 def _dev_i32(name: str, t: torch.Tensor) -> torch.Tensor:
-    _need(t.is_cuda, f"{name} must live on the GPU")
-    if t.dtype != torch.int32:
+    if not t.is_cuda:
+        raise ValueError(f"{name} must live on the GPU")
+    if t.dtype is not torch.int32:
         t = t.to(torch.int32)  # device-side cast, no host sync
-    return t.contiguous()
+    return t if t.is_contiguous() else t.contiguous()
 
 
 def _rows(name: str, t: torch.Tensor) -> int:
     """Token stride of a [T, H, D] tensor whose [H, D] block is contiguous."""
-    _need(t.dim() == 3, f"{name} must be [tokens, heads, head_dim]")
-    _need(t.stride(2) == 1 and t.stride(1) == t.shape[2], f"{name}: [heads, head_dim] block must be contiguous")
-    return t.stride(0) if t.shape[0] > 1 else max(t.stride(0), t.shape[1] * t.shape[2])
+    shape, stride = t.shape, t.stride()
+    if len(shape) != 3:
+        raise ValueError(f"{name} must be [tokens, heads, head_dim]")
+    if stride[2] != 1 or stride[1] != shape[2]:
+        raise ValueError(f"{name}: [heads, head_dim] block must be contiguous")
+    return stride[0] if shape[0] > 1 else max(stride[0], shape[1] * shape[2])
 
 
 def pool_geometry(kv_pool: torch.Tensor, page_size: int = PAGE_SIZE):
     """(num_slots, num_kv_heads, head_dim, num_pages, page_bytes) of a [slots, 2*Hkv, D] pool."""
-    _need(kv_pool.dim() == 3 and kv_pool.is_contiguous(), "kv_pool must be contiguous [slots, 2*Hkv, D]")
-    slots, two_h, d = kv_pool.shape
-    _need(two_h % 2 == 0, "kv_pool dim 1 must be 2 * num_kv_heads")
-    _need(slots % page_size == 0, "kv_pool slots must be a multiple of page_size")
+    shape = kv_pool.shape
+    if len(shape) != 3 or not kv_pool.is_contiguous():
+        raise ValueError("kv_pool must be contiguous [slots, 2*Hkv, D]")
+    slots, two_h, d = shape
+    if two_h % 2 != 0:
+        raise ValueError("kv_pool dim 1 must be 2 * num_kv_heads")
+    if slots % page_size != 0:
+        raise ValueError("kv_pool slots must be a multiple of page_size")
     return slots, two_h // 2, d, slots // page_size, page_size * two_h * d * kv_pool.element_size()
 
 
@@ -102,11 +120,14 @@ def kv_append(k: torch.Tensor, v: torch.Tensor, slot_mapping: torch.Tensor, kv_p
     """kv_pool[slot_mapping[t]] = concat(k[t], v[t]) for every token t (bit exact, in place)."""
     _dev_half("k", k), _dev_half("v", v), _dev_half("kv_pool", kv_pool)
     slots, hkv, d, _, _ = pool_geometry(kv_pool, 1)
-    _need(k.shape == v.shape, "k and v must have the same shape")
-    _need(k.shape[1] == hkv and k.shape[2] == d, f"k/v heads {tuple(k.shape[1:])} do not match pool ({hkv}, {d})")
+    if not (k.shape == v.shape):
+        raise ValueError("k and v must have the same shape")
+    if not (k.shape[1] == hkv and k.shape[2] == d):
+        raise ValueError(f"k/v heads {tuple(k.shape[1:])} do not match pool ({hkv}, {d})")
     slot_mapping = _dev_i32("slot_mapping", slot_mapping)
     t = k.shape[0]
-    _need(slot_mapping.numel() == t, "slot_mapping must hold one slot per token")
+    if not (slot_mapping.numel() == t):
+        raise ValueError("slot_mapping must hold one slot per token")
     lib = _lib.load()
     _lib.check(lib.litekv_kv_append(_ptr(k), _ptr(v), _rows("k", k), _rows("v", v), _ptr(slot_mapping),
                                     _ptr(kv_pool), t, hkv, d, slots, _stream()))
@@ -168,24 +189,32 @@ def qk_norm_rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, slot_
     else:
         _dev_half("kv_pool", kv_pool)
     t, hq = q.shape[0], q.shape[1]
-    _need(q.dim() == 3 and q.shape[2] == d, "q must be [T, Hq, D]")
-    _need(k.shape == (t, hkv, d) and v.shape == (t, hkv, d), "k / v must be [T, Hkv, D] matching the pool")
-    _need((q_norm_weight is None) == (k_norm_weight is None), "q_norm_weight and k_norm_weight go together")
-    _need((cos is None) == (sin is None), "cos and sin go together")
+    if not (q.dim() == 3 and q.shape[2] == d):
+        raise ValueError("q must be [T, Hq, D]")
+    if not (k.shape == (t, hkv, d) and v.shape == (t, hkv, d)):
+        raise ValueError("k / v must be [T, Hkv, D] matching the pool")
+    if not ((q_norm_weight is None) == (k_norm_weight is None)):
+        raise ValueError("q_norm_weight and k_norm_weight go together")
+    if not ((cos is None) == (sin is None)):
+        raise ValueError("cos and sin go together")
     if q_norm_weight is not None:
         _dev_half("q_norm_weight", q_norm_weight), _dev_half("k_norm_weight", k_norm_weight)
-        _need(q_norm_weight.numel() == d and k_norm_weight.numel() == d and q_norm_weight.is_contiguous()
-              and k_norm_weight.is_contiguous(), "norm weights must be contiguous [D]")
+        if not (q_norm_weight.numel() == d and k_norm_weight.numel() == d
+                and q_norm_weight.is_contiguous() and k_norm_weight.is_contiguous()):
+            raise ValueError("norm weights must be contiguous [D]")
     cs_stride = 0
     if cos is not None:
         _dev_half("cos", cos), _dev_half("sin", sin)
-        cos, sin = cos.reshape(-1, cos.shape[-1]), sin.reshape(-1, sin.shape[-1])
-        _need(cos.shape == sin.shape and cos.shape[0] == t and cos.shape[1] >= d // 2, "cos / sin must be [T, >= D/2]")
-        _need(cos.stride(1) == 1 and sin.stride(1) == 1 and cos.stride(0) == sin.stride(0),
-              "cos / sin rows must be contiguous with equal row strides")
+        if cos.dim() != 2 or sin.dim() != 2:
+            cos, sin = cos.reshape(-1, cos.shape[-1]), sin.reshape(-1, sin.shape[-1])
+        if not (cos.shape == sin.shape and cos.shape[0] == t and cos.shape[1] >= d // 2):
+            raise ValueError("cos / sin must be [T, >= D/2]")
+        if not (cos.stride(1) == 1 and sin.stride(1) == 1 and cos.stride(0) == sin.stride(0)):
+            raise ValueError("cos / sin rows must be contiguous with equal row strides")
         cs_stride = cos.stride(0)
     slot_mapping = _dev_i32("slot_mapping", slot_mapping)
-    _need(slot_mapping.numel() == t, "slot_mapping must hold one slot per token")
+    if not (slot_mapping.numel() == t):
+        raise ValueError("slot_mapping must hold one slot per token")
     lib = _lib.load()
     if fp8:
         _lib.check(_q8_entry(lib, "qk_norm_rope_append", kv_pool)(
@@ -492,7 +521,7 @@ def decode_advance(request_tables: torch.Tensor, request_ids: torch.Tensor, seq_
 
 def _segment(dst: torch.Tensor, src: torch.Tensor) -> Optional[tuple]:
     """(src, dst, rows, row bytes, src pitch, dst pitch) of a copy litekv_copy_segments can take, or None."""
-    if not (src.is_cuda and src.dtype == dst.dtype and src.shape == dst.shape and src.device == dst.device):
+    if not (src.is_cuda and src.dtype is dst.dtype and src.shape == dst.shape and src.get_device() == dst.get_device()):
         return None
     size = dst.element_size()
     if src.is_contiguous() and dst.is_contiguous():
@@ -546,17 +575,21 @@ def decode_step(q: torch.Tensor, kv_pool: torch.Tensor, plan: DecodePlan,
     fp8 = is_quantised_pool(kv_pool)
     if not fp8:
         _dev_half("kv_pool", kv_pool)
-    _need(q.dim() == 3 and q.stride(2) == 1 and q.stride(1) == q.shape[2], "q must be [B, Hq, D] with contiguous heads")
+    if not (q.dim() == 3 and q.stride(2) == 1 and q.stride(1) == q.shape[2]):
+        raise ValueError("q must be [B, Hq, D] with contiguous heads")
     b, hq, d = q.shape
     _, hkv, dk, n_pages, _ = pool_geometry(kv_pool, plan.page_size)
-    _need(d == dk, "q and kv_pool differ in head_dim")
-    _need((b, hq, hkv, n_pages) == (plan.batch, plan.num_q_heads, plan.num_kv_heads, plan.num_pages),
-          "plan was made for another batch / head / pool geometry")
-    _need((k_new is None) == (v_new is None), "k_new and v_new go together")
+    if not (d == dk):
+        raise ValueError("q and kv_pool differ in head_dim")
+    if not ((b, hq, hkv, n_pages) == (plan.batch, plan.num_q_heads, plan.num_kv_heads, plan.num_pages)):
+        raise ValueError("plan was made for another batch / head / pool geometry")
+    if not ((k_new is None) == (v_new is None)):
+        raise ValueError("k_new and v_new go together")
     kn_stride = vn_stride = 0
     if k_new is not None:
         _dev_half("k_new", k_new), _dev_half("v_new", v_new)
-        _need(k_new.shape == (b, hkv, d) and v_new.shape == (b, hkv, d), "k_new / v_new must be [B, Hkv, D]")
+        if not (k_new.shape == (b, hkv, d) and v_new.shape == (b, hkv, d)):
+            raise ValueError("k_new / v_new must be [B, Hkv, D]")
         kn_stride, vn_stride = _rows("k_new", k_new), _rows("v_new", v_new)
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(d)
@@ -564,7 +597,8 @@ def decode_step(q: torch.Tensor, kv_pool: torch.Tensor, plan: DecodePlan,
         out = torch.empty((b, hq, d), dtype=torch.float16, device=q.device)
     else:
         _dev_half("out", out)
-        _need(out.shape == (b, hq, d) and out.is_contiguous(), "out must be contiguous [B, Hq, D]")
+        if not (out.shape == (b, hq, d) and out.is_contiguous()):
+            raise ValueError("out must be contiguous [B, Hq, D]")
     q_stride = q.stride(0) if b > 1 else max(q.stride(0), hq * d)
     lib = _lib.load()
     if fp8:
@@ -624,20 +658,27 @@ def paged_decode(q: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Tens
     _dev_half("q", q)
     if not is_quantised_pool(kv_pool):
         _dev_half("kv_pool", kv_pool)
-    _need(q.dim() == 3 and q.stride(2) == 1 and q.stride(1) == q.shape[2], "q must be [B, Hq, D] with contiguous heads")
+    if not (q.dim() == 3 and q.stride(2) == 1 and q.stride(1) == q.shape[2]):
+        raise ValueError("q must be [B, Hq, D] with contiguous heads")
     b, hq, d = q.shape
     _, hkv, dk, n_pages, _ = pool_geometry(kv_pool, page_size)
-    _need(d == dk, "q and kv_pool differ in head_dim")
-    _need(stage in _STAGES, f"unknown stage {stage!r}")
+    if not (d == dk):
+        raise ValueError("q and kv_pool differ in head_dim")
+    if not (stage in _STAGES):
+        raise ValueError(f"unknown stage {stage!r}")
     if schedule is None:
         split_args = (num_splits, max_splits, min_pages_per_split)
         schedule = "splits" if any(x is not None for x in split_args) or stage != "both" else "balanced"
-    _need(schedule in ("balanced", "splits"), f"unknown schedule {schedule!r}")
+    if not (schedule in ("balanced", "splits")):
+        raise ValueError(f"unknown schedule {schedule!r}")
 
-    _need((k_new is None) == (v_new is None), "k_new and v_new go together")
+    if not ((k_new is None) == (v_new is None)):
+        raise ValueError("k_new and v_new go together")
     if schedule == "balanced":
-        _need(stage == "both", "the balanced schedule is a single launch")
-        _need(k_new is None, "the balanced schedule appends through decode_step")
+        if not (stage == "both"):
+            raise ValueError("the balanced schedule is a single launch")
+        if not (k_new is None):
+            raise ValueError("the balanced schedule appends through decode_step")
         if plan is None:
             plan = DecodePlan(block_table, seq_lens, hq, hkv, n_pages, chunks, page_size, shared_pages,
                               kv_dtype=kv_pool.dtype)
@@ -646,18 +687,22 @@ def paged_decode(q: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Tens
     fp8 = is_quantised_pool(kv_pool)
     if fp8:
         _dev_fp8_pool(kv_pool, kv_scales, hkv)
-        _need(stage == "both", "an fp8 pool is read by both stages in one call")
-    _need(block_table.dim() == 2 and block_table.shape[0] == b, "block_table must be [B, max_blocks]")
+        if not (stage == "both"):
+            raise ValueError("an fp8 pool is read by both stages in one call")
+    if not (block_table.dim() == 2 and block_table.shape[0] == b):
+        raise ValueError("block_table must be [B, max_blocks]")
     block_table = _dev_i32("block_table", block_table)
     seq_lens = _dev_i32("seq_lens", seq_lens)
-    _need(seq_lens.numel() == b, "seq_lens must be [B]")
+    if not (seq_lens.numel() == b):
+        raise ValueError("seq_lens must be [B]")
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(d)
     if out is None:
         out = torch.empty((b, hq, d), dtype=torch.float16, device=q.device)
     else:
         _dev_half("out", out)
-        _need(out.shape == (b, hq, d) and out.is_contiguous(), "out must be contiguous [B, Hq, D]")
+        if not (out.shape == (b, hq, d) and out.is_contiguous()):
+            raise ValueError("out must be contiguous [B, Hq, D]")
     lib = _lib.load()
     q_stride = q.stride(0) if b > 1 else max(q.stride(0), hq * d)
     if max_splits is None or min_pages_per_split is None:
@@ -668,9 +713,11 @@ def paged_decode(q: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Tens
         workspace = decode_workspace(b, hq, max_splits, q.device)
     ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     if k_new is not None:
-        _need(stage == "both", "the fused append belongs to the call that runs both stages")
+        if not (stage == "both"):
+            raise ValueError("the fused append belongs to the call that runs both stages")
         _dev_half("k_new", k_new), _dev_half("v_new", v_new)
-        _need(k_new.shape == (b, hkv, d) and v_new.shape == (b, hkv, d), "k_new / v_new must be [B, Hkv, D]")
+        if not (k_new.shape == (b, hkv, d) and v_new.shape == (b, hkv, d)):
+            raise ValueError("k_new / v_new must be [B, Hkv, D]")
         rows = (_ptr(k_new), _ptr(v_new), _rows("k_new", k_new), _rows("v_new", v_new))
         tail = (_ptr(out), _ptr(workspace), ws_bytes, b, hq, hkv, d, page_size, n_pages, max_splits,
                 min_pages_per_split, float(softmax_scale), _stream())
@@ -746,20 +793,24 @@ def paged_prefill(q: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Ten
     fp8 = is_quantised_pool(kv_pool)
     if not fp8:
         _dev_half("kv_pool", kv_pool)
-        _need(kv_scales is None, "kv_scales belong to an fp8 pool")
+        if not (kv_scales is None):
+            raise ValueError("kv_scales belong to an fp8 pool")
     q_stride = _rows("q", q)
     t, hq, d = q.shape
     _, hkv, dk, n_pages, _ = pool_geometry(kv_pool, page_size)
     if fp8:
         _dev_fp8_pool(kv_pool, kv_scales, hkv)
-    _need(d == dk, "q and kv_pool differ in head_dim")
+    if not (d == dk):
+        raise ValueError("q and kv_pool differ in head_dim")
     cu_q_lens = _dev_i32("cu_q_lens", cu_q_lens)
     b = cu_q_lens.numel() - 1
-    _need(block_table.dim() == 2 and block_table.shape[0] == b, "block_table must be [B, max_blocks]")
+    if not (block_table.dim() == 2 and block_table.shape[0] == b):
+        raise ValueError("block_table must be [B, max_blocks]")
     block_table = _dev_i32("block_table", block_table)
     if context_lens is not None:
         context_lens = _dev_i32("context_lens", context_lens)
-        _need(context_lens.numel() == b, "context_lens must be [B]")
+        if not (context_lens.numel() == b):
+            raise ValueError("context_lens must be [B]")
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(d)
     if out is None:
@@ -776,8 +827,9 @@ def paged_prefill(q: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Ten
         need = paged_prefill_workspace_floats(t, hq, d, key_slices)
         if workspace is None:
             workspace = torch.empty(need, dtype=torch.float32, device=q.device)
-        _need(workspace.is_cuda and workspace.dtype == torch.float32 and workspace.is_contiguous() and
-              workspace.numel() >= need, f"workspace must be {need} contiguous float32 on the device")
+        if not (workspace.is_cuda and workspace.dtype == torch.float32
+                and workspace.is_contiguous() and workspace.numel() >= need):
+            raise ValueError(f"workspace must be {need} contiguous float32 on the device")
     if fp8:
         if key_slices > 1:
             _lib.check(lib.litekv_paged_prefill_split_q8(
@@ -819,12 +871,14 @@ def varlen_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, seq_starts
     _dev_half("q", q), _dev_half("k", k), _dev_half("v", v)
     q_stride, k_stride, v_stride = _rows("q", q), _rows("k", k), _rows("v", v)
     t, hq, d = q.shape
-    _need(k.shape == v.shape and k.shape[0] == t and k.shape[2] == d, "k/v shape mismatch")
+    if not (k.shape == v.shape and k.shape[0] == t and k.shape[2] == d):
+        raise ValueError("k/v shape mismatch")
     hkv = k.shape[1]
     seq_starts = _dev_i32("seq_starts", seq_starts)
     seq_lens = _dev_i32("seq_lens", seq_lens)
     b = seq_lens.numel()
-    _need(seq_starts.numel() == b, "seq_starts and seq_lens differ in length")
+    if not (seq_starts.numel() == b):
+        raise ValueError("seq_starts and seq_lens differ in length")
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(d)
     if out is None:
