@@ -508,16 +508,25 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
     half_t *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_lse,
     int32_t num_q_heads, int32_t num_kv_heads, int32_t group_all, int32_t slices, int32_t max_splits,
     int32_t min_pages_per_split, int32_t num_pages, int32_t page_shift, float scale_log2) {
+  // All arguments in one go: left alone the compiler reads them block by block, each group a
+  // scalar round trip of its own in front of the requests that need it.
+  const int wg_waves = blockDim.x >> 6;
+  asm volatile("" ::"s"(q), "s"(q_batch_stride), "s"(kv), "s"(scales), "s"(block_table), "s"(bt_stride),
+               "s"(seq_lens), "s"(k_new), "s"(v_new), "s"(k_new_stride), "s"(v_new_stride), "s"(out),
+               "s"(part_o), "s"(part_lse), "s"(num_q_heads), "s"(num_kv_heads), "s"(group_all), "s"(slices),
+               "s"(max_splits), "s"(min_pages_per_split), "s"(num_pages), "s"(page_shift), "s"(scale_log2),
+               "s"(wg_waves));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int n = lane & 15;   // query head inside the slice (column of S^T)
   const int g = lane >> 4;   // lane group: owns tokens 4g..4g+3 of a page
   // a kv head with more than 16 query heads is served in slices of up to 16 (see head_slice)
-  const HeadSlice hs = head_slice(blockIdx.x * (blockDim.x >> 6) + wave, slices, group_all);
+  const HeadSlice hs = head_slice(blockIdx.x * wg_waves + wave, slices, group_all);
   const int h = hs.kv_head;
   const int group = hs.q_heads;
   const int split = blockIdx.y;
   half_t *vstage = split_vstage + wave * (kPageSize * kVPitch);
+  const int hq0 = hs.q_head0;
   int b = blockIdx.z, len;
   if constexpr (ORDERED) {
     const int64_t capacity = (int64_t)bt_stride << (page_shift + 4);
@@ -527,10 +536,49 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
     len = __builtin_amdgcn_readfirstlane(len);
     // a length beyond the row keeps its own value for the masks below
     if (len >= capacity) len = seq_lens[b];
-  } else {
-    len = seq_lens[b];
   }
-  const int hq0 = hs.q_head0;
+  // 64 entries of the sequence's block-table row, one per lane (entries win0 + lane), read back
+  // with v_readlane: a page id costs no load in the page loop, whose LDS waits would also wait for
+  // a scalar one. The first 64 are requested here, next to the length and q and before anything
+  // waits: where they are the whole row (a thousand tokens in pages of 16), the first page is one
+  // round trip to memory earlier than with ids read once the length has said which. Together
+  // with the merge's requests (paged_decode_merge_kernel) and the arguments read in one go, per
+  // layer: one sequence of 778 tokens, 16/8 heads, 16 splits 10.0 -> 9.6 us; twelve of 100 to 3000
+  // tokens, 32/8 heads of 64 17.9 -> 17.4 us.
+  const int32_t *table = block_table + (int64_t)b * bt_stride;
+  int win0 = 0;
+  int ids = table[lane < bt_stride ? lane : bt_stride - 1];
+  constexpr bool FP8 = KV != kKvF16;  // 8-bit codes (either format): the layout they share
+  typedef typename KvStore<KV>::elem Elem;
+  typedef typename KvStore<KV>::page Page;
+  half8_t qf[4];
+  {
+    // Every lane loads, lanes past the group the group's last head: their columns are computed and
+    // never stored. (A load under a lane condition would end the straight run of requests.)
+    const half_t *row = q + (int64_t)b * q_batch_stride + (int64_t)(hq0 + (n < group ? n : group - 1)) * kHD +
+                        (FP8 ? 16 : 8) * g;
+#pragma unroll
+    for (int kk = 0; kk < kKSteps; ++kk) {  // the d order of load_q / load_q_fp8_order
+      qf[kk] = *(const half8_t *)(row + (FP8 ? 64 * (kk >> 1) + 8 * (kk & 1) : 32 * kk));
+    }
+  }
+  // Fused append: the wavefront that attends the sequence's last page writes the step's token
+  // into it.
+  uint4_t k_row[4] = {}, v_row[2] = {};
+  if constexpr (APPEND) {
+    load_new_rows<FP8>(k_row, v_row, k_new + (int64_t)b * k_new_stride + (int64_t)h * kHD,
+                       v_new + (int64_t)b * v_new_stride + (int64_t)h * kHD, n, g);
+  }
+  float v_scale = 1.0f, k_inv = 1.0f, v_inv = 1.0f;
+  if constexpr (FP8) {  // the K scale joins the softmax scale, the V scale the normalisation
+    const float ks = scales[h];
+    scale_log2 *= ks;
+    v_scale = scales[num_kv_heads + h];
+    k_inv = 1.0f / ks;  // the step's new rows are quantised with the reciprocals
+    v_inv = 1.0f / v_scale;
+  }
+  asm volatile("" ::: "memory");  // the requests above stay above
+  if constexpr (!ORDERED) len = as_uniform(seq_lens)[b];
   half_t *out_row = out + ((int64_t)b * num_q_heads + hq0) * kHD;
   if (len <= 0) {
     if (split == 0 && n < group) {
@@ -546,28 +594,6 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
   const int p0 = (int)(((int64_t)split * pages) / n_splits);
   const int p1 = (int)(((int64_t)(split + 1) * pages) / n_splits);
 
-  constexpr bool FP8 = KV != kKvF16;  // 8-bit codes (either format): the layout they share
-  typedef typename KvStore<KV>::elem Elem;
-  typedef typename KvStore<KV>::page Page;
-  half8_t qf[4];
-  float v_scale = 1.0f, k_inv = 1.0f, v_inv = 1.0f;
-  if constexpr (FP8) {  // the K scale joins the softmax scale, the V scale the normalisation
-    load_q_fp8_order(qf, q + (int64_t)b * q_batch_stride + (int64_t)hq0 * kHD, n, g, group);
-    const float ks = scales[h];
-    scale_log2 *= ks;
-    v_scale = scales[num_kv_heads + h];
-    k_inv = 1.0f / ks;  // the step's new rows are quantised with the reciprocals
-    v_inv = 1.0f / v_scale;
-  } else {
-    load_q(qf, q + (int64_t)b * q_batch_stride + (int64_t)hq0 * kHD, n, g, group);
-  }
-  // Fused append: the wavefront that attends the sequence's last page writes the step's token
-  // into it. Its rows are requested here, before the pages.
-  uint4_t k_row[4] = {}, v_row[2] = {};
-  if constexpr (APPEND) {
-    load_new_rows<FP8>(k_row, v_row, k_new + (int64_t)b * k_new_stride + (int64_t)h * kHD,
-                       v_new + (int64_t)b * v_new_stride + (int64_t)h * kHD, n, g);
-  }
 
   const int64_t row_stride = (int64_t)2 * num_kv_heads * kHD;  // elements per slot
   // this lane's row and column inside page 0 (see PageRegs / PageRegsFp8)
@@ -576,24 +602,29 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
                            q8_v_row(n, g) * row_stride
                      : kv + (int64_t)(num_kv_heads + h) * kHD + 8 * (n & (kVCols - 1)) + g * row_stride;
   const half_t *vt_lane = &vstage[(4 * g + (n >> 2)) * kVPitch + 4 * (n & 3)];
-  const int32_t *table = block_table + (int64_t)b * bt_stride;
 
   HeadState st;
   st.reset();
   Page buf[DEPTH];
 
-  // Page ids are wavefront-uniform: they travel through scalar loads one step ahead of their
-  // use. Requests past the range still issue their loads (16 bytes of its last page), which keeps
+  // Requests past the range still issue their loads (16 bytes of its last page), which keeps
   // the number of vector loads in flight a compile-time constant, so each wait names exactly the
   // page it needs and never drains the younger prefetches.
   // A length beyond what a block-table row can name (the host cannot check lengths that live on
   // the device) re-reads the row's last entry instead of reading past it, and appends nothing.
   const bool fits_table = pages <= (bt_stride << page_shift);
+  // Ids are asked for in rising order, and past the range the last one's again, so the window only
+  // moves forward. (Its load is waited for inside the branch: see wait_vector_loads.)
   auto page_id = [&](int p) {
     const int pp = p < p1 ? p : p1 - 1;
     int at = pp >> page_shift;
     at = at < bt_stride ? at : bt_stride - 1;
-    return sub_page_id(table[at], pp, page_shift, num_pages);
+    if (at - win0 >= kWave) {
+      win0 = at;
+      ids = table[at + lane < bt_stride ? at + lane : bt_stride - 1];
+      wait_vector_loads();
+    }
+    return sub_page_id(__builtin_amdgcn_readlane(ids, at - win0), pp, page_shift, num_pages);
   };
   int pid_next = page_id(p0);
   auto request = [&](int p, Page &r) {
@@ -670,6 +701,32 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
               part_lse + cell, max_splits, n, g, group, v_scale);
 }
 
+// Folds up to kFewPieces partial rows of one query head whose elements 2 * lane, 2 * lane + 1 are
+// in r and whose log-sum-exps are in the lanes (lane s that of partial s, -inf past the last).
+constexpr int kFewPieces = 16;
+__device__ __forceinline__ void fold_few(const float2 (&r)[kFewPieces], float l, int n_parts,
+                                         half_t *out_row, int lane) {
+  float mx = l;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, xor_lane(mx, off));
+  const float w = fast_exp2((l - mx) * kLog2e);
+  float den = w;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) den += xor_lane(den, off);
+  float num0 = 0.f, num1 = 0.f;
+#pragma unroll
+  for (int s = 0; s < kFewPieces; ++s) {
+    if (s < n_parts) {
+      const float ws = __shfl(w, s, kWave);
+      num0 += ws * r[s].x;
+      num1 += ws * r[s].y;
+    }
+  }
+  const float inv = 1.0f / den;
+  typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+  if (2 * lane < kHD) *(half2_t *)(out_row + 2 * lane) = half2_t{(half_t)(num0 * inv), (half_t)(num1 * inv)};
+}
+
 // Merges partial rows of one query head into its final fp16 row; run by one whole wavefront.
 // The partials come in two runs: n1 of them at lse1[s * lse1_stride], po1[s * po1_stride .. +D),
 // then n2 more at lse2 / po2 (n2 may be 0). Lane s holds the weight of partial s (blocks of 64
@@ -694,37 +751,18 @@ __device__ __forceinline__ void merge_row(const float *__restrict__ lse1, int64_
     if (!TWO_RUNS || s < n1) return po1 + (int64_t)s * po1_stride;
     return po2 + (int64_t)(s - n1) * po2_stride;
   };
-  if (n_parts <= 16) {
+  if (n_parts <= kFewPieces) {
     // The usual case (a sequence spans a few chunks, with or without the slices of a shared
     // prefix): every row and the log-sum-exps are requested at once, so the launch waits for one
     // round trip to memory instead of one per group of rows. Same weights and the same order of
     // additions as the general path below.
-    float2 r[16];
+    float2 r[kFewPieces];
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
+    for (int s = 0; s < kFewPieces; ++s) {
       r[s] = float2{0.f, 0.f};
       if (s < n_parts) r[s] = *(const float2 *)(row_of(s) + mcol);
     }
-    const float l = lane < n_parts ? lse_of(lane) : -INFINITY;
-    float mx = l;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, xor_lane(mx, off));
-    const float w = fast_exp2((l - mx) * kLog2e);
-    float den = w;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) den += xor_lane(den, off);
-    float num0 = 0.f, num1 = 0.f;
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      if (s < n_parts) {
-        const float ws = __shfl(w, s, kWave);
-        num0 += ws * r[s].x;
-        num1 += ws * r[s].y;
-      }
-    }
-    const float inv = 1.0f / den;
-    typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-    if (live_col) *(half2_t *)(out_row + mcol) = half2_t{(half_t)(num0 * inv), (half_t)(num1 * inv)};
+    fold_few(r, lane < n_parts ? lse_of(lane) : -INFINITY, n_parts, out_row, lane);
     return;
   }
   float mx = -INFINITY;
@@ -773,11 +811,30 @@ __global__ __launch_bounds__(kWave) void paged_decode_merge_kernel(
     int32_t max_splits, int32_t min_pages_per_split) {
   const int hq = blockIdx.x;
   const int b = blockIdx.y;
+  const int64_t cell0 = ((int64_t)b * num_q_heads + hq) * max_splits;
+  if (max_splits <= kFewPieces) {
+    // Every partial row the head could have is requested together with the length that says how
+    // many it has, one round trip to memory instead of two; those past the last are not added.
+    const int lane = threadIdx.x;
+    const float *row0 = part_o + cell0 * kHD + (2 * lane < kHD ? 2 * lane : 0);
+    float2 r[kFewPieces];
+#pragma unroll
+    for (int s = 0; s < kFewPieces; ++s) {
+      r[s] = float2{0.f, 0.f};
+      if (s < max_splits) r[s] = *(const float2 *)(row0 + (int64_t)s * kHD);
+    }
+    const float l = part_lse[cell0 + (lane < max_splits ? lane : 0)];
+    asm volatile("" ::: "memory");  // the requests above stay above
+    const int n = as_uniform(seq_lens)[b];
+    const int n_splits = splits_for_pages(pages_of(n), max_splits, min_pages_per_split);
+    if (n <= 0 || n_splits == 1) return;  // the split kernel already wrote the final row
+    fold_few(r, lane < n_splits ? l : -INFINITY, n_splits, out + ((int64_t)b * num_q_heads + hq) * kHD, lane);
+    return;
+  }
   const int len = seq_lens[b];
   if (len <= 0) return;
   const int n_splits = splits_for_pages(pages_of(len), max_splits, min_pages_per_split);
   if (n_splits == 1) return;  // the split kernel already wrote the final row
-  const int64_t cell0 = ((int64_t)b * num_q_heads + hq) * max_splits;
   merge_row<false>(part_lse + cell0, 1, part_o + cell0 * kHD, kHD, n_splits, nullptr, 0,
                    nullptr, 0, 0, out + ((int64_t)b * num_q_heads + hq) * kHD, threadIdx.x);
 }

@@ -1,0 +1,36 @@
+"""GPU: the splits schedule reads a block-table row through a window of 64 entries per wavefront and
+its merge requests every partial row a head could have. Rows of just under, exactly and just over
+one and two windows, in one to sixteen splits, beside sequences of one page and of none, against the
+oracle; unwritten partial rows hold NaN."""
+
+import pytest
+import torch
+
+from llama_lite_npu_amd import ops, workloads
+from oracle import c_oracle
+from tests.parity import assert_attention_close, to_np16
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("splits", [1, 2, 4, 16])
+@pytest.mark.parametrize("pages", [3, 63, 64, 65, 127, 129, 193])
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (40, 8)])
+def test_rows_around_the_window(hq, hkv, pages, splits):
+    lens = [16 * pages - 3, 0, 5, 16 * (pages - 2), 16 * pages - 1]   # tokens before the step's own
+    print(f"row window: heads {hq}/{hkv} pages {pages} splits {splits}", flush=True)
+    case = workloads.make_decode_case("window", 77, lens, hq, hkv, device=DEV)
+    plan = ops.DecodePlan(case.block_table, case.seq_lens, hq, hkv, case.num_pages)
+    plan.set_schedule(splits)
+    if plan.split_workspace is not None:
+        plan.split_workspace.fill_(float("nan"))
+    pool = case.kv_pool.clone()
+    out = ops.decode_step(case.q, pool, plan, case.k_new, case.v_new, case.softmax_scale)
+    want = case.kv_pool.clone()
+    ops.kv_append(case.k_new, case.v_new, case.slot_mapping, want)
+    torch.cuda.synchronize()
+    assert torch.equal(pool.view(torch.int16), want.view(torch.int16))
+    ref = c_oracle.paged_decode(to_np16(case.q), to_np16(pool), case.block_table.cpu().numpy(),
+                                case.seq_lens.cpu().numpy(), case.softmax_scale)
+    assert_attention_close(out, ref, f"pages {pages} splits {splits}")
