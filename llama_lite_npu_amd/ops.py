@@ -301,11 +301,14 @@ SPLIT_COUNTS = (4, 8, 16)
 
 
 def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, total_pages: int, token_bytes: int,
-                              page_size: int = PAGE_SIZE, heads_per_kv_head: int = 8) -> dict:
+                              page_size: int = PAGE_SIZE, heads_per_kv_head: int = 8,
+                              head_dim: int = HEAD_DIM) -> dict:
     """Estimated microseconds per layer of every decode schedule a step could take, keyed as
     ``decode_schedule`` returns them. Fits to 554 measured shapes on an MI355X (1 to 2048 sequences
     of 32 to 16384 tokens: equal, ragged, one long among short; 64/8 and 16/8 heads; every
-    schedule replayed from a graph; ``tune_decode_schedule`` re-measures the table):
+    schedule replayed from a graph; ``tune_decode_schedule`` re-measures the table) and to 425 more
+    for what depends on the pool's format, the head dim and the number of kv heads (1 to 128
+    sequences of up to 32768 tokens; 64/8, 16/8 and 32/4 heads of 128, 32/8 of 64; fp16, fp8, int8):
 
     * 1, one wavefront per (sequence, kv head), one launch: 4.3 us + the largest (a 3.6-norm) of the
       longest sequence's dependent chain of 16-token steps at 0.58 us each -- up to half as much
@@ -313,14 +316,18 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
       memory paths with the chain's --, the placement of the launch's wavefronts at 2.9 ns each,
       and the bytes at 5.7 MB/us (unbalanced streams).
     * 4 / 8 / 16 splits per sequence + the merge launch, for launches of at most 2048 wavefronts:
-      6.8 us for the two launches, the chain of a split against the bytes at 6.1 MB/us (a 3.1-norm),
+      6.5 us for the two launches, the chain of a split against the bytes at 6.1 MB/us (a 3.1-norm),
       1.3 ns per wavefront; where the bytes dominate, uneven sequences make uneven splits, which
       the balanced cut does not have: up to 15 % more with the bytes' share.
     * 0, balanced (fused step + merge): 7.6 us, 0.17 us per piece the merge folds for the longest
-      sequence (up to 36; 0.06 us where a step of few rows shares a long row out among several
-      workgroups), 3.4 ns + 0.26 ns per query head for every sequence, and the bytes at
-      6.8 MB/us against the chain inside one of the 256 chunks; a tenth more with over 8 query
-      heads per kv head (two column tiles, twice the rows to merge)."""
+      sequence (up to 36; 0.06 to 0.15 us where a step of few rows shares a long row out among
+      several workgroups, by how many rows those are; half as much with rows of 64), 3.4 ns +
+      0.26 ns per query head for every sequence, and the bytes at 6.8 MB/us against the chain
+      inside one chunk -- 256 chunks for 8 kv heads, 512 for 4, whose workgroups hold two --; a
+      tenth more with over 8 query heads per kv head (two column tiles, twice the rows to merge).
+
+    A step over a page of codes takes 1.1 to 1.3 times as long as over fp16 rows (the conversion),
+    over rows of 64 elements 0.8 to 0.9 times."""
     steps = max(1, page_size // PAGE_SIZE)                 # the kernels step by 16 tokens
     chain = max_pages * steps
     total = total_pages * steps
@@ -329,39 +336,49 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
     slices = (heads_per_kv_head + 15) // 16                # wavefronts per kv head
     norm = lambda p, *xs: sum(x ** p for x in xs) ** (1.0 / p)
     lone = batch * num_kv_heads * slices                   # wavefronts of a launch with one per sequence
-    pieces = chain / max(1.0, total / 256.0)
+    heads = num_kv_heads * slices
+    groups = (heads + 7) // 8                              # workgroups of up to 8 wavefronts per chunk
+    chunks = (256 + groups - 1) // groups * max(1, 8 // heads)
+    narrow = head_dim < HEAD_DIM
+    codes = token_bytes < 4 * num_kv_heads * head_dim      # a pool of 8-bit codes
+    pieces = chain / max(1.0, total / chunks)
     # rows of more than 16 pieces are merged by several workgroups each while the step has few rows
-    per_piece = 0.057 if pieces > 16 and batch * num_q_heads <= 256 else 0.170
+    rows = batch * num_q_heads * head_dim / (256.0 * HEAD_DIM)
+    per_piece = 0.055 + 0.09 * rows if pieces > 16 and rows <= 1.0 else 0.170
+    per_piece *= 0.57 if narrow else 1.0
+    step = (0.87 if narrow else 1.0) * (1.12 if codes else 1.0)
     estimates = {
         0: (7.6 + per_piece * min(pieces, 36.0) + (3.4e-3 + 2.6e-4 * num_q_heads) * batch
-            + norm(2.0, nbytes / 6.81e6, 0.82 * ((total + 255) // 256))) * (1.1 if heads_per_kv_head > 8 else 1.0),
-        1: 4.27 + norm(3.6, 0.584 * chain * (1.0 + 0.49 * min(1.0, lone / 2048.0)), 2.9e-3 * lone, nbytes / 5.70e6),
+            + norm(2.0, nbytes / 6.81e6, 0.82 * step * -(-total // chunks))) * (1.1 if heads_per_kv_head > 8 else 1.0),
     }
+    step = (0.81 if narrow else 1.0) * (1.16 if codes else 1.0)
+    estimates[1] = 4.27 + norm(3.6, 0.584 * step * chain * (1.0 + 0.49 * min(1.0, lone / 2048.0)), 2.9e-3 * lone,
+                               nbytes / 5.70e6)
+    step = (0.82 if narrow else 1.0) * (1.27 if codes else 1.0)
     for n in SPLIT_COUNTS:
         wavefronts = batch * n * num_kv_heads * slices
         if wavefronts > 2048:
             continue
-        split_chain = 0.634 * ((chain + n - 1) // n)
+        split_chain = 0.634 * step * ((chain + n - 1) // n)
         stream = nbytes / 6.06e6
-        estimates[n] = ((6.76 + norm(3.1, split_chain, stream) + 1.3e-3 * wavefronts)
+        estimates[n] = ((6.5 + norm(3.1, split_chain, stream) + 1.3e-3 * wavefronts)
                         * (1.0 + 0.15 * stream / (split_chain + stream)))
     return estimates
 
 
 def decode_schedule(batch: int, num_kv_heads: int, max_pages: int, total_pages: int, token_bytes: int,
                     page_size: int = PAGE_SIZE, heads_per_kv_head: int = 8, current: Optional[int] = None,
-                    hysteresis: float = 1.0) -> int:
+                    hysteresis: float = 1.0, head_dim: int = HEAD_DIM) -> int:
     """Which decode schedule a step should take, from what the host knows about it: 0 = balanced,
     1 = one wavefront per (sequence, kv head) in one launch, 4 / 8 / 16 = that many splits per
     sequence and the merge launch: the smallest of ``decode_schedule_estimates``. Choosing by this
-    rule is 1.1 % slower on average than always choosing the fastest schedule on the measured
-    shapes (30 % at worst; 1.3 to 1.7 % and 27 to 32 % on three head layouts the constants were not
-    fitted on); always balanced is 19 % slower on average. ``current``: the schedule
+    rule is 1.0 % slower on average than always choosing the fastest schedule on the measured
+    shapes (33 % at worst: 4 sequences of 80 tokens, 8.4 against 6.4 us). ``current``: the schedule
     in use; another must be estimated ``hysteresis`` times faster to replace it."""
     if batch <= 0 or total_pages <= 0 or max_pages <= 0:
         return 0
     estimates = decode_schedule_estimates(batch, num_kv_heads, max_pages, total_pages, token_bytes, page_size,
-                                          heads_per_kv_head)
+                                          heads_per_kv_head, head_dim)
     if current in estimates:
         estimates[current] /= hysteresis
     return min(estimates, key=estimates.get)
@@ -388,7 +405,8 @@ class DecodePlan:
         ``host_seq_lens``: the lengths as the host knows them; with them the plan picks the
         per-sequence schedule (and its split count) where ``decode_schedule`` says so. ``token_bytes``:
         K + V bytes of one token in the pool (default: fp16). ``kv_dtype``: the pool's element type
-        (default fp16); with a shared prefix it decides how the default chunk count is chosen."""
+        (default fp16); with a shared prefix it decides how the default chunk count is chosen, and
+        with ``token_bytes`` it tells the width of the heads, which the schedule depends on."""
         lib = _lib.load()
         self.shared_pages = int(shared_pages)
         self.kv_dtype = kv_dtype
@@ -396,6 +414,9 @@ class DecodePlan:
         self.splits = 1
         self.split_workspace: Optional[torch.Tensor] = None
         self.token_bytes = int(token_bytes) if token_bytes is not None else 2 * int(num_kv_heads) * HEAD_DIM * 2
+        # what the schedule is chosen by: rows of 64 where bytes and element type say so, else of 128
+        self.head_dim = 64 if kv_dtype is not None and self.token_bytes == 2 * num_kv_heads * 64 * kv_dtype.itemsize \
+            else HEAD_DIM
         _need(0 <= self.shared_pages <= block_table.shape[1], "shared_pages out of range")
         _need(block_table.dim() == 2, "block_table must be [B, max_blocks]")
         self.block_table = _dev_i32("block_table", block_table)
@@ -453,9 +474,10 @@ class DecodePlan:
         if not pages:
             self.set_schedule(0)
             return False
+        narrow = {} if self.head_dim == HEAD_DIM else {"head_dim": self.head_dim}
         self.set_schedule(decode_schedule(self.batch, self.num_kv_heads, max(pages), sum(pages), self.token_bytes,
                                           self.page_size, self.num_q_heads // self.num_kv_heads,
-                                          current=self.schedule, hysteresis=hysteresis))
+                                          current=self.schedule, hysteresis=hysteresis, **narrow))
         return self.per_sequence
 
     def refresh(self, block_table: Optional[torch.Tensor] = None, seq_lens: Optional[torch.Tensor] = None) -> None:

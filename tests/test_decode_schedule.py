@@ -2,6 +2,8 @@
 measurements behind its constants showed, at the sizes the benchmark configurations name.
 0 = balanced, 1 = one wavefront per (sequence, kv head), 4 / 8 / 16 = splits per sequence + merge."""
 
+import pytest
+
 from llama_lite_npu_amd.ops import SPLIT_COUNTS, decode_schedule, decode_schedule_estimates
 
 TOK = 4096  # K + V bytes of a token: 8 kv heads, fp16
@@ -108,3 +110,17 @@ def test_page_size_does_not_change_the_choice_for_the_same_tokens():
         picks = {decode_schedule(batch, 8, tokens // ps, batch * tokens // ps, TOK, page_size=ps)
                  for ps in (16, 64, 256)}
         assert len(picks) == 1, (batch, tokens, picks)
+
+
+@pytest.mark.parametrize("batch,hkv,group,head_dim,code_bytes,longest,mean,want", [
+    (128, 4, 8, 128, 1, 32464, 19636, 0),    # int8, 428 us per layer against 571 in 4 splits
+    (42, 4, 8, 128, 1, 23920, 16034, 0),     # int8, 126 against 198 in 8 splits
+    (12, 8, 4, 64, 2, 2909, 1573, 0),        # rows of 64: 16 us against 18 in 16 splits
+    (12, 8, 2, 128, 2, 512, 484, 8),         # 11.6 us against 14.8 balanced
+    (1, 8, 2, 128, 2, 779, 779, 16),
+])
+def test_the_choice_knows_the_pool_format_the_head_dim_and_the_kv_heads(batch, hkv, group, head_dim, code_bytes,
+                                                                        longest, mean, want):
+    pick = decode_schedule(batch, hkv, pages(longest), batch * pages(mean), 2 * hkv * head_dim * code_bytes,
+                           heads_per_kv_head=group, head_dim=head_dim)
+    assert pick in ((8, 16) if want in (8, 16) else (want,))
