@@ -561,6 +561,10 @@ def _segment(dst: torch.Tensor, src: torch.Tensor) -> Optional[tuple]:
     return entry if aligned and rows * row_bytes <= 1 << 30 else None
 
 
+# One type for every launch: ctypes drops an array type nobody holds and takes 30 us to make it again.
+_SegmentArray = ctypes.c_int64 * (6 * 8)
+
+
 def copy_tensors(pairs: Sequence[tuple]) -> None:
     """dst.copy_(src) for every (dst, src): small device tensors of equal type and shape go eight to a
     launch, whatever else there is one by one."""
@@ -575,7 +579,7 @@ def copy_tensors(pairs: Sequence[tuple]) -> None:
         count += 1
     for i in range(0, count, 8):
         part = segments[6 * i:6 * (i + 8)]
-        _lib.check(_lib.load().litekv_copy_segments((ctypes.c_int64 * len(part))(*part), len(part) // 6, _stream()))
+        _lib.check(_lib.load().litekv_copy_segments(_SegmentArray(*part), len(part) // 6, _stream()))
 
 
 def decode_step(q: torch.Tensor, kv_pool: torch.Tensor, plan: DecodePlan,
