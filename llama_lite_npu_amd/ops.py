@@ -543,7 +543,8 @@ def decode_advance(request_tables: torch.Tensor, request_ids: torch.Tensor, seq_
 
 def _segment(dst: torch.Tensor, src: torch.Tensor) -> Optional[tuple]:
     """(src, dst, rows, row bytes, src pitch, dst pitch) of a copy litekv_copy_segments can take, or None."""
-    if not (src.is_cuda and src.dtype is dst.dtype and src.shape == dst.shape and src.get_device() == dst.get_device()):
+    if not (src.is_cuda and src.dtype is dst.dtype and src.shape == dst.shape
+            and src.get_device() == dst.get_device() == torch._C._cuda_getDevice()):   # a launch goes to the current device
         return None
     size = dst.element_size()
     if src.is_contiguous() and dst.is_contiguous():
