@@ -540,8 +540,8 @@ int litekv_decode_advance(const int32_t *request_tables, int64_t request_table_s
  *                 [cu_q_lens[b], cu_q_lens[b+1])
  *   context_lens  [B] int32 or NULL
  *   max_q_len     host upper bound of the per-sequence query length (grid)
- *   softmax_scale natural scale; callers holding the reference's
- *                 log2(e)-folded scale (lite_llama/models/qwen3.py:295-298)
+ *   softmax_scale natural scale, above 0 (head_dim 32 and 256 take any value);
+ *                 callers holding the reference's log2(e)-folded scale (lite_llama/models/qwen3.py:295-298)
  *                 divide it out first
  */
 int litekv_paged_prefill(const void *q, int64_t q_token_stride,

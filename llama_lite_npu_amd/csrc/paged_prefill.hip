@@ -30,11 +30,14 @@ static int validate_prefill(const char *what, const void *q, int64_t q_stride, c
 }
 
 // Whether a 256-wide prefill goes to the tiled kernel: all of them but rows it cannot address
-// (16-byte stores of the output, 32-bit offsets into q), which stay with the general kernel. Four
-// prompts of 300 to 2048 tokens, 16 / 4 heads: 9198 us there, without matrix instructions and with
-// every K row read by one lane at a time, 81 us here.
-[[maybe_unused]] static bool tiled_256(int64_t q_stride, int64_t out_stride, int32_t num_kv_heads) {
-  return q_stride < (1 << 25) && out_stride % 8 == 0 && num_kv_heads <= 1024;
+// (16-byte stores of the output, 32-bit offsets into q) and scales its arithmetic is not made for
+// (tile_scale: 0, below 0, not a number), which stay with the general kernel. Four prompts of 300
+// to 2048 tokens, 16 / 4 heads: 9198 us there, without matrix instructions and with every K row
+// read by one lane at a time, 81 us here.
+[[maybe_unused]] static bool tiled_256(int64_t q_stride, int64_t out_stride, int32_t num_kv_heads,
+                                       float softmax_scale) {
+  return q_stride < (1 << 25) && out_stride % 8 == 0 && num_kv_heads <= 1024 &&
+         tile_scale(softmax_scale * kLog2eP);
 }
 
 // How a GQA group of `group` heads is cut into workgroups.
@@ -162,7 +165,8 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
                  "%s: key slices take head_dim 64 or 128", what);
 #if LITEKV_HD == 128
   const PrefillBuild *build = head_dim == 64 ? &hd64_prefill()
-                              : head_dim == 256 && tiled_256(q_token_stride, out_token_stride, num_kv_heads)
+                              : head_dim == 256 && tiled_256(q_token_stride, out_token_stride, num_kv_heads,
+                                                                 softmax_scale)
                                   ? &hd256_prefill()
                                   : nullptr;
   if (build != nullptr) {  // another head dim's build of this file
@@ -290,7 +294,7 @@ static int launch_varlen_prefill(const void *q, int64_t q_token_stride, const vo
 #if LITEKV_HD == 128
   const PrefillBuild *build =
       head_dim == 64 ? &hd64_prefill()
-      : head_dim == 256 && tiled_256(q_token_stride, out_token_stride, num_kv_heads) &&
+      : head_dim == 256 && tiled_256(q_token_stride, out_token_stride, num_kv_heads, softmax_scale) &&
               k_token_stride < (1 << 25) && v_token_stride < (1 << 25)
           ? &hd256_prefill()
           : nullptr;

@@ -62,6 +62,7 @@
 #include "common.h"
 #include "head_dim.h"
 #include "kv_fp8.h"
+#include "prefill_rows.h"
 
 namespace litekv {
 inline namespace LITEKV_HD_NS {
@@ -93,6 +94,12 @@ constexpr int kWgPerCu = kHD == 64 ? 3 : kHD == 128 ? 2 : 1;
 constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 
 constexpr float kLog2eP = 1.4426950408889634f;
+
+// Scales (times log2 e, times the K scale of a pool of codes) the tile arithmetic is made for: it
+// takes maxima of unscaled scores (wrong below 0), and seeds the accumulators with a quotient by
+// the scale (no number at 0, lost below fp32's normal range). Head dim 256 takes any scale, so what
+// lies outside goes another way there.
+__host__ __device__ constexpr bool tile_scale(float k_mul) { return k_mul >= 0x1p-100f && k_mul <= 0x1p100f; }
 
 // Where the keys of a sequence live.
 struct PagedSource {
@@ -152,6 +159,36 @@ constexpr int kPagedPrefill = 0, kPackedPrefill = 1, kSharedPrefix = 2, kPagedPr
 // over a long history) cuts every block's keys into `key_slices` runs of tiles, one workgroup
 // each; a slice leaves a normalised fp32 partial row + log-sum-exp per (query row, head), and a
 // merge launch folds the slices of a row (prefill_split_merge_kernel in paged_prefill.hip).
+
+// Head dim 256: 16 query rows from row0 on (of the q_len of sequence b, which start at q_start behind
+// ctx cached tokens) of query head hq, in fp32 (prefill_rows.h); kv head h, `lds` as there.
+template <int KV, bool PAGED>
+__device__ __forceinline__ void tile_by_rows(uint32_t lds, const half_t *q, int64_t q_stride, half_t *out,
+                                             int64_t out_stride, const PagedSource &paged,
+                                             const PackedSource &packed, int b, int q_start, int q_len, int ctx,
+                                             int row0, int hq, int h, float scale_log2) {
+  constexpr bool CODES = KV != kKvF16;
+  auto kv_row = [&](int tok, bool value) -> const void * {
+    if constexpr (PAGED) {
+      const int shift = 4 + paged.page_shift;
+      int at = tok >> shift;
+      at = at < paged.bt_stride ? at : paged.bt_stride - 1;  // a length beyond the row re-reads its last entry
+      int pid = paged.block_table[(int64_t)b * paged.bt_stride + at];
+      pid = pid < 0 ? 0 : (pid >= paged.num_pages ? paged.num_pages - 1 : pid);
+      const int64_t slot = ((int64_t)pid << shift) + (tok & ((1 << shift) - 1));
+      return (const char *)paged.kv +
+             (slot * 2 * paged.num_kv_heads + (value ? paged.num_kv_heads : 0) + h) * kHD * (CODES ? 1 : 2);
+    } else {
+      return value ? packed.v + (int64_t)(q_start + tok) * packed.v_stride + h * kHD
+                   : packed.k + (int64_t)(q_start + tok) * packed.k_stride + h * kHD;
+    }
+  };
+  const int64_t at = (int64_t)hq * kHD;
+  prefill_rows::attend_rows<KV>(lds, q + (int64_t)(q_start + row0) * q_stride + at, q_stride,
+                                out + (int64_t)(q_start + row0) * out_stride + at, out_stride,
+                                q_len - row0 < 16 ? q_len - row0 : 16, ctx + row0 + 1, kv_row, scale_log2,
+                                CODES ? paged.scales[h] : 1.0f, CODES ? paged.scales[paged.num_kv_heads + h] : 1.0f);
+}
 
 // The body of the kernel, run by a workgroup of W wavefronts that stands at (block_x, block_y,
 // block_z) of a grid block_y runs over grid_y values of; k_lds is the LDS byte address of its
@@ -281,6 +318,22 @@ __device__ __forceinline__ void prefill_tile_body(
     }
   }
   const int n_tiles = (kv_end + kKvTile - 1) / kKvTile - tile0;
+
+  if constexpr (kHD == 256 && FP8) {
+    if (!tile_scale(k_mul)) {  // the K scale's doing: the launch looked at softmax_scale itself
+      constexpr uint32_t kOwn = (uint32_t)tile_lds_bytes<W>() / W;
+      static_assert(prefill_rows::kLdsBytes <= kOwn, "every wavefront has its own part of the staging area");
+      for (int t = wave * kColTiles; t < (wave + 1) * kColTiles; ++t) {
+        const int head = t / row_tiles;
+        const int row0 = m0 + (t - head * row_tiles) * 16;
+        if (head < heads_here && row0 < q_len) {
+          tile_by_rows<KV, PAGED>(k_lds + wave * kOwn, q, q_stride, out, out_stride, paged, packed, b, q_start, q_len,
+                                  ctx, row0, h * group + head0 + head, h, scale_log2);
+        }
+      }
+      return;
+    }
+  }
 
   // ---- staging addresses -------------------------------------------------------------------
   // Direct-load instruction i of wavefront w fills tile rows kRowsPerWave * w + 4i .. +3 (one
