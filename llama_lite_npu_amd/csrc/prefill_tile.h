@@ -160,13 +160,18 @@ constexpr int kPagedPrefill = 0, kPackedPrefill = 1, kSharedPrefix = 2, kPagedPr
 // each; a slice leaves a normalised fp32 partial row + log-sum-exp per (query row, head), and a
 // merge launch folds the slices of a row (prefill_split_merge_kernel in paged_prefill.hip).
 
-// Head dim 256: 16 query rows from row0 on (of the q_len of sequence b, which start at q_start behind
-// ctx cached tokens) of query head hq, in fp32 (prefill_rows.h); kv head h, `lds` as there.
+// Head dim 256: the 16 query rows of column tile t of a block (see prefill_tile_body, whose names these
+// are), in fp32 (prefill_rows.h); `lds` as there.
 template <int KV, bool PAGED>
 __device__ __forceinline__ void tile_by_rows(uint32_t lds, const half_t *q, int64_t q_stride, half_t *out,
                                              int64_t out_stride, const PagedSource &paged,
                                              const PackedSource &packed, int b, int q_start, int q_len, int ctx,
-                                             int row0, int hq, int h, float scale_log2) {
+                                             int m0, int t, int row_tiles, int head0, int heads_here, int group,
+                                             int h, float scale_log2) {
+  const int head = t / row_tiles;
+  const int row0 = m0 + (t - head * row_tiles) * 16;
+  if (head >= heads_here || row0 >= q_len) return;
+  const int hq = h * group + head0 + head;
   constexpr bool CODES = KV != kKvF16;
   auto kv_row = [&](int tok, bool value) -> const void * {
     if constexpr (PAGED) {
@@ -319,17 +324,14 @@ __device__ __forceinline__ void prefill_tile_body(
   }
   const int n_tiles = (kv_end + kKvTile - 1) / kKvTile - tile0;
 
+  // a wavefront's own quarter of the staging area, for what it does before and after the tiles
+  constexpr uint32_t kOwnLds = (uint32_t)tile_lds_bytes<W>() / W;
+  static_assert(kHD != 256 || prefill_rows::kLdsBytes <= kOwnLds, "a tile by rows fits a wavefront's part");
   if constexpr (kHD == 256 && FP8) {
     if (!tile_scale(k_mul)) {  // the K scale's doing: the launch looked at softmax_scale itself
-      constexpr uint32_t kOwn = (uint32_t)tile_lds_bytes<W>() / W;
-      static_assert(prefill_rows::kLdsBytes <= kOwn, "every wavefront has its own part of the staging area");
       for (int t = wave * kColTiles; t < (wave + 1) * kColTiles; ++t) {
-        const int head = t / row_tiles;
-        const int row0 = m0 + (t - head * row_tiles) * 16;
-        if (head < heads_here && row0 < q_len) {
-          tile_by_rows<KV, PAGED>(k_lds + wave * kOwn, q, q_stride, out, out_stride, paged, packed, b, q_start, q_len,
-                                  ctx, row0, h * group + head0 + head, h, scale_log2);
-        }
+        tile_by_rows<KV, PAGED>(k_lds + wave * kOwnLds, q, q_stride, out, out_stride, paged, packed, b, q_start, q_len,
+                                ctx, m0, t, row_tiles, head0, heads_here, group, h, scale_log2);
       }
       return;
     }
@@ -868,15 +870,23 @@ __device__ __forceinline__ void prefill_tile_body(
       __builtin_amdgcn_sched_barrier(0);
       // Region 3: the second half's MFMAs beside the first half's exponentials; the first
       // half's V fragments are requested on the way.
+      // (Head dim 256: the exponentials stand in front of the MFMAs in the source here and below; behind
+      // them, the scheduler started them late and a tile took 3 % longer.)
       half8_t vf[kJTiles];
+      if constexpr (kHD == 256) {
+        exponentials_seeded(st, pk, pk_lo, 0);
+        exponentials_seeded(st, pk, pk_lo, 1);
+      }
 #pragma unroll
       for (int i = 0; i < kJTiles; ++i) {
 #pragma unroll
         for (int u = 0; u < kColTiles; ++u) st1[i & 1][u] = mfma_16x16x32(kf1[i], qf[u][i >> 1], st1[i & 1][u]);
         vf[i] = load_vfrag(i, 0);
       }
-      exponentials_seeded(st, pk, pk_lo, 0);
-      exponentials_seeded(st, pk, pk_lo, 1);
+      if constexpr (kHD != 256) {
+        exponentials_seeded(st, pk, pk_lo, 0);
+        exponentials_seeded(st, pk, pk_lo, 1);
+      }
       const bool over_a = overflowed(pk);
 #pragma unroll
       for (int i = 0; i < kJTiles; ++i) {
@@ -888,6 +898,10 @@ __device__ __forceinline__ void prefill_tile_body(
       // Block 2: second product of the first half beside the second half's exponentials; each
       // fragment register takes the second half's fragment as soon as its MFMAs are issued.
       half8_t vf2[kJTiles];
+      if constexpr (kHD == 256) {
+        exponentials_seeded(st1, pk1, pk1_lo, 0);
+        exponentials_seeded(st1, pk1, pk1_lo, 1);
+      }
 #pragma unroll
       for (int u = 0; u < kColTiles; ++u) dsum[u] = mfma_p(ones, pk[u], pk_lo[u], dsum[u]);
 #pragma unroll
@@ -896,8 +910,10 @@ __device__ __forceinline__ void prefill_tile_body(
         for (int u = 0; u < kColTiles; ++u) acc[j][u] = mfma_p(vf[j], pk[u], pk_lo[u], acc[j][u]);
         vf2[j] = load_vfrag(j, 1);
       }
-      exponentials_seeded(st1, pk1, pk1_lo, 0);
-      exponentials_seeded(st1, pk1, pk1_lo, 1);
+      if constexpr (kHD != 256) {
+        exponentials_seeded(st1, pk1, pk1_lo, 0);
+        exponentials_seeded(st1, pk1, pk1_lo, 1);
+      }
       const bool over_b = overflowed(pk1);
 #pragma unroll
       for (int i = 0; i < kJTiles; ++i) {
@@ -945,7 +961,8 @@ __device__ __forceinline__ void prefill_tile_body(
     // (the K/V tiles are done with) and leave as whole 256-byte rows, 4 rows per instruction.
     constexpr int kOutPitch = 2 * kHD + 16;  // bytes; at 128: 68 dwords, a half-wave's 8-byte writes hit 64 banks
     __syncthreads();                              // every wavefront is done reading the last tile
-    const uint32_t mine = ((wave & 2) ? v_lds : k_lds) + (uint32_t)((wave & 1) * kColTiles * 16 * kOutPitch);
+    const uint32_t mine = kHD == 256 ? k_lds + (uint32_t)wave * kOwnLds
+                                     : ((wave & 2) ? v_lds : k_lds) + (uint32_t)((wave & 1) * kColTiles * 16 * kOutPitch);
 #pragma unroll
     for (int u = 0; u < kColTiles; ++u) {
       const float inv = v_scale / dsum[u][0];
@@ -959,6 +976,8 @@ __device__ __forceinline__ void prefill_tile_body(
     }
     // lane l carries chunk l % kChunks of row l / kChunks + kRowsPerLoad * step
     const int chunk = slot, r4 = r_loc;
+    // Head dim 256: not 0 (but not a number) once an output of the tile was not finite
+    float odd[kColTiles] = {};
 #pragma unroll
     for (int u = 0; u < kColTiles; ++u) {
 #pragma unroll
@@ -971,6 +990,28 @@ __device__ __forceinline__ void prefill_tile_body(
         if (head < heads_here && qrow_idx < q_len) {
           *(half8_t *)(out + (int64_t)(q_start + qrow_idx) * out_stride + (int64_t)out_head[u] * kHD +
                        8 * chunk) = row;
+        }
+        if constexpr (kHD == 256) {
+#pragma unroll
+          for (int i = 0; i < 8; i += 2) {
+            odd[u] = __builtin_amdgcn_fdot2(half2_t{row[i], row[i + 1]}, half2_t{0, 0}, odd[u], false);
+          }
+        }
+      }
+    }
+    if constexpr (kHD == 256) {
+      // A tile with an output that is not finite is attended again row by row, over what was just
+      // written. An infinite value times a probability of 0 -- of a row that may not see its key, or
+      // the second part of a probability that fp16 holds exactly -- is NaN above and must not be.
+      // (Looking costs a v_dot2_f32_f16 for two outputs, on the way to their store; as an fp32 add per
+      // output in front of the conversion it cost 2.5 % of a prompt of 300 to 2048 tokens.)
+      static_assert(kColTiles == 2, "");
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd[0] + odd[1] != 0.f) != 0, false)) {
+        __builtin_amdgcn_s_waitcnt(wait_vm(0));  // the rows' first stores come first
+#pragma unroll 1
+        for (int u = 0; u < kColTiles; ++u) {
+          tile_by_rows<FP8 ? KV : kKvF16, PAGED>(mine, q, q_stride, out, out_stride, paged, packed, b, q_start, q_len, ctx,
+                                                 m0, wave * kColTiles + u, row_tiles, head0, heads_here, group, h, scale_log2);
         }
       }
     }

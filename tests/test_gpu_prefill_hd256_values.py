@@ -63,3 +63,64 @@ def test_any_k_scale(fmt, hq, lens, ctx, page_size):
     torch.cuda.synchronize()
     values = torch.from_numpy(oracle.dequantize_pool(codes.numpy(), scales.numpy()))
     assert_attention_close(out, _reference(case, 0.0625, values).numpy(), f"K scales over {fmt}")
+
+
+def _plant(case, key, element, value, which):
+    """The packed row `key` gets `value` in one element of kv head 1 (k or v), in the pool as well."""
+    (case.k if which == "k" else case.v)[key, 1, element] = value
+    ops.kv_append(case.k, case.v, case.slot_mapping, case.kv_pool)
+
+
+def _rows_with_values(out, ref, key, element, want, group):
+    """`out` is `ref`, but for the rows from `key` on of the heads of kv head 1: `want` in `element`."""
+    ref = ref.clone()
+    ref[key:, group:2 * group, element] = want
+    got = out.double().cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
+    fine = torch.isfinite(ref)
+    assert torch.equal(got[~fine & ~torch.isnan(ref)], ref[~fine & ~torch.isnan(ref)])
+    assert_attention_close(torch.where(fine, got, 0.0), torch.where(fine, ref, 0.0).numpy(), "finite part")
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("hq,length,key", [(16, 200, 40), (16, 200, 130), (8, 190, 0), (28, 70, 69), (4, 150, 127)])
+def test_an_infinite_value_reaches_the_rows_that_see_it(hq, length, key, value):
+    """V of one key, one element: rows from that key on get it (a weight is above 0 at these scores), no
+    earlier row and no other element does, wherever the key stands in its tile."""
+    print(f"prefill 256, {value} in V of key {key} of {length}, {hq} heads", flush=True)
+    case = _case(63, [length], hq, 4)
+    ref = _reference(case, 0.0625)
+    _plant(case, key, 77, value, "v")
+    for out in (_paged(case, 0.0625), _packed(case, 0.0625)):
+        torch.cuda.synchronize()
+        _rows_with_values(out, ref, key, 77, value, hq // 4)
+
+
+def test_a_value_that_is_not_a_number_in_a_pool_of_codes():
+    case = _case(64, [90], 16, 4, [100])
+    gen = torch.Generator().manual_seed(5)
+    codes = torch.randint(-128, 128, case.kv_pool.shape, generator=gen, dtype=torch.int16).to(torch.uint8) & 0xBF
+    scales = torch.full((8,), 0.5)
+    ref = _reference(case, 0.0625, torch.from_numpy(fp8.dequantize_pool(codes.numpy(), scales.numpy())))
+    slot = int(case.slot_mapping[50])
+    codes[slot, 4 + 1, 33] = 0x7F                                   # V of the chunk's row 50, kv head 1
+    out = _paged(case, 0.0625, codes.to(DEV), kv_scales=scales.to(DEV))
+    torch.cuda.synchronize()
+    _rows_with_values(out, ref, 50, 33, float("nan"), 4)
+
+
+def test_an_infinite_key_and_query():
+    """A score of -inf takes the key out of the row, one of +inf (or a query that is not a number) makes
+    the row not a number; rows beside it in the tile stay as they are."""
+    case = _case(65, [150], 16, 4)
+    case.q[90, 5, 3] = float("nan")
+    case.q[:, 4:8, 20] = case.q[:, 4:8, 20].abs().clamp(min=0.25) * -1
+    case.q[100, 6, 20] = 0.5
+    _plant(case, 30, 20, float("inf"), "k")
+    ref = _reference(case, 0.0625)                                  # softmax of -inf is 0, of +inf NaN
+    assert int(torch.isnan(ref).any(-1).sum()) == 2
+    for out in (_paged(case, 0.0625), _packed(case, 0.0625)):
+        torch.cuda.synchronize()
+        got = out.double().cpu()
+        assert torch.equal(torch.isnan(got), torch.isnan(ref)) and not bool(torch.isinf(got).any())
+        assert_attention_close(got.nan_to_num(0.0), ref.nan_to_num(0.0).numpy(), "rows beside it")
