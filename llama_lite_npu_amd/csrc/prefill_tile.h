@@ -32,7 +32,7 @@
 // exponent: a probability costs one multiply, one v_exp_f32 and half a packed conversion. q is not
 // pre-multiplied by c: rounding q * c to fp16 would cost the scores 2^-12 of every channel's
 // share. Whether the running maximum still holds is checked on the packed fp16
-// probabilities (any above 2^8, or not finite, sends the sub-tile to general_tile), not by a
+// probabilities (any above 2^8 -- 2^kMaxP --, or not finite, sends the sub-tile to general_tile), not by a
 // column maximum over the fp32 scores.
 //
 // The accumulators are only ever rescaled in straight-line code (general_tile): a conditional
@@ -83,10 +83,19 @@ __device__ __forceinline__ int k_swz(int r) { return kHD >= 128 ? (r & 15) : ((r
 __device__ __forceinline__ int v_swz(int r) { return kHD >= 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); }
 
 // At head dim 256 a probability reaches the second product as two fp16 numbers, its rounding and
-// what the rounding left (22 bits together), each with an MFMA of its own: prompts of that width
-// have always been attended with fp32 probabilities. It costs half as many MFMAs again (the V
-// fragments and their LDS reads are shared).
+// what the rounding left, each with an MFMA of its own: prompts of that width have always been
+// attended with fp32 probabilities. It costs half as many MFMAs again (the V fragments and their LDS
+// reads are shared). The two hold p within 2^-23 of its value (v_exp_f32 is good for about as much),
+// or within 2^-25, half of fp16's smallest step, if that is more. What the second bound means for a
+// row depends on where its largest probability lies: it is put at 2^kMaxBias instead of 1, and may
+// grow to 2^kMaxP before the row is rescaled, so that the bound is at most 2^-34 of it. (At 1, a
+// row that is the sum over 12 000 keys 22.4 powers of two less likely than one of value 0 was off
+// by 1.4e-2 of itself; at 2^9 by 4e-5, a twelfth of the output's own rounding. 2^9 costs nothing;
+// with 2^11 rows outgrow their bound more often, and four prompts of 300 to 2048 tokens, 16 / 4
+// heads, take 2.5 % longer, with 2^13 a third.)
 constexpr bool kTwoPartP = kHD == 256;
+constexpr int kMaxBias = kTwoPartP ? 9 : 0;
+constexpr int kMaxP = kTwoPartP ? 15 : 8;
 // Workgroups per compute unit: bounded by registers at 64 and 128 (about 150 and 235 per lane), by
 // LDS at 256 (two tiles of K and of V are 128 KiB), where a lane may then use all 512 registers.
 constexpr int kWgPerCu = kHD == 64 ? 3 : kHD == 128 ? 2 : 1;
@@ -654,7 +663,7 @@ __device__ __forceinline__ void prefill_tile_body(
     if constexpr (kTwoPartP) c = mfma_16x16x32(a, lo, c);
     return c;
   };
-  // True if any probability of the sub-tile exceeds 2^8 (or is not finite): the running maximum
+  // True if any probability of the sub-tile exceeds 2^kMaxP (or is not finite): the running maximum
   // is then too low for these keys and the sub-tile has to be redone with a rescale. Probabilities
   // are non-negative, so their fp16 bit patterns order like their values.
   auto overflowed = [&](const half8_t (&pk)[kColTiles]) -> bool {
@@ -668,7 +677,7 @@ __device__ __forceinline__ void prefill_tile_body(
                                                   __builtin_shufflevector(mx4, mx4, 2, 3));
     const uint32_t bits = __builtin_bit_cast(uint32_t, mx2);
     const uint32_t top = (bits & 0xffffu) > (bits >> 16) ? (bits & 0xffffu) : (bits >> 16);
-    return __builtin_amdgcn_ballot_w64(top > 0x5C00u) != 0;  // 0x5C00 = 256.0
+    return __builtin_amdgcn_ballot_w64(top > (uint32_t)(15 + kMaxP) << 10) != 0;  // fp16 bits of 2^kMaxP
   };
   // O^T += V^T . P^T,  l += 1^T . P^T for keys 32 s2 .. +31 of the staged V tile.
   auto accumulate_sub = [&](int s2) {
@@ -775,7 +784,7 @@ __device__ __forceinline__ void prefill_tile_body(
 #pragma unroll
       for (int u = 0; u < kColTiles; ++u) {
         mask_sub(u, key0);
-        const float m_new = vmax2(m_run[u], column_max(u));
+        const float m_new = vmax2(m_run[u], column_max(u) - (float)kMaxBias);
         const float alpha = fast_exp2(m_run[u] - m_new);
         m_run[u] = m_new;
         const float sd = -m_new * k_mul_inv;
@@ -790,7 +799,7 @@ __device__ __forceinline__ void prefill_tile_body(
   };
 
   // Fast tiles kt .. kt_end-1: they proceed only while no column maximum exceeds the running one
-  // by more than 8 (p stays below 2^8: far inside fp16 and fp32 range), so the accumulators are
+  // by more than 8 (6 at head dim 256; p stays below 2^kMaxP, inside fp16 and fp32 range), so the accumulators are
   // touched by nothing but MFMAs. Returns 0 at kt_end, else 1 + the sub-tile of tile kt that
   // has to be redone with a rescale.
   int kt = 1;

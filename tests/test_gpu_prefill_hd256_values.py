@@ -124,3 +124,36 @@ def test_an_infinite_key_and_query():
         got = out.double().cpu()
         assert torch.equal(torch.isnan(got), torch.isnan(ref)) and not bool(torch.isinf(got).any())
         assert_attention_close(got.nan_to_num(0.0), ref.nan_to_num(0.0).numpy(), "rows beside it")
+
+
+@pytest.mark.parametrize("first", [True, False], ids=["likeliest first", "likeliest last"])
+@pytest.mark.parametrize("below,history", [(14.4, 3000), (22.4, 12000), (24.4, 20000)])
+def test_many_unlikely_keys_behind_one_of_no_value(below, history, first):
+    """One key `below` powers of two likelier than each of the history's others, of value 0 in half of the
+    elements: there the row is the sum over the others, so their probabilities must keep their bits.
+
+    Bound: fp16's rounding of the output, 2^-11 of it; probabilities that are off by 2^-34 of the
+    likeliest's, all to one side, times the largest value; fp32 sums over steps of 32 keys, one
+    rounding (2^-24 of the sum) each, and as much again for scores and exponentials."""
+    print(f"prefill 256, {history} keys {below} powers of two below one, first {first}", flush=True)
+    case = _case(66, [20], 8, 2, [history])
+    gen = torch.Generator().manual_seed(7)
+    n = history + 20
+    slots = (case.block_table[0].long().cpu()[torch.arange(n) // 16] * 16 + torch.arange(n) % 16)
+    k, v = torch.zeros((n, 2, D)), 20 + torch.randn((n, 2, D), generator=gen)
+    log2e = 1.4426950408889634
+    k[:, :, 0] = -(below + torch.rand((n, 2), generator=gen) * 0.4 - 0.2) / log2e
+    at = 0 if first else history - 1
+    k[at, :, 0], v[at, :, :D // 2] = 0.0, 0.0
+    pool = case.kv_pool.cpu()
+    pool[slots] = torch.cat([k, v], 1).half()
+    case.kv_pool.copy_(pool)
+    case.q[:] = 0.0
+    case.q[:, :, 0] = 16.0
+    out = _paged(case, 0.0625)
+    torch.cuda.synchronize()
+    ref = _reference(case, 0.0625)
+    bound = (2.0 ** -11 + 2 * (n / 32) * 2.0 ** -24) * ref.abs() + n * 2.0 ** -34 * float(v.max())
+    off = (out.double().cpu() - ref).abs()
+    print(f"  largest error {float((off / ref.abs()).max()):.2e} of the value", flush=True)
+    assert bool((off <= bound).all()), float((off / bound).max())
