@@ -142,7 +142,9 @@ int litekv_page_copy(void *kv_pool, const int32_t *src_ids,
  *   q            [B][Hq][D] fp16, batch stride q_batch_stride, heads contiguous
  *   block_table  [B][block_table_stride] int32 page ids (the per-page
  *                equivalent of the reference's per-token
- *                b_req_tokens_table, paged_attention.py:166-170)
+ *                b_req_tokens_table, paged_attention.py:166-170); any of
+ *                its entries may be read, those past a sequence's last page
+ *                without effect
  *   seq_lens     [B] int32, tokens to attend over (already counting the token
  *                appended this step, model_executor.py:893-911); 0 gives zeros
  *   out          [B][Hq][D] fp16, contiguous

@@ -93,6 +93,19 @@ def _dev_i32(name: str, t: torch.Tensor) -> torch.Tensor:
     return t if t.is_contiguous() else t.contiguous()
 
 
+def _table_rows(t: torch.Tensor) -> tuple:
+    """(block table, entries per row) as the kernels take it: they may read a row to the end of its
+    stride, whatever the lengths are, so no row may be said to reach past the tensor's storage. (The
+    one row of a view counts as contiguous with any stride; a view of some columns of a wider table
+    ends within its last row.)"""
+    width, stride = t.shape[1], t.stride(0)
+    if stride == width or t.shape[0] == 1:
+        return t, max(1, width)
+    if t.storage_offset() + t.shape[0] * stride > t.untyped_storage().nbytes() // t.element_size():
+        return t.contiguous(), max(1, width)
+    return t, stride
+
+
 def _rows(name: str, t: torch.Tensor) -> int:
     """Token stride of a [T, H, D] tensor whose [H, D] block is contiguous."""
     shape, stride = t.shape, t.stride()
@@ -425,7 +438,7 @@ class DecodePlan:
         _need(self.seq_lens.numel() == self.batch, "seq_lens must be [B]")
         self.num_q_heads, self.num_kv_heads = int(num_q_heads), int(num_kv_heads)
         self.num_pages, self.page_size = int(num_pages), int(page_size)
-        self.bt_stride = int(self.block_table.stride(0))
+        self.block_table, self.bt_stride = _table_rows(self.block_table)
         if chunks is not None:
             self.chunks = int(chunks)
         elif self.shared_pages > 0 and block_table.shape[0] > 0:
@@ -484,8 +497,8 @@ class DecodePlan:
         """Recomputes the cuts after the tables or lengths changed (same shapes). Nothing to do
         while the plan is on the per-sequence schedule."""
         if block_table is not None:
-            bt = _dev_i32("block_table", block_table)
-            _need(bt.shape == self.block_table.shape and bt.stride(0) == self.bt_stride, "block_table shape changed")
+            bt, stride = _table_rows(_dev_i32("block_table", block_table))
+            _need(bt.shape == self.block_table.shape and stride == self.bt_stride, "block_table shape changed")
             self.block_table = bt
         if seq_lens is not None:
             sl = _dev_i32("seq_lens", seq_lens)
@@ -718,7 +731,7 @@ def paged_decode(q: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Tens
             raise ValueError("an fp8 pool is read by both stages in one call")
     if not (block_table.dim() == 2 and block_table.shape[0] == b):
         raise ValueError("block_table must be [B, max_blocks]")
-    block_table = _dev_i32("block_table", block_table)
+    block_table, bt_stride = _table_rows(_dev_i32("block_table", block_table))
     seq_lens = _dev_i32("seq_lens", seq_lens)
     if not (seq_lens.numel() == b):
         raise ValueError("seq_lens must be [B]")
@@ -750,19 +763,19 @@ def paged_decode(q: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Tens
                 min_pages_per_split, float(softmax_scale), _stream())
         if fp8:
             _lib.check(_q8_entry(lib, "paged_decode_append", kv_pool)(_ptr(q), q_stride, _ptr(kv_pool), _ptr(kv_scales),
-                                                          _ptr(block_table), block_table.stride(0), _ptr(seq_lens),
+                                                          _ptr(block_table), bt_stride, _ptr(seq_lens),
                                                           *rows, *tail))
         else:
             _lib.check(lib.litekv_paged_decode_append(_ptr(q), q_stride, _ptr(kv_pool), _ptr(block_table),
-                                                      block_table.stride(0), _ptr(seq_lens), *rows, *tail))
+                                                      bt_stride, _ptr(seq_lens), *rows, *tail))
     elif fp8:
         _lib.check(_q8_entry(lib, "paged_decode", kv_pool)(_ptr(q), q_stride, _ptr(kv_pool), _ptr(kv_scales), _ptr(block_table),
-                                               block_table.stride(0), _ptr(seq_lens), _ptr(out), _ptr(workspace),
+                                               bt_stride, _ptr(seq_lens), _ptr(out), _ptr(workspace),
                                                ws_bytes, b, hq, hkv, d, page_size, n_pages, max_splits,
                                                min_pages_per_split, float(softmax_scale), _stream()))
     elif stage in ("both", "split"):
         fn = lib.litekv_paged_decode if stage == "both" else lib.litekv_paged_decode_split
-        _lib.check(fn(_ptr(q), q_stride, _ptr(kv_pool), _ptr(block_table), block_table.stride(0),
+        _lib.check(fn(_ptr(q), q_stride, _ptr(kv_pool), _ptr(block_table), bt_stride,
                       _ptr(seq_lens), _ptr(out), _ptr(workspace), ws_bytes, b, hq, hkv, d, page_size,
                       n_pages, max_splits, min_pages_per_split, float(softmax_scale), _stream()))
     else:
@@ -790,12 +803,13 @@ def paged_decode_static(q: torch.Tensor, kv_pool: torch.Tensor, block_table: tor
         _need(t.is_cuda and t.dtype == torch.int32, f"{name} must be an int32 device tensor")
     _need(block_table.dim() == 2 and block_table.shape[0] == b and block_table.stride(1) == 1,
           "block_table must be [B, max_blocks]")
+    block_table, bt_stride = _table_rows(block_table)
     _need(seq_lens.numel() == b and seq_lens.is_contiguous(), "seq_lens must be contiguous [B]")
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(d)
     q_stride = q.stride(0) if b > 1 else max(q.stride(0), hq * d)
     _lib.check(_lib.load().litekv_paged_decode_static(
-        _ptr(q), q_stride, _ptr(kv_pool), _ptr(block_table), block_table.stride(0), _ptr(seq_lens),
+        _ptr(q), q_stride, _ptr(kv_pool), _ptr(block_table), bt_stride, _ptr(seq_lens),
         _ptr(out), b, hq, hkv, d, page_size, n_pages, int(max_splits), int(min_pages_per_split),
         float(softmax_scale), _stream()))
     return out

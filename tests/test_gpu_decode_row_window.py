@@ -34,3 +34,26 @@ def test_rows_around_the_window(hq, hkv, pages, splits):
     ref = c_oracle.paged_decode(to_np16(case.q), to_np16(pool), case.block_table.cpu().numpy(),
                                 case.seq_lens.cpu().numpy(), case.softmax_scale)
     assert_attention_close(out, ref, f"pages {pages} splits {splits}")
+
+
+@pytest.mark.parametrize("splits", [0, 1, 4])
+def test_rows_that_end_with_their_table(splits):
+    """Views of some columns of a wider table, the last row's included: as the copied table."""
+    print(f"table views, {splits} splits", flush=True)
+    for lens in ([300, 40, 200], [150]):
+        case = workloads.make_decode_case("views", 78, lens, 16, 8, device=DEV)
+        b, width = case.block_table.shape
+        wide = torch.full((b, width + 1500), case.num_pages - 1, dtype=torch.int32, device=DEV)
+        wide[:, 1500:] = case.block_table
+        outs = []
+        for table in (case.block_table, wide[:, 1500:]):
+            plan = ops.DecodePlan(table, case.seq_lens, 16, 8, case.num_pages)
+            plan.set_schedule(splits)
+            plan.refresh()
+            outs.append(ops.decode_step(case.q, case.kv_pool.clone(), plan, case.k_new, case.v_new, case.softmax_scale))
+            out = torch.empty_like(case.q)
+            if splits > 0:
+                outs.append(ops.paged_decode_static(case.q, case.kv_pool, table, case.seq_lens, out, splits, 1))
+        torch.cuda.synchronize()
+        half = len(outs) // 2
+        assert all(torch.equal(a, b) for a, b in zip(outs[:half], outs[half:]))
