@@ -511,7 +511,7 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
   // All arguments in one go: left alone the compiler reads them block by block, each group a
   // scalar round trip of its own in front of the requests that need it.
   const int wg_waves = blockDim.x >> 6;
-  asm volatile("" ::"s"(q), "s"(q_batch_stride), "s"(kv), "s"(scales), "s"(block_table), "s"(bt_stride),
+  if constexpr (!ORDERED) asm volatile("" ::"s"(q), "s"(q_batch_stride), "s"(kv), "s"(scales), "s"(block_table), "s"(bt_stride),
                "s"(seq_lens), "s"(k_new), "s"(v_new), "s"(k_new_stride), "s"(v_new_stride), "s"(out),
                "s"(part_o), "s"(part_lse), "s"(num_q_heads), "s"(num_kv_heads), "s"(group_all), "s"(slices),
                "s"(max_splits), "s"(min_pages_per_split), "s"(num_pages), "s"(page_shift), "s"(scale_log2),
@@ -545,14 +545,14 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
   // with the merge's requests (paged_decode_merge_kernel) and the arguments read in one go, per
   // layer: one sequence of 778 tokens, 16/8 heads, 16 splits 10.0 -> 9.6 us; twelve of 100 to 3000
   // tokens, 32/8 heads of 64 17.9 -> 17.4 us.
-  const int32_t *table = block_table + (int64_t)b * bt_stride;
-  int win0 = 0;
-  int ids = table[lane < bt_stride ? lane : bt_stride - 1];
+  auto row_of_table = [&]() { return block_table + (int64_t)b * bt_stride; };
+  int win0 = 0, ids = 0;
+  if constexpr (!ORDERED) ids = row_of_table()[lane < bt_stride ? lane : bt_stride - 1];
   constexpr bool FP8 = KV != kKvF16;  // 8-bit codes (either format): the layout they share
   typedef typename KvStore<KV>::elem Elem;
   typedef typename KvStore<KV>::page Page;
   half8_t qf[4];
-  {
+  if constexpr (!ORDERED) {
     // Every lane loads, lanes past the group the group's last head: their columns are computed and
     // never stored. (A load under a lane condition would end the straight run of requests.)
     const half_t *row = q + (int64_t)b * q_batch_stride + (int64_t)(hq0 + (n < group ? n : group - 1)) * kHD +
@@ -570,15 +570,18 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
                        v_new + (int64_t)b * v_new_stride + (int64_t)h * kHD, n, g);
   }
   float v_scale = 1.0f, k_inv = 1.0f, v_inv = 1.0f;
-  if constexpr (FP8) {  // the K scale joins the softmax scale, the V scale the normalisation
+  auto read_scales = [&]() {  // the K scale joins the softmax scale, the V scale the normalisation
     const float ks = scales[h];
     scale_log2 *= ks;
     v_scale = scales[num_kv_heads + h];
     k_inv = 1.0f / ks;  // the step's new rows are quantised with the reciprocals
     v_inv = 1.0f / v_scale;
+  };
+  if constexpr (!ORDERED) {
+    if constexpr (FP8) read_scales();
+    asm volatile("" ::: "memory");  // the requests above stay above
+    len = as_uniform(seq_lens)[b];
   }
-  asm volatile("" ::: "memory");  // the requests above stay above
-  if constexpr (!ORDERED) len = as_uniform(seq_lens)[b];
   half_t *out_row = out + ((int64_t)b * num_q_heads + hq0) * kHD;
   if (len <= 0) {
     if (split == 0 && n < group) {
@@ -593,7 +596,15 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
   if (split >= n_splits) return;
   const int p0 = (int)(((int64_t)split * pages) / n_splits);
   const int p1 = (int)(((int64_t)(split + 1) * pages) / n_splits);
-
+  if constexpr (ORDERED) {
+    const half_t *q_rows = q + (int64_t)b * q_batch_stride + (int64_t)hq0 * kHD;
+    if constexpr (FP8) {
+      load_q_fp8_order(qf, q_rows, n, g, group);
+      read_scales();
+    } else {
+      load_q(qf, q_rows, n, g, group);
+    }
+  }
 
   const int64_t row_stride = (int64_t)2 * num_kv_heads * kHD;  // elements per slot
   // this lane's row and column inside page 0 (see PageRegs / PageRegsFp8)
@@ -602,6 +613,7 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
                            q8_v_row(n, g) * row_stride
                      : kv + (int64_t)(num_kv_heads + h) * kHD + 8 * (n & (kVCols - 1)) + g * row_stride;
   const half_t *vt_lane = &vstage[(4 * g + (n >> 2)) * kVPitch + 4 * (n & 3)];
+  const int32_t *table = row_of_table();
 
   HeadState st;
   st.reset();
@@ -615,10 +627,15 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
   const bool fits_table = pages <= (bt_stride << page_shift);
   // Ids are asked for in rising order, and past the range the last one's again, so the window only
   // moves forward. (Its load is waited for inside the branch: see wait_vector_loads.)
+  // ORDERED launches hold more wavefronts than the device, of long splits, and know the length
+  // first: there an id per page, through scalar loads a step ahead of their use, is faster than
+  // the window and requests in front of the length (16 splits, 32 / 4 heads: 64 sequences of 4k to
+  // 16k tokens 230.6 against 237.6 us, 128 of 8k to 32k 816 against 824).
   auto page_id = [&](int p) {
     const int pp = p < p1 ? p : p1 - 1;
     int at = pp >> page_shift;
     at = at < bt_stride ? at : bt_stride - 1;
+    if constexpr (ORDERED) return sub_page_id(table[at], pp, page_shift, num_pages);
     if (at - win0 >= kWave) {
       win0 = at;
       ids = table[at + lane < bt_stride ? at + lane : bt_stride - 1];
