@@ -821,17 +821,22 @@ __device__ __forceinline__ void merge_row(const float *__restrict__ lse1, int64_
   if (live_col) *(half2_t *)(out_row + mcol) = half2_t{(half_t)(num0 * inv), (half_t)(num1 * inv)};
 }
 
-// Schedule "splits" merge: one wavefront per (query head, sequence).
+// Schedule "splits" merge: one wavefront per (query head, sequence). `all_rows`: request every partial
+// row a head could have before the length is known. That is one round trip to memory instead of two,
+// but for short sequences also rows that do not count: taken while all of the launch's partial rows
+// together are at most 8 MiB, which the L2 caches hold as the split kernel left them. Split kernel and
+// merge, 16 splits, 64 / 8 heads: 16 sequences of 2000 tokens 30.3 us with all rows, 31.3 with the
+// length first; 64 sequences, 4 of 4000 tokens among 30-token ones, 42.4 against 38.7, 128
+// sequences of the kind 80.0 against 73.3.
+constexpr int64_t kAllRowsBytes = 8 << 20;
 __global__ __launch_bounds__(kWave) void paged_decode_merge_kernel(
     const int32_t *__restrict__ seq_lens, half_t *__restrict__ out,
     const float *__restrict__ part_o, const float *__restrict__ part_lse, int32_t num_q_heads,
-    int32_t max_splits, int32_t min_pages_per_split) {
+    int32_t max_splits, int32_t min_pages_per_split, int32_t all_rows) {
   const int hq = blockIdx.x;
   const int b = blockIdx.y;
   const int64_t cell0 = ((int64_t)b * num_q_heads + hq) * max_splits;
-  if (max_splits <= kFewPieces) {
-    // Every partial row the head could have is requested together with the length that says how
-    // many it has, one round trip to memory instead of two; those past the last are not added.
+  if (all_rows) {  // (max_splits <= kFewPieces; rows past the last that counts are not added)
     const int lane = threadIdx.x;
     const float *row0 = part_o + cell0 * kHD + (2 * lane < kHD ? 2 * lane : 0);
     float2 r[kFewPieces];
@@ -848,7 +853,7 @@ __global__ __launch_bounds__(kWave) void paged_decode_merge_kernel(
     fold_few(r, lane < n_splits ? l : -INFINITY, n_splits, out + ((int64_t)b * num_q_heads + hq) * kHD, lane);
     return;
   }
-  const int len = seq_lens[b];
+  const int len = as_uniform(seq_lens)[b];
   if (len <= 0) return;
   const int n_splits = splits_for_pages(pages_of(len), max_splits, min_pages_per_split);
   if (n_splits == 1) return;  // the split kernel already wrote the final row
@@ -1578,10 +1583,12 @@ static int launch_merge(const DecodeArgs &a, int32_t max_splits, int32_t min_pag
   }
   const float *part_o = static_cast<const float *>(a.workspace);
   const float *part_lse = part_o + (size_t)a.batch * a.num_q_heads * max_splits * a.head_dim;
+  const bool all_rows = max_splits <= kFewPieces &&
+                        (int64_t)a.batch * a.num_q_heads * max_splits * kHD * (int64_t)sizeof(float) <= kAllRowsBytes;
   hipLaunchKernelGGL(paged_decode_merge_kernel, dim3((unsigned)a.num_q_heads, (unsigned)a.batch),
                      dim3(kWave), 0, static_cast<hipStream_t>(a.stream), a.seq_lens,
                      static_cast<half_t *>(a.out), part_o, part_lse, a.num_q_heads, max_splits,
-                     min_16_token_pages(min_pages_per_split, a.page_size));
+                     min_16_token_pages(min_pages_per_split, a.page_size), (int32_t)all_rows);
   return check_launch(what);
 }
 

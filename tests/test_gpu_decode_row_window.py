@@ -57,3 +57,30 @@ def test_rows_that_end_with_their_table(splits):
         torch.cuda.synchronize()
         half = len(outs) // 2
         assert all(torch.equal(a, b) for a, b in zip(outs[:half], outs[half:]))
+
+
+@pytest.mark.parametrize("batch,hq,hkv", [(16, 64, 8), (17, 64, 8), (33, 32, 4)])
+@pytest.mark.parametrize("splits", [16, 17])
+def test_merge_on_either_side_of_its_rule(batch, hq, hkv, splits):
+    """16 rows a head are requested before the length up to 8 MiB of them (16 x 64 heads); more rows, and
+    more splits, after it: the same fold in fp32, so the sequences both batches hold agree to a step of
+    the output's fp16."""
+    print(f"merge: {batch} sequences, {hq}/{hkv} heads, {splits} splits", flush=True)
+    lens = [30, 0, 4000, 700, 17, 255, 256, 257, 1, 2000, 33, 48] * 3
+    case = workloads.make_decode_case("merge", 79, lens[:batch], hq, hkv, device=DEV)
+    outs = []
+    for rows in (slice(0, 12), slice(0, batch)):
+        plan = ops.DecodePlan(case.block_table[rows].contiguous(), case.seq_lens[rows].contiguous(), hq, hkv,
+                              case.num_pages)
+        plan.set_schedule(splits)
+        plan.split_workspace.fill_(float("nan"))
+        outs.append(ops.decode_step(case.q[rows], case.kv_pool.clone(), plan, case.k_new[rows], case.v_new[rows],
+                                    case.softmax_scale))
+    torch.cuda.synchronize()
+    few, many = outs[0].float(), outs[1][:12].float()
+    assert bool(((few - many).abs() <= 2.0 ** -10 * few.abs() + 2.0 ** -24).all())
+    pool = case.kv_pool.clone()
+    ops.kv_append(case.k_new, case.v_new, case.slot_mapping, pool)
+    ref = c_oracle.paged_decode(to_np16(case.q), to_np16(pool), case.block_table.cpu().numpy(),
+                                case.seq_lens.cpu().numpy(), case.softmax_scale)
+    assert_attention_close(outs[1], ref, f"{batch} sequences, {splits} splits")
