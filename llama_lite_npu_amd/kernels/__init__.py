@@ -62,7 +62,7 @@ def flash_decoding(q, k_cache, v_cache, qk_scale, b_req_tokens_table, b_seq_len,
     hkv, d = k_cache.shape[1], k_cache.shape[2]
     max_pages = cols // PAGE_SIZE
     splits = ops.decode_schedule(b, hkv, max_pages, b * max_pages, 2 * hkv * d * q.element_size(),
-                                 heads_per_kv_head=q.shape[1] // hkv)
+                                 heads_per_kv_head=q.shape[1] // hkv, head_dim=d)
     if splits:
         return ops.paged_decode(q, pool, table, b_seq_len, float(qk_scale), num_splits=splits, schedule="splits")
     return ops.paged_decode(q, pool, table, b_seq_len, float(qk_scale))

@@ -387,7 +387,8 @@ def decode_schedule(batch: int, num_kv_heads: int, max_pages: int, total_pages: 
     sequence and the merge launch: the smallest of ``decode_schedule_estimates``. Choosing by this
     rule is 1.0 % slower on average than always choosing the fastest schedule on the measured
     shapes (33 % at worst: 4 sequences of 80 tokens, 8.4 against 6.4 us). ``current``: the schedule
-    in use; another must be estimated ``hysteresis`` times faster to replace it."""
+    in use; another must be estimated ``hysteresis`` times faster to replace it. ``head_dim`` tells rows
+    of 64 fp16 elements from 128 codes, which ``token_bytes`` alone does not."""
     if batch <= 0 or total_pages <= 0 or max_pages <= 0:
         return 0
     estimates = decode_schedule_estimates(batch, num_kv_heads, max_pages, total_pages, token_bytes, page_size,
@@ -395,6 +396,12 @@ def decode_schedule(batch: int, num_kv_heads: int, max_pages: int, total_pages: 
     if current in estimates:
         estimates[current] /= hysteresis
     return min(estimates, key=estimates.get)
+
+
+def pool_head_dim(token_bytes: int, num_kv_heads: int, kv_dtype: Optional[torch.dtype] = None) -> int:
+    """What ``decode_schedule`` takes for the width of a pool's heads: 64 where the K + V bytes of a token
+    and the element type (None: fp16) say so, else 128, also for the widths the rule does not serve."""
+    return 64 if token_bytes == 2 * num_kv_heads * 64 * (2 if kv_dtype is None else kv_dtype.itemsize) else HEAD_DIM
 
 
 class DecodePlan:
@@ -427,9 +434,7 @@ class DecodePlan:
         self.splits = 1
         self.split_workspace: Optional[torch.Tensor] = None
         self.token_bytes = int(token_bytes) if token_bytes is not None else 2 * int(num_kv_heads) * HEAD_DIM * 2
-        # what the schedule is chosen by: rows of 64 where bytes and element type say so, else of 128
-        self.head_dim = 64 if kv_dtype is not None and self.token_bytes == 2 * num_kv_heads * 64 * kv_dtype.itemsize \
-            else HEAD_DIM
+        self.head_dim = pool_head_dim(self.token_bytes, int(num_kv_heads), kv_dtype)
         _need(0 <= self.shared_pages <= block_table.shape[1], "shared_pages out of range")
         _need(block_table.dim() == 2, "block_table must be [B, max_blocks]")
         self.block_table = _dev_i32("block_table", block_table)
@@ -487,10 +492,11 @@ class DecodePlan:
         if not pages:
             self.set_schedule(0)
             return False
-        narrow = {} if self.head_dim == HEAD_DIM else {"head_dim": self.head_dim}
+        # the rule is told what its defaults do not say
+        differs = {} if self.head_dim == HEAD_DIM else {"head_dim": self.head_dim}
         self.set_schedule(decode_schedule(self.batch, self.num_kv_heads, max(pages), sum(pages), self.token_bytes,
                                           self.page_size, self.num_q_heads // self.num_kv_heads,
-                                          current=self.schedule, hysteresis=hysteresis, **narrow))
+                                          current=self.schedule, hysteresis=hysteresis, **differs))
         return self.per_sequence
 
     def refresh(self, block_table: Optional[torch.Tensor] = None, seq_lens: Optional[torch.Tensor] = None) -> None:

@@ -3,8 +3,9 @@ measurements behind its constants showed, at the sizes the benchmark configurati
 0 = balanced, 1 = one wavefront per (sequence, kv head), 4 / 8 / 16 = splits per sequence + merge."""
 
 import pytest
+import torch
 
-from llama_lite_npu_amd.ops import SPLIT_COUNTS, decode_schedule, decode_schedule_estimates
+from llama_lite_npu_amd.ops import SPLIT_COUNTS, decode_schedule, decode_schedule_estimates, pool_head_dim
 
 TOK = 4096  # K + V bytes of a token: 8 kv heads, fp16
 
@@ -124,3 +125,26 @@ def test_the_choice_knows_the_pool_format_the_head_dim_and_the_kv_heads(batch, h
     pick = decode_schedule(batch, hkv, pages(longest), batch * pages(mean), 2 * hkv * head_dim * code_bytes,
                            heads_per_kv_head=group, head_dim=head_dim)
     assert pick in ((8, 16) if want in (8, 16) else (want,))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("batch,tokens", [(1, 300), (24, 128), (4, 80), (12, 2900), (64, 512), (128, 64)])
+def test_flash_decoding_asks_for_the_width_it_is_given(monkeypatch, batch, tokens, d):
+    """Rows of 64 fp16 elements have the bytes of 128 codes: the wrapper says which it has."""
+    from llama_lite_npu_amd import kernels, ops
+
+    hq, hkv = 32, 8
+    taken = []
+    monkeypatch.setattr(ops, "paged_decode", lambda *a, **kw: taken.append(kw.get("num_splits", 0)))
+    pool = torch.zeros((16, 2 * hkv, d), dtype=torch.float16)
+    kernels.flash_decoding(torch.zeros((batch, hq, d), dtype=torch.float16), pool[:, :hkv], pool[:, hkv:], 0.1,
+                           torch.zeros((batch, tokens), dtype=torch.int32), torch.full((batch,), tokens), tokens)
+    assert taken == [decode_schedule(batch, hkv, pages(tokens), batch * pages(tokens), 2 * hkv * d * 2,
+                                     heads_per_kv_head=hq // hkv, head_dim=d)]
+
+
+def test_a_plan_without_an_element_type_is_one_of_fp16():
+    assert pool_head_dim(2 * 8 * 64 * 2, 8) == 64 and pool_head_dim(2 * 8 * 128 * 2, 8) == 128
+    assert pool_head_dim(2 * 8 * 64 * 2, 8, torch.float16) == 64
+    assert pool_head_dim(2 * 8 * 128, 8, torch.int8) == 128 and pool_head_dim(2 * 8 * 64, 8, torch.uint8) == 64
+    assert pool_head_dim(2 * 4 * 256 * 2, 4) == 128                    # the rule's widths are 64 and 128
