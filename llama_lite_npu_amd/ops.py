@@ -313,9 +313,16 @@ def prefix_chunks(batch: int, num_q_heads: int, num_kv_heads: int, shared_pages:
 SPLIT_COUNTS = (4, 8, 16)
 
 
+def _whole_device_chunks(num_kv_heads: int, cus: int = 256) -> int:
+    """``balanced_chunks`` of a device with so many compute units (no device is asked)."""
+    per_group = min(num_kv_heads, 8)                       # kv heads of a workgroup, a wavefront each
+    groups = (num_kv_heads + 7) // 8
+    return (cus + groups - 1) // groups * (8 // per_group)
+
+
 def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, total_pages: int, token_bytes: int,
                               page_size: int = PAGE_SIZE, heads_per_kv_head: int = 8,
-                              head_dim: int = HEAD_DIM) -> dict:
+                              head_dim: int = HEAD_DIM, chunks: Optional[int] = None) -> dict:
     """Estimated microseconds per layer of every decode schedule a step could take, keyed as
     ``decode_schedule`` returns them. Fits to 554 measured shapes on an MI355X (1 to 2048 sequences
     of 32 to 16384 tokens: equal, ragged, one long among short; 64/8 and 16/8 heads; every
@@ -336,8 +343,11 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
       sequence (up to 36; 0.06 to 0.15 us where a step of few rows shares a long row out among
       several workgroups, by how many rows those are; half as much with rows of 64), 3.4 ns +
       0.26 ns per query head for every sequence, and the bytes at 6.8 MB/us against the chain
-      inside one chunk -- 256 chunks for 8 kv heads, 512 for 4, whose workgroups hold two --; a
-      tenth more with over 8 query heads per kv head (two column tiles, twice the rows to merge).
+      inside one of ``chunks`` (a plan's own count; else what ``balanced_chunks`` gives 256 compute
+      units: 256 for 8 kv heads, 512 for 4, whose workgroups hold two); with over 8 query heads per
+      kv head a tenth more (two column tiles) and the partial rows beyond 8 MB, written and read
+      at 3 MB/us (117 shapes of 8 to 64 query heads per kv head, 1 to 8 kv heads: 2 to 3 % over the
+      fastest schedule; 8 sequences of 4000 tokens, 32/1 heads, 2048 chunks: 31 us, 17 without).
 
     A step over a page of codes takes 1.1 to 1.3 times as long as over fp16 rows (the conversion),
     over rows of 64 elements 0.8 to 0.9 times."""
@@ -349,9 +359,7 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
     slices = (heads_per_kv_head + 15) // 16                # wavefronts per kv head
     norm = lambda p, *xs: sum(x ** p for x in xs) ** (1.0 / p)
     lone = batch * num_kv_heads * slices                   # wavefronts of a launch with one per sequence
-    heads = num_kv_heads * slices
-    groups = (heads + 7) // 8                              # workgroups of up to 8 wavefronts per chunk
-    chunks = (256 + groups - 1) // groups * max(1, 8 // heads)
+    chunks = _whole_device_chunks(num_kv_heads) if chunks is None else chunks
     narrow = head_dim < HEAD_DIM
     codes = token_bytes < 4 * num_kv_heads * head_dim      # a pool of 8-bit codes
     pieces = chain / max(1.0, total / chunks)
@@ -360,9 +368,11 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
     per_piece = 0.055 + 0.09 * rows if pieces > 16 and rows <= 1.0 else 0.170
     per_piece *= 0.57 if narrow else 1.0
     step = (0.87 if narrow else 1.0) * (1.12 if codes else 1.0)
+    partials = (min(total, chunks) + batch) * num_q_heads * head_dim * 4.0
     estimates = {
         0: (7.6 + per_piece * min(pieces, 36.0) + (3.4e-3 + 2.6e-4 * num_q_heads) * batch
-            + norm(2.0, nbytes / 6.81e6, 0.82 * step * -(-total // chunks))) * (1.1 if heads_per_kv_head > 8 else 1.0),
+            + norm(2.0, nbytes / 6.81e6, 0.82 * step * -(-total // chunks))) * (1.1 if heads_per_kv_head > 8 else 1.0)
+           + (max(0.0, 2.0 * partials - 16.8e6) / 3.0e6 if heads_per_kv_head > 8 else 0.0),
     }
     step = (0.81 if narrow else 1.0) * (1.16 if codes else 1.0)
     estimates[1] = 4.27 + norm(3.6, 0.584 * step * chain * (1.0 + 0.49 * min(1.0, lone / 2048.0)), 2.9e-3 * lone,
@@ -381,18 +391,19 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
 
 def decode_schedule(batch: int, num_kv_heads: int, max_pages: int, total_pages: int, token_bytes: int,
                     page_size: int = PAGE_SIZE, heads_per_kv_head: int = 8, current: Optional[int] = None,
-                    hysteresis: float = 1.0, head_dim: int = HEAD_DIM) -> int:
+                    hysteresis: float = 1.0, head_dim: int = HEAD_DIM, chunks: Optional[int] = None) -> int:
     """Which decode schedule a step should take, from what the host knows about it: 0 = balanced,
     1 = one wavefront per (sequence, kv head) in one launch, 4 / 8 / 16 = that many splits per
     sequence and the merge launch: the smallest of ``decode_schedule_estimates``. Choosing by this
     rule is 1.0 % slower on average than always choosing the fastest schedule on the measured
     shapes (33 % at worst: 4 sequences of 80 tokens, 8.4 against 6.4 us). ``current``: the schedule
     in use; another must be estimated ``hysteresis`` times faster to replace it. ``head_dim`` tells rows
-    of 64 fp16 elements from 128 codes, which ``token_bytes`` alone does not."""
+    of 64 fp16 elements from 128 codes, which ``token_bytes`` alone does not; ``chunks``: a plan's own
+    count, see ``decode_schedule_estimates``."""
     if batch <= 0 or total_pages <= 0 or max_pages <= 0:
         return 0
     estimates = decode_schedule_estimates(batch, num_kv_heads, max_pages, total_pages, token_bytes, page_size,
-                                          heads_per_kv_head, head_dim)
+                                          heads_per_kv_head, head_dim, chunks)
     if current in estimates:
         estimates[current] /= hysteresis
     return min(estimates, key=estimates.get)
@@ -494,6 +505,8 @@ class DecodePlan:
             return False
         # the rule is told what its defaults do not say
         differs = {} if self.head_dim == HEAD_DIM else {"head_dim": self.head_dim}
+        if self.chunks != _whole_device_chunks(self.num_kv_heads):
+            differs["chunks"] = self.chunks
         self.set_schedule(decode_schedule(self.batch, self.num_kv_heads, max(pages), sum(pages), self.token_bytes,
                                           self.page_size, self.num_q_heads // self.num_kv_heads,
                                           current=self.schedule, hysteresis=hysteresis, **differs))

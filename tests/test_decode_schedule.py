@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from llama_lite_npu_amd.ops import SPLIT_COUNTS, decode_schedule, decode_schedule_estimates, pool_head_dim
+from llama_lite_npu_amd import _lib, ops
 
 TOK = 4096  # K + V bytes of a token: 8 kv heads, fp16
 
@@ -131,7 +132,7 @@ def test_the_choice_knows_the_pool_format_the_head_dim_and_the_kv_heads(batch, h
 @pytest.mark.parametrize("batch,tokens", [(1, 300), (24, 128), (4, 80), (12, 2900), (64, 512), (128, 64)])
 def test_flash_decoding_asks_for_the_width_it_is_given(monkeypatch, batch, tokens, d):
     """Rows of 64 fp16 elements have the bytes of 128 codes: the wrapper says which it has."""
-    from llama_lite_npu_amd import kernels, ops
+    from llama_lite_npu_amd import kernels
 
     hq, hkv = 32, 8
     taken = []
@@ -148,3 +149,29 @@ def test_a_plan_without_an_element_type_is_one_of_fp16():
     assert pool_head_dim(2 * 8 * 64 * 2, 8, torch.float16) == 64
     assert pool_head_dim(2 * 8 * 128, 8, torch.int8) == 128 and pool_head_dim(2 * 8 * 64, 8, torch.uint8) == 64
     assert pool_head_dim(2 * 4 * 256 * 2, 4) == 128                    # the rule's widths are 64 and 128
+
+
+@pytest.mark.parametrize("hkv", [1, 2, 3, 4, 5, 8, 9, 16])
+def test_the_rule_counts_the_chunks_a_launch_has(hkv):
+    """Of 256 compute units, which is also what the library takes where it finds no device."""
+    if not torch.cuda.is_available():
+        assert ops._whole_device_chunks(hkv) == _lib.load().litekv_paged_decode_balanced_chunks(hkv)
+    for group in (8, 16, 32, 64):              # slices of a kv head's query heads do not change the count
+        shape = (16, hkv, 100, 1600, 4 * hkv * 128)
+        same = decode_schedule_estimates(*shape, heads_per_kv_head=group, chunks=ops._whole_device_chunks(hkv))
+        assert decode_schedule_estimates(*shape, heads_per_kv_head=group) == same
+        few = decode_schedule_estimates(*shape, heads_per_kv_head=group, chunks=7)
+        assert few[0] > same[0] and {k: v for k, v in few.items() if k} == {k: v for k, v in same.items() if k}
+
+
+@pytest.mark.parametrize("hq,hkv,batch,tokens,want", [
+    (32, 1, 8, 4000, (16,)),        # 18.8 us against 31.2 balanced (2048 chunks of 32 partial rows each)
+    (32, 1, 16, 8000, (16,)),       # 31.3 against 48.0
+    (32, 2, 128, 2000, (4, 8)),     # 50.5 and 56.1 against 62.8
+    (64, 1, 2, 16000, (16,)),       # 46.8 against 55.2
+    (32, 1, 1, 2000, (0, 16)),      # 11.9 balanced
+])
+def test_wide_groups_are_charged_for_their_partial_rows(hq, hkv, batch, tokens, want):
+    pick = decode_schedule(batch, hkv, pages(tokens + 1), batch * pages(tokens + 1), 4 * hkv * 128,
+                           heads_per_kv_head=hq // hkv)
+    assert pick in want
