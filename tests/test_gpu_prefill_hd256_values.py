@@ -157,3 +157,39 @@ def test_many_unlikely_keys_behind_one_of_no_value(below, history, first):
     off = (out.double().cpu() - ref).abs()
     print(f"  largest error {float((off / ref.abs()).max()):.2e} of the value", flush=True)
     assert bool((off <= bound).all()), float((off / bound).max())
+
+
+def _spiked(case, at):
+    """Key `at` of sequence 0 scores about 2^40 above the others for every query head that follows it."""
+    case.q[:, :, :4] = 4.0
+    case.k[at, :, :4] = 28.0
+    ops.kv_append(case.k, case.v, case.slot_mapping, case.kv_pool)
+
+
+@pytest.mark.parametrize("fmt", ["f16", "packed", "fp8", "int8"])
+@pytest.mark.parametrize("hq,lens,ctx,page_size,at", [(16, [150, 1, 33], [70, 0, 5], 16, 90), (28, [40], [47], 32, 3)])
+def test_general_kernel_in_every_form(fmt, hq, lens, ctx, page_size, at):
+    """Outputs whose rows are not 16-byte aligned stay with the general kernel: every source of keys, one
+    key that takes the whole weight, nothing written beside the rows."""
+    if fmt == "packed":
+        ctx = None
+    print(f"prefill 256, general kernel, {fmt}, {hq} heads, {lens}", flush=True)
+    case = _case(67, lens, hq, 4, ctx, page_size)
+    _spiked(case, at)
+    wide = torch.zeros((case.q.shape[0], hq * D + 4), dtype=torch.float16, device=DEV)
+    out = wide[:, :hq * D].unflatten(1, (hq, D))
+    values = None
+    if fmt == "packed":
+        ops.varlen_prefill(case.q, case.k, case.v, case.cu_q_lens[:-1], case.seq_lens, case.max_q_len, 0.0625, out=out)
+    elif fmt == "f16":
+        _paged(case, 0.0625, out=out)
+    else:
+        scales = torch.tensor([28.0 / 100] * 4 + [0.04] * 4)
+        pool = torch.zeros(case.kv_pool.shape, dtype=torch.uint8 if fmt == "fp8" else torch.int8, device=DEV)
+        every = torch.arange(pool.shape[0], dtype=torch.int32, device=DEV)
+        ops.kv_append_quantised(case.kv_pool[:, :4], case.kv_pool[:, 4:], every, pool, scales.to(DEV))
+        _paged(case, 0.0625, pool, out=out, kv_scales=scales.to(DEV))
+        values = torch.from_numpy((fp8 if fmt == "fp8" else int8).dequantize_pool(pool.cpu().numpy(), scales.numpy()))
+    torch.cuda.synchronize()
+    assert_attention_close(out, _reference(case, 0.0625, values).numpy(), f"general kernel, {fmt}")
+    assert bool((wide[:, hq * D:] == 0).all())

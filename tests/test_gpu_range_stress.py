@@ -10,7 +10,8 @@ running maximum follows only part of the keys still passes them. Two kinds of in
 
 Both run over pool format {fp16, fp8, int8} x head dim {64, 128} x {balanced schedule,
 per-sequence splits, fused append on either schedule, shared prefix, paged prefill, chunk over
-cached history}, and over head dims 32 and 256 on the general kernel. The reference for a pool of
+cached history}, and over head dims 32 and 256 on the general kernel, but for 256-wide prefills, which
+the tiled kernel takes (the general kernel's are in test_gpu_prefill_hd256_values.py). The reference for a pool of
 8-bit codes is the fp32 oracle applied to the decoded pool (codes are exact in fp16, the scale is
 applied in fp32), so quantisation error is not part of the comparison.
 """
@@ -276,7 +277,7 @@ def test_chunk_over_history_spike(fmt, d, hq, hkv):
 @pytest.mark.parametrize("d", [32, 256])
 @pytest.mark.parametrize("fmt", ["f16", "int8"])
 def test_general_kernel_spikes(d, fmt):
-    """Head dims 32 and 256 (the general kernel): decode on both schedules, fused append of a
+    """Head dims 32 and 256 (the general kernel; the prefill at 256 is the tiled one's): decode on both schedules, fused append of a
     spiking row, prefill and a chunk over history."""
     print(f"stress general kernel d={d} fmt={fmt}", flush=True)
     hq, hkv = 8, 2
