@@ -901,7 +901,7 @@ __device__ __forceinline__ void prefill_tile_body(
       for (int i = 0; i < kJTiles; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, kTwoPartP ? 6 : 5, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
       }
       if (over_a) return 1;
       // Block 2: second product of the first half beside the second half's exponentials; each
@@ -928,7 +928,7 @@ __device__ __forceinline__ void prefill_tile_body(
       for (int i = 0; i < kJTiles; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, kTwoPartP ? 4 : 2, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, kTwoPartP ? 6 : 5, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
       }
       __builtin_amdgcn_sched_group_barrier(0x008, kTwoPartP ? 4 : 2, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
