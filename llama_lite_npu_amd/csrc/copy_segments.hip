@@ -3,7 +3,7 @@
 //
 // Launch-bound: seven arrays of a few hundred bytes each. As seven copies on the stream they ran
 // one after the other in front of every replayed step: 28 layers for one sequence of 778 tokens took
-// 293 us a step with them and 281 with this launch, the graph alone 272.
+// 293 us a step with them and 281 with this launch.
 // One grid row per array; a block takes 4 KiB of it (a thread four 4-byte words: block-table rows
 // have any width, so rows are only 4-byte aligned), the largest array decides how many.
 #include "common.h"

@@ -326,7 +326,7 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
     """Estimated microseconds per layer of every decode schedule a step could take, keyed as
     ``decode_schedule`` returns them. Fits to 554 measured shapes on an MI355X (1 to 2048 sequences
     of 32 to 16384 tokens: equal, ragged, one long among short; 64/8 and 16/8 heads; every
-    schedule replayed from a graph; ``tune_decode_schedule`` re-measures the table) and to 425 more
+    schedule replayed from a graph; ``tune_decode_schedule`` re-measures such tables) and to 425 more
     for what depends on the pool's format, the head dim and the number of kv heads (1 to 128
     sequences of up to 32768 tokens; 64/8, 16/8 and 32/4 heads of 128, 32/8 of 64; fp16, fp8, int8):
 
@@ -395,8 +395,8 @@ def decode_schedule(batch: int, num_kv_heads: int, max_pages: int, total_pages: 
     """Which decode schedule a step should take, from what the host knows about it: 0 = balanced,
     1 = one wavefront per (sequence, kv head) in one launch, 4 / 8 / 16 = that many splits per
     sequence and the merge launch: the smallest of ``decode_schedule_estimates``. Choosing by this
-    rule is 1.0 % slower on average than always choosing the fastest schedule on the measured
-    shapes (33 % at worst: 4 sequences of 80 tokens, 8.4 against 6.4 us). ``current``: the schedule
+    rule is 1.1 to 2.0 % slower on average than always choosing the fastest schedule over the shapes of
+    a head layout and pool format, 17 to 32 % at worst (``tune_decode_schedule``). ``current``: the schedule
     in use; another must be estimated ``hysteresis`` times faster to replace it. ``head_dim`` tells rows
     of 64 fp16 elements from 128 codes, which ``token_bytes`` alone does not; ``chunks``: a plan's own
     count, see ``decode_schedule_estimates``."""
