@@ -511,11 +511,13 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
   // All arguments in one go: left alone the compiler reads them block by block, each group a
   // scalar round trip of its own in front of the requests that need it.
   const int wg_waves = blockDim.x >> 6;
-  if constexpr (!ORDERED) asm volatile("" ::"s"(q), "s"(q_batch_stride), "s"(kv), "s"(scales), "s"(block_table), "s"(bt_stride),
-               "s"(seq_lens), "s"(k_new), "s"(v_new), "s"(k_new_stride), "s"(v_new_stride), "s"(out),
-               "s"(part_o), "s"(part_lse), "s"(num_q_heads), "s"(num_kv_heads), "s"(group_all), "s"(slices),
-               "s"(max_splits), "s"(min_pages_per_split), "s"(num_pages), "s"(page_shift), "s"(scale_log2),
-               "s"(wg_waves));
+  if constexpr (!ORDERED) {
+    asm volatile("" ::"s"(q), "s"(q_batch_stride), "s"(kv), "s"(scales), "s"(block_table), "s"(bt_stride),
+                 "s"(seq_lens), "s"(k_new), "s"(v_new), "s"(k_new_stride), "s"(v_new_stride), "s"(out),
+                 "s"(part_o), "s"(part_lse), "s"(num_q_heads), "s"(num_kv_heads), "s"(group_all), "s"(slices),
+                 "s"(max_splits), "s"(min_pages_per_split), "s"(num_pages), "s"(page_shift), "s"(scale_log2),
+                 "s"(wg_waves));
+  }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int n = lane & 15;   // query head inside the slice (column of S^T)

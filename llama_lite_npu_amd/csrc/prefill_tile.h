@@ -32,7 +32,7 @@
 // exponent: a probability costs one multiply, one v_exp_f32 and half a packed conversion. q is not
 // pre-multiplied by c: rounding q * c to fp16 would cost the scores 2^-12 of every channel's
 // share. Whether the running maximum still holds is checked on the packed fp16
-// probabilities (any above 2^8 -- 2^kMaxP --, or not finite, sends the sub-tile to general_tile), not by a
+// probabilities (any above 2^kMaxP, or not finite, sends the sub-tile to general_tile), not by a
 // column maximum over the fp32 scores.
 //
 // The accumulators are only ever rescaled in straight-line code (general_tile): a conditional
@@ -90,7 +90,7 @@ __device__ __forceinline__ int v_swz(int r) { return kHD >= 128 ? 2 * (r & 7) : 
 // row depends on where its largest probability lies: it is put at 2^kMaxBias instead of 1, and may
 // grow to 2^kMaxP before the row is rescaled, so that the bound is at most 2^-34 of it. (At 1, a
 // row that is the sum over 12 000 keys 22.4 powers of two less likely than one of value 0 was off
-// by 1.4e-2 of itself; at 2^9 by 4e-5, a twelfth of the output's own rounding. 2^9 costs nothing;
+// by 1.4e-2 of itself; at 2^9 by 3e-5, a sixteenth of the output's own rounding. 2^9 costs nothing;
 // with 2^11 rows outgrow their bound more often, and four prompts of 300 to 2048 tokens, 16 / 4
 // heads, take 2.5 % longer, with 2^13 a third.)
 constexpr bool kTwoPartP = kHD == 256;
@@ -799,8 +799,8 @@ __device__ __forceinline__ void prefill_tile_body(
   };
 
   // Fast tiles kt .. kt_end-1: they proceed only while no column maximum exceeds the running one
-  // by more than 8 (6 at head dim 256; p stays below 2^kMaxP, inside fp16 and fp32 range), so the accumulators are
-  // touched by nothing but MFMAs. Returns 0 at kt_end, else 1 + the sub-tile of tile kt that
+  // by more than 8 (6 at head dim 256; p stays below 2^kMaxP, inside fp16 and fp32 range), so the
+  // accumulators are touched by nothing but MFMAs. Returns 0 at kt_end, else 1 + the sub-tile of tile kt that
   // has to be redone with a rescale.
   int kt = 1;
   auto fast_tiles = [&](int kt_end, auto masked_tag) -> int {
@@ -1012,8 +1012,7 @@ __device__ __forceinline__ void prefill_tile_body(
       // A tile with an output that is not finite is attended again row by row, over what was just
       // written. An infinite value times a probability of 0 -- of a row that may not see its key, or
       // the second part of a probability that fp16 holds exactly -- is NaN above and must not be.
-      // (Looking costs a v_dot2_f32_f16 for two outputs, on the way to their store; as an fp32 add per
-      // output in front of the conversion it cost 2.5 % of a prompt of 300 to 2048 tokens.)
+      // (Looking is a v_dot2_f32_f16 for two outputs on the way to their store: nothing to measure.)
       static_assert(kColTiles == 2, "");
       if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd[0] + odd[1] != 0.f) != 0, false)) {
         __builtin_amdgcn_s_waitcnt(wait_vm(0));  // the rows' first stores come first

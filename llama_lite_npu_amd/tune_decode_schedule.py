@@ -67,8 +67,8 @@ def main() -> int:
     token_bytes = 2 * hkv * args.head_dim * dtype.itemsize
     scales = torch.full((2 * hkv,), 0.02, dtype=torch.float32, device=DEV) if codes else None
     schedules = (0, 1) + ops.SPLIT_COUNTS
-    print(f"heads {hq}/{hkv} of {args.head_dim}, {args.kv_dtype} pool, pages of {args.page_size}; us per layer: balanced, then per-sequence in "
-          f"{', '.join(map(str, schedules[1:]))} splits", flush=True)
+    print(f"heads {hq}/{hkv} of {args.head_dim}, {args.kv_dtype} pool, pages of {args.page_size}; us per layer: "
+          f"balanced, then per-sequence in {', '.join(map(str, schedules[1:]))} splits", flush=True)
     ratio_rule, ratio_balanced, worst, shapes = 0.0, 0.0, 0.0, 0
     for b in batches:
         for hi in lengths:
