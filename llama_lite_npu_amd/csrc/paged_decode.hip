@@ -291,6 +291,119 @@ __device__ __forceinline__ void attend_page(HeadState &st, const PageRegsQ8<KV> 
   });
 }
 
+// Two neighbouring pages p, p + 1 in one step: tokens 16p .. 16p+31 of which those before `end`
+// count (page p holds at least one of them). A page on its own is one dependent chain (scores,
+// maximum over the lane groups, exponentials, second product); here the two pages' chains run
+// beside each other, with one maximum, one look at the reference maximum and half as many MFMAs in
+// the second product, whose k index runs over both pages: k = 8g + i is token 4g + i of page p for
+// i < 4 and of page p + 1 behind. `stage_v` writes 32 rows.
+template <typename StageV, typename Refill>
+__device__ __forceinline__ void attend_pair_core(HeadState &st, const half8_t (&ka)[4], const half8_t (&kb)[4],
+                                                 const half8_t (&qf)[4], const half_t *vt_lane, int p, int end,
+                                                 int g, float scale_log2, StageV stage_v, Refill refill) {
+  const bool tail = (p + 2) * kPageSize > end;  // wavefront-uniform
+  wave_lds_fence();
+  stage_v(tail);
+  wave_lds_fence();
+
+  const float4_t zero = float4_t{0.f, 0.f, 0.f, 0.f};
+  float4_t s[2] = {mfma_16x16x32(ka[0], qf[0], zero), mfma_16x16x32(kb[0], qf[0], zero)};
+  float4_t s1[2] = {mfma_16x16x32(ka[kKSteps / 2], qf[kKSteps / 2], zero),
+                    mfma_16x16x32(kb[kKSteps / 2], qf[kKSteps / 2], zero)};
+  if constexpr (kKSteps == 4) {
+    s[0] = mfma_16x16x32(ka[1], qf[1], s[0]);
+    s[1] = mfma_16x16x32(kb[1], qf[1], s[1]);
+    s1[0] = mfma_16x16x32(ka[3], qf[3], s1[0]);
+    s1[1] = mfma_16x16x32(kb[3], qf[3], s1[1]);
+  }
+  refill();
+  float sv[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) sv[i] = (s[i >> 2][i & 3] + s1[i >> 2][i & 3]) * scale_log2;
+  if (tail) {
+    const int tok0 = p * kPageSize + 4 * g;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sv[i] = (tok0 + (i >> 2) * kPageSize + (i & 3) < end) ? sv[i] : -INFINITY;
+  }
+  float mx = fmaxf(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])), fmaxf(fmaxf(sv[4], sv[5]), fmaxf(sv[6], sv[7])));
+  mx = max_over_lane_groups(mx);
+  // as in attend_core
+  if (__builtin_amdgcn_ballot_w64(mx > st.m + kMaxSlack) != 0) {
+    const float m_new = fmaxf(st.m, mx);
+    const float alpha = fast_exp2(st.m - m_new);
+    st.d *= alpha;
+#pragma unroll
+    for (int j = 0; j < kJTiles; ++j) {
+      st.acc[j][0] *= alpha;
+      st.acc[j][1] *= alpha;
+      st.acc[j][2] *= alpha;
+      st.acc[j][3] *= alpha;
+    }
+    st.m = m_new;
+  }
+  half8_t pt;
+  float sum[2] = {0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float pr = fast_exp2(sv[i] - st.m);
+    sum[i >> 2] += pr;
+    pt[i] = (half_t)pr;
+  }
+  st.d += sum[0] + sum[1];
+#pragma unroll
+  for (int j = 0; j < kJTiles; ++j) {
+    typedef __attribute__((address_space(3))) short4_t lds_short4_t;
+    typedef short short8_t __attribute__((ext_vector_type(8)));
+    const short4_t a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t *)(vt_lane + 16 * j));
+    const short4_t b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t *)(vt_lane + kPageSize * kVPitch + 16 * j));
+    st.acc[j] = mfma_16x16x32(__builtin_bit_cast(half8_t, short8_t{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}),
+                              pt, st.acc[j]);
+  }
+}
+
+template <typename Refill>
+__device__ __forceinline__ void attend_pair(HeadState &st, const PageRegs &r0, const PageRegs &r1,
+                                            const half8_t (&qf)[4], half_t *vstage, const half_t *vt_lane, int p,
+                                            int end, int n, int g, float scale_log2, Refill refill) {
+  attend_pair_core(st, r0.k, r1.k, qf, vt_lane, p, end, g, scale_log2, [&](bool tail) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      half8_t x = i < 4 ? r0.v[i & 3] : r1.v[i & 3];
+      // Slots past the end hold arbitrary bits: keep them out of the MFMA.
+      if (tail && p * kPageSize + 4 * i + g >= end) x = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      *(half8_t *)(&vstage[(4 * i + g) * kVPitch + 8 * n]) = x;
+    }
+  }, refill);
+}
+
+template <int KV, typename Refill>
+__device__ __forceinline__ void attend_pair(HeadState &st, const PageRegsQ8<KV> &r0, const PageRegsQ8<KV> &r1,
+                                            const half8_t (&qf)[4], half_t *vstage, const half_t *vt_lane, int p,
+                                            int end, int n, int g, float scale_log2, Refill refill) {
+  half8_t ka[4], kb[4];
+#pragma unroll
+  for (int kk = 0; kk < kKSteps; ++kk) {
+    ka[kk] = codes_to_half<KV>(uint2_t{r0.k[kk >> 1][2 * (kk & 1)], r0.k[kk >> 1][2 * (kk & 1) + 1]});
+    kb[kk] = codes_to_half<KV>(uint2_t{r1.k[kk >> 1][2 * (kk & 1)], r1.k[kk >> 1][2 * (kk & 1) + 1]});
+  }
+  attend_pair_core(st, ka, kb, qf, vt_lane, p, end, g, scale_log2, [&](bool tail) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 8 * i + q8_v_row(n, g);
+      const uint4_t v = i < 2 ? r0.v[i & 1] : r1.v[i & 1];
+      half8_t lo = codes_to_half<KV>(uint2_t{v[0], v[1]});
+      half8_t hi = codes_to_half<KV>(uint2_t{v[2], v[3]});
+      if (tail && p * kPageSize + row >= end) {
+        lo = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        hi = lo;
+      }
+      half_t *dst = &vstage[row * kVPitch + 16 * q8_v_col(n)];
+      *(half8_t *)dst = lo;
+      *(half8_t *)(dst + 8) = hi;
+    }
+  }, refill);
+}
+
 // Writes the normalised state either as the final fp16 row or as an fp32 partial + log-sum-exp.
 // Head n of the group writes out_row + n*D, or part_row + n*part_head_stride and
 // part_lse_cell + n*lse_head_stride.
@@ -494,12 +607,31 @@ __device__ __forceinline__ int sequence_of_rank(const int32_t *seq_lens, int bat
   return r;  // not reached for r < batch
 }
 
-extern __shared__ __attribute__((aligned(16))) half_t split_vstage[];  // [waves][kPageSize * kVPitch]
+extern __shared__ __attribute__((aligned(16))) half_t split_vstage[];  // [waves][2 * kPageSize * kVPitch]
 // ORDERED: blockIdx.z is a rank by length instead of the sequence (see sequence_of_rank); an
 // instantiation of its own, so that launches bound by the dispatch of many short workgroups keep
 // the short prologue.
-template <int DEPTH, int KV, bool APPEND, bool ORDERED = false>
-__global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
+//
+// Two pages per step (attend_pair). A page on its own is one dependent chain, of which a wavefront
+// with a SIMD to itself waits out every part: 0.60 us a page (0.50 of them without the copies
+// described below), 0.42 us as half of a pair (one sequence of 4096 tokens, 64 / 8 heads: one
+// wavefront 160 -> 112 us, 16 splits 18.6 -> 14.5).
+//
+// DEEP: two steps' pages in flight instead of one, requested again after the step instead of in the
+// middle of it, once the scores are under way and V is in LDS. Four pages' registers leave two
+// wavefronts per SIMD where the other form has three, or four over codes, and every launch requests four
+// pages however few its splits have: see the rule in launch_split. Both give the same bits.
+//
+// The second launch bound keeps the accumulators in ordinary registers. Without one the compiler
+// expects a wavefront to be alone with all 512, puts every MFMA result into AGPRs and copies all 32
+// accumulators and the scores out and back on every page: 304 moves in the loop of two pages (the
+// kernel as it was with nothing but the bound: one wavefront 160 -> 139 us, 8 x 512 tokens in 8 splits 11.5 ->
+// 10.7). It is the number of wavefronts per SIMD that the registers allow anyway.
+constexpr int split_waves_per_simd(int kv, bool append, bool deep) {
+  return deep || (kv == kKvFp8 && append) ? 2 : 3;
+}
+template <int KV, bool APPEND, bool DEEP, bool ORDERED = false>
+__global__ __launch_bounds__(kSplitWaves *kWave, split_waves_per_simd(KV, APPEND, DEEP)) void paged_decode_split_kernel(
     const half_t *__restrict__ q, int64_t q_batch_stride,
     typename KvStore<KV>::elem *__restrict__ kv, const float *__restrict__ scales,
     const int32_t *__restrict__ block_table, int32_t bt_stride,
@@ -518,6 +650,8 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
                  "s"(max_splits), "s"(min_pages_per_split), "s"(num_pages), "s"(page_shift), "s"(scale_log2),
                  "s"(wg_waves));
   }
+  constexpr int STEP = 2;                        // pages per step
+  constexpr int DEPTH = DEEP ? 2 * STEP : STEP;  // pages in flight
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int n = lane & 15;   // query head inside the slice (column of S^T)
@@ -527,7 +661,7 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
   const int h = hs.kv_head;
   const int group = hs.q_heads;
   const int split = blockIdx.y;
-  half_t *vstage = split_vstage + wave * (kPageSize * kVPitch);
+  half_t *vstage = split_vstage + wave * (2 * kPageSize * kVPitch);
   const int hq0 = hs.q_head0;
   int b = blockIdx.z, len;
   if constexpr (ORDERED) {
@@ -652,13 +786,16 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
     request_page(r, k_lane, v_lane, page_off, row_stride, p >= p1, kv);
   };
 
+  // Pages past the split's last count for nothing (a pair's second page), whosever they are.
+  const int end = len < p1 * kPageSize ? len : p1 * kPageSize;
 #pragma unroll
   for (int dd = 0; dd < DEPTH; ++dd) request(p0 + dd, buf[dd]);
   for (int p = p0; p < p1; p += DEPTH) {
 #pragma unroll
-    for (int dd = 0; dd < DEPTH; ++dd) {
-      if (p + dd < p1) {
-        if (APPEND && fits_table && (p + dd + 1) * kPageSize >= len) {
+    for (int first = 0; first < DEPTH; first += STEP) {
+#pragma unroll
+      for (int dd = first; dd < first + STEP; ++dd) {
+        if (APPEND && fits_table && p + dd < p1 && (p + dd + 1) * kPageSize >= len) {
           // The sequence's last page: the step's new token (logical position len - 1) goes to
           // the pool and replaces the stale values this wavefront loaded before the write; an
           // fp8 pool gets the codes the append kernel would store and is attended as stored.
@@ -709,9 +846,19 @@ __global__ __launch_bounds__(kSplitWaves *kWave) void paged_decode_split_kernel(
             }
           }
         }
-        attend_page(st, buf[dd], qf, vstage, vt_lane, p + dd, len, n, g, scale_log2);
       }
-      request(p + dd + DEPTH, buf[dd]);
+      auto refill = [&]() {
+        request(p + first + DEPTH, buf[first]);
+        request(p + first + 1 + DEPTH, buf[first + 1]);
+      };
+      if (p + first < p1) {
+        attend_pair(st, buf[first], buf[first + 1], qf, vstage, vt_lane, p + first, end, n, g, scale_log2, [&]() {
+          // the last step asks for nothing (with two steps in flight a request left out would leave the
+          // waits of the loop without the count of the requests behind the one they wait for)
+          if (!DEEP && p + first + DEPTH < p1) refill();
+        });
+      }
+      if constexpr (DEEP) refill();
     }
   }
 
@@ -1509,14 +1656,20 @@ static int launch_split(const DecodeArgs &a, int32_t max_splits, int32_t min_pag
   while (waves > 1 && (units / waves < 512 || slice_heads % waves != 0)) waves >>= 1;
   const dim3 grid((unsigned)(slice_heads / waves), (unsigned)max_splits, (unsigned)a.batch);
   const dim3 block((unsigned)(waves * kWave));
-  const size_t lds = (size_t)waves * kPageSize * kVPitch * sizeof(half_t);
+  const int64_t row_pages = (int64_t)a.block_table_stride << page_shift_of(a.page_size);
+  // Two steps' pages in flight (DEEP) while the launch has half a wavefront per SIMD of an fp16 pool, one
+  // of a pool of codes (whose pages take half the registers and requests, and more work per byte), and
+  // a split can have two pages at all. Geometric means over 239 / 209 shapes, 64 / 8 heads, of the time
+  // against one step's pages: 512 wavefronts 0.94 to 0.99 (codes 0.87 to 0.94), 1024: 1.05 (0.96 to
+  // 1.00), 2048: 1.04 to 1.05 (1.03 to 1.09), 4096: 1.06 to 1.10 (1.02 to 1.05).
+  const bool deep = units <= (fp8_scales != nullptr ? 1024 : 512) && row_pages > max_splits;
+  const size_t lds = (size_t)waves * 2 * kPageSize * kVPitch * sizeof(half_t);
   // Sequences from the longest down once the launch has more workgroups than the device holds at
   // a time (see sequence_of_rank; a launch that is resident at once ends with its longest piece
   // in any order), for block tables wide enough that a split can be 16 pages long: finding its
   // sequence costs a wavefront about a microsecond, which pieces of a page or two would not
   // return (200 sequences of 64 to 256 tokens in 16 splits: 82 us in batch order, 120 us ranked;
   // 256 sequences of 128 to 1024 tokens in 4 splits: 150 against 134 us).
-  const int64_t row_pages = (int64_t)a.block_table_stride << page_shift_of(a.page_size);
   const bool longest_first = max_splits > 1 && a.k_new == nullptr && a.batch <= kMaxOrderedBatch &&
                              units / waves > 3 * (int64_t)device_cus() &&
                              row_pages >= 16 * (int64_t)max_splits;
@@ -1547,11 +1700,17 @@ static int launch_split(const DecodeArgs &a, int32_t max_splits, int32_t min_pag
   auto by_append = [&](auto kv_tag, auto *kv) {
     constexpr int KV = decltype(kv_tag)::value;
     if (a.k_new != nullptr) {
-      launch(paged_decode_split_kernel<LITEKV_DECODE_DEPTH, KV, true>, kv);
+      if (deep) {
+        launch(paged_decode_split_kernel<KV, true, true>, kv);
+      } else {
+        launch(paged_decode_split_kernel<KV, true, false>, kv);
+      }
     } else if (longest_first) {
-      launch(paged_decode_split_kernel<LITEKV_DECODE_DEPTH, KV, false, true>, kv);
+      launch(paged_decode_split_kernel<KV, false, false, true>, kv);
+    } else if (deep) {
+      launch(paged_decode_split_kernel<KV, false, true>, kv);
     } else {
-      launch(paged_decode_split_kernel<LITEKV_DECODE_DEPTH, KV, false>, kv);
+      launch(paged_decode_split_kernel<KV, false, false>, kv);
     }
   };
   if (fp8_scales != nullptr && format == kKvInt8) {

@@ -328,19 +328,20 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
     of 32 to 16384 tokens: equal, ragged, one long among short; 64/8 and 16/8 heads; every
     schedule replayed from a graph; ``tune_decode_schedule`` re-measures such tables) and to 425 more
     for what depends on the pool's format, the head dim and the number of kv heads (1 to 128
-    sequences of up to 32768 tokens; 64/8, 16/8 and 32/4 heads of 128, 32/8 of 64; fp16, fp8, int8):
+    sequences of up to 32768 tokens; 64/8, 16/8 and 32/4 heads of 128, 32/8 of 64; fp16, fp8, int8);
+    the per-sequence ones to 1613 (1 to 2048 sequences, up to 140 000 tokens; the same layouts and formats):
 
     * 1, one wavefront per (sequence, kv head), one launch: 4.3 us + the largest (a 3.6-norm) of the
-      longest sequence's dependent chain of 16-token steps at 0.58 us each -- up to half as much
-      again when the launch has 2048 wavefronts or more, whose loads share the compute units'
-      memory paths with the chain's --, the placement of the launch's wavefronts at 2.9 ns each,
-      and the bytes at 5.7 MB/us (unbalanced streams).
+      longest sequence's dependent chain of 16-token steps at 0.41 us each -- up to 80 % more
+      when the launch has 2048 wavefronts or more, whose loads share the compute units'
+      memory paths with the chain's --, the placement of the launch's wavefronts at 2.4 ns each,
+      and the bytes at 6.0 MB/us (unbalanced streams).
     * 4 / 8 / 16 splits per sequence + the merge launch, for launches of at most 2048 wavefronts:
-      6.5 us for the two launches, the chain of a split against the bytes at 6.1 MB/us (a 3.1-norm),
-      1.3 ns per wavefront; where the bytes dominate, uneven sequences make uneven splits, which
-      the balanced cut does not have: up to 15 % more with the bytes' share.
+      5.9 us for the two launches, the chain of a split at 0.44 to 0.66 us a step against the bytes at
+      6.4 MB/us (a 3.1-norm), 1.1 ns per wavefront (codes: 1.4); where the bytes dominate, uneven sequences make
+      uneven splits, which the balanced cut does not have: up to 18 % more with the bytes' share.
     * 0, balanced (fused step + merge): 7.6 us, 0.17 us per piece the merge folds for the longest
-      sequence (up to 36; 0.06 to 0.15 us where a step of few rows shares a long row out among
+      sequence (up to 36; 0.07 to 0.10 us where a step of few rows shares a long row out among
       several workgroups, by how many rows those are; half as much with rows of 64), 3.4 ns +
       0.26 ns per query head for every sequence, and the bytes at 6.8 MB/us against the chain
       inside one of ``chunks`` (a plan's own count; else what ``balanced_chunks`` gives 256 compute
@@ -349,7 +350,7 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
       at 3 MB/us (117 shapes of 8 to 64 query heads per kv head, 1 to 8 kv heads: 2 to 3 % over the
       fastest schedule; 8 sequences of 4000 tokens, 32/1 heads, 2048 chunks: 31 us, 17 without).
 
-    A step over a page of codes takes 1.1 to 1.3 times as long as over fp16 rows (the conversion),
+    A step over a page of codes takes 1.1 to 1.35 times as long as over fp16 rows (the conversion),
     over rows of 64 elements 0.8 to 0.9 times."""
     steps = max(1, page_size // PAGE_SIZE)                 # the kernels step by 16 tokens
     chain = max_pages * steps
@@ -365,7 +366,7 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
     pieces = chain / max(1.0, total / chunks)
     # rows of more than 16 pieces are merged by several workgroups each while the step has few rows
     rows = batch * num_q_heads * head_dim / (256.0 * HEAD_DIM)
-    per_piece = 0.055 + 0.09 * rows if pieces > 16 and rows <= 1.0 else 0.170
+    per_piece = 0.07 + 0.03 * rows if pieces > 16 and rows <= 1.0 else 0.170
     per_piece *= 0.57 if narrow else 1.0
     step = (0.87 if narrow else 1.0) * (1.12 if codes else 1.0)
     partials = (min(total, chunks) + batch) * num_q_heads * head_dim * 4.0
@@ -374,18 +375,26 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
             + norm(2.0, nbytes / 6.81e6, 0.82 * step * -(-total // chunks))) * (1.1 if heads_per_kv_head > 8 else 1.0)
            + (max(0.0, 2.0 * partials - 16.8e6) / 3.0e6 if heads_per_kv_head > 8 else 0.0),
     }
-    step = (0.81 if narrow else 1.0) * (1.16 if codes else 1.0)
-    estimates[1] = 4.27 + norm(3.6, 0.584 * step * chain * (1.0 + 0.49 * min(1.0, lone / 2048.0)), 2.9e-3 * lone,
-                               nbytes / 5.70e6)
-    step = (0.82 if narrow else 1.0) * (1.27 if codes else 1.0)
+    if narrow and not codes:
+        estimates[0] *= 0.93
+    # the per-sequence kernels: two steps' pages in flight instead of one up to so many wavefronts
+    deep = 1024 if codes else 512
+    step = (0.82 if narrow else 1.0) * (1.29 if codes else 1.0)
+    page = 0.41 * (1.0 + 0.8 * min(1.0, lone / 2048.0))
+    estimates[1] = 4.28 * (0.85 if narrow else 1.0) + norm(3.6, page * step * chain, 2.4e-3 * lone, nbytes / 5.96e6)
+    step = (0.82 if narrow else 1.0) * (1.33 if codes else 1.0)
     for n in SPLIT_COUNTS:
         wavefronts = batch * n * num_kv_heads * slices
         if wavefronts > 2048:
             continue
-        split_chain = 0.634 * step * ((chain + n - 1) // n)
-        stream = nbytes / 6.06e6
-        estimates[n] = ((6.5 + norm(3.1, split_chain, stream) + 1.3e-3 * wavefronts)
-                        * (1.0 + 0.15 * stream / (split_chain + stream)))
+        page = 0.54
+        if wavefronts > deep:
+            page = 0.464 * (1.0 + 0.12 * wavefronts / 2048.0) if codes else 0.44 * (1.0 + 0.5 * wavefronts / 2048.0)
+        split_chain = page * step * ((chain + n - 1) // n)
+        stream = nbytes / 6.4e6
+        estimates[n] = ((5.9 * (1.08 if narrow else 1.0) + norm(3.1, split_chain, stream)
+                         + (1.4e-3 if codes else 1.1e-3) * wavefronts)
+                        * (1.0 + 0.18 * stream / (split_chain + stream)))
     return estimates
 
 
@@ -395,8 +404,8 @@ def decode_schedule(batch: int, num_kv_heads: int, max_pages: int, total_pages: 
     """Which decode schedule a step should take, from what the host knows about it: 0 = balanced,
     1 = one wavefront per (sequence, kv head) in one launch, 4 / 8 / 16 = that many splits per
     sequence and the merge launch: the smallest of ``decode_schedule_estimates``. Choosing by this
-    rule is 1.1 to 2.0 % slower on average than always choosing the fastest schedule over the shapes of
-    a head layout and pool format, 17 to 32 % at worst (``tune_decode_schedule``). ``current``: the schedule
+    rule is 1.1 to 2.3 % slower on average than always choosing the fastest schedule over the shapes of
+    a head layout and pool format, 19 to 36 % at worst (``tune_decode_schedule``). ``current``: the schedule
     in use; another must be estimated ``hysteresis`` times faster to replace it. ``head_dim`` tells rows
     of 64 fp16 elements from 128 codes, which ``token_bytes`` alone does not; ``chunks``: a plan's own
     count, see ``decode_schedule_estimates``."""
