@@ -93,26 +93,8 @@ static size_t prefill_split_workspace_bytes(int64_t num_tokens, int32_t num_q_he
   return (size_t)key_slices * (size_t)num_tokens * (size_t)num_q_heads * (kHD + 1) * sizeof(float);
 }
 
-// Key slices for a paged prefill whose row blocks alone would not fill the device, if the longest
-// row sees `max_kv_len` keys: the count (at most kMaxPrefillKeySlices) with the smallest estimated
-// time, 1 (do not split) unless that is at least 5 % less than unsplit. The estimate, in
-// microseconds, head dim 128 (fits to one request's chunk of 64 to 512 rows over 0 to 32k cached
-// tokens, 64 query / 8 kv heads): a workgroup walks max_kv_len / 64 / n key tiles at 1.0 us each
-// while it has its compute unit to itself and at 1.7 us once the launch has more workgroups than
-// compute units (two share one), times the rounds the launch needs on the device's resident
-// slots; a cut costs the merge launch, 6 us, and a partial row (fp32) written and read back per
-// query row, head and slice at 6 MB/us. (One chunk over 32k tokens, plain against sliced:
-// 128 rows 527 -> 176 us, 256 rows 533 -> 298 us, 512 rows 609 -> 551 us; 128 rows over 2048 tokens
-// 40 -> 30 us in four slices; 512 rows over 2048 tokens in two slices 49 -> 60 us and 128 rows of a
-// fresh prompt in eight 14 -> 29 us, which the estimate rules out.)
-static int32_t prefill_key_slices(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads,
-                                  int32_t max_q_len, int64_t max_kv_len) {
-  if (batch <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 ||
-      max_q_len <= 0 || max_kv_len <= 0 || num_q_heads / num_kv_heads > kMaxGroup) {
-    return 1;
-  }
-  const PrefillShape s = prefill_shape(num_q_heads / num_kv_heads, max_q_len);
-  const int64_t wgs = (int64_t)num_kv_heads * s.head_splits * s.row_blocks * batch;
+// Compute units of the current device.
+static int device_cus() {
   static thread_local int cached_device = -1, cached_cus = 0;  // compute units of the current device
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) dev = -2;
@@ -125,7 +107,42 @@ static int32_t prefill_key_slices(int32_t batch, int32_t num_q_heads, int32_t nu
     cached_device = dev;
     cached_cus = cus;
   }
-  const int64_t cus = cached_cus;
+  return cached_cus;
+}
+
+// Whether the blocks of a launch of `wgs` workgroups (counted as if every sequence had max_q_len rows)
+// whose rows see at most `max_keys` keys are attended by two groups of wavefronts each
+// (varlen_prefill_two_group_kernel): where a workgroup would have its compute unit to itself, from 9 key
+// tiles on. The meeting of the groups costs 1.2 us, halving the keys saves 0.14 us a tile (rows of
+// 64: 0.18). One request, 64 / 8 heads, us with one group and with two: 64 rows over 512 tokens 15.0, 15.4; 128
+// rows 16.5, 16.0; 128 rows over 2048 40.1, 35.4; 512 rows over 8192 174.9, 154.8; 256 rows of a fresh prompt
+// 10.6, 11.1, 512 rows 15.7, 15.8. (More workgroups than compute units share them two by two as it is.)
+static bool two_key_groups(int64_t wgs, int64_t max_keys) {
+  return kHD != 256 && max_keys > 8 * kKvTile && wgs <= device_cus();
+}
+
+// Key slices for a paged prefill whose row blocks alone would not fill the device, if the longest
+// row sees `max_kv_len` keys: the count (at most kMaxPrefillKeySlices) with the smallest estimated
+// time, 1 (do not split) unless that is at least 5 % less than unsplit. The estimate, in
+// microseconds, head dim 128 (fits to one request's chunk of 64 to 512 rows over 0 to 32k cached
+// tokens, 64 query / 8 kv heads): a workgroup walks max_kv_len / 64 / n key tiles at 1.0 us each
+// while it has its compute unit to itself and at 1.7 us once the launch has more workgroups than
+// compute units (two share one), times the rounds the launch needs on the device's resident
+// slots; a cut costs the merge launch, 6 us, and a partial row (fp32) written and read back per
+// query row, head and slice at 6 MB/us. (An unsliced launch of so few workgroups runs in two groups of wavefronts by now, at
+// 0.80 to 0.95 us a tile: where that moves the choice the two are within 5 %. One chunk over 30 000 tokens, plain against sliced:
+// 128 rows 379 -> 142 us, 256 rows 394 -> 275 us, 512 rows 480 -> 485 us; 128 rows over 2048 tokens
+// 35 -> 30 us in four slices; 512 rows over 2048 tokens in two slices 48 -> 62 us and 128 rows of a
+// fresh prompt in eight 14 -> 29 us, which the estimate rules out.)
+static int32_t prefill_key_slices(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads,
+                                  int32_t max_q_len, int64_t max_kv_len) {
+  if (batch <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 ||
+      max_q_len <= 0 || max_kv_len <= 0 || num_q_heads / num_kv_heads > kMaxGroup) {
+    return 1;
+  }
+  const PrefillShape s = prefill_shape(num_q_heads / num_kv_heads, max_q_len);
+  const int64_t wgs = (int64_t)num_kv_heads * s.head_splits * s.row_blocks * batch;
+  const int64_t cus = device_cus();
   const int64_t slots = cus * kWgPerCu;
   if (2 * wgs > slots) return 1;
   const double tile_us = kHD == 64 ? 0.6 : 1.0;
@@ -267,19 +284,31 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
   const PrefillShape s = prefill_shape(group, max_q_len);
   LITEKV_REQUIRE(s.row_blocks <= 65535u, "%s: max_q_len %d too large", what, max_q_len);
   const dim3 grid((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch);
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(kTiledWaves * kWave), 0, static_cast<hipStream_t>(stream),
-                       static_cast<const half_t *>(q), q_token_stride, static_cast<half_t *>(out),
-                       out_token_stride, paged, packed, PrefixTask{}, cu_q_lens,
-                       (const int32_t *)nullptr, context_lens, group, s.head_splits, s.heads_per_wg,
-                       s.row_tiles, softmax_scale * kLog2eP, 1);
+  auto launch = [&](auto mode_tag) {
+    constexpr int MODE = decltype(mode_tag)::value;
+    auto with = [&](auto kernel, int waves) {
+      hipLaunchKernelGGL(kernel, grid, dim3(waves * kWave), 0, static_cast<hipStream_t>(stream),
+                         static_cast<const half_t *>(q), q_token_stride, static_cast<half_t *>(out),
+                         out_token_stride, paged, packed, PrefixTask{}, cu_q_lens,
+                         (const int32_t *)nullptr, context_lens, group, s.head_splits, s.heads_per_wg,
+                         s.row_tiles, softmax_scale * kLog2eP, 1);
+    };
+#if LITEKV_HD != 256
+    // (lengths live on the device: behind a history, as many keys as a block-table row can name)
+    const int64_t max_keys = context_lens != nullptr ? (int64_t)block_table_stride * page_size : max_q_len;
+    if (two_key_groups((int64_t)grid.x * grid.y * grid.z, max_keys)) {
+      with(varlen_prefill_two_group_kernel<MODE>, 2 * kTiledWaves);
+      return;
+    }
+#endif
+    with(varlen_prefill_tiled_kernel<MODE>, kTiledWaves);
   };
   if (format == kKvInt8) {
-    launch(varlen_prefill_tiled_kernel<kPagedPrefillInt8>);
+    launch(std::integral_constant<int, kPagedPrefillInt8>{});
   } else if (format == kKvFp8) {
-    launch(varlen_prefill_tiled_kernel<kPagedPrefillFp8>);
+    launch(std::integral_constant<int, kPagedPrefillFp8>{});
   } else {
-    launch(varlen_prefill_tiled_kernel<kPagedPrefill>);
+    launch(std::integral_constant<int, kPagedPrefill>{});
   }
   return check_launch(what);
 }
@@ -349,16 +378,21 @@ static int launch_varlen_prefill(const void *q, int64_t q_token_stride, const vo
   const int group = num_q_heads / num_kv_heads;
   const PrefillShape s = prefill_shape(group, max_seq_len);
   LITEKV_REQUIRE(s.row_blocks <= 65535u, "varlen_prefill: max_seq_len %d too large", max_seq_len);
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel,
-                       dim3((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch),
-                       dim3(kTiledWaves * kWave), 0, static_cast<hipStream_t>(stream),
+  const dim3 grid((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch);
+  auto launch = [&](auto kernel, int waves) {
+    hipLaunchKernelGGL(kernel, grid, dim3(waves * kWave), 0, static_cast<hipStream_t>(stream),
                        static_cast<const half_t *>(q), q_token_stride, static_cast<half_t *>(out),
                        out_token_stride, paged, packed, PrefixTask{}, seq_starts, seq_lens,
                        (const int32_t *)nullptr, group, s.head_splits, s.heads_per_wg, s.row_tiles,
                        softmax_scale * kLog2eP, 1);
   };
-  launch(varlen_prefill_tiled_kernel<kPackedPrefill>);
+#if LITEKV_HD != 256
+  if (two_key_groups((int64_t)grid.x * grid.y * grid.z, max_seq_len)) {
+    launch(varlen_prefill_two_group_kernel<kPackedPrefill>, 2 * kTiledWaves);
+    return check_launch("varlen_prefill");
+  }
+#endif
+  launch(varlen_prefill_tiled_kernel<kPackedPrefill>, kTiledWaves);
   return check_launch("varlen_prefill");
 }
 }  // namespace LITEKV_HD_NS

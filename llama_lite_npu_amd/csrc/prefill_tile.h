@@ -211,9 +211,9 @@ __device__ __forceinline__ void tile_by_rows(uint32_t lds, const half_t *q, int6
 template <int W>
 constexpr int tile_lds_bytes() { return (W == kWideWaves ? 6 : 4) * kTileHalfs * 2; }
 
-template <int MODE, int W>
+template <int MODE, int W, int KG = 1>
 __device__ __forceinline__ void prefill_tile_body(
-    const uint32_t k_lds, const int block_x, const int block_y, const int block_z, const int grid_y,
+    const uint32_t lds_base, const int block_x, const int block_y, const int block_z, const int grid_y,
     const half_t *__restrict__ q, int64_t q_stride, half_t *__restrict__ out, int64_t out_stride,
     const PagedSource &paged, const PackedSource &packed, const PrefixTask &prefix,
     const int32_t *__restrict__ q_starts_or_cu, const int32_t *__restrict__ q_lens_or_null,
@@ -242,12 +242,16 @@ __device__ __forceinline__ void prefill_tile_body(
   // instructions that takes per operand.
   constexpr int kRowsPerWave = kKvTile / W;
   constexpr int kLoads = kRowsPerWave / kRowsPerLoad;
+  static_assert(KG == 1 || (KG == 2 && W == kTiledWaves && !KSPLIT && !SHARED && kHD != 256), "two key groups: a prefill");
+  const int wave_in_wg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kgroup = KG == 2 ? wave_in_wg / W : 0;  // which half of the keys this wavefront attends
+  const uint32_t k_lds = lds_base + (uint32_t)(kgroup * tile_lds_bytes<W>());
   // Two tiles of K, then two of V: tile t sits in half t % 2. (Eight wavefronts have a third
   // region of the same size behind them: room for their partial rows.)
   const uint32_t v_lds = k_lds + 4u * kTileHalfs;  // LDS byte addresses
 
   const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wave_in_wg - kgroup * W;
   const int lane = tid & 63;
   const int n = lane & 15;
   const int g = lane >> 4;
@@ -274,6 +278,7 @@ __device__ __forceinline__ void prefill_tile_body(
   //   tile0   first key tile (tiles are counted from it)   last_key  last key that exists
   int q_start = 0, q_len = 0, m0 = 0, ctx = 0, kv_end, diag, last_key;
   int tile0 = 0;
+  int wg_barriers = 0;  // two key groups: barriers of the one with more tiles
   if constexpr (SHARED) {
     const int key_begin = block_z * prefix.keys_per_split;
     if (key_begin >= prefix.prefix_keys) return;
@@ -299,6 +304,21 @@ __device__ __forceinline__ void prefill_tile_body(
     kv_end = ctx + m0 + rows;
     diag = ctx + m0;
     last_key = ctx + q_len - 1;
+    if constexpr (KG == 2) {
+      // The first group takes the first half of the tiles, the second the rest: as in a launch over key
+      // slices, from no later than the last tile that every row of the block sees in full. (A block of
+      // so few keys leaves the first group without any.)
+      const int total = (kv_end + kKvTile - 1) / kKvTile;
+      const int plain = (diag + 1) / kKvTile;
+      const int last_start = plain > 0 ? plain - 1 : 0;
+      const int mid = (total + 1) / 2 < last_start ? (total + 1) / 2 : last_start;
+      wg_barriers = mid > total - mid ? mid : total - mid;
+      if (kgroup == 0) {
+        kv_end = mid * kKvTile;
+      } else {
+        tile0 = mid;
+      }
+    }
     if constexpr (KSPLIT) {
       // The tiles every row of the block sees in full (`plain` of them) are shared out among the
       // slices; the last slice also takes the tiles at the diagonal, and starts no later than
@@ -964,6 +984,61 @@ __device__ __forceinline__ void prefill_tile_body(
     }
   }
 
+  if constexpr (KG == 2) {
+    // Each group finishes one of a wavefront's two column tiles: it hands the other's accumulators,
+    // denominators and maxima to the wavefront of the same columns in the other group, through the
+    // staging area, and folds in what it is given.
+    typedef __attribute__((address_space(3))) float4_t lds_float4_t;
+    typedef __attribute__((address_space(3))) float lds_float_t;
+    for (int i = n_tiles > 1 ? n_tiles : 1; i < wg_barriers; ++i) __syncthreads();
+    __syncthreads();  // every wavefront is done with its last tile
+    constexpr uint32_t kHandBytes = 64 * (16 * kJTiles + 8);  // per wavefront: [kJTiles][64] float4, then [2][64] floats
+    constexpr int kOutPitch = 2 * kHD + 16;
+    static_assert(2 * W * (kHandBytes + 16 * kOutPitch) <= 2 * tile_lds_bytes<W>(), "fits the staging area");
+    const uint32_t give = lds_base + (uint32_t)wave_in_wg * kHandBytes;
+    const uint32_t take = lds_base + (uint32_t)(wave_in_wg ^ W) * kHandBytes;
+#pragma unroll
+    for (int u = 0; u < kColTiles; ++u) {
+      if (u != kgroup) {
+#pragma unroll
+        for (int j = 0; j < kJTiles; ++j) *(lds_float4_t *)(uintptr_t)(give + 1024u * j + 16u * lane) = acc[j][u];
+        *(lds_float_t *)(uintptr_t)(give + 1024u * kJTiles + 4u * lane) = dsum[u][0];
+        *(lds_float_t *)(uintptr_t)(give + 1024u * kJTiles + 256u + 4u * lane) = m_run[u];
+      }
+    }
+    __syncthreads();
+    const float d_in = *(const lds_float_t *)(uintptr_t)(take + 1024u * kJTiles + 4u * lane);
+    const float m_in = *(const lds_float_t *)(uintptr_t)(take + 1024u * kJTiles + 256u + 4u * lane);
+    const float m_own = kgroup ? m_run[1] : m_run[0];
+    const float d_own = kgroup ? dsum[1][0] : dsum[0][0];
+    const float m_all = vmax2(m_own, m_in);  // finite: the second group's rows all see a key
+    const float w_own = fast_exp2(m_own - m_all), w_in = fast_exp2(m_in - m_all);
+    const float inv = v_scale / (d_own * w_own + d_in * w_in);
+    const uint32_t mine = lds_base + 2u * W * kHandBytes + (uint32_t)(wave_in_wg * 16 * kOutPitch);
+#pragma unroll
+    for (int j = 0; j < kJTiles; ++j) {
+      const float4_t in = *(const lds_float4_t *)(uintptr_t)(take + 1024u * j + 16u * lane);
+      const float4_t own = kgroup ? acc[j][1] : acc[j][0];
+      half4_t o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = (half_t)((own[i] * w_own + in[i] * w_in) * inv);
+      *(__attribute__((address_space(3))) half4_t *)(uintptr_t)(mine + (uint32_t)(n * kOutPitch + 8 * g) + 32u * j) = o;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int t = wave * kColTiles + kgroup;
+    const int head = t / row_tiles;
+    const int row0 = m0 + (t - head * row_tiles) * 16;
+    half_t *o_tile = out + (int64_t)(q_start + row0) * out_stride + (int64_t)(h * group + head0 + head) * kHD + 8 * slot;
+#pragma unroll
+    for (int step = 0; step < kLoadsPerWave; ++step) {
+      const int r = kRowsPerLoad * step + r_loc;
+      const half8_t row = *(const lds_half8_t *)(uintptr_t)(mine + (uint32_t)(r * kOutPitch + 16 * slot));
+      if (head < heads_here && row0 + r < q_len) *(half8_t *)(o_tile + (int64_t)r * out_stride) = row;
+    }
+    return;
+  }
   if constexpr (!SHARED && !KSPLIT) {
     // The accumulators hold O^T: a lane has 4 consecutive d of one row, so stored directly every
     // store instruction would touch 16 rows with 32 bytes each. The rows go through LDS instead
@@ -1111,6 +1186,27 @@ __global__ __launch_bounds__(kTiledWaves *kWave, kWgPerCu) void varlen_prefill_t
                                prefix, q_starts_or_cu, q_lens_or_null, context_lens, group, head_splits,
                                heads_per_wg, row_tiles, scale_log2);
   }
+}
+
+// The same for a launch of no more workgroups than compute units: eight wavefronts, two groups of four
+// that attend half of the block's keys each (see KG in prefill_tile_body). One workgroup of four on a
+// compute unit is a lone wavefront per SIMD, whose softmax and barrier waits nothing covers; this gives
+// every SIMD two and halves the chain of tiles. The groups meet in LDS, where key slices (separate
+// workgroups) pay for partial rows in memory and a merge launch. One request's chunk of 512 rows, 64 / 8
+// heads, over 7601 cached tokens: 159 -> 132 us (826 -> 994 TFLOP/s); 32 / 8 heads of 64, over 8192: 107 ->
+// 85. Bound by the tile loop's instruction mix, as the launch of many workgroups is.
+template <int MODE>
+__global__ __launch_bounds__(2 * kTiledWaves *kWave, 2) void varlen_prefill_two_group_kernel(
+    const half_t *__restrict__ q, int64_t q_stride, half_t *__restrict__ out, int64_t out_stride,
+    PagedSource paged, PackedSource packed, PrefixTask prefix,
+    const int32_t *__restrict__ q_starts_or_cu, const int32_t *__restrict__ q_lens_or_null,
+    const int32_t *__restrict__ context_lens, int32_t group, int32_t head_splits,
+    int32_t heads_per_wg, int32_t row_tiles, float scale_log2, int32_t) {
+  __shared__ __attribute__((aligned(1024))) half_t lds_all[tile_lds_bytes<kTiledWaves>()];  // two staging areas
+  prefill_tile_body<MODE, kTiledWaves, 2>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, (int)blockIdx.y,
+                             (int)blockIdx.z, (int)gridDim.y, q, q_stride, out, out_stride, paged, packed,
+                             prefix, q_starts_or_cu, q_lens_or_null, context_lens, group, head_splits,
+                             heads_per_wg, row_tiles, scale_log2);
 }
 
 }  // namespace prefill_tile

@@ -1,0 +1,96 @@
+"""GPU: a prefill of few workgroups whose rows may see over 512 keys is attended by two groups of
+wavefronts per block, each over half of its key tiles. Blocks of one tile (the first group has none)
+up to odd and even numbers of them, ragged last blocks and tiles, every pool format, both head dims,
+paged and packed: against float64 arithmetic, and against the one-group launch of the same rows."""
+
+import pytest
+import torch
+
+from llama_lite_npu_amd import ops
+from tests.parity import assert_attention_close
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+# (rows of the chunk, keys cached before it): the tiles of a block go from 1 to 12
+SHAPES = [(1, 0), (70, 0), (17, 47), (16, 48), (64, 64), (33, 95), (1, 127), (129, 128), (130, 250), (5, 700), (150, 511)]
+
+
+def _reference(q, k, v, ctx, scale):
+    q, k, v = q.double().cpu(), k.double().cpu(), v.double().cpu()
+    group = q.shape[1] // k.shape[1]
+    visible = torch.arange(k.shape[0])[None, :] <= ctx + torch.arange(q.shape[0])[:, None]
+    out = torch.empty_like(q)
+    for h in range(q.shape[1]):
+        s = (q[:, h] @ k[:, h // group].T * scale).masked_fill(~visible, float("-inf"))
+        out[:, h] = torch.softmax(s, 1) @ v[:, h // group]
+    return out
+
+
+@pytest.mark.parametrize("hq,hkv", [(8, 1), (4, 2), (3, 3), (10, 1)])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("fmt", ["f16", "fp8", "int8"])
+def test_two_groups(fmt, head_dim, hq, hkv):
+    print(f"two key groups: {fmt} pool, {hq}/{hkv} heads of {head_dim}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    rows = [r for r, _ in SHAPES]
+    ctx = [c for _, c in SHAPES]
+    pages = [-(-(r + c) // 16) for r, c in SHAPES]
+    perm = torch.randperm(sum(pages), generator=gen, device=DEV).to(torch.int32)
+    width = max(pages)
+    table = torch.zeros((len(SHAPES), width), dtype=torch.int32, device=DEV)
+    at = 0
+    for b, n in enumerate(pages):
+        table[b, :n] = perm[at:at + n]
+        at += n
+    kv = torch.randn((sum(pages) * 16, 2 * hkv, head_dim), generator=gen, dtype=torch.float16, device=DEV)
+    pool, scales, values = kv, None, kv
+    if fmt != "f16":
+        scales = torch.full((2 * hkv,), 0.035, device=DEV)
+        pool = torch.empty(kv.shape, dtype=torch.uint8 if fmt == "fp8" else torch.int8, device=DEV)
+        slots = torch.arange(kv.shape[0], dtype=torch.int32, device=DEV)
+        ops.kv_append_quantised(kv[:, :hkv], kv[:, hkv:], slots, pool, scales)
+        values = (pool if fmt == "int8" else pool.view(torch.float8_e4m3fn)).double() * 0.035
+    q = torch.randn((sum(rows), hq, head_dim), generator=gen, dtype=torch.float16, device=DEV)
+    scale = head_dim ** -0.5
+    out, one = torch.empty_like(q), torch.empty_like(q)
+    first = 0
+    for b, (r, c) in enumerate(SHAPES):
+        cu = torch.tensor([0, r], dtype=torch.int32, device=DEV)
+        ctx_b = torch.tensor([c], dtype=torch.int32, device=DEV)
+        part = slice(first, first + r)
+        # the row of the whole table names over 512 keys; its own pages alone may not
+        ops.paged_prefill(q[part], pool, table[b:b + 1], cu, ctx_b, r, scale, out=out[part], kv_scales=scales, key_slices=1)
+        own = table[b:b + 1, :min(pages[b], 32)].contiguous()
+        if pages[b] <= 32:
+            ops.paged_prefill(q[part], pool, own, cu, ctx_b, r, scale, out=one[part], kv_scales=scales, key_slices=1)
+        else:
+            one[part] = out[part]
+        first += r
+    cu = torch.tensor([0] + rows, dtype=torch.int32).cumsum(0).to(torch.int32).to(DEV)
+    batch = ops.paged_prefill(q, pool, table, cu, torch.tensor(ctx, dtype=torch.int32, device=DEV), max(rows), scale,
+                              kv_scales=scales, key_slices=1)
+    torch.cuda.synchronize()
+    assert torch.equal(batch, out)
+    assert_attention_close(out, one.float().cpu().numpy(), "one group")
+    first = 0
+    for b, (r, c) in enumerate(SHAPES):
+        slot = torch.cat([table[b, t // 16, None].long() * 16 + t % 16 for t in range(r + c)])
+        ref = _reference(q[first:first + r], values[slot, :hkv], values[slot, hkv:], c, scale)
+        assert_attention_close(out[first:first + r], ref.numpy(), f"rows {r} ctx {c}")
+        first += r
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_two_groups_over_packed_rows(head_dim):
+    print(f"two key groups, packed, heads of {head_dim}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(6)
+    lens, hq, hkv = [513, 1, 64, 65, 130], 6, 2
+    q, k, v = (torch.randn((sum(lens), h, head_dim), generator=gen, dtype=torch.float16, device=DEV) for h in (hq, hkv, hkv))
+    starts = torch.tensor([0] + lens[:-1], dtype=torch.int32).cumsum(0).to(torch.int32).to(DEV)
+    out = ops.varlen_prefill(q, k, v, starts, torch.tensor(lens, dtype=torch.int32, device=DEV), max(lens))
+    torch.cuda.synchronize()
+    first = 0
+    for n in lens:
+        s = slice(first, first + n)
+        assert_attention_close(out[s], _reference(q[s], k[s], v[s], 0, head_dim ** -0.5).numpy(), f"length {n}")
+        first += n
