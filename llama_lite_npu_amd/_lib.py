@@ -222,6 +222,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_calls = None
 
 
 class LiteKVError(RuntimeError):
@@ -248,6 +249,20 @@ def load() -> ctypes.CDLL:
         raise LiteKVError(f"liblitekv ABI {got} != binding ABI {ABI_VERSION}; rebuild the library")
     _lib = lib
     return lib
+
+
+def calls():
+    """The native form of the wrappers that run per layer of a prefill (csrc/torch_calls.cpp)."""
+    global _calls
+    if _calls is None:
+        load()
+        try:
+            from . import _calls as module
+        except ImportError as e:
+            raise LiteKVError(f"{__package__}._calls: {e}: build it with `python -m llama_lite_npu_amd.build` "
+                              "(there is no fallback implementation)") from e
+        _calls = module
+    return _calls
 
 
 def check(status: int) -> None:

@@ -12,11 +12,13 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 CSRC = Path(__file__).resolve().parent / "csrc"
 LIB_PATH = CSRC / "liblitekv.so"
+CALLS_PATH = CSRC.parent / "_calls.so"          # csrc/torch_calls.cpp, a Python module
 OBJ_DIR = CSRC / "build"
 
 SOURCES = (
@@ -119,5 +121,30 @@ def build_library(force: bool = False, extra_flags: tuple[str, ...] = ()) -> Pat
     return LIB_PATH
 
 
+def build_calls(force: bool = False) -> Path:
+    """Compiles the Python module of the calls that take PyTorch tensors (host code, no kernel); returns its
+    path. It finds liblitekv.so next to its source."""
+    import torch
+    from torch.utils import cpp_extension
+
+    src = CSRC / "torch_calls.cpp"
+    deps = [src, CSRC.parents[1] / "include" / "litekv.h"]
+    if not force and CALLS_PATH.exists() and all(d.stat().st_mtime <= CALLS_PATH.stat().st_mtime for d in deps):
+        return CALLS_PATH
+    torch_lib = Path(torch.__file__).resolve().parent / "lib"
+    includes = [CSRC.parents[1] / "include", sysconfig.get_paths()["include"], *cpp_extension.include_paths()]
+    tmp = CALLS_PATH.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-isystem{i}" for i in includes),
+           str(src), "-o", str(tmp), f"-L{torch_lib}", "-ltorch_python", "-ltorch_cpu", "-lc10",
+           f"-L{CSRC}", f"-l:{LIB_PATH.name}", f"-Wl,-rpath,$ORIGIN/{CSRC.name}"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"build of {CALLS_PATH.name} failed:\n{proc.stdout}{proc.stderr}")
+    os.replace(tmp, CALLS_PATH)
+    return CALLS_PATH
+
+
 if __name__ == "__main__":
     print(build_library(force=True))
+    print(build_calls(force=True))

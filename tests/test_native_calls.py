@@ -1,0 +1,127 @@
+"""The native form of the per-layer prefill calls (csrc/torch_calls.cpp): it answers None to whatever
+is not a plain call, and the wrappers then behave as they do without it -- the same results bit for
+bit, the same errors."""
+
+import pytest
+import torch
+
+from llama_lite_npu_amd import _lib, ops
+
+DEV = "cuda:0"
+
+
+def test_anything_but_a_plain_call_is_left_alone():
+    calls = _lib.calls()
+    x = torch.zeros((2, 4, 128), dtype=torch.float16)
+    pool = torch.zeros((32, 4, 128), dtype=torch.float16)
+    idx = torch.zeros(2, dtype=torch.int32)
+    assert calls.qk_norm_rope_append() is None and calls.paged_prefill(1, 2) is None
+    assert calls.qk_norm_rope_append(x, x, x, idx, pool, None, None, None, None, 1e-6, None, 0) is None   # on the CPU
+    assert calls.qk_norm_rope_append(*[None] * 12) is None and calls.paged_prefill(*["q"] * 11) is None
+    assert calls.paged_prefill(x, pool, idx[None], idx, None, 2, 1.0, 16, None, None, 0) is None
+
+
+class _NoCalls:
+    @staticmethod
+    def qk_norm_rope_append(*a):
+        return None
+
+    @staticmethod
+    def paged_prefill(*a):
+        return None
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+def _state(fmt, d, hq=8, hkv=2, rows=37):
+    gen = torch.Generator(device=DEV).manual_seed(d + rows)
+    r = lambda *s: torch.randn(s, generator=gen, device=DEV, dtype=torch.float16)
+    dtype = {"f16": torch.float16, "fp8": torch.uint8, "e4m3": torch.float8_e4m3fn, "int8": torch.int8}[fmt]
+    st = dict(q=r(rows, hq, d), k=r(rows, hkv, d), v=r(rows, hkv, d), qw=1 + r(d) / 8, kw=1 + r(d) / 8, cos=r(rows, d),
+              sin=r(rows, d), pool=torch.zeros((96, 2 * hkv, d), dtype=dtype, device=DEV),
+              scales=None if fmt == "f16" else torch.full((2 * hkv,), 0.03, device=DEV),
+              slots=torch.randperm(48, generator=gen, device=DEV)[:rows].to(torch.int32),
+              table=torch.tensor([[1, 0, 2]], dtype=torch.int32, device=DEV),
+              cu=torch.tensor([0, rows], dtype=torch.int32, device=DEV), ctx=None, max_q=rows, scale=d ** -0.5)
+    return st
+
+
+def _run(st):
+    q = ops.qk_norm_rope_append(st["q"], st["k"], st["v"], st["slots"], st["pool"], st["qw"], st["kw"], st["cos"], st["sin"],
+                                1e-6, kv_scales=st["scales"])
+    out = ops.paged_prefill(q, st["pool"], st["table"], st["cu"], st["ctx"], st["max_q"], st["scale"], page_size=16,
+                            kv_scales=st["scales"], max_kv_len=st["max_q"])
+    torch.cuda.synchronize()
+    return [out, st["q"].clone(), st["pool"].view(torch.int16 if st["pool"].dtype == torch.float16 else torch.uint8).clone()]
+
+
+def _strided_q(st):      # q as a slice of a wider projection
+    wide = torch.randn((37, 12, st["q"].shape[2]), device=DEV, dtype=torch.float16)
+    wide[:, 2:10] = st["q"]
+    st["q"] = wide[:, 2:10]
+
+
+CHANGES = {
+    "plain": lambda st: None,
+    "q rows of a wider tensor": _strided_q,
+    "no norm": lambda st: st.update(qw=None, kw=None),
+    "no rotary": lambda st: st.update(cos=None, sin=None),
+    "parameters": lambda st: st.update(qw=torch.nn.Parameter(st["qw"]), kw=torch.nn.Parameter(st["kw"])),
+    "long cos": lambda st: st.update(cos=torch.cat([st["cos"]] * 2, 1), sin=torch.cat([st["sin"]] * 2, 1)),
+    "cos with a batch dim": lambda st: st.update(cos=st["cos"][None], sin=st["sin"][None]),
+    "int64 slots": lambda st: st.update(slots=st["slots"].long()),
+    "int64 table": lambda st: st.update(table=st["table"].long()),
+    "a view of a table": lambda st: st.update(table=torch.cat([st["table"]] * 2, 1)[:, :3]),
+    "history": lambda st: st.update(ctx=torch.tensor([5], dtype=torch.int32, device=DEV)),
+    "a subclass": lambda st: st.update(q=st["q"].as_subclass(_Sub)),
+    # refused
+    "q in bf16": lambda st: st.update(q=st["q"].bfloat16()),
+    "k of another length": lambda st: st.update(k=st["k"][:-1]),
+    "one norm": lambda st: st.update(kw=None),
+    "short cos": lambda st: st.update(cos=st["cos"][:, :8], sin=st["sin"][:, :8]),
+    "slots too few": lambda st: st.update(slots=st["slots"][:-1]),
+    "scales of the wrong size": lambda st: st.update(scales=torch.ones(3, device=DEV)),
+    "heads not contiguous": lambda st: st.update(q=st["q"].transpose(0, 1).contiguous().transpose(0, 1)),
+    "misaligned q": lambda st: st.update(q=torch.zeros(st["q"].numel() + 1, device=DEV, dtype=torch.float16)[1:].view_as(st["q"])),
+    "table of another batch": lambda st: st.update(table=torch.cat([st["table"]] * 2)),
+    "odd pool": lambda st: st.update(pool=st["pool"][:, :3].contiguous()),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["f16", "fp8", "e4m3", "int8"])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_the_wrappers_do_the_same_with_and_without_it(fmt, d, monkeypatch):
+    print(f"native calls: {fmt} pool, heads of {d}", flush=True)
+    for name, change in CHANGES.items():
+        results = []
+        for native in (True, False):
+            st = _state(fmt, d)
+            change(st)
+            with monkeypatch.context() as m:
+                if not native:
+                    m.setattr(_lib, "calls", lambda: _NoCalls)
+                try:
+                    results.append(_run(st))
+                except (ValueError, _lib.LiteKVError) as e:
+                    results.append(f"{type(e).__name__}: {e}")
+        a, b = results
+        if isinstance(b, str):
+            assert a == b, name
+        else:
+            assert all(torch.equal(x, y) for x, y in zip(a, b)), name
+
+
+@pytest.mark.gpu
+def test_a_plain_call_is_taken():
+    print("native calls: taken", flush=True)
+    st = _state("f16", 128)
+    calls = _lib.calls()
+    stream = torch.cuda.current_stream().cuda_stream
+    assert calls.qk_norm_rope_append(st["q"], st["k"], st["v"], st["slots"], st["pool"], st["qw"], st["kw"], st["cos"],
+                                     st["sin"], 1e-6, None, stream) is True
+    out = calls.paged_prefill(st["q"], st["pool"], st["table"], st["cu"], None, 37, st["scale"], 16, None, 37, stream)
+    torch.cuda.synchronize()
+    assert out.shape == st["q"].shape and out.dtype == torch.float16 and bool(torch.isfinite(out).all())
