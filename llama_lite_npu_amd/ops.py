@@ -341,7 +341,7 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
       memory paths with the chain's --, the placement of the launch's wavefronts at 2.4 ns each,
       and the bytes at 6.0 MB/us (unbalanced streams).
     * 4 / 8 / 16 splits per sequence + the merge launch, for launches of at most 2048 wavefronts:
-      5.9 us for the two launches, the chain of a split at 0.44 to 0.66 us a step against the bytes at
+      5.9 us for the two launches, the chain of a split at 0.44 to 0.67 us a step against the bytes at
       6.4 MB/us (a 3.1-norm), 1.1 ns per wavefront (codes: 1.4); where the bytes dominate, uneven sequences make
       uneven splits, which the balanced cut does not have: up to 18 % more with the bytes' share.
     * 0, balanced (fused step + merge): 7.6 us, 0.17 us per piece the merge folds for the longest
@@ -393,7 +393,7 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
             continue
         page = 0.54
         if wavefronts > deep:
-            page = 0.464 * (1.0 + 0.12 * wavefronts / 2048.0) if codes else 0.44 * (1.0 + 0.5 * wavefronts / 2048.0)
+            page = 0.6 * (1.0 + 0.12 * wavefronts / 2048.0) if codes else 0.44 * (1.0 + 0.5 * wavefronts / 2048.0)
         split_chain = page * step * ((chain + n - 1) // n)
         stream = nbytes / 6.4e6
         estimates[n] = ((5.9 * (1.08 if narrow else 1.0) + norm(3.1, split_chain, stream)
@@ -408,7 +408,7 @@ def decode_schedule(batch: int, num_kv_heads: int, max_pages: int, total_pages: 
     """Which decode schedule a step should take, from what the host knows about it: 0 = balanced,
     1 = one wavefront per (sequence, kv head) in one launch, 4 / 8 / 16 = that many splits per
     sequence and the merge launch: the smallest of ``decode_schedule_estimates``. Choosing by this
-    rule is 1.1 to 2.3 % slower on average than always choosing the fastest schedule over the shapes of
+    rule is 1.1 to 2.6 % slower on average than always choosing the fastest schedule over the shapes of
     a head layout and pool format, 19 to 36 % at worst (``tune_decode_schedule``). ``current``: the schedule
     in use; another must be estimated ``hysteresis`` times faster to replace it. ``head_dim`` tells rows
     of 64 fp16 elements from 128 codes, which ``token_bytes`` alone does not; ``chunks``: a plan's own
