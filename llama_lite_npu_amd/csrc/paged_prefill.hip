@@ -45,11 +45,11 @@ struct PrefillShape {
   int head_splits, heads_per_wg, row_tiles;
   unsigned row_blocks;
 };
-static PrefillShape prefill_shape(int group, int max_q_len) {
+static PrefillShape prefill_shape(int group, int max_q_len, int wg_col_tiles = kWgColTiles) {
   PrefillShape s;
-  s.head_splits = (group + kWgColTiles - 1) / kWgColTiles;
+  s.head_splits = (group + wg_col_tiles - 1) / wg_col_tiles;
   s.heads_per_wg = (group + s.head_splits - 1) / s.head_splits;
-  s.row_tiles = kWgColTiles / s.heads_per_wg;
+  s.row_tiles = wg_col_tiles / s.heads_per_wg;
   s.row_blocks = (unsigned)((max_q_len + 16 * s.row_tiles - 1) / (16 * s.row_tiles));
   return s;
 }
@@ -112,13 +112,24 @@ static int device_cus() {
 
 // Whether the blocks of a launch of `wgs` workgroups (counted as if every sequence had max_q_len rows)
 // whose rows see at most `max_keys` keys are attended by two groups of wavefronts each
-// (varlen_prefill_two_group_kernel): where a workgroup would have its compute unit to itself, from 9 key
-// tiles on. The meeting of the groups costs 1.2 us, halving the keys saves 0.14 us a tile (rows of
-// 64: 0.18). One request, 64 / 8 heads, us with one group and with two: 64 rows over 512 tokens 15.0, 15.4; 128
-// rows 16.5, 16.0; 128 rows over 2048 40.1, 35.4; 512 rows over 8192 174.9, 154.8; 256 rows of a fresh prompt
-// 10.6, 11.1, 512 rows 15.7, 15.8. (More workgroups than compute units share them two by two as it is.)
+// (varlen_prefill_two_group_kernel): where a workgroup would have its compute unit to itself (and
+// narrow_launch does not take it), from 9 key tiles on. The meeting of the groups costs 1.2 us, halving the
+// keys saves 0.14 us a tile (rows of 64: 0.18). One request, 64 / 8 heads, us with one group and with two: 512
+// rows over 512 tokens 25.3, 24.0, over 2048 54.2, 48.1, over 8192 174.9, 154.8; 512 rows of a fresh prompt 15.7,
+// 15.8. (More workgroups than compute units share them two by two as it is.)
 static bool two_key_groups(int64_t wgs, int64_t max_keys) {
   return kHD != 256 && max_keys > 8 * kKvTile && wgs <= device_cus();
+}
+
+// Whether a launch of `wgs` workgroups of 128 columns runs with 64 columns a workgroup, one column tile
+// per wavefront, instead: where that still leaves at most one workgroup per compute unit. Twice as many
+// wavefronts with half of a key tile's products and exponentials each, 0.70 us a tile instead of 0.94
+// (two groups of wavefronts: 0.80 to 0.85), and less to load, normalise and store around them. One
+// request, us with 128 columns and with 64: 203 rows of a fresh prompt, 16 / 8 heads, 9.2, 7.6; 64 rows, 64 / 8 heads,
+// 5.3, 4.4; 128 rows over 2048 tokens 40.1, 30.5; 32 / 8 heads of 64, 256 rows 7.3, 5.8. With more
+// workgroups the K and V tiles staged twice cost as much as that saves (400 rows, 64 / 8 heads: 200 workgroups).
+static bool narrow_launch(int64_t wgs) {
+  return kHD != 256 && 2 * wgs <= device_cus();
 }
 
 // Key slices for a paged prefill whose row blocks alone would not fill the device, if the longest
@@ -126,13 +137,14 @@ static bool two_key_groups(int64_t wgs, int64_t max_keys) {
 // time, 1 (do not split) unless that is at least 5 % less than unsplit. The estimate, in
 // microseconds, head dim 128 (fits to one request's chunk of 64 to 512 rows over 0 to 32k cached
 // tokens, 64 query / 8 kv heads): a workgroup walks max_kv_len / 64 / n key tiles at 1.0 us each
-// while it has its compute unit to itself and at 1.7 us once the launch has more workgroups than
-// compute units (two share one), times the rounds the launch needs on the device's resident
-// slots; a cut costs the merge launch, 6 us, and a partial row (fp32) written and read back per
-// query row, head and slice at 6 MB/us. (An unsliced launch of so few workgroups runs in two groups of wavefronts by now, at
-// 0.80 to 0.95 us a tile: where that moves the choice the two are within 5 %. One chunk over 30 000 tokens, plain against sliced:
-// 128 rows 379 -> 142 us, 256 rows 394 -> 275 us, 512 rows 480 -> 485 us; 128 rows over 2048 tokens
-// 35 -> 30 us in four slices; 512 rows over 2048 tokens in two slices 48 -> 62 us and 128 rows of a
+// while it has its compute unit to itself (0.75 us with 64 columns, narrow_launch) and at 1.7 us once
+// the launch has more workgroups than compute units (two share one), times the rounds the launch needs
+// on the device's resident slots; a cut costs the merge launch, 6 us, and a partial row (fp32) written and read back per
+// query row, head and slice at 6 MB/us. (An unsliced launch of 129 to 256 workgroups runs in two groups of
+// wavefronts, at 0.95 us a tile: where that moves the choice the two are within 5 %. One chunk over 30 000
+// tokens, plain against sliced:
+// 128 rows 364 -> 148 us, 256 rows 388 -> 269 us, 512 rows 480 -> 485 us; 128 rows over 2048 tokens
+// 30.5 -> 25.5 us in four slices; 512 rows over 2048 tokens in two slices 48 -> 62 us and 128 rows of a
 // fresh prompt in eight 14 -> 29 us, which the estimate rules out.)
 static int32_t prefill_key_slices(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads,
                                   int32_t max_q_len, int64_t max_kv_len) {
@@ -150,7 +162,9 @@ static int32_t prefill_key_slices(int32_t batch, int32_t num_q_heads, int32_t nu
   const double partial_us = (double)batch * max_q_len * num_q_heads * (kHD + 1) * 2.0 * sizeof(float) / 6.0e6;
   auto estimate = [&](int64_t n) {
     const int64_t resident = wgs * n;
-    const double per_tile = resident <= cus ? tile_us : 1.7 * tile_us * (double)((resident + slots - 1) / slots);
+    const double per_tile = narrow_launch(resident) ? 0.75 * tile_us
+                            : resident <= cus       ? tile_us
+                                                    : 1.7 * tile_us * (double)((resident + slots - 1) / slots);
     return tiles / (double)n * per_tile + (n > 1 ? 6.0 + partial_us * (double)n : 0.0);
   };
   const double unsplit = estimate(1);
@@ -251,7 +265,14 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
     LITEKV_REQUIRE(split.workspace != nullptr && aligned16(split.workspace) && split.workspace_bytes >= need,
                    "%s: workspace of %zu bytes needed for %d key slices, got %zu", what, need, slices,
                    split.workspace_bytes);
-    const PrefillShape s = prefill_shape(group, max_q_len);
+    PrefillShape s = prefill_shape(group, max_q_len);
+    // 64 columns a workgroup (narrow_launch); short slices (at most 16 tiles, as far as the block table can
+    // say) up to twice as many: 128 rows, 64 / 8 heads, in 4 slices over 2048 tokens 29.6, 25.5 us, over 8192
+    // 54.7, 56.2, over 30 000 169.7, 181.0.
+    const int64_t wgs = (int64_t)num_kv_heads * s.head_splits * s.row_blocks * slices * batch;
+    const bool narrow = narrow_launch(wgs) || (wgs <= device_cus() && (int64_t)block_table_stride * page_size <=
+                                                                          (int64_t)slices * 16 * kKvTile);
+    if (narrow) s = prefill_shape(group, max_q_len, kTiledWaves);
     LITEKV_REQUIRE((uint64_t)s.row_blocks * slices <= 65535u, "%s: max_q_len %d too large for %d key slices",
                    what, max_q_len, slices);
     float *part_o = static_cast<float *>(split.workspace);
@@ -265,12 +286,20 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
                          context_lens, group, s.head_splits, s.heads_per_wg, s.row_tiles,
                          softmax_scale * kLog2eP, slices);
     };
+    auto by_width = [&](auto mode_tag) {
+      constexpr int MODE = decltype(mode_tag)::value;
+      if (narrow) {
+        launch_slices(varlen_prefill_tiled_kernel<MODE, 1>);
+      } else {
+        launch_slices(varlen_prefill_tiled_kernel<MODE>);
+      }
+    };
     if (format == kKvInt8) {
-      launch_slices(varlen_prefill_tiled_kernel<kPagedPrefillSplitInt8>);
+      by_width(std::integral_constant<int, kPagedPrefillSplitInt8>{});
     } else if (format == kKvFp8) {
-      launch_slices(varlen_prefill_tiled_kernel<kPagedPrefillSplitFp8>);
+      by_width(std::integral_constant<int, kPagedPrefillSplitFp8>{});
     } else {
-      launch_slices(varlen_prefill_tiled_kernel<kPagedPrefillSplit>);
+      by_width(std::integral_constant<int, kPagedPrefillSplit>{});
     }
     int rc2 = check_launch(what);
     if (rc2 != LITEKV_OK) return rc2;
@@ -281,9 +310,9 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
     return check_launch(what);
   }
 #endif  // LITEKV_HD != 256
-  const PrefillShape s = prefill_shape(group, max_q_len);
+  PrefillShape s = prefill_shape(group, max_q_len);
   LITEKV_REQUIRE(s.row_blocks <= 65535u, "%s: max_q_len %d too large", what, max_q_len);
-  const dim3 grid((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch);
+  dim3 grid((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch);
   auto launch = [&](auto mode_tag) {
     constexpr int MODE = decltype(mode_tag)::value;
     auto with = [&](auto kernel, int waves) {
@@ -296,7 +325,14 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
 #if LITEKV_HD != 256
     // (lengths live on the device: behind a history, as many keys as a block-table row can name)
     const int64_t max_keys = context_lens != nullptr ? (int64_t)block_table_stride * page_size : max_q_len;
-    if (two_key_groups((int64_t)grid.x * grid.y * grid.z, max_keys)) {
+    const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
+    if (narrow_launch(wgs)) {
+      s = prefill_shape(group, max_q_len, kTiledWaves);
+      grid = dim3((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch);
+      with(varlen_prefill_tiled_kernel<MODE, 1>, kTiledWaves);
+      return;
+    }
+    if (two_key_groups(wgs, max_keys)) {
       with(varlen_prefill_two_group_kernel<MODE>, 2 * kTiledWaves);
       return;
     }
@@ -376,9 +412,9 @@ static int launch_varlen_prefill(const void *q, int64_t q_token_stride, const vo
   PackedSource packed{static_cast<const half_t *>(k), static_cast<const half_t *>(v),
                       k_token_stride, v_token_stride, seq_starts};
   const int group = num_q_heads / num_kv_heads;
-  const PrefillShape s = prefill_shape(group, max_seq_len);
+  PrefillShape s = prefill_shape(group, max_seq_len);
   LITEKV_REQUIRE(s.row_blocks <= 65535u, "varlen_prefill: max_seq_len %d too large", max_seq_len);
-  const dim3 grid((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch);
+  dim3 grid((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch);
   auto launch = [&](auto kernel, int waves) {
     hipLaunchKernelGGL(kernel, grid, dim3(waves * kWave), 0, static_cast<hipStream_t>(stream),
                        static_cast<const half_t *>(q), q_token_stride, static_cast<half_t *>(out),
@@ -387,7 +423,14 @@ static int launch_varlen_prefill(const void *q, int64_t q_token_stride, const vo
                        softmax_scale * kLog2eP, 1);
   };
 #if LITEKV_HD != 256
-  if (two_key_groups((int64_t)grid.x * grid.y * grid.z, max_seq_len)) {
+  const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
+  if (narrow_launch(wgs)) {
+    s = prefill_shape(group, max_seq_len, kTiledWaves);
+    grid = dim3((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch);
+    launch(varlen_prefill_tiled_kernel<kPackedPrefill, 1>, kTiledWaves);
+    return check_launch("varlen_prefill");
+  }
+  if (two_key_groups(wgs, max_seq_len)) {
     launch(varlen_prefill_two_group_kernel<kPackedPrefill>, 2 * kTiledWaves);
     return check_launch("varlen_prefill");
   }

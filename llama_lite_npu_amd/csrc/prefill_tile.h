@@ -211,7 +211,7 @@ __device__ __forceinline__ void tile_by_rows(uint32_t lds, const half_t *q, int6
 template <int W>
 constexpr int tile_lds_bytes() { return (W == kWideWaves ? 6 : 4) * kTileHalfs * 2; }
 
-template <int MODE, int W, int KG = 1>
+template <int MODE, int W, int KG = 1, int CT = kColTiles>
 __device__ __forceinline__ void prefill_tile_body(
     const uint32_t lds_base, const int block_x, const int block_y, const int block_z, const int grid_y,
     const half_t *__restrict__ q, int64_t q_stride, half_t *__restrict__ out, int64_t out_stride,
@@ -242,6 +242,8 @@ __device__ __forceinline__ void prefill_tile_body(
   // instructions that takes per operand.
   constexpr int kRowsPerWave = kKvTile / W;
   constexpr int kLoads = kRowsPerWave / kRowsPerLoad;
+  static_assert(CT == kColTiles || (CT == 1 && KG == 1 && W == kTiledWaves && !SHARED && kHD != 256),
+                "one column tile a wavefront: a prefill");
   static_assert(KG == 1 || (KG == 2 && W == kTiledWaves && !KSPLIT && !SHARED && kHD != 256), "two key groups: a prefill");
   const int wave_in_wg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kgroup = KG == 2 ? wave_in_wg / W : 0;  // which half of the keys this wavefront attends
@@ -333,7 +335,7 @@ __device__ __forceinline__ void prefill_tile_body(
       t_end = key_slice == key_slices - 1 ? total : (t_end < last_start ? t_end : last_start);
       if (t_end <= t_begin) {
         // Nothing for this slice: its partial rows say so (log-sum-exp -inf, a row of zeros).
-        for (int t = wave * kColTiles; t < wave * kColTiles + kColTiles; ++t) {
+        for (int t = wave * CT; t < wave * CT + CT; ++t) {
           const int head = t / row_tiles;
           const int row = m0 + (t - head * row_tiles) * 16 + n;
           if (head < heads_here && row < q_len) {
@@ -358,7 +360,7 @@ __device__ __forceinline__ void prefill_tile_body(
   static_assert(kHD != 256 || prefill_rows::kLdsBytes <= kOwnLds, "a tile by rows fits a wavefront's part");
   if constexpr (kHD == 256 && FP8) {
     if (!tile_scale(k_mul)) {  // the K scale's doing: the launch looked at softmax_scale itself
-      for (int t = wave * kColTiles; t < (wave + 1) * kColTiles; ++t) {
+      for (int t = wave * CT; t < (wave + 1) * CT; ++t) {
         tile_by_rows<KV, PAGED>(k_lds + wave * kOwnLds, q, q_stride, out, out_stride, paged, packed, b, q_start, q_len,
                                 ctx, m0, t, row_tiles, head0, heads_here, group, h, scale_log2);
       }
@@ -484,8 +486,8 @@ __device__ __forceinline__ void prefill_tile_body(
     static_assert(SHARED || W == kTiledWaves, "the q rows of four wavefronts fit a tile half of K and of V");
     q_lds = ((wave & 2) ? v_lds : k_lds) + (uint32_t)(kTileHalfs * 2 + (wave & 1) * (64 * kHD));
 #pragma unroll
-    for (int u = 0; u < kColTiles; ++u) {
-      const int t = wave * kColTiles + u;
+    for (int u = 0; u < CT; ++u) {
+      const int t = wave * CT + u;
       const int head = t / row_tiles;
       const int row0 = m0 + (t - head * row_tiles) * 16;
       const int hq = h * group + head0 + (head < heads_here ? head : 0);
@@ -507,18 +509,18 @@ __device__ __forceinline__ void prefill_tile_body(
   issue_tile(0);
 
   // ---- this wavefront's columns: tile t = head (t / row_tiles), rows 16 * (t % row_tiles) ..
-  half8_t qf[kColTiles][kKSteps];
-  int q_pos[kColTiles];
-  int out_row[kColTiles];   // packed row index, or -1
-  int out_head[kColTiles];
+  half8_t qf[CT][kKSteps];
+  int q_pos[CT];
+  int out_row[CT];   // packed row index, or -1
+  int out_head[CT];
 #pragma unroll
-  for (int u = 0; u < kColTiles; ++u) {
-    const int t = wave * kColTiles + u;
+  for (int u = 0; u < CT; ++u) {
+    const int t = wave * CT + u;
     bool ok;
     int hq;
     const half_t *qrow;
     if constexpr (SHARED) {
-      const int col = block_y * (16 * kColTiles * W) + 16 * t + n;  // (sequence, head) pair
+      const int col = block_y * (16 * CT * W) + 16 * t + n;  // (sequence, head) pair
       ok = col < prefix.batch * group;
       const int seq = ok ? col / group : 0;
       hq = h * group + (ok ? col - seq * group : 0);
@@ -550,7 +552,7 @@ __device__ __forceinline__ void prefill_tile_body(
       __builtin_amdgcn_s_waitcnt(wait_vm(2 * kLoads));
     }
 #pragma unroll
-    for (int u = 0; u < kColTiles; ++u) {
+    for (int u = 0; u < CT; ++u) {
 #pragma unroll
       for (int kk = 0; kk < kKSteps; ++kk) {
         qf[u][kk] = *(const lds_half8_t *)(uintptr_t)(
@@ -559,14 +561,14 @@ __device__ __forceinline__ void prefill_tile_body(
     }
   }
 
-  float4_t acc[kJTiles][kColTiles];
-  float4_t dsum[kColTiles];
-  float m_run[kColTiles];
+  float4_t acc[kJTiles][CT];
+  float4_t dsum[CT];
+  float m_run[CT];
   // Seed of the score accumulators in the fast tiles: -m_run (divided by k_mul), in all four
   // elements, so that the MFMA result is already the exponent.
-  float4_t seed[kColTiles];
+  float4_t seed[CT];
 #pragma unroll
-  for (int u = 0; u < kColTiles; ++u) {
+  for (int u = 0; u < CT; ++u) {
     m_run[u] = -INFINITY;
     seed[u] = float4_t{0.f, 0.f, 0.f, 0.f};
     dsum[u] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -599,23 +601,23 @@ __device__ __forceinline__ void prefill_tile_body(
     flip = -flip;
   };
 
-  float4_t st[2][kColTiles];
-  half8_t pk[kColTiles];
-  half8_t pk_lo[kColTiles];  // kTwoPartP: what the rounding of pk left
+  float4_t st[2][CT];
+  half8_t pk[CT];
+  half8_t pk_lo[CT];  // kTwoPartP: what the rounding of pk left
 
   // S^T of 32 keys (rows 32 s2 .. +31 of the staged K tile) against this wavefront's columns.
-  auto scores_into = [&](float4_t (&st)[2][kColTiles], int s2, auto seeded_tag) {
+  auto scores_into = [&](float4_t (&st)[2][CT], int s2, auto seeded_tag) {
     constexpr bool SEEDED = decltype(seeded_tag)::value;
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
 #pragma unroll
-      for (int u = 0; u < kColTiles; ++u) st[m][u] = SEEDED ? seed[u] : float4_t{0.f, 0.f, 0.f, 0.f};
+      for (int u = 0; u < CT; ++u) st[m][u] = SEEDED ? seed[u] : float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kk = 0; kk < kKSteps; ++kk) {
         const half8_t a =
             *(const lds_half8_t *)(uintptr_t)(k_addr[kk] + 2u * (32 * s2 + 16 * m) * kHD);
 #pragma unroll
-        for (int u = 0; u < kColTiles; ++u) st[m][u] = mfma_16x16x32(a, qf[u][kk], st[m][u]);
+        for (int u = 0; u < CT; ++u) st[m][u] = mfma_16x16x32(a, qf[u][kk], st[m][u]);
       }
     }
   };
@@ -631,7 +633,7 @@ __device__ __forceinline__ void prefill_tile_body(
     }
   };
   // Column maxima of `st`, in scaled (log2) units.
-  auto column_max_of = [&](const float4_t (&st)[2][kColTiles], int u) {
+  auto column_max_of = [&](const float4_t (&st)[2][CT], int u) {
     float mx = vmax3(st[0][u][0], st[0][u][1], st[0][u][2]);
     mx = vmax3(mx, st[0][u][3], st[1][u][0]);
     mx = vmax3(mx, st[1][u][1], st[1][u][2]);
@@ -652,8 +654,8 @@ __device__ __forceinline__ void prefill_tile_body(
       lo[at + 1] = pl[1];
     }
   };
-  auto exponentials_of = [&](const float4_t (&st)[2][kColTiles], half8_t (&pk)[kColTiles],
-                             half8_t (&pk_lo)[kColTiles], int u) {
+  auto exponentials_of = [&](const float4_t (&st)[2][CT], half8_t (&pk)[CT],
+                             half8_t (&pk_lo)[CT], int u) {
     const float neg_m = -m_run[u];
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
@@ -666,8 +668,8 @@ __device__ __forceinline__ void prefill_tile_body(
     }
   };
   // Fast path: the scores were seeded with -m / k_mul, so they are the exponents up to that factor.
-  auto exponentials_seeded = [&](const float4_t (&st)[2][kColTiles], half8_t (&pk)[kColTiles],
-                                 half8_t (&pk_lo)[kColTiles], int u) {
+  auto exponentials_seeded = [&](const float4_t (&st)[2][CT], half8_t (&pk)[CT],
+                                 half8_t (&pk_lo)[CT], int u) {
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
 #pragma unroll
@@ -686,9 +688,9 @@ __device__ __forceinline__ void prefill_tile_body(
   // True if any probability of the sub-tile exceeds 2^kMaxP (or is not finite): the running maximum
   // is then too low for these keys and the sub-tile has to be redone with a rescale. Probabilities
   // are non-negative, so their fp16 bit patterns order like their values.
-  auto overflowed = [&](const half8_t (&pk)[kColTiles]) -> bool {
+  auto overflowed = [&](const half8_t (&pk)[CT]) -> bool {
     typedef _Float16 half8v __attribute__((ext_vector_type(8)));
-    const half8v mx8 = __builtin_elementwise_max(pk[0], pk[1]);
+    const half8v mx8 = CT == 1 ? pk[0] : __builtin_elementwise_max(pk[0], pk[CT - 1]);
     typedef _Float16 half4v __attribute__((ext_vector_type(4)));
     const half4v lo4 = __builtin_shufflevector(mx8, mx8, 0, 1, 2, 3);
     const half4v hi4 = __builtin_shufflevector(mx8, mx8, 4, 5, 6, 7);
@@ -702,7 +704,7 @@ __device__ __forceinline__ void prefill_tile_body(
   // O^T += V^T . P^T,  l += 1^T . P^T for keys 32 s2 .. +31 of the staged V tile.
   auto accumulate_sub = [&](int s2) {
 #pragma unroll
-    for (int u = 0; u < kColTiles; ++u) dsum[u] = mfma_p(ones, pk[u], pk_lo[u], dsum[u]);
+    for (int u = 0; u < CT; ++u) dsum[u] = mfma_p(ones, pk[u], pk_lo[u], dsum[u]);
 #pragma unroll
     for (int j = 0; j < kJTiles; ++j) {
       const uint32_t at = v_addr[j] + 2u * 32 * s2 * kHD;
@@ -712,7 +714,7 @@ __device__ __forceinline__ void prefill_tile_body(
       const short8_t both = short8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       const half8_t a = __builtin_bit_cast(half8_t, both);
 #pragma unroll
-      for (int u = 0; u < kColTiles; ++u) acc[j][u] = mfma_p(a, pk[u], pk_lo[u], acc[j][u]);
+      for (int u = 0; u < CT; ++u) acc[j][u] = mfma_p(a, pk[u], pk_lo[u], acc[j][u]);
     }
   };
   // V^T fragment j (A operand: d rows 16j.., keys 32 s2 + {4g..4g+3, 16+4g..}) of the staged tile.
@@ -727,8 +729,8 @@ __device__ __forceinline__ void prefill_tile_body(
   auto scores_sub = [&](int s2) { scores_into(st, s2, std::false_type{}); };
   auto column_max = [&](int u) { return column_max_of(st, u); };
   auto exponentials = [&](int u) { exponentials_of(st, pk, pk_lo, u); };
-  float4_t st1[2][kColTiles];  // scores of the second half of a fast tile
-  half8_t pk1[kColTiles], pk1_lo[kColTiles];
+  float4_t st1[2][CT];  // scores of the second half of a fast tile
+  half8_t pk1[CT], pk1_lo[CT];
 
   // Publishes tile kt (already requested) and requests tile kt + 1 into the other half.
   auto sync_and_prefetch = [&](int kt, bool issue_next = true) {
@@ -802,7 +804,7 @@ __device__ __forceinline__ void prefill_tile_body(
       if (key0 >= kv_end) break;  // nothing visible in the second half
       scores_sub(s2);
 #pragma unroll
-      for (int u = 0; u < kColTiles; ++u) {
+      for (int u = 0; u < CT; ++u) {
         mask_sub(u, key0);
         const float m_new = vmax2(m_run[u], column_max(u) - (float)kMaxBias);
         const float alpha = fast_exp2(m_run[u] - m_new);
@@ -834,11 +836,11 @@ __device__ __forceinline__ void prefill_tile_body(
         if (MASKED && key0 >= kv_end) break;
         scores_into(st, s2, std::true_type{});
         if (MASKED) {
-          mask_sub(0, key0);
-          mask_sub(1, key0);
+#pragma unroll
+          for (int u = 0; u < CT; ++u) mask_sub(u, key0);
         }
-        exponentials_seeded(st, pk, pk_lo, 0);
-        exponentials_seeded(st, pk, pk_lo, 1);
+#pragma unroll
+        for (int u = 0; u < CT; ++u) exponentials_seeded(st, pk, pk_lo, u);
         if (overflowed(pk)) return 1 + s2;
         accumulate_sub(s2);
       }
@@ -874,7 +876,7 @@ __device__ __forceinline__ void prefill_tile_body(
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
 #pragma unroll
-        for (int u = 0; u < kColTiles; ++u) st[m][u] = st1[m][u] = seed[u];
+        for (int u = 0; u < CT; ++u) st[m][u] = st1[m][u] = seed[u];
       }
       __builtin_amdgcn_sched_barrier(0);
       // Region 2: the first half's MFMAs; each fragment register takes the second half's
@@ -884,7 +886,7 @@ __device__ __forceinline__ void prefill_tile_body(
 #pragma unroll
       for (int i = 0; i < kJTiles; ++i) {
 #pragma unroll
-        for (int u = 0; u < kColTiles; ++u) st[i & 1][u] = mfma_16x16x32(kf[i], qf[u][i >> 1], st[i & 1][u]);
+        for (int u = 0; u < CT; ++u) st[i & 1][u] = mfma_16x16x32(kf[i], qf[u][i >> 1], st[i & 1][u]);
         kf1[i] = load_kfrag(1, i);
         if constexpr (!FP8) {
           if (i % kIssueEvery == kIssueEvery - 1) issue_rows(i / kIssueEvery);
@@ -892,7 +894,7 @@ __device__ __forceinline__ void prefill_tile_body(
       }
 #pragma unroll
       for (int i = 0; i < kJTiles; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, CT, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         if (!FP8 && i % kIssueEvery == kIssueEvery - 1) __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
       }
@@ -903,23 +905,23 @@ __device__ __forceinline__ void prefill_tile_body(
       // them, the scheduler started them late and a tile took 3 % longer.)
       half8_t vf[kJTiles];
       if constexpr (kHD == 256) {
-        exponentials_seeded(st, pk, pk_lo, 0);
-        exponentials_seeded(st, pk, pk_lo, 1);
+#pragma unroll
+        for (int u = 0; u < CT; ++u) exponentials_seeded(st, pk, pk_lo, u);
       }
 #pragma unroll
       for (int i = 0; i < kJTiles; ++i) {
 #pragma unroll
-        for (int u = 0; u < kColTiles; ++u) st1[i & 1][u] = mfma_16x16x32(kf1[i], qf[u][i >> 1], st1[i & 1][u]);
+        for (int u = 0; u < CT; ++u) st1[i & 1][u] = mfma_16x16x32(kf1[i], qf[u][i >> 1], st1[i & 1][u]);
         vf[i] = load_vfrag(i, 0);
       }
       if constexpr (kHD != 256) {
-        exponentials_seeded(st, pk, pk_lo, 0);
-        exponentials_seeded(st, pk, pk_lo, 1);
+#pragma unroll
+        for (int u = 0; u < CT; ++u) exponentials_seeded(st, pk, pk_lo, u);
       }
       const bool over_a = overflowed(pk);
 #pragma unroll
       for (int i = 0; i < kJTiles; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, CT, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
         __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
       }
@@ -928,38 +930,38 @@ __device__ __forceinline__ void prefill_tile_body(
       // fragment register takes the second half's fragment as soon as its MFMAs are issued.
       half8_t vf2[kJTiles];
       if constexpr (kHD == 256) {
-        exponentials_seeded(st1, pk1, pk1_lo, 0);
-        exponentials_seeded(st1, pk1, pk1_lo, 1);
+#pragma unroll
+        for (int u = 0; u < CT; ++u) exponentials_seeded(st1, pk1, pk1_lo, u);
       }
 #pragma unroll
-      for (int u = 0; u < kColTiles; ++u) dsum[u] = mfma_p(ones, pk[u], pk_lo[u], dsum[u]);
+      for (int u = 0; u < CT; ++u) dsum[u] = mfma_p(ones, pk[u], pk_lo[u], dsum[u]);
 #pragma unroll
       for (int j = 0; j < kJTiles; ++j) {
 #pragma unroll
-        for (int u = 0; u < kColTiles; ++u) acc[j][u] = mfma_p(vf[j], pk[u], pk_lo[u], acc[j][u]);
+        for (int u = 0; u < CT; ++u) acc[j][u] = mfma_p(vf[j], pk[u], pk_lo[u], acc[j][u]);
         vf2[j] = load_vfrag(j, 1);
       }
       if constexpr (kHD != 256) {
-        exponentials_seeded(st1, pk1, pk1_lo, 0);
-        exponentials_seeded(st1, pk1, pk1_lo, 1);
+#pragma unroll
+        for (int u = 0; u < CT; ++u) exponentials_seeded(st1, pk1, pk1_lo, u);
       }
       const bool over_b = overflowed(pk1);
 #pragma unroll
       for (int i = 0; i < kJTiles; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, kTwoPartP ? 4 : 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, kTwoPartP ? 2 * CT : CT, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
         __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
       }
-      __builtin_amdgcn_sched_group_barrier(0x008, kTwoPartP ? 4 : 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, kTwoPartP ? 2 * CT : CT, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
       if (over_b) return 2;
       // Block 3: second product of the second half.
 #pragma unroll
-      for (int u = 0; u < kColTiles; ++u) dsum[u] = mfma_p(ones, pk1[u], pk1_lo[u], dsum[u]);
+      for (int u = 0; u < CT; ++u) dsum[u] = mfma_p(ones, pk1[u], pk1_lo[u], dsum[u]);
 #pragma unroll
       for (int j = 0; j < kJTiles; ++j) {
 #pragma unroll
-        for (int u = 0; u < kColTiles; ++u) acc[j][u] = mfma_p(vf2[j], pk1[u], pk1_lo[u], acc[j][u]);
+        for (int u = 0; u < CT; ++u) acc[j][u] = mfma_p(vf2[j], pk1[u], pk1_lo[u], acc[j][u]);
       }
     }
     return 0;
@@ -998,7 +1000,7 @@ __device__ __forceinline__ void prefill_tile_body(
     const uint32_t give = lds_base + (uint32_t)wave_in_wg * kHandBytes;
     const uint32_t take = lds_base + (uint32_t)(wave_in_wg ^ W) * kHandBytes;
 #pragma unroll
-    for (int u = 0; u < kColTiles; ++u) {
+    for (int u = 0; u < CT; ++u) {
       if (u != kgroup) {
 #pragma unroll
         for (int j = 0; j < kJTiles; ++j) *(lds_float4_t *)(uintptr_t)(give + 1024u * j + 16u * lane) = acc[j][u];
@@ -1027,7 +1029,7 @@ __device__ __forceinline__ void prefill_tile_body(
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int t = wave * kColTiles + kgroup;
+    const int t = wave * CT + kgroup;
     const int head = t / row_tiles;
     const int row0 = m0 + (t - head * row_tiles) * 16;
     half_t *o_tile = out + (int64_t)(q_start + row0) * out_stride + (int64_t)(h * group + head0 + head) * kHD + 8 * slot;
@@ -1046,9 +1048,9 @@ __device__ __forceinline__ void prefill_tile_body(
     constexpr int kOutPitch = 2 * kHD + 16;  // bytes; at 128: 68 dwords, a half-wave's 8-byte writes hit 64 banks
     __syncthreads();                              // every wavefront is done reading the last tile
     const uint32_t mine = kHD == 256 ? k_lds + (uint32_t)wave * kOwnLds
-                                     : ((wave & 2) ? v_lds : k_lds) + (uint32_t)((wave & 1) * kColTiles * 16 * kOutPitch);
+                                     : ((wave & 2) ? v_lds : k_lds) + (uint32_t)((wave & 1) * CT * 16 * kOutPitch);
 #pragma unroll
-    for (int u = 0; u < kColTiles; ++u) {
+    for (int u = 0; u < CT; ++u) {
       const float inv = v_scale / dsum[u][0];
       const uint32_t at = mine + (uint32_t)((u * 16 + n) * kOutPitch + 8 * g);
 #pragma unroll
@@ -1061,14 +1063,14 @@ __device__ __forceinline__ void prefill_tile_body(
     // lane l carries chunk l % kChunks of row l / kChunks + kRowsPerLoad * step
     const int chunk = slot, r4 = r_loc;
     // Head dim 256: not 0 (but not a number) once an output of the tile was not finite
-    float odd[kColTiles] = {};
+    float odd[CT] = {};
 #pragma unroll
-    for (int u = 0; u < kColTiles; ++u) {
+    for (int u = 0; u < CT; ++u) {
 #pragma unroll
       for (int step = 0; step < kLoadsPerWave; ++step) {
         const int r = kRowsPerLoad * step + r4;
         const half8_t row = *(const lds_half8_t *)(uintptr_t)(mine + (uint32_t)((u * 16 + r) * kOutPitch + 16 * chunk));
-        const int t = wave * kColTiles + u;
+        const int t = wave * CT + u;
         const int head = t / row_tiles;
         const int qrow_idx = m0 + (t - head * row_tiles) * 16 + r;
         if (head < heads_here && qrow_idx < q_len) {
@@ -1088,13 +1090,12 @@ __device__ __forceinline__ void prefill_tile_body(
       // written. An infinite value times a probability of 0 -- of a row that may not see its key, or
       // the second part of a probability that fp16 holds exactly -- is NaN above and must not be.
       // (Looking is a v_dot2_f32_f16 for two outputs on the way to their store: nothing to measure.)
-      static_assert(kColTiles == 2, "");
-      if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd[0] + odd[1] != 0.f) != 0, false)) {
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd[0] + odd[CT - 1] != 0.f) != 0, false)) {
         __builtin_amdgcn_s_waitcnt(wait_vm(0));  // the rows' first stores come first
 #pragma unroll 1
-        for (int u = 0; u < kColTiles; ++u) {
+        for (int u = 0; u < CT; ++u) {
           tile_by_rows<FP8 ? KV : kKvF16, PAGED>(mine, q, q_stride, out, out_stride, paged, packed, b, q_start, q_len, ctx,
-                                                 m0, wave * kColTiles + u, row_tiles, head0, heads_here, group, h, scale_log2);
+                                                 m0, wave * CT + u, row_tiles, head0, heads_here, group, h, scale_log2);
         }
       }
     }
@@ -1113,7 +1114,7 @@ __device__ __forceinline__ void prefill_tile_body(
     const uint32_t mine = k_lds + (uint32_t)(wave * 16 * kPartPitch);
     typedef __attribute__((address_space(3))) float4_t lds_float4_t;
 #pragma unroll
-    for (int u = 0; u < kColTiles; ++u) {
+    for (int u = 0; u < CT; ++u) {
       const float inv = v_scale / dsum[u][0];
       // the partial row of this lane's column (the same in its four lane groups), or -1
       const int piece = SHARED ? block_z : key_slice;  // which partial of the row this block writes
@@ -1149,7 +1150,7 @@ __device__ __forceinline__ void prefill_tile_body(
     return;
   }
 #pragma unroll
-  for (int u = 0; u < kColTiles; ++u) {
+  for (int u = 0; u < CT; ++u) {
     const float inv = v_scale / dsum[u][0];
     if (out_row[u] >= 0) {
       half_t *o = out + (int64_t)out_row[u] * out_stride + (int64_t)out_head[u] * kHD + 4 * g;
@@ -1163,7 +1164,9 @@ __device__ __forceinline__ void prefill_tile_body(
   }
 }
 
-template <int MODE>
+// CT: column tiles per wavefront. One instead of two, 64 score columns a workgroup, for launches that would
+// leave most of the device idle (see narrow_launch in paged_prefill.hip). Bound by the chain of its few key tiles.
+template <int MODE, int CT = kColTiles>
 __global__ __launch_bounds__(kTiledWaves *kWave, kWgPerCu) void varlen_prefill_tiled_kernel(
     const half_t *__restrict__ q, int64_t q_stride, half_t *__restrict__ out, int64_t out_stride,
     PagedSource paged, PackedSource packed, PrefixTask prefix,
@@ -1175,13 +1178,13 @@ __global__ __launch_bounds__(kTiledWaves *kWave, kWgPerCu) void varlen_prefill_t
                 MODE == kPagedPrefillSplitInt8) {
     // blockIdx.y = row block * key_slices + slice: the slices of a block are neighbours
     const int by = (int)blockIdx.y / key_slices;
-    prefill_tile_body<MODE, kTiledWaves>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, by,
+    prefill_tile_body<MODE, kTiledWaves, 1, CT>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, by,
                                (int)blockIdx.z, (int)gridDim.y / key_slices, q, q_stride, out, out_stride,
                                paged, packed, prefix, q_starts_or_cu, q_lens_or_null, context_lens, group,
                                head_splits, heads_per_wg, row_tiles, scale_log2,
                                (int)blockIdx.y - by * key_slices, key_slices);
   } else {
-    prefill_tile_body<MODE, kTiledWaves>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, (int)blockIdx.y,
+    prefill_tile_body<MODE, kTiledWaves, 1, CT>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, (int)blockIdx.y,
                                (int)blockIdx.z, (int)gridDim.y, q, q_stride, out, out_stride, paged, packed,
                                prefix, q_starts_or_cu, q_lens_or_null, context_lens, group, head_splits,
                                heads_per_wg, row_tiles, scale_log2);

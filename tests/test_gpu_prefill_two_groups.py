@@ -1,7 +1,8 @@
-"""GPU: a prefill of few workgroups whose rows may see over 512 keys is attended by two groups of
-wavefronts per block, each over half of its key tiles. Blocks of one tile (the first group has none)
-up to odd and even numbers of them, ragged last blocks and tiles, every pool format, both head dims,
-paged and packed: against float64 arithmetic, and against the one-group launch of the same rows."""
+"""GPU: a prefill of at most as many workgroups as compute units whose rows may see over 512 keys is
+attended by two groups of wavefronts per block, each over half of its key tiles; one of at most half as many
+workgroups with one column tile per wavefront. Blocks of one tile (the first group has none) up to odd
+and even numbers of them, ragged last blocks and tiles, every pool format, both head dims, paged and
+packed, in a batch (two groups) and sequence by sequence (one column tile): against float64 arithmetic."""
 
 import pytest
 import torch
@@ -52,31 +53,34 @@ def test_two_groups(fmt, head_dim, hq, hkv):
         values = (pool if fmt == "int8" else pool.view(torch.float8_e4m3fn)).double() * 0.035
     q = torch.randn((sum(rows), hq, head_dim), generator=gen, dtype=torch.float16, device=DEV)
     scale = head_dim ** -0.5
-    out, one = torch.empty_like(q), torch.empty_like(q)
+    one = torch.empty_like(q)
     first = 0
     for b, (r, c) in enumerate(SHAPES):
-        cu = torch.tensor([0, r], dtype=torch.int32, device=DEV)
-        ctx_b = torch.tensor([c], dtype=torch.int32, device=DEV)
         part = slice(first, first + r)
-        # the row of the whole table names over 512 keys; its own pages alone may not
-        ops.paged_prefill(q[part], pool, table[b:b + 1], cu, ctx_b, r, scale, out=out[part], kv_scales=scales, key_slices=1)
-        own = table[b:b + 1, :min(pages[b], 32)].contiguous()
-        if pages[b] <= 32:
-            ops.paged_prefill(q[part], pool, own, cu, ctx_b, r, scale, out=one[part], kv_scales=scales, key_slices=1)
-        else:
-            one[part] = out[part]
+        ops.paged_prefill(q[part], pool, table[b:b + 1], torch.tensor([0, r], dtype=torch.int32, device=DEV),
+                          torch.tensor([c], dtype=torch.int32, device=DEV), r, scale, out=one[part], kv_scales=scales,
+                          key_slices=1)
         first += r
-    cu = torch.tensor([0] + rows, dtype=torch.int32).cumsum(0).to(torch.int32).to(DEV)
-    batch = ops.paged_prefill(q, pool, table, cu, torch.tensor(ctx, dtype=torch.int32, device=DEV), max(rows), scale,
-                              kv_scales=scales, key_slices=1)
+    # the batch, as often as makes it more than half as many workgroups as there are compute units
+    splits = -(-(hq // hkv) // 8)
+    block_rows = 16 * (8 // -(-(hq // hkv) // splits))
+    wgs = hkv * splits * -(-max(rows) // block_rows) * len(rows)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    copies = cus // 2 // wgs + 1
+    assert cus < 2 * wgs * copies <= 2 * cus
+    cu = torch.tensor([0] + rows * copies, dtype=torch.int32).cumsum(0).to(torch.int32).to(DEV)
+    batch = ops.paged_prefill(q.repeat(copies, 1, 1), pool, table.repeat(copies, 1), cu,
+                              torch.tensor(ctx * copies, dtype=torch.int32, device=DEV), max(rows), scale, kv_scales=scales,
+                              key_slices=1)
     torch.cuda.synchronize()
-    assert torch.equal(batch, out)
-    assert_attention_close(out, one.float().cpu().numpy(), "one group")
+    for out in batch.split(sum(rows)):
+        assert torch.equal(out, batch[:sum(rows)])
     first = 0
     for b, (r, c) in enumerate(SHAPES):
         slot = torch.cat([table[b, t // 16, None].long() * 16 + t % 16 for t in range(r + c)])
-        ref = _reference(q[first:first + r], values[slot, :hkv], values[slot, hkv:], c, scale)
-        assert_attention_close(out[first:first + r], ref.numpy(), f"rows {r} ctx {c}")
+        ref = _reference(q[first:first + r], values[slot, :hkv], values[slot, hkv:], c, scale).numpy()
+        assert_attention_close(batch[first:first + r], ref, f"two groups, rows {r} ctx {c}")
+        assert_attention_close(one[first:first + r], ref, f"one column tile, rows {r} ctx {c}")
         first += r
 
 
