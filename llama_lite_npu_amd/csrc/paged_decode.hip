@@ -56,8 +56,8 @@ constexpr int kVPitch = 128 + 8;     // fp16 elements per staged V row (272 byte
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
-// Pages a wavefront keeps in flight in registers (K fragments and V rows of DEPTH pages are
-// requested before the oldest one is consumed).
+// Pages a wavefront of the balanced schedule keeps in flight in registers (K fragments and V rows of
+// DEPTH pages are requested before the oldest one is consumed).
 #ifndef LITEKV_DECODE_DEPTH
 #define LITEKV_DECODE_DEPTH 2
 #endif
@@ -619,8 +619,8 @@ extern __shared__ __attribute__((aligned(16))) half_t split_vstage[];  // [waves
 //
 // DEEP: two steps' pages in flight instead of one, requested again after the step instead of in the
 // middle of it, once the scores are under way and V is in LDS. Four pages' registers leave two
-// wavefronts per SIMD where the other form has three, or four over codes, and every launch requests four
-// pages however few its splits have: see the rule in launch_split. Both give the same bits.
+// wavefronts per SIMD where the other form has three, and every split requests four pages however few
+// it has: see the rule in launch_split. Both give the same bits.
 //
 // The second launch bound keeps the accumulators in ordinary registers. Without one the compiler
 // expects a wavefront to be alone with all 512, puts every MFMA result into AGPRs and copies all 32
@@ -1659,9 +1659,10 @@ static int launch_split(const DecodeArgs &a, int32_t max_splits, int32_t min_pag
   const int64_t row_pages = (int64_t)a.block_table_stride << page_shift_of(a.page_size);
   // Two steps' pages in flight (DEEP) while the launch has half a wavefront per SIMD of an fp16 pool, one
   // of a pool of codes (whose pages take half the registers and requests, and more work per byte), and
-  // a split can have two pages at all. Geometric means over 239 / 209 shapes, 64 / 8 heads, of the time
-  // against one step's pages: 512 wavefronts 0.94 to 0.99 (codes 0.87 to 0.94), 1024: 1.05 (0.96 to
-  // 1.00), 2048: 1.04 to 1.05 (1.03 to 1.09), 4096: 1.06 to 1.10 (1.02 to 1.05).
+  // a split can have two pages at all. Time against a page per step in the same registers, geometric
+  // means over 239 shapes of fp16 pools (209 of codes), 64 / 8 heads: DEEP 256 wavefronts 0.88 to 0.96 (0.87 to
+  // 0.94), 512: 0.96 to 1.01 (0.87 to 0.95), 1024: 1.06 to 1.09 (0.96 to 1.01), 2048: 1.07 to 1.10 (0.98 to
+  // 0.99); one step's pages 1024: 1.00 to 1.02, 2048: 1.02 to 1.04 (0.91 to 0.96).
   const bool deep = units <= (fp8_scales != nullptr ? 1024 : 512) && row_pages > max_splits;
   const size_t lds = (size_t)waves * 2 * kPageSize * kVPitch * sizeof(half_t);
   // Sequences from the longest down once the launch has more workgroups than the device holds at
