@@ -409,7 +409,7 @@ def decode_schedule(batch: int, num_kv_heads: int, max_pages: int, total_pages: 
     1 = one wavefront per (sequence, kv head) in one launch, 4 / 8 / 16 = that many splits per
     sequence and the merge launch: the smallest of ``decode_schedule_estimates``. Choosing by this
     rule is 1.1 to 2.6 % slower on average than always choosing the fastest schedule over the shapes of
-    a head layout and pool format, 19 to 36 % at worst (``tune_decode_schedule``). ``current``: the schedule
+    a head layout and pool format, 19 to 43 % at worst (``tune_decode_schedule``). ``current``: the schedule
     in use; another must be estimated ``hysteresis`` times faster to replace it. ``head_dim`` tells rows
     of 64 fp16 elements from 128 codes, which ``token_bytes`` alone does not; ``chunks``: a plan's own
     count, see ``decode_schedule_estimates``."""
