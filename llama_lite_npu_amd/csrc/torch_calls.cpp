@@ -3,9 +3,11 @@
 // layer against 12 us of kernels), and there most of a call was Python: some sixty attribute reads
 // on tensors and twenty conversions by ctypes. One prompt of 203 tokens, 28 layers, 16 / 8 heads: 543 -> 359 us.
 //
-// A function takes what it recognises as a plain, well-formed call and says so; anything else
-// (another dtype, a shape that does not fit, a tensor subclass, an error of the library) it leaves
-// alone and answers None, and the wrapper goes through its own checks, conversions and messages.
+// A function takes what it recognises as a plain, well-formed call; anything else (another dtype, a
+// shape that does not fit, a tensor subclass) it leaves alone and answers None, and the wrapper goes
+// through its own checks, conversions and messages. None says that the library was not called: what it
+// answered goes back as it is, since a launch error is reported after the launch (and may be an older
+// one of the thread), and the epilogue, which works in place, must not run twice.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -90,7 +92,7 @@ int unlocked(Call call) {
 }
 
 // (q, k, v, slot_mapping, kv_pool, q_norm_weight, k_norm_weight, cos, sin, eps, kv_scales, stream)
-// -> True if launched, else None
+// -> True if launched, the library's status if that is not 0, or None
 PyObject *qk_norm_rope_append(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 12) Py_RETURN_NONE;
   try {
@@ -146,16 +148,17 @@ PyObject *qk_norm_rope_append(PyObject *, PyObject *const *a, Py_ssize_t n) {
                                                  (int32_t)hq, (int32_t)pool.hkv, (int32_t)d, pool.slots, (float)eps, stream);
       }
     });
-    if (rc != 0) Py_RETURN_NONE;
+    if (rc != 0) return PyLong_FromLong(rc);
     Py_RETURN_TRUE;
   } catch (...) {  // (a tensor without storage, under a transform: the wrapper meets the same and says so)
+    PyErr_Clear();
     Py_RETURN_NONE;
   }
 }
 
 // (q, kv_pool, block_table, cu_q_lens, context_lens, max_q_len, softmax_scale, page_size, kv_scales,
-//  max_kv_len or None, stream) -> the output, or None. A launch that is to be cut along its keys is
-// left to the wrapper as well.
+//  max_kv_len or None, stream) -> the output, or the library's status if that is not 0, or None. A launch
+// that is to be cut along its keys is left to the wrapper as well.
 PyObject *paged_prefill(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 11) Py_RETURN_NONE;
   try {
@@ -197,6 +200,7 @@ PyObject *paged_prefill(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const int32_t *ctxp = static_cast<const int32_t *>(address(ctx));
     const float *scales = static_cast<const float *>(pool.scales);
     void *op = address(&out);
+    PyObject *result = THPVariable_Wrap(std::move(out));  // (before the launch: it may throw)
     const int32_t ts = (int32_t)table->stride(0);
     const int64_t pages = pool.slots / page;
     const int rc = unlocked([&] {
@@ -214,9 +218,11 @@ PyObject *paged_prefill(PyObject *, PyObject *const *a, Py_ssize_t n) {
                                            stream);
       }
     });
-    if (rc != 0) Py_RETURN_NONE;
-    return THPVariable_Wrap(std::move(out));
+    if (rc == 0) return result;
+    Py_DECREF(result);
+    return PyLong_FromLong(rc);
   } catch (...) {
+    PyErr_Clear();
     Py_RETURN_NONE;
   }
 }

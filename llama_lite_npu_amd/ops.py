@@ -194,9 +194,13 @@ def qk_norm_rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, slot_
     k [T, Hkv, D] on its way into the pool, plus the append of v: one launch for the reference's
     skip_rmsnorm x2 + rope_emb_forward + cat + update_kv_buffer. cos / sin are [T, >= D/2] rows of
     each token's position. An fp8 pool (with its ``kv_scales``) receives the quantised rows. Returns q."""
-    if q.is_cuda and _lib.calls().qk_norm_rope_append(q, k, v, slot_mapping, kv_pool, q_norm_weight, k_norm_weight,
-                                                      cos, sin, rms_eps, kv_scales, _stream()):
-        return q
+    if q.is_cuda:
+        done = _lib.calls().qk_norm_rope_append(q, k, v, slot_mapping, kv_pool, q_norm_weight, k_norm_weight, cos, sin,
+                                                rms_eps, kv_scales, _stream())
+        if done is not None:
+            if done is not True:        # a status: q may have been written all the same, so never a second time
+                _lib.check(done)
+            return q
     # (not a plain call: found out below)
     _dev_half("q", q), _dev_half("k", k), _dev_half("v", v)
     slots, hkv, d, _, _ = pool_geometry(kv_pool, 1)
@@ -866,6 +870,8 @@ def paged_prefill(q: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Ten
         done = _lib.calls().paged_prefill(q, kv_pool, block_table, cu_q_lens, context_lens, max_q_len, softmax_scale,
                                           page_size, kv_scales, max_kv_len, _stream())
         if done is not None:
+            if type(done) is int:
+                _lib.check(done)
             return done
     # (not a plain call, or one that is cut along its keys)
     _dev_half("q", q)

@@ -125,3 +125,56 @@ def test_a_plain_call_is_taken():
     out = calls.paged_prefill(st["q"], st["pool"], st["table"], st["cu"], None, 37, st["scale"], 16, None, 37, stream)
     torch.cuda.synchronize()
     assert out.shape == st["q"].shape and out.dtype == torch.float16 and bool(torch.isfinite(out).all())
+
+
+class _LaunchError:
+    """Native calls that reached the library and brought back a launch status."""
+
+    def __init__(self):
+        self.calls = 0
+
+    def _status(self, *a):
+        self.calls += 1
+        return 2
+
+    qk_norm_rope_append = paged_prefill = _status
+
+
+class _Library:
+    """Stands for liblitekv: any entry point but litekv_last_error is a second launch."""
+
+    def __getattr__(self, name):
+        raise AssertionError(f"{name} called after the native call had reached the library")
+
+    @staticmethod
+    def litekv_last_error():
+        return b"launch failed"
+
+
+def test_a_launch_error_is_raised_and_nothing_is_launched_again(monkeypatch):
+    native = _LaunchError()
+    monkeypatch.setattr(_lib, "calls", lambda: native)
+    monkeypatch.setattr(_lib, "load", lambda: _Library())
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    q = type("OnTheGpu", (), {"is_cuda": True, "dtype": torch.float16})()
+    with pytest.raises(_lib.LiteKVError, match="status 2: launch failed"):
+        ops.qk_norm_rope_append(q, q, q, None, q)
+    with pytest.raises(_lib.LiteKVError, match="status 2: launch failed"):
+        ops.paged_prefill(q, q, None, None, None, 1, 1.0)
+    assert native.calls == 2
+
+
+@pytest.mark.gpu
+def test_a_status_of_the_library_comes_back():
+    print("native calls: statuses", flush=True)
+    st = _state("f16", 128)
+    CHANGES["misaligned q"](st)         # the library's own check
+    calls, before = _lib.calls(), st["q"].clone()
+    stream = torch.cuda.current_stream().cuda_stream
+    for status in (calls.qk_norm_rope_append(st["q"], st["k"], st["v"], st["slots"], st["pool"], st["qw"], st["kw"], st["cos"],
+                                             st["sin"], 1e-6, None, stream),
+                   calls.paged_prefill(st["q"], st["pool"], st["table"], st["cu"], None, 37, st["scale"], 16, None, 37, stream)):
+        assert type(status) is int and status == 1
+        with pytest.raises(_lib.LiteKVError, match="align"):
+            _lib.check(status)
+    assert torch.equal(st["q"], before)
