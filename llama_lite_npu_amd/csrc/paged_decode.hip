@@ -296,27 +296,29 @@ __device__ __forceinline__ void attend_page(HeadState &st, const PageRegsQ8<KV> 
 // maximum over the lane groups, exponentials, second product); here the two pages' chains run
 // beside each other, with one maximum, one look at the reference maximum and half as many MFMAs in
 // the second product, whose k index runs over both pages: k = 8g + i is token 4g + i of page p for
-// i < 4 and of page p + 1 behind. `stage_v` writes 32 rows.
-template <typename StageV, typename Refill>
-__device__ __forceinline__ void attend_pair_core(HeadState &st, const half8_t (&ka)[4], const half8_t (&kb)[4],
-                                                 const half8_t (&qf)[4], const half_t *vt_lane, int p, int end,
-                                                 int g, float scale_log2, StageV stage_v, Refill refill) {
+// i < 4 and of page p + 1 behind. `keys(u)` gives page u's K fragments, `stage_v(u, tail)` writes its
+// V rows; page u's registers are free where `refill(u)` is called, before page 1's are waited for.
+template <typename Keys, typename StageV, typename Refill>
+__device__ __forceinline__ void attend_pair_core(HeadState &st, const half8_t (&qf)[4], const half_t *vt_lane, int p,
+                                                 int end, int g, float scale_log2, Keys keys, StageV stage_v,
+                                                 Refill refill) {
   const bool tail = (p + 2) * kPageSize > end;  // wavefront-uniform
   wave_lds_fence();
-  stage_v(tail);
-  wave_lds_fence();
-
-  const float4_t zero = float4_t{0.f, 0.f, 0.f, 0.f};
-  float4_t s[2] = {mfma_16x16x32(ka[0], qf[0], zero), mfma_16x16x32(kb[0], qf[0], zero)};
-  float4_t s1[2] = {mfma_16x16x32(ka[kKSteps / 2], qf[kKSteps / 2], zero),
-                    mfma_16x16x32(kb[kKSteps / 2], qf[kKSteps / 2], zero)};
-  if constexpr (kKSteps == 4) {
-    s[0] = mfma_16x16x32(ka[1], qf[1], s[0]);
-    s[1] = mfma_16x16x32(kb[1], qf[1], s[1]);
-    s1[0] = mfma_16x16x32(ka[3], qf[3], s1[0]);
-    s1[1] = mfma_16x16x32(kb[3], qf[3], s1[1]);
+  float4_t s[2], s1[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    stage_v(u, tail);
+    half8_t kf[4];
+    keys(u, kf);
+    s[u] = mfma_16x16x32(kf[0], qf[0], float4_t{0.f, 0.f, 0.f, 0.f});
+    s1[u] = mfma_16x16x32(kf[kKSteps / 2], qf[kKSteps / 2], float4_t{0.f, 0.f, 0.f, 0.f});
+    if constexpr (kKSteps == 4) {
+      s[u] = mfma_16x16x32(kf[1], qf[1], s[u]);
+      s1[u] = mfma_16x16x32(kf[3], qf[3], s1[u]);
+    }
+    refill(u);
   }
-  refill();
+  wave_lds_fence();
   float sv[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) sv[i] = (s[i >> 2][i & 3] + s1[i >> 2][i & 3]) * scale_log2;
@@ -365,13 +367,17 @@ template <typename Refill>
 __device__ __forceinline__ void attend_pair(HeadState &st, const PageRegs &r0, const PageRegs &r1,
                                             const half8_t (&qf)[4], half_t *vstage, const half_t *vt_lane, int p,
                                             int end, int n, int g, float scale_log2, Refill refill) {
-  attend_pair_core(st, r0.k, r1.k, qf, vt_lane, p, end, g, scale_log2, [&](bool tail) {
+  attend_pair_core(st, qf, vt_lane, p, end, g, scale_log2, [&](int u, half8_t (&kf)[4]) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      half8_t x = i < 4 ? r0.v[i & 3] : r1.v[i & 3];
+    for (int kk = 0; kk < kKSteps; ++kk) kf[kk] = u == 0 ? r0.k[kk] : r1.k[kk];
+  }, [&](int u, bool tail) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      half8_t x = u == 0 ? r0.v[i] : r1.v[i];
+      const int row = u * kPageSize + 4 * i + g;
       // Slots past the end hold arbitrary bits: keep them out of the MFMA.
-      if (tail && p * kPageSize + 4 * i + g >= end) x = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-      *(half8_t *)(&vstage[(4 * i + g) * kVPitch + 8 * n]) = x;
+      if (tail && p * kPageSize + row >= end) x = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      *(half8_t *)(&vstage[row * kVPitch + 8 * n]) = x;
     }
   }, refill);
 }
@@ -380,17 +386,17 @@ template <int KV, typename Refill>
 __device__ __forceinline__ void attend_pair(HeadState &st, const PageRegsQ8<KV> &r0, const PageRegsQ8<KV> &r1,
                                             const half8_t (&qf)[4], half_t *vstage, const half_t *vt_lane, int p,
                                             int end, int n, int g, float scale_log2, Refill refill) {
-  half8_t ka[4], kb[4];
+  attend_pair_core(st, qf, vt_lane, p, end, g, scale_log2, [&](int u, half8_t (&kf)[4]) {
 #pragma unroll
-  for (int kk = 0; kk < kKSteps; ++kk) {
-    ka[kk] = codes_to_half<KV>(uint2_t{r0.k[kk >> 1][2 * (kk & 1)], r0.k[kk >> 1][2 * (kk & 1) + 1]});
-    kb[kk] = codes_to_half<KV>(uint2_t{r1.k[kk >> 1][2 * (kk & 1)], r1.k[kk >> 1][2 * (kk & 1) + 1]});
-  }
-  attend_pair_core(st, ka, kb, qf, vt_lane, p, end, g, scale_log2, [&](bool tail) {
+    for (int kk = 0; kk < kKSteps; ++kk) {
+      const uint4_t x = u == 0 ? r0.k[kk >> 1] : r1.k[kk >> 1];
+      kf[kk] = codes_to_half<KV>(uint2_t{x[2 * (kk & 1)], x[2 * (kk & 1) + 1]});
+    }
+  }, [&](int u, bool tail) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 8 * i + q8_v_row(n, g);
-      const uint4_t v = i < 2 ? r0.v[i & 1] : r1.v[i & 1];
+    for (int i = 0; i < 2; ++i) {
+      const int row = u * kPageSize + 8 * i + q8_v_row(n, g);
+      const uint4_t v = u == 0 ? r0.v[i] : r1.v[i];
       half8_t lo = codes_to_half<KV>(uint2_t{v[0], v[1]});
       half8_t hi = codes_to_half<KV>(uint2_t{v[2], v[3]});
       if (tail && p * kPageSize + row >= end) {
@@ -617,21 +623,34 @@ extern __shared__ __attribute__((aligned(16))) half_t split_vstage[];  // [waves
 // described below), 0.42 us as half of a pair (one sequence of 4096 tokens, 64 / 8 heads: one
 // wavefront 160 -> 112 us, 16 splits 18.6 -> 14.5).
 //
-// DEEP: two steps' pages in flight instead of one, requested again after the step instead of in the
-// middle of it, once the scores are under way and V is in LDS. Four pages' registers leave two
-// wavefronts per SIMD where the other form has three, and every split requests four pages however few
-// it has: see the rule in launch_split. Both give the same bits.
+// One step's pages are in flight, a page's registers requested again as soon as its scores are under way
+// and its V is in LDS, while the other page is still on its way. DEEP: two steps' pages, requested again
+// after the step: longer ahead, at two wavefronts per SIMD. Both give the same bits. The steps behind
+// which a split has nothing left to request are written out behind the loops, and a split of one step
+// requests one: requests for nothing (16 bytes per lane of the last page, to keep the count of requests in
+// flight) cost launches of short splits up to 9 % (8 sequences of 256 tokens, 64 / 8 heads over fp8, 16 splits:
+// 11.2 us with them, 10.0 without; 10.7 with a page per step).
 //
-// The second launch bound keeps the accumulators in ordinary registers. Without one the compiler
-// expects a wavefront to be alone with all 512, puts every MFMA result into AGPRs and copies all 32
-// accumulators and the scores out and back on every page: 304 moves in the loop of two pages (the
-// kernel as it was with nothing but the bound: one wavefront 160 -> 139 us, 8 x 512 tokens in 8 splits 11.5 ->
-// 10.7). It is the number of wavefronts per SIMD that the registers allow anyway.
-constexpr int split_waves_per_simd(int kv, bool append, bool deep) {
-  return deep || (kv == kKvFp8 && append) ? 2 : 3;
+// The wavefronts per SIMD are fixed from below and from above. From below, so that the accumulators stay
+// in ordinary registers: left alone the compiler expects a wavefront to be alone with all 512, puts every
+// MFMA result into AGPRs and copies all 32 accumulators and the scores out and back on every page: 304
+// moves in the loop of two pages (one page per step, one wavefront 160 -> 139 us without them). From above for
+// launches of more wavefronts than the device holds: at three per SIMD ragged batches of fp16 rows with the
+// append lose up to 8 % against two (64 / 8 heads, 64 sequences of 2048 tokens and less, 8 splits 83.2 us at
+// two, 88.5 at three), equal ones are the same; without append, in batch order, three are up to 6 % faster (512
+// sequences of 128 tokens 52.5 us, 55.4 at two). Over codes three; a fourth costs up to 16 % (fp8, one of 512 sequences
+// long 11.2 -> 13.0 us). Rows of 64: only over fp8 with the append three (64 sequences of 4096 tokens, 32 / 8
+// heads, 16 splits 78.3 us, 83.7 at four).
+constexpr int split_waves_per_simd(int kv, bool append, bool deep, bool ordered) {
+  return deep || (kv == kKvF16 && (append || ordered)) ? 2 : 3;
+}
+constexpr int split_most_waves(int kv, bool append, bool deep, bool ordered) {
+  return kHD == 128 ? split_waves_per_simd(kv, append, deep, ordered) : kv == kKvFp8 && append ? 3 : 8;
 }
 template <int KV, bool APPEND, bool DEEP, bool ORDERED = false>
-__global__ __launch_bounds__(kSplitWaves *kWave, split_waves_per_simd(KV, APPEND, DEEP)) void paged_decode_split_kernel(
+__global__ __launch_bounds__(kSplitWaves *kWave)
+    __attribute__((amdgpu_waves_per_eu(split_waves_per_simd(KV, APPEND, DEEP, ORDERED),
+                                       split_most_waves(KV, APPEND, DEEP, ORDERED)))) void paged_decode_split_kernel(
     const half_t *__restrict__ q, int64_t q_batch_stride,
     typename KvStore<KV>::elem *__restrict__ kv, const float *__restrict__ scales,
     const int32_t *__restrict__ block_table, int32_t bt_stride,
@@ -650,8 +669,6 @@ __global__ __launch_bounds__(kSplitWaves *kWave, split_waves_per_simd(KV, APPEND
                  "s"(max_splits), "s"(min_pages_per_split), "s"(num_pages), "s"(page_shift), "s"(scale_log2),
                  "s"(wg_waves));
   }
-  constexpr int STEP = 2;                        // pages per step
-  constexpr int DEPTH = DEEP ? 2 * STEP : STEP;  // pages in flight
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int n = lane & 15;   // query head inside the slice (column of S^T)
@@ -753,7 +770,7 @@ __global__ __launch_bounds__(kSplitWaves *kWave, split_waves_per_simd(KV, APPEND
 
   HeadState st;
   st.reset();
-  Page buf[DEPTH];
+  Page buf[DEEP ? 4 : 2];
 
   // Requests past the range still issue their loads (16 bytes of its last page), which keeps
   // the number of vector loads in flight a compile-time constant, so each wait names exactly the
@@ -788,78 +805,97 @@ __global__ __launch_bounds__(kSplitWaves *kWave, split_waves_per_simd(KV, APPEND
 
   // Pages past the split's last count for nothing (a pair's second page), whosever they are.
   const int end = len < p1 * kPageSize ? len : p1 * kPageSize;
+  auto request_pair = [&](int p, auto at) {
+    request(p, buf[at]);
+    request(p + 1, buf[at + 1]);
+  };
+  auto no_refill = [](int) {};
+  constexpr std::integral_constant<int, 0> first_pair{};
+  constexpr std::integral_constant<int, 2> second_pair{};
+  // Pages p, p + 1 where they may be the sequence's last.
+  auto last_pair = [&](int p, auto at) {
 #pragma unroll
-  for (int dd = 0; dd < DEPTH; ++dd) request(p0 + dd, buf[dd]);
-  for (int p = p0; p < p1; p += DEPTH) {
+    for (int u = 0; u < 2; ++u) {
+      if (APPEND && fits_table && p + u < p1 && (p + u + 1) * kPageSize >= len) {
+        // The sequence's last page: the step's new token (logical position len - 1) goes to
+        // the pool and replaces the stale values this wavefront loaded before the write; an
+        // fp8 pool gets the codes the append kernel would store and is attended as stored.
+        // (The pages are named by compile-time numbers: behind a function taking one by reference, or
+        // with a value stored under a condition on i, the pages in flight end up in scratch memory.)
+        const int t_new = (len - 1) & (kPageSize - 1);
+        const int64_t slot_off = ((int64_t)page_id(p + u) * kPageSize + t_new) * row_stride;
+        Page &r = buf[at + u];
+        if constexpr (FP8) {
+          if (n == t_new) {
+            uint8_t *dst = kv + slot_off + (int64_t)h * kHD + 16 * g;
 #pragma unroll
-    for (int first = 0; first < DEPTH; first += STEP) {
-#pragma unroll
-      for (int dd = first; dd < first + STEP; ++dd) {
-        if (APPEND && fits_table && p + dd < p1 && (p + dd + 1) * kPageSize >= len) {
-          // The sequence's last page: the step's new token (logical position len - 1) goes to
-          // the pool and replaces the stale values this wavefront loaded before the write; an
-          // fp8 pool gets the codes the append kernel would store and is attended as stored.
-          // (Written out here: behind a function taking the page by reference the page
-          // registers of both pages in flight end up in scratch memory.)
-          const int t_new = (len - 1) & (kPageSize - 1);
-          const int64_t slot_off = ((int64_t)page_id(p + dd) * kPageSize + t_new) * row_stride;
-          Page &r = buf[dd];
-          if constexpr (FP8) {
-            if (n == t_new) {
-              uint8_t *dst = kv + slot_off + (int64_t)h * kHD + 16 * g;
-#pragma unroll
-              for (int j = 0; j < kHD / 64; ++j) {
-                const uint2_t lo = half_to_codes<KV>(__builtin_bit_cast(half8_t, k_row[2 * j]), k_inv);
-                const uint2_t hi = half_to_codes<KV>(__builtin_bit_cast(half8_t, k_row[2 * j + 1]), k_inv);
-                const uint4_t x = uint4_t{lo[0], lo[1], hi[0], hi[1]};
-                r.k[j] = x;
-                *(uint4_t *)(dst + 64 * j) = x;
-              }
-            }
-            if (q8_v_row(n, g) == (t_new & 7)) {
-              const uint2_t lo = half_to_codes<KV>(__builtin_bit_cast(half8_t, v_row[0]), v_inv);
-              const uint2_t hi = half_to_codes<KV>(__builtin_bit_cast(half8_t, v_row[1]), v_inv);
+            for (int j = 0; j < kHD / 64; ++j) {
+              const uint2_t lo = half_to_codes<KV>(__builtin_bit_cast(half8_t, k_row[2 * j]), k_inv);
+              const uint2_t hi = half_to_codes<KV>(__builtin_bit_cast(half8_t, k_row[2 * j + 1]), k_inv);
               const uint4_t x = uint4_t{lo[0], lo[1], hi[0], hi[1]};
-              *(uint4_t *)(kv + slot_off + (int64_t)(num_kv_heads + h) * kHD + 16 * (q8_v_col(n) & (kHD / 16 - 1))) = x;
-#pragma unroll
-              for (int i = 0; i < 2; ++i) {
-                if (i == (t_new >> 3)) r.v[i] = x;
-              }
+              r.k[j] = x;
+              *(uint4_t *)(dst + 64 * j) = x;
             }
-          } else {
-            if (n == t_new) {
-              half_t *dst = kv + slot_off + (int64_t)h * kHD + 8 * g;
+          }
+          if (q8_v_row(n, g) == (t_new & 7)) {
+            const uint2_t lo = half_to_codes<KV>(__builtin_bit_cast(half8_t, v_row[0]), v_inv);
+            const uint2_t hi = half_to_codes<KV>(__builtin_bit_cast(half8_t, v_row[1]), v_inv);
+            const uint4_t x = uint4_t{lo[0], lo[1], hi[0], hi[1]};
+            *(uint4_t *)(kv + slot_off + (int64_t)(num_kv_heads + h) * kHD + 16 * (q8_v_col(n) & (kHD / 16 - 1))) = x;
 #pragma unroll
-              for (int kk = 0; kk < kKSteps; ++kk) {
-                const half8_t x = __builtin_bit_cast(half8_t, k_row[kk]);
-                r.k[kk] = x;
-                *(half8_t *)(dst + 32 * kk) = x;
-              }
+            for (int i = 0; i < 2; ++i) {
+              r.v[i] = i == (t_new >> 3) ? x : r.v[i];
             }
-            if (g == (t_new & 3)) {
-              const half8_t x = __builtin_bit_cast(half8_t, v_row[0]);
-              *(half8_t *)(kv + slot_off + (int64_t)(num_kv_heads + h) * kHD + 8 * (n & (kVCols - 1))) = x;
+          }
+        } else {
+          if (n == t_new) {
+            half_t *dst = kv + slot_off + (int64_t)h * kHD + 8 * g;
 #pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                if (i == (t_new >> 2)) r.v[i] = x;
-              }
+            for (int kk = 0; kk < kKSteps; ++kk) {
+              const half8_t x = __builtin_bit_cast(half8_t, k_row[kk]);
+              r.k[kk] = x;
+              *(half8_t *)(dst + 32 * kk) = x;
+            }
+          }
+          if (g == (t_new & 3)) {
+            const half8_t x = __builtin_bit_cast(half8_t, v_row[0]);
+            *(half8_t *)(kv + slot_off + (int64_t)(num_kv_heads + h) * kHD + 8 * (n & (kVCols - 1))) = x;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              r.v[i] = i == (t_new >> 2) ? x : r.v[i];
             }
           }
         }
       }
-      auto refill = [&]() {
-        request(p + first + DEPTH, buf[first]);
-        request(p + first + 1 + DEPTH, buf[first + 1]);
-      };
-      if (p + first < p1) {
-        attend_pair(st, buf[first], buf[first + 1], qf, vstage, vt_lane, p + first, end, n, g, scale_log2, [&]() {
-          // the last step asks for nothing (with two steps in flight a request left out would leave the
-          // waits of the loop without the count of the requests behind the one they wait for)
-          if (!DEEP && p + first + DEPTH < p1) refill();
-        });
-      }
-      if constexpr (DEEP) refill();
     }
+    attend_pair(st, buf[at], buf[at + 1], qf, vstage, vt_lane, p, end, n, g, scale_log2, no_refill);
+  };
+  // (A request left out inside a loop, under a condition, would leave the loop's waits without the count of
+  // the requests behind the one they wait for.)
+  int p = p0;
+  request_pair(p, first_pair);
+  if constexpr (DEEP) {
+    if (p1 - p0 > 2) {
+      request_pair(p + 2, second_pair);
+      for (; p + 4 < p1; p += 4) {
+        attend_pair(st, buf[0], buf[1], qf, vstage, vt_lane, p, end, n, g, scale_log2, no_refill);
+        request_pair(p + 4, first_pair);
+        attend_pair(st, buf[2], buf[3], qf, vstage, vt_lane, p + 2, end, n, g, scale_log2, no_refill);
+        request_pair(p + 6, second_pair);
+      }
+      last_pair(p, first_pair);
+      if (p + 2 < p1) last_pair(p + 2, second_pair);
+    } else {
+      last_pair(p, first_pair);
+    }
+  } else {
+    for (; p + 2 < p1; p += 2) {
+      attend_pair(st, buf[0], buf[1], qf, vstage, vt_lane, p, end, n, g, scale_log2, [&](int u) {
+        request(p + 2 + u, buf[u]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    }
+    last_pair(p, first_pair);
   }
 
   const int64_t cell = ((int64_t)b * num_q_heads + hq0) * max_splits + split;
@@ -1657,13 +1693,12 @@ static int launch_split(const DecodeArgs &a, int32_t max_splits, int32_t min_pag
   const dim3 grid((unsigned)(slice_heads / waves), (unsigned)max_splits, (unsigned)a.batch);
   const dim3 block((unsigned)(waves * kWave));
   const int64_t row_pages = (int64_t)a.block_table_stride << page_shift_of(a.page_size);
-  // Two steps' pages in flight (DEEP) while the launch has half a wavefront per SIMD of an fp16 pool, one
-  // of a pool of codes (whose pages take half the registers and requests, and more work per byte), and
-  // a split can have two pages at all. Time against a page per step in the same registers, geometric
-  // means over 239 shapes of fp16 pools (209 of codes), 64 / 8 heads: DEEP 256 wavefronts 0.88 to 0.96 (0.87 to
-  // 0.94), 512: 0.96 to 1.01 (0.87 to 0.95), 1024: 1.06 to 1.09 (0.96 to 1.01), 2048: 1.07 to 1.10 (0.98 to
-  // 0.99); one step's pages 1024: 1.00 to 1.02, 2048: 1.02 to 1.04 (0.91 to 0.96).
-  const bool deep = units <= (fp8_scales != nullptr ? 1024 : 512) && row_pages > max_splits;
+  // Two steps' pages in flight (DEEP) while the launch has at most half a wavefront per SIMD, and a split can
+  // have two pages at all. Time against the kernel of a page per step, geometric means over 24 to 30
+  // shapes each, 64 / 8 heads, fp16 rows (fp8): DEEP 256 wavefronts 0.71 to 0.85, 512 0.81 to 0.90 (0.73 to 0.86);
+  // without 512 0.88 to 0.95, 1024 0.91 to 0.95 (0.80 to 0.90, with 0.85 to 0.92), 2048 0.97 to 0.98 (0.94 to 0.97), 4096
+  // 0.97 (0.94 to 0.97).
+  const bool deep = units <= 512 && row_pages > max_splits;
   const size_t lds = (size_t)waves * 2 * kPageSize * kVPitch * sizeof(half_t);
   // Sequences from the longest down once the launch has more workgroups than the device holds at
   // a time (see sequence_of_rank; a launch that is resident at once ends with its longest piece
