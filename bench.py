@@ -633,7 +633,7 @@ def time_chunk_prefill(device: str, rows: int = 128, history: int = 32768, hq: i
 
     def timed(key_slices):
         run = lambda: ops.paged_prefill(q, pool, table, cu, ctx, rows, None, out=out, key_slices=key_slices,
-                                        workspace=ws if key_slices > 1 else None)
+                                        max_kv_len=history + rows, workspace=ws if key_slices > 1 else None)
         for _ in range(3):
             run()
         torch.cuda.synchronize()

@@ -50,7 +50,7 @@ extern "C" {
 #define LITEKV_ERR_INVALID_ARGUMENT 1
 #define LITEKV_ERR_LAUNCH 2
 
-#define LITEKV_ABI_VERSION 3
+#define LITEKV_ABI_VERSION 4
 
 /* ABI version of the loaded library (LITEKV_ABI_VERSION at build time). */
 int litekv_abi_version(void);
@@ -554,6 +554,29 @@ int litekv_paged_prefill(const void *q, int64_t q_token_stride,
                          int32_t num_q_heads, int32_t num_kv_heads,
                          int32_t head_dim, int32_t page_size, int64_t num_pages,
                          int32_t max_q_len, float softmax_scale, void *stream);
+
+/*
+ * The same, or litekv_paged_prefill_fp8 / _int8 below where kv_scales is not
+ * NULL (_int8 when pool_is_int8 is not 0), for a caller that knows on the host
+ * how many keys its longest row sees (history + chunk): max_kv_len, 0 where it
+ * does not. The kernel's form goes by it, what is computed does not: behind a
+ * history, a launch of no more workgroups than compute units shares the keys of
+ * a block among twice as many wavefronts where there are enough of them. (The
+ * entry points without it attend as for few.)
+ */
+int litekv_paged_prefill_bounded(const void *q, int64_t q_token_stride,
+                                 const void *kv_pool, const float *kv_scales,
+                                 int32_t pool_is_int8,
+                                 const int32_t *block_table,
+                                 int32_t block_table_stride,
+                                 const int32_t *cu_q_lens,
+                                 const int32_t *context_lens, void *out,
+                                 int64_t out_token_stride, int32_t batch,
+                                 int32_t num_q_heads, int32_t num_kv_heads,
+                                 int32_t head_dim, int32_t page_size,
+                                 int64_t num_pages, int32_t max_q_len,
+                                 int64_t max_kv_len, float softmax_scale,
+                                 void *stream);
 
 /*
  * The same for launches with too few query rows to fill the device: one

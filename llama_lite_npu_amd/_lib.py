@@ -18,7 +18,7 @@ import torch  # noqa: F401
 
 LIB_PATH = Path(__file__).resolve().parent / "csrc" / "liblitekv.so"
 
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 # name -> (restype, argtypes); mirrors include/litekv.h declaration by declaration.
 SIGNATURES = {
@@ -197,6 +197,11 @@ SIGNATURES = {
         [c_void_p, c_int64, c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_int64,
          c_int32, c_int32, c_int32, c_int32, c_int32, c_int64, c_int32, c_int64, c_int32, c_void_p, c_size_t,
          c_float, c_void_p],
+    ),
+    "litekv_paged_prefill_bounded": (
+        c_int32,
+        [c_void_p, c_int64, c_void_p, c_void_p, c_int32, c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_int64,
+         c_int32, c_int32, c_int32, c_int32, c_int32, c_int64, c_int32, c_int64, c_float, c_void_p],
     ),
     "litekv_paged_prefill_split_q8": (
         c_int32,

@@ -131,10 +131,11 @@ struct DecodeArgs {
 // A paged prefill whose blocks are cut into key slices (see kPagedPrefillSplit in prefill_tile.h):
 // how many, the workspace for the slices' partial rows, and the query rows of the launch.
 struct PrefillKeySplit {
-  int32_t key_slices = 1;   // 1: no split, nothing else is read
+  int32_t key_slices = 1;   // 1: no split, the next three are not read
   void *workspace = nullptr;
   size_t workspace_bytes = 0;
   int64_t num_tokens = 0;   // query rows of the launch (cu_q_lens[batch])
+  int64_t max_kv_len = 0;   // the most keys a row sees as the host knows it, 0: it does not
 };
 constexpr int kMaxPrefillKeySlices = 8;
 

@@ -110,15 +110,20 @@ static int device_cus() {
   return cached_cus;
 }
 
-// Whether the blocks of a launch of `wgs` workgroups (counted as if every sequence had max_q_len rows)
-// whose rows see at most `max_keys` keys are attended by two groups of wavefronts each
-// (varlen_prefill_two_group_kernel): where a workgroup would have its compute unit to itself (and
-// narrow_launch does not take it), from 9 key tiles on. The meeting of the groups costs 1.2 us, halving the
-// keys saves 0.14 us a tile (rows of 64: 0.18). One request, 64 / 8 heads, us with one group and with two: 512
-// rows over 512 tokens 25.3, 24.0, over 2048 54.2, 48.1, over 8192 174.9, 154.8; 512 rows of a fresh prompt 15.7,
-// 15.8. (More workgroups than compute units share them two by two as it is.)
-static bool two_key_groups(int64_t wgs, int64_t max_keys) {
-  return kHD != 256 && max_keys > 8 * kKvTile && wgs <= device_cus();
+// Whether the blocks of a launch of `wgs` workgroups (counted as if every sequence had max_q_len rows, in
+// `row_blocks` blocks) whose rows see up to `max_keys` keys are attended by two groups of wavefronts each
+// (varlen_prefill_two_group_kernel): where a workgroup would have its compute unit to itself, narrow_launch
+// does not take it, and half of the key tiles saves more than the larger workgroup and the meeting of
+// the groups cost. That is from 10 tiles on; over codes, whose conversion the groups share, from 4; where
+// a sequence has one or two blocks of 128-wide fp16 rows and the launch streams its K and V, from 24. Time with
+// two groups / one, 136 to 256 workgroups, 1 to 32 sequences, 64 / 8, 16 / 8 and 32 / 4 heads: 4 tiles 0.97 to 1.04
+// (fp8 0.94 to 0.99), 9 1.01 to 1.04 (0.95 to 0.97), 10 0.96 to 1.02, 16 0.92 to 0.98, 32 0.88 to 0.95, 128 0.85 to
+// 0.94; one or two blocks a sequence: 9 1.03 to 1.09, 16 0.96 to 1.03, 24 0.94 to 1.00; 32 / 8 heads of 64: 9 1.00 to 1.03,
+// 10 0.94 to 0.98, 128 0.79 to 0.91. (The width of a block table says little about the keys: 8 chunks of 64 rows,
+// nothing cached, in a table of 2048 pages took 8.2 us in two groups, 6.6 in one.)
+static bool two_key_groups(int64_t wgs, unsigned row_blocks, int64_t max_keys, bool codes) {
+  const int from = codes ? 4 : kHD == 128 && row_blocks <= 2 ? 24 : 10;
+  return kHD != 256 && max_keys > (from - 1) * kKvTile && wgs <= device_cus();
 }
 
 // Whether a launch of `wgs` workgroups of 128 columns runs with 64 columns a workgroup, one column tile
@@ -323,8 +328,7 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
                          s.row_tiles, softmax_scale * kLog2eP, 1);
     };
 #if LITEKV_HD != 256
-    // (lengths live on the device: behind a history, as many keys as a block-table row can name)
-    const int64_t max_keys = context_lens != nullptr ? (int64_t)block_table_stride * page_size : max_q_len;
+    const int64_t max_keys = context_lens != nullptr ? split.max_kv_len : max_q_len;
     const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
     if (narrow_launch(wgs)) {
       s = prefill_shape(group, max_q_len, kTiledWaves);
@@ -332,7 +336,7 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
       with(varlen_prefill_tiled_kernel<MODE, 1>, kTiledWaves);
       return;
     }
-    if (two_key_groups(wgs, max_keys)) {
+    if (two_key_groups(wgs, s.row_blocks, max_keys, fp8)) {
       with(varlen_prefill_two_group_kernel<MODE>, 2 * kTiledWaves);
       return;
     }
@@ -430,7 +434,7 @@ static int launch_varlen_prefill(const void *q, int64_t q_token_stride, const vo
     launch(varlen_prefill_tiled_kernel<kPackedPrefill, 1>, kTiledWaves);
     return check_launch("varlen_prefill");
   }
-  if (two_key_groups(wgs, max_seq_len)) {
+  if (two_key_groups(wgs, s.row_blocks, max_seq_len, false)) {
     launch(varlen_prefill_two_group_kernel<kPackedPrefill>, 2 * kTiledWaves);
     return check_launch("varlen_prefill");
   }
@@ -467,6 +471,26 @@ extern "C" int litekv_paged_prefill(const void *q, int64_t q_token_stride, const
                                       out_token_stride, batch, num_q_heads, num_kv_heads, head_dim,
                                       page_size, num_pages, max_q_len, softmax_scale, stream,
                                       litekv::kKvF16, litekv::PrefillKeySplit{});
+}
+
+extern "C" int litekv_paged_prefill_bounded(const void *q, int64_t q_token_stride, const void *kv_pool,
+                                            const float *kv_scales, int32_t pool_is_int8,
+                                            const int32_t *block_table, int32_t block_table_stride,
+                                            const int32_t *cu_q_lens, const int32_t *context_lens,
+                                            void *out, int64_t out_token_stride, int32_t batch,
+                                            int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                            int32_t page_size, int64_t num_pages, int32_t max_q_len,
+                                            int64_t max_kv_len, float softmax_scale, void *stream) {
+  const int format = kv_scales == nullptr ? litekv::kKvF16 : pool_is_int8 ? litekv::kKvInt8 : litekv::kKvFp8;
+  const char *what = format == litekv::kKvF16    ? "paged_prefill"
+                     : format == litekv::kKvInt8 ? "paged_prefill_int8"
+                                                 : "paged_prefill_fp8";
+  litekv::PrefillKeySplit split;
+  split.max_kv_len = max_kv_len;
+  return litekv::launch_paged_prefill(what, q, q_token_stride, kv_pool, kv_scales, block_table,
+                                      block_table_stride, cu_q_lens, context_lens, out,
+                                      out_token_stride, batch, num_q_heads, num_kv_heads, head_dim,
+                                      page_size, num_pages, max_q_len, softmax_scale, stream, format, split);
 }
 
 extern "C" size_t litekv_paged_prefill_split_workspace_bytes(int64_t num_tokens, int32_t num_q_heads,

@@ -204,19 +204,9 @@ PyObject *paged_prefill(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const int32_t ts = (int32_t)table->stride(0);
     const int64_t pages = pool.slots / page;
     const int rc = unlocked([&] {
-      switch (pool.format) {
-        case kF16:
-          return litekv_paged_prefill(qp, qs, pp, tp, ts, cup, ctxp, op, hq * d, (int32_t)b, (int32_t)hq, (int32_t)pool.hkv,
-                                      (int32_t)d, (int32_t)page, pages, (int32_t)max_q, (float)scale, stream);
-        case kFp8:
-          return litekv_paged_prefill_fp8(qp, qs, pp, scales, tp, ts, cup, ctxp, op, hq * d, (int32_t)b, (int32_t)hq,
-                                          (int32_t)pool.hkv, (int32_t)d, (int32_t)page, pages, (int32_t)max_q, (float)scale,
-                                          stream);
-        default:
-          return litekv_paged_prefill_int8(qp, qs, pp, scales, tp, ts, cup, ctxp, op, hq * d, (int32_t)b, (int32_t)hq,
-                                           (int32_t)pool.hkv, (int32_t)d, (int32_t)page, pages, (int32_t)max_q, (float)scale,
-                                           stream);
-      }
+      return litekv_paged_prefill_bounded(qp, qs, pp, scales, pool.format == kInt8, tp, ts, cup, ctxp, op, hq * d, (int32_t)b,
+                                          (int32_t)hq, (int32_t)pool.hkv, (int32_t)d, (int32_t)page, pages, (int32_t)max_q,
+                                          max_kv < 0 ? 0 : max_kv, (float)scale, stream);
     });
     if (rc == 0) return result;
     Py_DECREF(result);

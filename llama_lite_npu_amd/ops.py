@@ -864,7 +864,7 @@ def paged_prefill(q: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Ten
     is cut along the keys as well: ``key_slices`` workgroups per row block and a merge launch
     (head_dim 64 / 128, any pool format). None lets the library choose from the launch shape and
     ``max_kv_len`` (the most keys a row sees: history + chunk, as the host knows it; without it
-    the launch is not cut); 1 switches it off. ``workspace`` (float32, see ``paged_prefill_workspace_floats``) is
+    the launch is not cut, and its form is the one for few keys); 1 switches it off. ``workspace`` (float32, see ``paged_prefill_workspace_floats``) is
     allocated when not given."""
     if q.is_cuda and out is None and key_slices is None and workspace is None and softmax_scale is not None:
         done = _lib.calls().paged_prefill(q, kv_pool, block_table, cu_q_lens, context_lens, max_q_len, softmax_scale,
@@ -915,30 +915,26 @@ def paged_prefill(q: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Ten
         if not (workspace.is_cuda and workspace.dtype == torch.float32
                 and workspace.is_contiguous() and workspace.numel() >= need):
             raise ValueError(f"workspace must be {need} contiguous float32 on the device")
+    if key_slices <= 1:
+        # (max_kv_len 0: not known)
+        _lib.check(lib.litekv_paged_prefill_bounded(
+            _ptr(q), q_stride, _ptr(kv_pool), _ptr(kv_scales), 1 if is_int8_pool(kv_pool) else 0, _ptr(block_table),
+            block_table.stride(0), _ptr(cu_q_lens), _ptr(context_lens), _ptr(out), _rows("out", out), b, hq, hkv, d,
+            page_size, n_pages, int(max_q_len), 0 if max_kv_len is None else int(max_kv_len), float(softmax_scale),
+            _stream()))
+        return out
     if fp8:
-        if key_slices > 1:
-            _lib.check(lib.litekv_paged_prefill_split_q8(
-                _ptr(q), q_stride, _ptr(kv_pool), _ptr(kv_scales), 1 if is_int8_pool(kv_pool) else 0,
-                _ptr(block_table), block_table.stride(0), _ptr(cu_q_lens), _ptr(context_lens), _ptr(out),
-                _rows("out", out), b, hq, hkv, d, page_size, n_pages, int(max_q_len), t, key_slices,
-                _ptr(workspace), workspace.numel() * 4, float(softmax_scale), _stream()))
-            return out
-        _lib.check(_q8_entry(lib, "paged_prefill", kv_pool)(_ptr(q), q_stride, _ptr(kv_pool), _ptr(kv_scales), _ptr(block_table),
-                                                block_table.stride(0), _ptr(cu_q_lens), _ptr(context_lens),
-                                                _ptr(out), _rows("out", out), b, hq, hkv, d, page_size, n_pages,
-                                                int(max_q_len), float(softmax_scale), _stream()))
+        _lib.check(lib.litekv_paged_prefill_split_q8(
+            _ptr(q), q_stride, _ptr(kv_pool), _ptr(kv_scales), 1 if is_int8_pool(kv_pool) else 0,
+            _ptr(block_table), block_table.stride(0), _ptr(cu_q_lens), _ptr(context_lens), _ptr(out),
+            _rows("out", out), b, hq, hkv, d, page_size, n_pages, int(max_q_len), t, key_slices,
+            _ptr(workspace), workspace.numel() * 4, float(softmax_scale), _stream()))
         return out
-    if key_slices > 1:
-        _lib.check(lib.litekv_paged_prefill_split(_ptr(q), q_stride, _ptr(kv_pool), _ptr(block_table),
-                                                  block_table.stride(0), _ptr(cu_q_lens), _ptr(context_lens),
-                                                  _ptr(out), _rows("out", out), b, hq, hkv, d, page_size, n_pages,
-                                                  int(max_q_len), t, key_slices, _ptr(workspace),
-                                                  workspace.numel() * 4, float(softmax_scale), _stream()))
-        return out
-    _lib.check(lib.litekv_paged_prefill(_ptr(q), q_stride, _ptr(kv_pool), _ptr(block_table),
-                                        block_table.stride(0), _ptr(cu_q_lens), _ptr(context_lens),
-                                        _ptr(out), _rows("out", out), b, hq, hkv, d, page_size, n_pages,
-                                        int(max_q_len), float(softmax_scale), _stream()))
+    _lib.check(lib.litekv_paged_prefill_split(_ptr(q), q_stride, _ptr(kv_pool), _ptr(block_table),
+                                              block_table.stride(0), _ptr(cu_q_lens), _ptr(context_lens),
+                                              _ptr(out), _rows("out", out), b, hq, hkv, d, page_size, n_pages,
+                                              int(max_q_len), t, key_slices, _ptr(workspace),
+                                              workspace.numel() * 4, float(softmax_scale), _stream()))
     return out
 
 

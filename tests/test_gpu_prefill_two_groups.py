@@ -1,6 +1,6 @@
-"""GPU: a prefill of at most as many workgroups as compute units whose rows may see over 512 keys is
-attended by two groups of wavefronts per block, each over half of its key tiles; one of at most half as many
-workgroups with one column tile per wavefront. Blocks of one tile (the first group has none) up to odd
+"""GPU: a prefill of at most as many workgroups as compute units whose longest row sees many keys (as the
+caller says) is attended by two groups of wavefronts per block, each over half of its key tiles; one of at
+most half as many workgroups with one column tile per wavefront. Blocks of one tile (the first group has none) up to odd
 and even numbers of them, ragged last blocks and tiles, every pool format, both head dims, paged and
 packed, in a batch (two groups) and sequence by sequence (one column tile): against float64 arithmetic."""
 
@@ -71,7 +71,7 @@ def test_two_groups(fmt, head_dim, hq, hkv):
     cu = torch.tensor([0] + rows * copies, dtype=torch.int32).cumsum(0).to(torch.int32).to(DEV)
     batch = ops.paged_prefill(q.repeat(copies, 1, 1), pool, table.repeat(copies, 1), cu,
                               torch.tensor(ctx * copies, dtype=torch.int32, device=DEV), max(rows), scale, kv_scales=scales,
-                              key_slices=1)
+                              key_slices=1, max_kv_len=4096)      # (the form goes by the bound, not by the lengths)
     torch.cuda.synchronize()
     for out in batch.split(sum(rows)):
         assert torch.equal(out, batch[:sum(rows)])
@@ -98,3 +98,41 @@ def test_two_groups_over_packed_rows(head_dim):
         s = slice(first, first + n)
         assert_attention_close(out[s], _reference(q[s], k[s], v[s], 0, head_dim ** -0.5).numpy(), f"length {n}")
         first += n
+
+
+@pytest.mark.parametrize("fmt,head_dim,rows,batch,keys,told", [
+    ("f16", 128, 60, 8, 64, True), ("f16", 128, 60, 8, 9 * 64, True),       # few keys
+    ("f16", 128, 16, 30, 23 * 64, True),                                    # one block a sequence
+    ("f16", 64, 100, 7, 9 * 64, True), ("fp8", 128, 60, 8, 3 * 64, True), ("int8", 64, 100, 7, 3 * 64, True),
+    ("f16", 128, 60, 8, 20 * 64, False), ("fp8", 64, 100, 7, 20 * 64, False),   # the caller does not say
+])
+def test_few_keys_in_a_wide_table_are_attended_by_one_group(fmt, head_dim, rows, batch, keys, told):
+    """A launch of more workgroups than compute units has one group a block: the same bits."""
+    print(f"one key group: {fmt} pool, heads of {head_dim}, {batch} x {rows} rows, {keys} keys, told {told}", flush=True)
+    hq, hkv = (64, 8) if head_dim == 128 else (32, 8)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    wgs = hkv * batch * -(-rows // (128 * hkv // hq))
+    assert cus < 2 * wgs <= 2 * cus
+    gen = torch.Generator(device=DEV).manual_seed(9)
+    pages = keys // 16
+    pool = torch.randn((batch * keys, 2 * hkv, head_dim), generator=gen, dtype=torch.float16, device=DEV)
+    scales = None
+    if fmt != "f16":
+        scales = torch.full((2 * hkv,), 0.035, device=DEV)
+        codes = torch.empty(pool.shape, dtype=torch.uint8 if fmt == "fp8" else torch.int8, device=DEV)
+        slots = torch.arange(batch * keys, dtype=torch.int32, device=DEV)
+        ops.kv_append_quantised(pool[:, :hkv], pool[:, hkv:], slots, codes, scales)
+        pool = codes
+    table = torch.zeros((batch, 2048), dtype=torch.int32, device=DEV)
+    table[:, :pages] = torch.randperm(batch * pages, generator=gen, device=DEV).to(torch.int32).view(batch, pages)
+    q = torch.randn((batch * rows, hq, head_dim), generator=gen, dtype=torch.float16, device=DEV)
+
+    def run(copies):
+        cu = torch.arange(0, (batch * copies + 1) * rows, rows, dtype=torch.int32, device=DEV)
+        ctx = torch.full((batch * copies,), keys - rows, dtype=torch.int32, device=DEV)
+        return ops.paged_prefill(q.repeat(copies, 1, 1), pool, table.repeat(copies, 1), cu, ctx, rows, head_dim ** -0.5,
+                                 kv_scales=scales, key_slices=1, max_kv_len=keys if told else None)
+
+    few, many = run(1), run(cus // wgs + 1)
+    torch.cuda.synchronize()
+    assert torch.equal(few, many[:few.shape[0]])
