@@ -112,8 +112,8 @@ static int device_cus() {
 
 // Whether the blocks of a launch of `wgs` workgroups (counted as if every sequence had max_q_len rows, in
 // `row_blocks` blocks) whose rows see up to `max_keys` keys are attended by two groups of wavefronts each
-// (varlen_prefill_two_group_kernel): where a workgroup would have its compute unit to itself, narrow_launch
-// does not take it, and half of the key tiles saves more than the larger workgroup and the meeting of
+// (varlen_prefill_two_group_kernel): where a workgroup would have its compute unit to itself, the narrow
+// form does not take it, and half of the key tiles saves more than the larger workgroup and the meeting of
 // the groups cost. That is from 10 tiles on; over codes, whose conversion the groups share, from 4; where
 // a sequence has one or two blocks of 128-wide fp16 rows and the launch streams its K and V, from 24. Time with
 // two groups / one, 136 to 256 workgroups, 1 to 32 sequences, 64 / 8, 16 / 8 and 32 / 4 heads: 4 tiles 0.97 to 1.04
@@ -133,8 +133,20 @@ static bool two_key_groups(int64_t wgs, unsigned row_blocks, int64_t max_keys, b
 // request, us with 128 columns and with 64: 203 rows of a fresh prompt, 16 / 8 heads, 9.2, 7.6; 64 rows, 64 / 8 heads,
 // 5.3, 4.4; 128 rows over 2048 tokens 40.1, 30.5; 32 / 8 heads of 64, 256 rows 7.3, 5.8. With more
 // workgroups the K and V tiles staged twice cost as much as that saves (400 rows, 64 / 8 heads: 200 workgroups).
-static bool narrow_launch(int64_t wgs) {
+static bool narrow_fits(int64_t wgs) {
   return kHD != 256 && 2 * wgs <= device_cus();
+}
+
+// Whether narrow workgroups would bring K and V in from memory twice at a cost: those of more than 4 heads per kv
+// head share the heads of a block, not its rows, and land on different XCDs, so where every sequence has one block
+// (of 128-wide fp16 rows) nothing else keeps its K and V near. From 7/16 of the compute units and 13 key tiles a
+// workgroup on (or where nobody says how many, 0) that costs more than the rest saves: 16 rows a sequence, 64 / 8
+// heads, time with 64 columns / with 128: 112 workgroups 16 tiles 0.97, 64 tiles 1.05, 128 workgroups 12 tiles 1.00, 16
+// 1.05, 32 1.12 (41 us with 128); 96 workgroups 0.82 to 0.96; 16 / 8 heads 0.84 to 0.96, codes and rows of 64 0.73 to
+// 0.87. In 8 key slices, two sequences of 30 000 tokens: 77.3 us with 128 columns, 84.1 with 64.
+static bool narrow_reads_twice(int64_t wgs, int group, unsigned row_blocks, int64_t max_keys, bool codes) {
+  return kHD == 128 && !codes && group > kTiledWaves && row_blocks == 1 && 16 * wgs >= 7 * device_cus() &&
+         (max_keys <= 0 || max_keys > 12 * kKvTile);
 }
 
 // Key slices for a paged prefill whose row blocks alone would not fill the device, if the longest
@@ -142,7 +154,7 @@ static bool narrow_launch(int64_t wgs) {
 // time, 1 (do not split) unless that is at least 5 % less than unsplit. The estimate, in
 // microseconds, head dim 128 (fits to one request's chunk of 64 to 512 rows over 0 to 32k cached
 // tokens, 64 query / 8 kv heads): a workgroup walks max_kv_len / 64 / n key tiles at 1.0 us each
-// while it has its compute unit to itself (0.75 us with 64 columns, narrow_launch) and at 1.7 us once
+// while it has its compute unit to itself (0.75 us with 64 columns, narrow_fits) and at 1.7 us once
 // the launch has more workgroups than compute units (two share one), times the rounds the launch needs
 // on the device's resident slots; a cut costs the merge launch, 6 us, and a partial row (fp32) written and read back per
 // query row, head and slice at 6 MB/us. (An unsliced launch of 129 to 256 workgroups runs in two groups of
@@ -167,7 +179,7 @@ static int32_t prefill_key_slices(int32_t batch, int32_t num_q_heads, int32_t nu
   const double partial_us = (double)batch * max_q_len * num_q_heads * (kHD + 1) * 2.0 * sizeof(float) / 6.0e6;
   auto estimate = [&](int64_t n) {
     const int64_t resident = wgs * n;
-    const double per_tile = narrow_launch(resident) ? 0.75 * tile_us
+    const double per_tile = narrow_fits(resident) ? 0.75 * tile_us
                             : resident <= cus       ? tile_us
                                                     : 1.7 * tile_us * (double)((resident + slots - 1) / slots);
     return tiles / (double)n * per_tile + (n > 1 ? 6.0 + partial_us * (double)n : 0.0);
@@ -271,12 +283,13 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
                    "%s: workspace of %zu bytes needed for %d key slices, got %zu", what, need, slices,
                    split.workspace_bytes);
     PrefillShape s = prefill_shape(group, max_q_len);
-    // 64 columns a workgroup (narrow_launch); short slices (at most 16 tiles, as far as the block table can
+    // 64 columns a workgroup (narrow_fits); short slices (at most 16 tiles, as far as the block table can
     // say) up to twice as many: 128 rows, 64 / 8 heads, in 4 slices over 2048 tokens 29.6, 25.5 us, over 8192
     // 54.7, 56.2, over 30 000 169.7, 181.0.
     const int64_t wgs = (int64_t)num_kv_heads * s.head_splits * s.row_blocks * slices * batch;
-    const bool narrow = narrow_launch(wgs) || (wgs <= device_cus() && (int64_t)block_table_stride * page_size <=
-                                                                          (int64_t)slices * 16 * kKvTile);
+    const int64_t slice_keys = (int64_t)block_table_stride * page_size / slices;  // at most, by the table
+    const bool narrow = (narrow_fits(wgs) || (wgs <= device_cus() && slice_keys <= 16 * kKvTile)) &&
+                        !narrow_reads_twice(wgs, group, s.row_blocks, slice_keys, fp8);
     if (narrow) s = prefill_shape(group, max_q_len, kTiledWaves);
     LITEKV_REQUIRE((uint64_t)s.row_blocks * slices <= 65535u, "%s: max_q_len %d too large for %d key slices",
                    what, max_q_len, slices);
@@ -330,7 +343,7 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
 #if LITEKV_HD != 256
     const int64_t max_keys = context_lens != nullptr ? split.max_kv_len : max_q_len;
     const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
-    if (narrow_launch(wgs)) {
+    if (narrow_fits(wgs) && !narrow_reads_twice(wgs, group, s.row_blocks, max_keys, fp8)) {
       s = prefill_shape(group, max_q_len, kTiledWaves);
       grid = dim3((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch);
       with(varlen_prefill_tiled_kernel<MODE, 1>, kTiledWaves);
@@ -428,7 +441,7 @@ static int launch_varlen_prefill(const void *q, int64_t q_token_stride, const vo
   };
 #if LITEKV_HD != 256
   const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
-  if (narrow_launch(wgs)) {
+  if (narrow_fits(wgs) && !narrow_reads_twice(wgs, group, s.row_blocks, max_seq_len, false)) {
     s = prefill_shape(group, max_seq_len, kTiledWaves);
     grid = dim3((unsigned)(num_kv_heads * s.head_splits), s.row_blocks, (unsigned)batch);
     launch(varlen_prefill_tiled_kernel<kPackedPrefill, 1>, kTiledWaves);

@@ -1165,7 +1165,7 @@ __device__ __forceinline__ void prefill_tile_body(
 }
 
 // CT: column tiles per wavefront. One instead of two, 64 score columns a workgroup, for launches that would
-// leave most of the device idle (see narrow_launch in paged_prefill.hip). Bound by the chain of its few key tiles.
+// leave most of the device idle (see narrow_fits in paged_prefill.hip). Bound by the chain of its few key tiles.
 template <int MODE, int CT = kColTiles>
 __global__ __launch_bounds__(kTiledWaves *kWave, kWgPerCu) void varlen_prefill_tiled_kernel(
     const half_t *__restrict__ q, int64_t q_stride, half_t *__restrict__ out, int64_t out_stride,
