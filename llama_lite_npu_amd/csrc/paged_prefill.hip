@@ -154,11 +154,14 @@ static bool narrow_reads_twice(int64_t wgs, int group, unsigned row_blocks, int6
 // time, 1 (do not split) unless that is at least 5 % less than unsplit. The estimate, in
 // microseconds, head dim 128 (fits to one request's chunk of 64 to 512 rows over 0 to 32k cached
 // tokens, 64 query / 8 kv heads): a workgroup walks max_kv_len / 64 / n key tiles at 1.0 us each
-// while it has its compute unit to itself (0.75 us with 64 columns, narrow_fits) and at 1.7 us once
-// the launch has more workgroups than compute units (two share one), times the rounds the launch needs
-// on the device's resident slots; a cut costs the merge launch, 6 us, and a partial row (fp32) written and read back per
-// query row, head and slice at 6 MB/us. (An unsliced launch of 129 to 256 workgroups runs in two groups of
-// wavefronts, at 0.95 us a tile: where that moves the choice the two are within 5 %. One chunk over 30 000
+// while it has its compute unit to itself (0.75 us with 64 columns, narrow_fits; 0.95 uncut in two groups of
+// wavefronts, two_key_groups) and at 1.7 us once the launch has more workgroups than compute units (two share
+// one), times the rounds the launch needs on the device's resident slots; a cut costs the merge launch, 6 us, and
+// a partial row (fp32) written and read back per query row, head and slice at 6 MB/us. Rows of 64: 0.6 us a
+// tile with 64 columns as with 128 (priced at 0.45, chunks of 8 to 64 rows over 1000 tokens were left uncut: 12.1 us, 8.6
+// in eight slices; over int8 15.7, 8.9). Over 1121 shapes (8 to 512 rows, 200 to 30 000 tokens, 1 to 4 chunks, the
+// layouts above and 32 / 8 heads of 64, codes among them) the choice takes 1.019 times as long as the best count, rows of
+// 64 1.020 (1.042 before). (One chunk over 30 000
 // tokens, plain against sliced:
 // 128 rows 364 -> 148 us, 256 rows 388 -> 269 us, 512 rows 480 -> 485 us; 128 rows over 2048 tokens
 // 30.5 -> 25.5 us in four slices; 512 rows over 2048 tokens in two slices 48 -> 62 us and 128 rows of a
@@ -179,9 +182,10 @@ static int32_t prefill_key_slices(int32_t batch, int32_t num_q_heads, int32_t nu
   const double partial_us = (double)batch * max_q_len * num_q_heads * (kHD + 1) * 2.0 * sizeof(float) / 6.0e6;
   auto estimate = [&](int64_t n) {
     const int64_t resident = wgs * n;
-    const double per_tile = narrow_fits(resident) ? 0.75 * tile_us
-                            : resident <= cus       ? tile_us
-                                                    : 1.7 * tile_us * (double)((resident + slots - 1) / slots);
+    const double per_tile = narrow_fits(resident) ? (kHD == 64 ? 1.0 : 0.75) * tile_us
+                            : n == 1 && two_key_groups(resident, s.row_blocks, max_kv_len, false) ? 0.95 * tile_us
+                            : resident <= cus ? tile_us
+                                              : 1.7 * tile_us * (double)((resident + slots - 1) / slots);
     return tiles / (double)n * per_tile + (n > 1 ? 6.0 + partial_us * (double)n : 0.0);
   };
   const double unsplit = estimate(1);
