@@ -631,26 +631,21 @@ extern __shared__ __attribute__((aligned(16))) half_t split_vstage[];  // [waves
 // flight) cost launches of short splits up to 9 % (8 sequences of 256 tokens, 64 / 8 heads over fp8, 16 splits:
 // 11.2 us with them, 10.0 without; 10.7 with a page per step).
 //
-// The wavefronts per SIMD are fixed from below and from above. From below, so that the accumulators stay
-// in ordinary registers: left alone the compiler expects a wavefront to be alone with all 512, puts every
+// The wavefronts per SIMD are fixed from below and, for codes, from above. From below, so that the accumulators
+// stay in ordinary registers: left alone the compiler expects a wavefront to be alone with all 512, puts every
 // MFMA result into AGPRs and copies all 32 accumulators and the scores out and back on every page: 304
-// moves in the loop of two pages (one page per step, one wavefront 160 -> 139 us without them). From above for
-// launches of more wavefronts than the device holds: at three per SIMD ragged batches of fp16 rows with the
-// append lose up to 8 % against two (64 / 8 heads, 64 sequences of 2048 tokens and less, 8 splits 83.2 us at
-// two, 88.5 at three), equal ones are the same; without append, in batch order, three are up to 6 % faster (512
-// sequences of 128 tokens 52.5 us, 55.4 at two). Over codes three; a fourth costs up to 16 % (fp8, one of 512 sequences
-// long 11.2 -> 13.0 us). Rows of 64: only over fp8 with the append three (64 sequences of 4096 tokens, 32 / 8
-// heads, 16 splits 78.3 us, 83.7 at four).
-constexpr int split_waves_per_simd(int kv, bool append, bool deep, bool ordered) {
-  return deep || (kv == kKvF16 && (append || ordered)) ? 2 : 3;
-}
-constexpr int split_most_waves(int kv, bool append, bool deep, bool ordered) {
-  return kHD == 128 ? split_waves_per_simd(kv, append, deep, ordered) : kv == kKvFp8 && append ? 3 : 8;
+// moves in the loop of two pages (one page per step, one wavefront 160 -> 139 us without them). From above
+// because a fourth wavefront over codes costs up to 16 % (fp8, one of 512 sequences long 11.2 -> 13.0 us); rows of 64
+// only over fp8 with the append (64 sequences of 4096 tokens, 32 / 8 heads, 16 splits 78.3 us, 83.7 at four).
+// For fp16 rows see two_per_simd in launch_split.
+constexpr int split_least_waves(bool deep) { return deep ? 2 : 3; }
+constexpr int split_most_waves(int kv, bool append, bool deep) {
+  return kHD == 128 ? split_least_waves(deep) : kv == kKvFp8 && append ? 3 : 8;
 }
 template <int KV, bool APPEND, bool DEEP, bool ORDERED = false>
 __global__ __launch_bounds__(kSplitWaves *kWave)
-    __attribute__((amdgpu_waves_per_eu(split_waves_per_simd(KV, APPEND, DEEP, ORDERED),
-                                       split_most_waves(KV, APPEND, DEEP, ORDERED)))) void paged_decode_split_kernel(
+    __attribute__((amdgpu_waves_per_eu(split_least_waves(DEEP), split_most_waves(KV, APPEND, DEEP)))) void
+paged_decode_split_kernel(
     const half_t *__restrict__ q, int64_t q_batch_stride,
     typename KvStore<KV>::elem *__restrict__ kv, const float *__restrict__ scales,
     const int32_t *__restrict__ block_table, int32_t bt_stride,
@@ -1699,7 +1694,6 @@ static int launch_split(const DecodeArgs &a, int32_t max_splits, int32_t min_pag
   // without 512 0.88 to 0.95, 1024 0.91 to 0.95 (0.80 to 0.90, with 0.85 to 0.92), 2048 0.97 to 0.98 (0.94 to 0.97), 4096
   // 0.97 (0.94 to 0.97).
   const bool deep = units <= 512 && row_pages > max_splits;
-  const size_t lds = (size_t)waves * 2 * kPageSize * kVPitch * sizeof(half_t);
   // Sequences from the longest down once the launch has more workgroups than the device holds at
   // a time (see sequence_of_rank; a launch that is resident at once ends with its longest piece
   // in any order), for block tables wide enough that a split can be 16 pages long: finding its
@@ -1709,6 +1703,16 @@ static int launch_split(const DecodeArgs &a, int32_t max_splits, int32_t min_pag
   const bool longest_first = max_splits > 1 && a.k_new == nullptr && a.batch <= kMaxOrderedBatch &&
                              units / waves > 3 * (int64_t)device_cus() &&
                              row_pages >= 16 * (int64_t)max_splits;
+  // Two wavefronts per SIMD instead of three, by the LDS a workgroup asks for, in launches of more than the
+  // device holds whose splits may have 8 pages or more of fp16 rows: a long split then shares its
+  // compute unit's memory path with fewer others. 64 / 8 heads, 4096 wavefronts and more, time with two / with
+  // three, one long sequence among short ones: splits of 8 pages and more 0.87 to 0.97 (64 sequences, 4096 tokens and
+  // 256, 8 splits 46.7 us, 50), 3 to 5 pages 1.03 to 1.13; ragged 0.96 to 1.02, 0.98 to 1.05; equal 0.99 to 1.04, 1.00 to
+  // 1.05. (In batch order without the append three are up to 6 % faster: 512 sequences of 128 tokens 52.5 us, 55.4.)
+  const bool two_per_simd = kHD == 128 && fp8_scales == nullptr && (a.k_new != nullptr || longest_first) &&
+                            units > 8 * (int64_t)device_cus() && row_pages >= 8 * (int64_t)max_splits;
+  size_t lds = (size_t)waves * 2 * kPageSize * kVPitch * sizeof(half_t);
+  if (two_per_simd) lds = (waves == 4 ? 56 : 18 * waves) * 1024;  // of 160 KiB: two workgroups of 4, four of 2, eight of 1
   LITEKV_REQUIRE((a.k_new == nullptr) == (a.v_new == nullptr), "%s: k_new and v_new go together", what);
   if (a.k_new != nullptr) {
     const int64_t row = (int64_t)a.num_kv_heads * a.head_dim;
