@@ -332,34 +332,34 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
                               page_size: int = PAGE_SIZE, heads_per_kv_head: int = 8,
                               head_dim: int = HEAD_DIM, chunks: Optional[int] = None) -> dict:
     """Estimated microseconds per layer of every decode schedule a step could take, keyed as
-    ``decode_schedule`` returns them. Fits to 554 measured shapes on an MI355X (1 to 2048 sequences
-    of 32 to 16384 tokens: equal, ragged, one long among short; 64/8 and 16/8 heads; every
-    schedule replayed from a graph; ``tune_decode_schedule`` re-measures such tables) and to 425 more
-    for what depends on the pool's format, the head dim and the number of kv heads (1 to 128
-    sequences of up to 32768 tokens; 64/8, 16/8 and 32/4 heads of 128, 32/8 of 64; fp16, fp8, int8);
-    the per-sequence ones to 1613 (1 to 2048 sequences, up to 140 000 tokens; the same layouts and formats):
+    ``decode_schedule`` returns them. Fits to 2681 measured shapes on an MI355X: a grid of 1 to 2048 sequences of 32 to
+    32768 tokens (equal, ragged, one long among short; ``tune_decode_schedule`` re-measures such tables) and 630
+    drawn ones (1 to 1500 sequences, those kinds and log-normal lengths, pages of 16 to 64); 64/8, 16/8 and 32/4 heads
+    of 128 and 32/8 of 64 over fp16, 64/8 over fp8, 32/4 and 32/8 of 64 over int8; every schedule replayed from a
+    graph.
 
-    * 1, one wavefront per (sequence, kv head), one launch: 4.3 us + the largest (a 3.6-norm) of the
-      longest sequence's dependent chain of 16-token steps at 0.41 us each -- up to 80 % more
-      when the launch has 2048 wavefronts or more, whose loads share the compute units'
-      memory paths with the chain's --, the placement of the launch's wavefronts at 2.4 ns each,
-      and the bytes at 6.0 MB/us (unbalanced streams).
+    * 1, one wavefront per (sequence, kv head), one launch: 4.45 us + the largest (a 2.8-norm) of the
+      longest sequence's dependent chain of 16-token steps at 0.40 to 0.42 us each -- 0.73 from 2048 wavefronts on,
+      four to a workgroup, whose loads share their compute unit's memory path --, the placement of the
+      launch's wavefronts at 1.6 ns each, and the bytes at 6.1 MB/us, up to 10 % more where the sequences
+      are uneven.
     * 4 / 8 / 16 splits per sequence + the merge launch, for launches of at most 2048 wavefronts:
-      5.9 us for the two launches, the chain of a split at 0.44 to 0.67 us a step against the bytes at
-      6.4 MB/us (a 3.1-norm), 1.1 ns per wavefront (codes: 1.4); where the bytes dominate, uneven sequences make
-      uneven splits, which the balanced cut does not have: up to 18 % more with the bytes' share.
-    * 0, balanced (fused step + merge): 7.6 us, 0.17 us per piece the merge folds for the longest
-      sequence (up to 36; 0.07 to 0.10 us where a step of few rows shares a long row out among
-      several workgroups, by how many rows those are; half as much with rows of 64), 3.4 ns +
-      0.26 ns per query head for every sequence, and the bytes at 6.8 MB/us against the chain
-      inside one of ``chunks`` (a plan's own count; else what ``balanced_chunks`` gives 256 compute
-      units: 256 for 8 kv heads, 512 for 4, whose workgroups hold two); with over 8 query heads per
-      kv head a tenth more (two column tiles) and the partial rows beyond 8 MB, written and read
+      6.3 us for the two launches, the chain of a split at 0.35 us a step with two steps' pages in flight (up to 512
+      wavefronts), 0.44 with one's, 0.59 at 2048, against the bytes at 6.65 MB/us (a 2.4-norm), 0.4 ns per wavefront
+      (codes: 1.0); where the bytes dominate, uneven sequences make uneven splits, which the balanced cut does not
+      have: 14 to 41 % more with the bytes' share.
+    * 0, balanced (fused step + merge): 7.8 us, 0.19 us per piece the merge folds for the longest
+      sequence (up to 23; 0.3 us more for each past 16 in a step of many rows; 0.04 to 0.13 us where a step
+      of few rows shares a long row out among several workgroups, by how many rows those are; half as much
+      with rows of 64), 1.8 ns + 0.21 ns per query head for every sequence, and the bytes at 7.0 MB/us
+      against the chain inside one of ``chunks`` (a plan's own count; else what ``balanced_chunks`` gives 256
+      compute units) at 0.52 us a step; with more than 8 query heads per kv head, 10 % more -- its page step
+      carries twice the exponentials -- and the partial rows beyond 8 MB, written and read back,
       at 3 MB/us (117 shapes of 8 to 64 query heads per kv head, 1 to 8 kv heads: 2 to 3 % over the
       fastest schedule; 8 sequences of 4000 tokens, 32/1 heads, 2048 chunks: 31 us, 17 without).
 
-    A step over a page of codes takes 1.1 to 1.35 times as long as over fp16 rows (the conversion),
-    over rows of 64 elements 0.8 to 0.9 times."""
+    A step over a page of codes takes 0.9 to 1.3 times as long as over fp16 rows (half the bytes, the conversion),
+    over rows of 64 elements 0.87 to 1.0 times."""
     steps = max(1, page_size // PAGE_SIZE)                 # the kernels step by 16 tokens
     chain = max_pages * steps
     total = total_pages * steps
@@ -371,38 +371,38 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
     chunks = _whole_device_chunks(num_kv_heads) if chunks is None else chunks
     narrow = head_dim < HEAD_DIM
     codes = token_bytes < 4 * num_kv_heads * head_dim      # a pool of 8-bit codes
-    pieces = chain / max(1.0, total / chunks)
+    uneven = min(1.0, chain * batch / max(1, total) - 1.0)
+    pieces = min(chain / max(1.0, total / chunks), 23.5)
     # rows of more than 16 pieces are merged by several workgroups each while the step has few rows
     rows = batch * num_q_heads * head_dim / (256.0 * HEAD_DIM)
-    per_piece = 0.07 + 0.03 * rows if pieces > 16 and rows <= 1.0 else 0.170
-    per_piece *= 0.57 if narrow else 1.0
-    step = (0.87 if narrow else 1.0) * (1.12 if codes else 1.0)
+    per_piece = 0.035 + 0.092 * rows if pieces > 16 and rows <= 1.0 else 0.191
+    merge = per_piece * (0.46 if narrow else 1.0) * pieces + (0.30 * max(0.0, pieces - 16.0) if rows > 1.0 else 0.0)
+    step = (0.865 if narrow else 1.0) * (1.27 if codes else 1.0)
     partials = (min(total, chunks) + batch) * num_q_heads * head_dim * 4.0
     estimates = {
-        0: (7.6 + per_piece * min(pieces, 36.0) + (3.4e-3 + 2.6e-4 * num_q_heads) * batch
-            + norm(2.0, nbytes / 6.81e6, 0.82 * step * -(-total // chunks))) * (1.1 if heads_per_kv_head > 8 else 1.0)
+        0: (7.84 + merge + (1.81e-3 + 2.12e-4 * num_q_heads) * batch
+            + norm(2.0, nbytes / 6.97e6, 0.517 * step * -(-total // chunks))) * (1.1 if heads_per_kv_head > 8 else 1.0)
            + (max(0.0, 2.0 * partials - 16.8e6) / 3.0e6 if heads_per_kv_head > 8 else 0.0),
     }
     if narrow and not codes:
-        estimates[0] *= 0.93
-    # the per-sequence kernels: two steps' pages in flight instead of one up to so many wavefronts
-    deep = 1024 if codes else 512
-    step = (0.82 if narrow else 1.0) * (1.29 if codes else 1.0)
-    page = 0.41 * (1.0 + 0.8 * min(1.0, lone / 2048.0))
-    estimates[1] = 4.28 * (0.85 if narrow else 1.0) + norm(3.6, page * step * chain, 2.4e-3 * lone, nbytes / 5.96e6)
-    step = (0.82 if narrow else 1.0) * (1.33 if codes else 1.0)
+        estimates[0] *= 0.984
+    # the per-sequence kernels: two steps' pages in flight up to 512 wavefronts, one's beyond; from 2048
+    # on four wavefronts share a workgroup
+    page = (0.40 if lone <= 512 else 0.419 if lone < 2048 else 0.419 * 1.745) * (0.905 if codes else 1.0)
+    chain_us, stream = page * chain, nbytes / 6.1e6
+    estimates[1] = (4.45 * (0.648 if narrow else 1.0) + norm(2.78, chain_us, 1.58e-3 * lone, stream)) * (
+        1.0 + 0.097 * uneven * stream / max(1e-9, chain_us + stream))
     for n in SPLIT_COUNTS:
         wavefronts = batch * n * num_kv_heads * slices
         if wavefronts > 2048:
             continue
-        page = 0.54
-        if wavefronts > deep:
-            page = 0.6 * (1.0 + 0.12 * wavefronts / 2048.0) if codes else 0.44 * (1.0 + 0.5 * wavefronts / 2048.0)
-        split_chain = page * step * ((chain + n - 1) // n)
-        stream = nbytes / 6.4e6
-        estimates[n] = ((5.9 * (1.08 if narrow else 1.0) + norm(3.1, split_chain, stream)
-                         + (1.4e-3 if codes else 1.1e-3) * wavefronts)
-                        * (1.0 + 0.18 * stream / (split_chain + stream)))
+        deep = wavefronts <= 512
+        page = 0.35 if deep else 0.443 if wavefronts < 2048 else 0.443 * 1.322
+        page *= (0.9 if narrow else 1.0) * ((1.14 if deep else 0.928) if codes else 1.0)
+        chain_us, stream = page * ((chain + n - 1) // n), nbytes / 6.65e6
+        estimates[n] = (6.29 * (0.96 if narrow else 1.0) + norm(2.37, chain_us, stream)
+                        + (1.03e-3 if codes else 4.4e-4) * wavefronts) * (
+            1.0 + (0.141 + 0.273 * uneven) * stream / max(1e-9, chain_us + stream))
     return estimates
 
 
@@ -412,8 +412,8 @@ def decode_schedule(batch: int, num_kv_heads: int, max_pages: int, total_pages: 
     """Which decode schedule a step should take, from what the host knows about it: 0 = balanced,
     1 = one wavefront per (sequence, kv head) in one launch, 4 / 8 / 16 = that many splits per
     sequence and the merge launch: the smallest of ``decode_schedule_estimates``. Choosing by this
-    rule is 1.1 to 2.6 % slower on average than always choosing the fastest schedule over the shapes of
-    a head layout and pool format, 19 to 43 % at worst (``tune_decode_schedule``). ``current``: the schedule
+    rule is 0.3 to 1.4 % slower on average than always choosing the fastest schedule over the shapes of
+    a head layout and pool format, 8 to 31 % at worst (3451 shapes, 770 of them not fitted to). ``current``: the schedule
     in use; another must be estimated ``hysteresis`` times faster to replace it. ``head_dim`` tells rows
     of 64 fp16 elements from 128 codes, which ``token_bytes`` alone does not; ``chunks``: a plan's own
     count, see ``decode_schedule_estimates``."""

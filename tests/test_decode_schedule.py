@@ -128,6 +128,28 @@ def test_the_choice_knows_the_pool_format_the_head_dim_and_the_kv_heads(batch, h
     assert pick in ((8, 16) if want in (8, 16) else (want,))
 
 
+@pytest.mark.parametrize("batch,hkv,group,head_dim,code_bytes,longest,rest,want", [
+    # one long sequence among short ones, us measured per layer: {0: balanced, 1, 4, 8, 16: wavefronts per sequence}
+    (128, 8, 8, 128, 2, 512, 32, (1, 4)),      # {0: 28.5, 1: 20.5, 4: 21.0}
+    (128, 8, 8, 128, 1, 512, 32, (1, 4)),      # {0: 26.4, 1: 18.9, 4: 18.4}
+    (128, 8, 8, 128, 1, 256, 16, (1,)),        # {0: 16.4, 1: 11.9, 4: 17.5}
+    (16, 8, 8, 128, 1, 2048, 128, (8, 16)),    # {0: 19.4, 1: 56.5, 4: 21.0, 8: 15.6, 16: 14.0}
+    (32, 4, 8, 128, 1, 2048, 128, (8, 16)),    # {0: 18.9, 1: 67.9, 4: 23.9, 8: 17.2, 16: 14.4}
+    (64, 4, 8, 128, 1, 1024, 64, (8, 16)),     # {0: 18.1, 1: 36.4, 4: 17.2, 8: 13.9, 16: 16.2}
+    (256, 4, 8, 128, 2, 512, 32, (1, 4)),      # {0: 27.3, 1: 21.0, 4: 21.2}
+    (128, 8, 4, 64, 2, 256, 16, (1, 4)),       # {0: 13.4, 1: 10.4, 4: 11.6}
+    # equal lengths
+    (64, 8, 8, 128, 1, 512, 512, (1, 4)),      # {0: 25.8, 1: 20.6, 4: 21.2, 8: 26.8}
+    (2, 8, 8, 128, 1, 64, 64, (1,)),           # {0: 9.9, 1: 6.2, 4: 7.1, 8: 7.8, 16: 7.9}
+    (2048, 8, 8, 128, 2, 256, 256, (0,)),      # {0: 389.4, 1: 425.4}
+])
+def test_steps_whose_choice_cost_a_quarter(batch, hkv, group, head_dim, code_bytes, longest, rest, want):
+    total = pages(longest + 1) + (batch - 1) * pages(rest + 1)
+    pick = decode_schedule(batch, hkv, pages(longest + 1), total, 2 * hkv * head_dim * code_bytes,
+                           heads_per_kv_head=group, head_dim=head_dim)
+    assert pick in want
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("batch,tokens", [(1, 300), (24, 128), (4, 80), (12, 2900), (64, 512), (128, 64)])
 def test_flash_decoding_asks_for_the_width_it_is_given(monkeypatch, batch, tokens, d):
