@@ -8,13 +8,14 @@ PyTorch fallback behind these functions.
 from __future__ import annotations
 
 import ctypes
+import re
 from ctypes import c_char_p, c_float, c_int32, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
 # PyTorch-ROCm ships its own HIP runtime under the soname the library links
 # against; importing torch first makes both share one runtime (and one set of
 # streams and allocations).
-import torch  # noqa: F401
+import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "csrc" / "liblitekv.so"
 
@@ -266,6 +267,12 @@ def calls():
         except ImportError as e:
             raise LiteKVError(f"{__package__}._calls: {e}: build it with `python -m llama_lite_npu_amd.build` "
                               "(there is no fallback implementation)") from e
+        # what it was compiled against: the library's prototypes, PyTorch's classes
+        for what, built, now in (("liblitekv ABI", getattr(module, "ABI_VERSION", None), ABI_VERSION),
+                                 ("PyTorch", getattr(module, "TORCH_VERSION", None), re.match(r"[\d.]+\d", torch.__version__)[0])):
+            if built != now:
+                raise LiteKVError(f"{__package__}._calls was built for {what} {built}, not {now}; rebuild it "
+                                  "(`python -m llama_lite_npu_amd.build`)")
         _calls = module
     return _calls
 

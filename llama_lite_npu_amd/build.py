@@ -1,9 +1,10 @@
-"""Builds liblitekv.so (HIP, gfx950) in-tree with hipcc.
+"""Builds liblitekv.so (HIP, gfx950) in-tree with hipcc, and the Python module of the calls that take
+PyTorch tensors (host code) with g++.
 
 Usage: ``python -m llama_lite_npu_amd.build`` or ``build_library(force=True)``.
 hipcc cross-compiles for gfx950 without a GPU, so this also runs on a CPU-only
-machine. The library lands next to its sources (``csrc/liblitekv.so``); nothing
-is installed outside the tree.
+machine. The library lands next to its sources (``csrc/liblitekv.so``), the module in the
+package; nothing is installed outside the tree.
 """
 
 from __future__ import annotations
@@ -18,7 +19,8 @@ from pathlib import Path
 
 CSRC = Path(__file__).resolve().parent / "csrc"
 LIB_PATH = CSRC / "liblitekv.so"
-CALLS_PATH = CSRC.parent / "_calls.so"          # csrc/torch_calls.cpp, a Python module
+# csrc/torch_calls.cpp; the suffix names the interpreter it is for, and another one does not find it
+CALLS_PATH = CSRC.parent / f"_calls{sysconfig.get_config_var('EXT_SUFFIX') or '.so'}"
 OBJ_DIR = CSRC / "build"
 
 SOURCES = (
@@ -99,8 +101,10 @@ def _compile(hipcc: str, src: Path, obj: Path, extra: tuple[str, ...]) -> None:
 
 
 def build_library(force: bool = False, extra_flags: tuple[str, ...] = ()) -> Path:
-    """Compiles every source and links liblitekv.so; returns its path."""
+    """Compiles every source and links liblitekv.so, then the module of the tensor calls; returns the
+    library's path."""
     if not force and not is_stale():
+        build_calls()
         return LIB_PATH
     hipcc = _hipcc()
     OBJ_DIR.mkdir(exist_ok=True)
@@ -118,22 +122,23 @@ def build_library(force: bool = False, extra_flags: tuple[str, ...] = ()) -> Pat
     if proc.returncode != 0:
         raise RuntimeError(f"link of liblitekv.so failed:\n{proc.stdout}{proc.stderr}")
     os.replace(tmp, LIB_PATH)
+    build_calls(force)
     return LIB_PATH
 
 
 def build_calls(force: bool = False) -> Path:
     """Compiles the Python module of the calls that take PyTorch tensors (host code, no kernel); returns its
     path. It finds liblitekv.so next to its source."""
-    import torch
-    from torch.utils import cpp_extension
-
     src = CSRC / "torch_calls.cpp"
     deps = [src, CSRC.parents[1] / "include" / "litekv.h"]
     if not force and CALLS_PATH.exists() and all(d.stat().st_mtime <= CALLS_PATH.stat().st_mtime for d in deps):
         return CALLS_PATH
+    import torch
+    from torch.utils import cpp_extension
+
     torch_lib = Path(torch.__file__).resolve().parent / "lib"
     includes = [CSRC.parents[1] / "include", sysconfig.get_paths()["include"], *cpp_extension.include_paths()]
-    tmp = CALLS_PATH.with_suffix(".so.tmp")
+    tmp = CALLS_PATH.with_name(CALLS_PATH.name + ".tmp")
     cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-isystem{i}" for i in includes),
            str(src), "-o", str(tmp), f"-L{torch_lib}", "-ltorch_python", "-ltorch_cpu", "-lc10",
@@ -147,4 +152,4 @@ def build_calls(force: bool = False) -> Path:
 
 if __name__ == "__main__":
     print(build_library(force=True))
-    print(build_calls(force=True))
+    print(CALLS_PATH)

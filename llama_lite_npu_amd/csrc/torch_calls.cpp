@@ -9,9 +9,11 @@
 // answered goes back as it is, since a launch error is reported after the launch (and may be an older
 // one of the thread), and the epilogue, which works in place, must not run twice.
 #include <Python.h>
+#include <stdio.h>
 
 #include <ATen/ATen.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include "litekv.h"
 
@@ -226,4 +228,15 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, methods, nul
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__calls(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__calls(void) {
+  PyObject *m = PyModule_Create(&module);
+  if (m == nullptr) return nullptr;
+  char torch_version[32];
+  snprintf(torch_version, sizeof(torch_version), "%d.%d.%d", TORCH_VERSION_MAJOR, TORCH_VERSION_MINOR, TORCH_VERSION_PATCH);
+  if (PyModule_AddIntConstant(m, "ABI_VERSION", LITEKV_ABI_VERSION) != 0 ||
+      PyModule_AddStringConstant(m, "TORCH_VERSION", torch_version) != 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

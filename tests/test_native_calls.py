@@ -2,10 +2,14 @@
 is not a plain call, and the wrappers then behave as they do without it -- the same results bit for
 bit, the same errors."""
 
+import sys
+import types
+
 import pytest
 import torch
 
-from llama_lite_npu_amd import _lib, ops
+import llama_lite_npu_amd
+from llama_lite_npu_amd import _lib, build, ops
 
 DEV = "cuda:0"
 
@@ -19,6 +23,27 @@ def test_anything_but_a_plain_call_is_left_alone():
     assert calls.qk_norm_rope_append(x, x, x, idx, pool, None, None, None, None, 1e-6, None, 0) is None   # on the CPU
     assert calls.qk_norm_rope_append(*[None] * 12) is None and calls.paged_prefill(*["q"] * 11) is None
     assert calls.paged_prefill(x, pool, idx[None], idx, None, 2, 1.0, 16, None, None, 0) is None
+
+
+@pytest.mark.parametrize("built", [dict(), dict(ABI_VERSION=_lib.ABI_VERSION - 1), dict(ABI_VERSION=_lib.ABI_VERSION, TORCH_VERSION="1.0.0")])
+def test_a_module_of_another_library_or_torch_is_refused(built, monkeypatch):
+    right = _lib.calls()
+    assert right.ABI_VERSION == _lib.ABI_VERSION and torch.__version__.startswith(right.TORCH_VERSION)
+    other = types.ModuleType("llama_lite_npu_amd._calls")
+    vars(other).update(built)
+    monkeypatch.setitem(sys.modules, other.__name__, other)
+    monkeypatch.setattr(llama_lite_npu_amd, "_calls", other)
+    monkeypatch.setattr(_lib, "_calls", None)
+    with pytest.raises(_lib.LiteKVError, match="was built for"):
+        _lib.calls()
+
+
+def test_building_the_library_builds_the_module(monkeypatch):
+    made = []
+    monkeypatch.setattr(build, "build_calls", lambda force=False: made.append(force))
+    monkeypatch.setattr(build, "is_stale", lambda: False)
+    build.build_library()
+    assert made == [False]
 
 
 class _NoCalls:
