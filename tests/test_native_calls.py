@@ -115,19 +115,45 @@ CHANGES = {
 }
 
 
+# What the native epilogue and the native prefill answer: T(aken), D(eclined), S(tatus of the library), - (not asked:
+# the wrapper had refused the call before). Any other entry is taken by both.
+ANSWERS = {
+    "cos with a batch dim": "DT", "int64 slots": "DT", "int64 table": "TD", "a subclass": "DD", "q in bf16": "D-",
+    "k of another length": "D-", "one norm": "D-", "short cos": "D-", "slots too few": "D-",
+    "heads not contiguous": "D-", "misaligned q": "S-", "table of another batch": "TD", "odd pool": "D-",
+}
+
+
+class _Recorded:
+    """The native calls and what they answered."""
+
+    def __init__(self, calls):
+        self.calls, self.answers = calls, ""
+
+    def _note(self, answer):
+        self.answers += "D" if answer is None else "S" if type(answer) is int else "T"
+        return answer
+
+    def qk_norm_rope_append(self, *a):
+        return self._note(self.calls.qk_norm_rope_append(*a))
+
+    def paged_prefill(self, *a):
+        return self._note(self.calls.paged_prefill(*a))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", ["f16", "fp8", "e4m3", "int8"])
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_the_wrappers_do_the_same_with_and_without_it(fmt, d, monkeypatch):
     print(f"native calls: {fmt} pool, heads of {d}", flush=True)
+    native_calls = _lib.calls()
     for name, change in CHANGES.items():
-        results = []
+        results, recorded = [], _Recorded(native_calls)
         for native in (True, False):
             st = _state(fmt, d)
             change(st)
             with monkeypatch.context() as m:
-                if not native:
-                    m.setattr(_lib, "calls", lambda: _NoCalls)
+                m.setattr(_lib, "calls", lambda: recorded if native else _NoCalls)
                 try:
                     results.append(_run(st))
                 except (ValueError, _lib.LiteKVError) as e:
@@ -137,6 +163,9 @@ def test_the_wrappers_do_the_same_with_and_without_it(fmt, d, monkeypatch):
             assert a == b, name
         else:
             assert all(torch.equal(x, y) for x, y in zip(a, b)), name
+        wrong_scales = "DD" if fmt == "f16" else "D-"       # an fp16 pool's epilogue does not look at them
+        want = wrong_scales if name == "scales of the wrong size" else ANSWERS.get(name, "TT")
+        assert recorded.answers.ljust(2, "-") == want, name
 
 
 @pytest.mark.gpu
