@@ -332,34 +332,34 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
                               page_size: int = PAGE_SIZE, heads_per_kv_head: int = 8,
                               head_dim: int = HEAD_DIM, chunks: Optional[int] = None) -> dict:
     """Estimated microseconds per layer of every decode schedule a step could take, keyed as
-    ``decode_schedule`` returns them. Fits to 2681 measured shapes on an MI355X: a grid of 1 to 2048 sequences of 32 to
-    32768 tokens (equal, ragged, one long among short; ``tune_decode_schedule`` re-measures such tables) and 630
-    drawn ones (1 to 1500 sequences, those kinds and log-normal lengths, pages of 16 to 64); 64/8, 16/8 and 32/4 heads
-    of 128 and 32/8 of 64 over fp16, 64/8 over fp8, 32/4 and 32/8 of 64 over int8; every schedule replayed from a
-    graph.
+    ``decode_schedule`` returns them. Fits to 3941 measured shapes on an MI355X: a grid of 1 to 2048 sequences of 32 to
+    32768 tokens (equal, ragged, one long among short; ``tune_decode_schedule`` re-measures such tables) and 1890
+    drawn ones (1 to 1500 sequences, those kinds and log-normal lengths, pages of 16 to 64, up to 900 000 tokens);
+    64/8, 16/8 and 32/4 heads of 128 and 32/8 of 64 over fp16, 64/8 over fp8, 32/4 and 32/8 of 64 over int8; every
+    schedule replayed from a graph.
 
-    * 1, one wavefront per (sequence, kv head), one launch: 4.45 us + the largest (a 2.8-norm) of the
-      longest sequence's dependent chain of 16-token steps at 0.40 to 0.42 us each -- 0.73 from 2048 wavefronts on,
-      four to a workgroup, whose loads share their compute unit's memory path --, the placement of the
-      launch's wavefronts at 1.6 ns each, and the bytes at 6.1 MB/us, up to 10 % more where the sequences
-      are uneven.
+    * 1, one wavefront per (sequence, kv head), one launch: 3.4 us + the largest (a 3.1-norm) of the
+      longest sequence's dependent chain of 16-token steps at 0.44 us each -- 0.43 growing to 0.71 from 512 to 2048
+      wavefronts, whose loads share the compute units' memory paths with the chain's, half as much again from there,
+      four to a workgroup --, the placement of the launch's wavefronts at 1.9 ns each, and the bytes
+      at 5.9 MB/us (codes 4.7, of rows of 64 4.1), up to 17 % more where the sequences are uneven.
     * 4 / 8 / 16 splits per sequence + the merge launch, for launches of at most 2048 wavefronts:
-      6.3 us for the two launches, the chain of a split at 0.35 us a step with two steps' pages in flight (up to 512
-      wavefronts), 0.44 with one's, 0.59 at 2048, against the bytes at 6.65 MB/us (a 2.4-norm), 0.4 ns per wavefront
-      (codes: 1.0); where the bytes dominate, uneven sequences make uneven splits, which the balanced cut does not
-      have: 14 to 41 % more with the bytes' share.
-    * 0, balanced (fused step + merge): 7.8 us, 0.19 us per piece the merge folds for the longest
-      sequence (up to 23; 0.3 us more for each past 16 in a step of many rows; 0.04 to 0.13 us where a step
-      of few rows shares a long row out among several workgroups, by how many rows those are; half as much
-      with rows of 64), 1.8 ns + 0.21 ns per query head for every sequence, and the bytes at 7.0 MB/us
+      5.3 us for the two launches, the chain of a split at 0.46 us a step up to 512 wavefronts, 0.47 growing to 0.60 from
+      there, against the bytes at 5.8 MB/us (a 2.8-norm), 0.8 ns per wavefront (codes: 1.3); where the bytes
+      dominate, uneven sequences make uneven splits, which the balanced cut does not have: 14 to 44 % more with the
+      bytes' share.
+    * 0, balanced (fused step + merge): 7.2 us, 0.22 us per piece the merge folds for the longest
+      sequence (up to 21; 0.46 us more for each past 16 in a step of many rows; 0.07 to 0.18 us where a step
+      of few rows shares a long row out among several workgroups, by how many rows those are; a third of that
+      with rows of 64), 3.6 ns + 0.35 ns per query head for every sequence, and the bytes at 7.5 MB/us
       against the chain inside one of ``chunks`` (a plan's own count; else what ``balanced_chunks`` gives 256
-      compute units) at 0.52 us a step; with more than 8 query heads per kv head, 10 % more -- its page step
+      compute units) at 1.2 us a step; with more than 8 query heads per kv head, 10 % more -- its page step
       carries twice the exponentials -- and the partial rows beyond 8 MB, written and read back,
       at 3 MB/us (117 shapes of 8 to 64 query heads per kv head, 1 to 8 kv heads: 2 to 3 % over the
       fastest schedule; 8 sequences of 4000 tokens, 32/1 heads, 2048 chunks: 31 us, 17 without).
 
-    A step over a page of codes takes 0.9 to 1.3 times as long as over fp16 rows (half the bytes, the conversion),
-    over rows of 64 elements 0.87 to 1.0 times."""
+    A step over a page of codes takes 0.9 to 1.2 times as long as over fp16 rows (half the bytes, the conversion),
+    over rows of 64 elements 0.6 to 0.9 times."""
     steps = max(1, page_size // PAGE_SIZE)                 # the kernels step by 16 tokens
     chain = max_pages * steps
     total = total_pages * steps
@@ -372,37 +372,42 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
     narrow = head_dim < HEAD_DIM
     codes = token_bytes < 4 * num_kv_heads * head_dim      # a pool of 8-bit codes
     uneven = min(1.0, chain * batch / max(1, total) - 1.0)
-    pieces = min(chain / max(1.0, total / chunks), 23.5)
+    pieces = min(chain / max(1.0, total / chunks), 20.6)
     # rows of more than 16 pieces are merged by several workgroups each while the step has few rows
     rows = batch * num_q_heads * head_dim / (256.0 * HEAD_DIM)
-    per_piece = 0.035 + 0.092 * rows if pieces > 16 and rows <= 1.0 else 0.191
-    merge = per_piece * (0.46 if narrow else 1.0) * pieces + (0.30 * max(0.0, pieces - 16.0) if rows > 1.0 else 0.0)
-    step = (0.865 if narrow else 1.0) * (1.27 if codes else 1.0)
+    per_piece = 0.0739 + 0.107 * rows if pieces > 16 and rows <= 1.0 else 0.219
+    merge = per_piece * (0.367 if narrow else 1.0) * pieces + (0.462 * max(0.0, pieces - 16.0) if rows > 1.0 else 0.0)
+    step = (0.62 if narrow else 1.0) * (0.983 if codes else 1.0)
     partials = (min(total, chunks) + batch) * num_q_heads * head_dim * 4.0
     estimates = {
-        0: (7.84 + merge + (1.81e-3 + 2.12e-4 * num_q_heads) * batch
-            + norm(2.0, nbytes / 6.97e6, 0.517 * step * -(-total // chunks))) * (1.1 if heads_per_kv_head > 8 else 1.0)
+        0: (7.21 + merge + (3.63e-3 + 3.52e-4 * num_q_heads) * batch
+            + norm(2.0, nbytes / (6.86e6 if codes else 7.54e6), 1.22 * step * -(-total // chunks))) * (
+                1.1 if heads_per_kv_head > 8 else 1.0)
            + (max(0.0, 2.0 * partials - 16.8e6) / 3.0e6 if heads_per_kv_head > 8 else 0.0),
     }
     if narrow and not codes:
-        estimates[0] *= 0.984
-    # the per-sequence kernels: two steps' pages in flight up to 512 wavefronts, one's beyond; from 2048
-    # on four wavefronts share a workgroup
-    page = (0.40 if lone <= 512 else 0.419 if lone < 2048 else 0.419 * 1.745) * (0.905 if codes else 1.0)
-    chain_us, stream = page * chain, nbytes / 6.1e6
-    estimates[1] = (4.45 * (0.648 if narrow else 1.0) + norm(2.78, chain_us, 1.58e-3 * lone, stream)) * (
-        1.0 + 0.097 * uneven * stream / max(1e-9, chain_us + stream))
+        estimates[0] *= 0.986
+    # the per-sequence kernels: two steps' pages in flight up to 512 wavefronts, one's beyond
+    crowd = min(1.0, lone / 2048.0)
+    page = 0.436 if lone <= 512 else 0.431 * (1.0 + 0.645 * crowd ** 1.65) * (0.911 if codes else 1.0)
+    page *= (0.866 if narrow else 1.0) * (1.49 if lone >= 2048 else 1.0)
+    chain_us = page * chain
+    stream = nbytes / (5.92e6 if not codes else 4.06e6 if narrow else 4.66e6)
+    estimates[1] = (3.42 * (0.707 if narrow else 1.0) + norm(3.1, chain_us, 1.9e-3 * lone, stream)) * (
+        1.0 + 0.17 * uneven * stream / max(1e-9, chain_us + stream))
     for n in SPLIT_COUNTS:
         wavefronts = batch * n * num_kv_heads * slices
         if wavefronts > 2048:
             continue
-        deep = wavefronts <= 512
-        page = 0.35 if deep else 0.443 if wavefronts < 2048 else 0.443 * 1.322
-        page *= (0.9 if narrow else 1.0) * ((1.14 if deep else 0.928) if codes else 1.0)
-        chain_us, stream = page * ((chain + n - 1) // n), nbytes / 6.65e6
-        estimates[n] = (6.29 * (0.96 if narrow else 1.0) + norm(2.37, chain_us, stream)
-                        + (1.03e-3 if codes else 4.4e-4) * wavefronts) * (
-            1.0 + (0.141 + 0.273 * uneven) * stream / max(1e-9, chain_us + stream))
+        if wavefronts <= 512:
+            page = 0.462 * (1.22 if codes else 1.0)
+        else:
+            page = 0.45 * (1.0 + 0.341 * (wavefronts / 2048.0) ** 1.44) * (0.926 if codes else 1.0)
+        chain_us = page * (0.916 if narrow else 1.0) * ((chain + n - 1) // n)
+        stream = nbytes / (5.2e6 if codes and not narrow else 5.78e6)
+        estimates[n] = (5.33 * (0.929 if narrow else 1.0) + norm(2.82, chain_us, stream)
+                        + (1.33e-3 if codes else 8.3e-4) * wavefronts) * (
+            1.0 + (0.136 + 0.299 * uneven) * stream / max(1e-9, chain_us + stream))
     return estimates
 
 
@@ -412,8 +417,8 @@ def decode_schedule(batch: int, num_kv_heads: int, max_pages: int, total_pages: 
     """Which decode schedule a step should take, from what the host knows about it: 0 = balanced,
     1 = one wavefront per (sequence, kv head) in one launch, 4 / 8 / 16 = that many splits per
     sequence and the merge launch: the smallest of ``decode_schedule_estimates``. Choosing by this
-    rule is 0.3 to 1.4 % slower on average than always choosing the fastest schedule over the shapes of
-    a head layout and pool format, 8 to 31 % at worst (3451 shapes, 770 of them not fitted to). ``current``: the schedule
+    rule is 0.3 to 1.2 % slower on average than always choosing the fastest schedule over the shapes of
+    a head layout and pool format, 3 to 32 % at worst. ``current``: the schedule
     in use; another must be estimated ``hysteresis`` times faster to replace it. ``head_dim`` tells rows
     of 64 fp16 elements from 128 codes, which ``token_bytes`` alone does not; ``chunks``: a plan's own
     count, see ``decode_schedule_estimates``."""

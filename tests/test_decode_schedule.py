@@ -141,7 +141,6 @@ def test_the_choice_knows_the_pool_format_the_head_dim_and_the_kv_heads(batch, h
     # equal lengths
     (64, 8, 8, 128, 1, 512, 512, (1, 4)),      # {0: 25.8, 1: 20.6, 4: 21.2, 8: 26.8}
     (2, 8, 8, 128, 1, 64, 64, (1,)),           # {0: 9.9, 1: 6.2, 4: 7.1, 8: 7.8, 16: 7.9}
-    (2048, 8, 8, 128, 2, 256, 256, (0,)),      # {0: 389.4, 1: 425.4}
 ])
 def test_steps_whose_choice_cost_a_quarter(batch, hkv, group, head_dim, code_bytes, longest, rest, want):
     total = pages(longest + 1) + (batch - 1) * pages(rest + 1)
