@@ -345,7 +345,7 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
       at 5.9 MB/us (codes 4.7, of rows of 64 4.1), up to 17 % more where the sequences are uneven.
     * 4 / 8 / 16 splits per sequence + the merge launch, for launches of at most 2048 wavefronts:
       5.3 us for the two launches, the chain of a split at 0.46 us a step up to 512 wavefronts, 0.47 growing to 0.60 from
-      there, against the bytes at 5.8 MB/us (a 2.8-norm), 0.8 ns per wavefront (codes: 1.3); where the bytes
+      there, against the bytes at 5.8 MB/us (codes 5.2; a 2.8-norm), 0.8 ns per wavefront (codes: 1.3); where the bytes
       dominate, uneven sequences make uneven splits, which the balanced cut does not have: 14 to 44 % more with the
       bytes' share.
     * 0, balanced (fused step + merge): 7.2 us, 0.22 us per piece the merge folds for the longest
@@ -404,7 +404,7 @@ def decode_schedule_estimates(batch: int, num_kv_heads: int, max_pages: int, tot
         else:
             page = 0.45 * (1.0 + 0.341 * (wavefronts / 2048.0) ** 1.44) * (0.926 if codes else 1.0)
         chain_us = page * (0.916 if narrow else 1.0) * ((chain + n - 1) // n)
-        stream = nbytes / (5.2e6 if codes and not narrow else 5.78e6)
+        stream = nbytes / (5.2e6 if codes else 5.78e6)
         estimates[n] = (5.33 * (0.929 if narrow else 1.0) + norm(2.82, chain_us, stream)
                         + (1.33e-3 if codes else 8.3e-4) * wavefronts) * (
             1.0 + (0.136 + 0.299 * uneven) * stream / max(1e-9, chain_us + stream))
