@@ -128,8 +128,8 @@ static bool two_key_groups(int64_t wgs, unsigned row_blocks, int64_t max_keys, b
 
 // Whether a launch of `wgs` workgroups of 128 columns runs with 64 columns a workgroup, one column tile
 // per wavefront, instead: where that still leaves at most one workgroup per compute unit. Twice as many
-// wavefronts with half of a key tile's products and exponentials each, 0.70 us a tile instead of 0.94
-// (two groups of wavefronts: 0.80 to 0.85), and less to load, normalise and store around them. One
+// wavefronts with half of a key tile's products and exponentials each, and less to load, normalise and store around
+// them: 0.68 to 0.95 of the time with 128 columns (32 to 128 workgroups, 1 to 128 key tiles, the layouts above). One
 // request, us with 128 columns and with 64: 203 rows of a fresh prompt, 16 / 8 heads, 9.2, 7.6; 64 rows, 64 / 8 heads,
 // 5.3, 4.4; 128 rows over 2048 tokens 40.1, 30.5; 32 / 8 heads of 64, 256 rows 7.3, 5.8. With more
 // workgroups the K and V tiles staged twice cost as much as that saves (400 rows, 64 / 8 heads: 200 workgroups).

@@ -1196,8 +1196,9 @@ __global__ __launch_bounds__(kTiledWaves *kWave, kWgPerCu) void varlen_prefill_t
 // compute unit is a lone wavefront per SIMD, whose softmax and barrier waits nothing covers; this gives
 // every SIMD two and halves the chain of tiles. The groups meet in LDS, where key slices (separate
 // workgroups) pay for partial rows in memory and a merge launch. One request's chunk of 512 rows, 64 / 8
-// heads, over 7601 cached tokens: 159 -> 132 us (826 -> 994 TFLOP/s); 32 / 8 heads of 64, over 8192: 107 ->
-// 85. Bound by the tile loop's instruction mix, as the launch of many workgroups is.
+// heads, over 7601 cached tokens: 159 -> 132 us (826 -> 994 TFLOP/s); 1008 rows, 32 / 8 heads of 64, over 7177: 105 ->
+// 89; 256 workgroups, 64 / 8 heads: 1.1 us a key tile with one group, 1.0 with two. Bound by the tile loop's
+// instruction mix, as the launch of many workgroups is.
 template <int MODE>
 __global__ __launch_bounds__(2 * kTiledWaves *kWave, 2) void varlen_prefill_two_group_kernel(
     const half_t *__restrict__ q, int64_t q_stride, half_t *__restrict__ out, int64_t out_stride,

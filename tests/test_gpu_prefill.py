@@ -322,10 +322,10 @@ def test_key_slices_are_chosen_for_launches_that_leave_the_device_idle():
     # 512 rows x 64/8 heads = 32 row blocks x 8 kv heads = 256 workgroups on 2 per compute unit
     assert rule(1, 64, 8, 128, 128, 32768) >= 4
     if cus == 256:
-        assert rule(1, 64, 8, 128, 512, 32768 + 512) == 2         # measured 609 -> 551 us
+        assert rule(1, 64, 8, 128, 512, 32768 + 512) == 2         # measured 609 -> 551 us; in two groups of wavefronts 468 uncut, 479 in two slices
         assert rule(1, 64, 8, 128, 128, 32768) == 8               # 64 workgroups: eight slices fill the slots
-        assert rule(1, 64, 8, 128, 128, 2048 + 128) == 4           # measured 40 -> 30 us
-        assert rule(1, 64, 8, 128, 64, 8192 + 64) == 8             # measured 130 -> 36 us
+        assert rule(1, 64, 8, 128, 128, 2048 + 128) == 4           # measured 40 -> 30 us (64 columns a workgroup: 30, 25 to 30)
+        assert rule(1, 64, 8, 128, 64, 8192 + 64) == 8             # measured 130 -> 36 us (64 columns: 102 uncut)
     assert rule(4, 64, 8, 128, 512, 32768) == 1                    # four such chunks fill it
     assert rule(1, 64, 8, 128, 512, 700) == 1                      # too few keys to share out
     assert rule(1, 64, 8, 128, 512, 2048 + 512) == 1               # two slices would not pay (49 -> 60 us)
