@@ -297,28 +297,51 @@ __device__ __forceinline__ void attend_page(HeadState &st, const PageRegsQ8<KV> 
 // beside each other, with one maximum, one look at the reference maximum and half as many MFMAs in
 // the second product, whose k index runs over both pages: k = 8g + i is token 4g + i of page p for
 // i < 4 and of page p + 1 behind. `keys(u)` gives page u's K fragments, `stage_v(u, tail)` writes its
-// V rows; page u's registers are free where `refill(u)` is called, before page 1's are waited for.
-template <typename Keys, typename StageV, typename Refill>
+// V rows; page u's registers are free where `refill(u)` is called: BY_PAGE page 0's before page 1's are
+// waited for, else both behind the scores of both.
+template <bool BY_PAGE, typename Keys, typename StageV, typename Refill>
 __device__ __forceinline__ void attend_pair_core(HeadState &st, const half8_t (&qf)[4], const half_t *vt_lane, int p,
                                                  int end, int g, float scale_log2, Keys keys, StageV stage_v,
                                                  Refill refill) {
   const bool tail = (p + 2) * kPageSize > end;  // wavefront-uniform
   wave_lds_fence();
   float4_t s[2], s1[2];
+  if constexpr (BY_PAGE) {
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    stage_v(u, tail);
-    half8_t kf[4];
-    keys(u, kf);
-    s[u] = mfma_16x16x32(kf[0], qf[0], float4_t{0.f, 0.f, 0.f, 0.f});
-    s1[u] = mfma_16x16x32(kf[kKSteps / 2], qf[kKSteps / 2], float4_t{0.f, 0.f, 0.f, 0.f});
-    if constexpr (kKSteps == 4) {
-      s[u] = mfma_16x16x32(kf[1], qf[1], s[u]);
-      s1[u] = mfma_16x16x32(kf[3], qf[3], s1[u]);
+    for (int u = 0; u < 2; ++u) {
+      stage_v(u, tail);
+      half8_t kf[4];
+      keys(u, kf);
+      s[u] = mfma_16x16x32(kf[0], qf[0], float4_t{0.f, 0.f, 0.f, 0.f});
+      s1[u] = mfma_16x16x32(kf[kKSteps / 2], qf[kKSteps / 2], float4_t{0.f, 0.f, 0.f, 0.f});
+      if constexpr (kKSteps == 4) {
+        s[u] = mfma_16x16x32(kf[1], qf[1], s[u]);
+        s1[u] = mfma_16x16x32(kf[3], qf[3], s1[u]);
+      }
+      refill(u);
     }
-    refill(u);
+    wave_lds_fence();
+  } else {
+    stage_v(0, tail);
+    stage_v(1, tail);
+    wave_lds_fence();
+    half8_t ka[4], kb[4];
+    keys(0, ka);
+    keys(1, kb);
+    const float4_t zero = float4_t{0.f, 0.f, 0.f, 0.f};
+    s[0] = mfma_16x16x32(ka[0], qf[0], zero);
+    s[1] = mfma_16x16x32(kb[0], qf[0], zero);
+    s1[0] = mfma_16x16x32(ka[kKSteps / 2], qf[kKSteps / 2], zero);
+    s1[1] = mfma_16x16x32(kb[kKSteps / 2], qf[kKSteps / 2], zero);
+    if constexpr (kKSteps == 4) {
+      s[0] = mfma_16x16x32(ka[1], qf[1], s[0]);
+      s[1] = mfma_16x16x32(kb[1], qf[1], s[1]);
+      s1[0] = mfma_16x16x32(ka[3], qf[3], s1[0]);
+      s1[1] = mfma_16x16x32(kb[3], qf[3], s1[1]);
+    }
+    refill(0);
+    refill(1);
   }
-  wave_lds_fence();
   float sv[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) sv[i] = (s[i >> 2][i & 3] + s1[i >> 2][i & 3]) * scale_log2;
@@ -363,11 +386,11 @@ __device__ __forceinline__ void attend_pair_core(HeadState &st, const half8_t (&
   }
 }
 
-template <typename Refill>
+template <bool BY_PAGE = true, typename Refill>
 __device__ __forceinline__ void attend_pair(HeadState &st, const PageRegs &r0, const PageRegs &r1,
                                             const half8_t (&qf)[4], half_t *vstage, const half_t *vt_lane, int p,
                                             int end, int n, int g, float scale_log2, Refill refill) {
-  attend_pair_core(st, qf, vt_lane, p, end, g, scale_log2, [&](int u, half8_t (&kf)[4]) {
+  attend_pair_core<BY_PAGE>(st, qf, vt_lane, p, end, g, scale_log2, [&](int u, half8_t (&kf)[4]) {
 #pragma unroll
     for (int kk = 0; kk < kKSteps; ++kk) kf[kk] = u == 0 ? r0.k[kk] : r1.k[kk];
   }, [&](int u, bool tail) {
@@ -382,11 +405,11 @@ __device__ __forceinline__ void attend_pair(HeadState &st, const PageRegs &r0, c
   }, refill);
 }
 
-template <int KV, typename Refill>
+template <bool BY_PAGE = true, int KV, typename Refill>
 __device__ __forceinline__ void attend_pair(HeadState &st, const PageRegsQ8<KV> &r0, const PageRegsQ8<KV> &r1,
                                             const half8_t (&qf)[4], half_t *vstage, const half_t *vt_lane, int p,
                                             int end, int n, int g, float scale_log2, Refill refill) {
-  attend_pair_core(st, qf, vt_lane, p, end, g, scale_log2, [&](int u, half8_t (&kf)[4]) {
+  attend_pair_core<BY_PAGE>(st, qf, vt_lane, p, end, g, scale_log2, [&](int u, half8_t (&kf)[4]) {
 #pragma unroll
     for (int kk = 0; kk < kKSteps; ++kk) {
       const uint4_t x = u == 0 ? r0.k[kk >> 1] : r1.k[kk >> 1];
@@ -624,7 +647,9 @@ extern __shared__ __attribute__((aligned(16))) half_t split_vstage[];  // [waves
 // wavefront 160 -> 112 us, 16 splits 18.6 -> 14.5).
 //
 // One step's pages are in flight, a page's registers requested again as soon as its scores are under way
-// and its V is in LDS, while the other page is still on its way. DEEP: two steps' pages, requested again
+// and its V is in LDS, while the other page is still on its way. (Long splits of fp16 rows, ORDERED: both pages'
+// together, which streams better: 128 sequences of 8k to 32k tokens, 32 / 4 heads, 16 splits 840 us page by page, 831;
+// one long sequence among 63 short ones 47.5, 48.7.) DEEP: two steps' pages, requested again
 // after the step: longer ahead, at two wavefronts per SIMD. Both give the same bits. The steps behind
 // which a split has nothing left to request are written out behind the loops, and a split of one step
 // requests one: requests for nothing (16 bytes per lane of the last page, to keep the count of requests in
@@ -865,6 +890,7 @@ paged_decode_split_kernel(
     }
     attend_pair(st, buf[at], buf[at + 1], qf, vstage, vt_lane, p, end, n, g, scale_log2, no_refill);
   };
+  constexpr bool BY_PAGE = !(ORDERED && KV == kKvF16);
   // (A request left out inside a loop, under a condition, would leave the loop's waits without the count of
   // the requests behind the one they wait for.)
   int p = p0;
@@ -885,9 +911,9 @@ paged_decode_split_kernel(
     }
   } else {
     for (; p + 2 < p1; p += 2) {
-      attend_pair(st, buf[0], buf[1], qf, vstage, vt_lane, p, end, n, g, scale_log2, [&](int u) {
+      attend_pair<BY_PAGE>(st, buf[0], buf[1], qf, vstage, vt_lane, p, end, n, g, scale_log2, [&](int u) {
         request(p + 2 + u, buf[u]);
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (BY_PAGE) __builtin_amdgcn_sched_barrier(0);
       });
     }
     last_pair(p, first_pair);
