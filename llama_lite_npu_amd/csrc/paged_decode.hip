@@ -649,7 +649,7 @@ extern __shared__ __attribute__((aligned(16))) half_t split_vstage[];  // [waves
 // One step's pages are in flight, a page's registers requested again as soon as its scores are under way
 // and its V is in LDS, while the other page is still on its way. (Long splits of fp16 rows, ORDERED: both pages'
 // together, which streams better: 128 sequences of 8k to 32k tokens, 32 / 4 heads, 16 splits 840 us page by page, 831;
-// one long sequence among 63 short ones 47.5, 48.7.) DEEP: two steps' pages, requested again
+// one long sequence among 63 short ones 46.7, 48.7.) DEEP: two steps' pages, requested again
 // after the step: longer ahead, at two wavefronts per SIMD. Both give the same bits. The steps behind
 // which a split has nothing left to request are written out behind the loops, and a split of one step
 // requests one: requests for nothing (16 bytes per lane of the last page, to keep the count of requests in
