@@ -33,7 +33,7 @@ static int validate_prefill(const char *what, const void *q, int64_t q_stride, c
 // (16-byte stores of the output, 32-bit offsets into q) and scales its arithmetic is not made for
 // (tile_scale: 0, below 0, not a number), which stay with the general kernel. Four prompts of 300
 // to 2048 tokens, 16 / 4 heads: 9198 us there, without matrix instructions and with every K row
-// read by one lane at a time, 82 us here.
+// read by one lane at a time, 76 us here.
 [[maybe_unused]] static bool tiled_256(int64_t q_stride, int64_t out_stride, int32_t num_kv_heads,
                                        float softmax_scale) {
   return q_stride < (1 << 25) && out_stride % 8 == 0 && num_kv_heads <= 1024 &&
@@ -358,7 +358,7 @@ static int launch_paged_prefill(const char *what, const void *q, int64_t q_token
       return;
     }
 #endif
-    with(varlen_prefill_tiled_kernel<MODE>, kTiledWaves);
+    with(varlen_prefill_tiled_kernel<MODE>, prefill_waves(MODE));
   };
   if (format == kKvInt8) {
     launch(std::integral_constant<int, kPagedPrefillInt8>{});
@@ -456,7 +456,7 @@ static int launch_varlen_prefill(const void *q, int64_t q_token_stride, const vo
     return check_launch("varlen_prefill");
   }
 #endif
-  launch(varlen_prefill_tiled_kernel<kPackedPrefill>, kTiledWaves);
+  launch(varlen_prefill_tiled_kernel<kPackedPrefill>, prefill_waves(kPackedPrefill));
   return check_launch("varlen_prefill");
 }
 }  // namespace LITEKV_HD_NS

@@ -1,5 +1,5 @@
 // The column tiles of a 256-wide prefill that the matrix pipeline of prefill_tile.h does not serve:
-// 16 neighbouring query rows of one query head, in fp32 without matrix instructions, as the general
+// neighbouring query rows of one query head (a tile has 16), in fp32 without matrix instructions, as the general
 // kernel (generic_attention.hip) computes them, whatever the scale and the values are. Run by one
 // whole wavefront in the place of its tile.
 //
@@ -15,8 +15,8 @@ namespace litekv {
 namespace prefill_rows {
 
 constexpr int kDim = 256;
-constexpr int kRows = 16;
-constexpr int kLdsBytes = (kRows * kDim + kWave * (kRows + 1)) * 4;  // per wavefront: 20.6 KiB
+// Per wavefront: 20.6 KiB for 16 rows attended together, 10.3 for 8. (A row's result does not depend on it.)
+constexpr int lds_bytes(int rows) { return (rows * kDim + kWave * (rows + 1)) * 4; }
 
 typedef __attribute__((address_space(3))) float lds_float_t;
 
@@ -27,16 +27,16 @@ __device__ __forceinline__ void lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// q, out: the tile's first row (`rows` of them, 1 .. 16); that row sees keys 0 .. keys0 - 1, each
+// q, out: the first row (`rows` of them, 1 .. ROWS); that row sees keys 0 .. keys0 - 1, each
 // further row one key more. kv_row(token, value): address of the token's K or V row of the kv head
-// (fp16, or codes of format KV). lds: kLdsBytes bytes of this wavefront's own.
-template <int KV, typename KvRow>
+// (fp16, or codes of format KV). lds: lds_bytes(ROWS) bytes of this wavefront's own.
+template <int KV, int ROWS, typename KvRow>
 __device__ __forceinline__ void attend_rows(uint32_t lds, const half_t *q, int64_t q_stride, half_t *out,
                                             int64_t out_stride, int rows, int keys0, KvRow kv_row,
                                             float scale_log2, float k_scale, float v_scale) {
   const int lane = threadIdx.x & (kWave - 1);
-  lds_float_t *qs = (lds_float_t *)(uintptr_t)lds;                         // [kRows][kDim]
-  lds_float_t *ps = (lds_float_t *)(uintptr_t)(lds + 4u * kRows * kDim);   // [kWave][kRows + 1]
+  lds_float_t *qs = (lds_float_t *)(uintptr_t)lds;                         // [ROWS][kDim]
+  lds_float_t *ps = (lds_float_t *)(uintptr_t)(lds + 4u * ROWS * kDim);   // [kWave][ROWS + 1]
   auto load8 = [&](const void *row, int d8) -> half8_t {
     if constexpr (KV == kKvF16) {
       return *((const half8_t *)row + d8);
@@ -46,7 +46,7 @@ __device__ __forceinline__ void attend_rows(uint32_t lds, const half_t *q, int64
   };
   lds_fence();
 #pragma unroll
-  for (int r = 0; r < kRows; ++r) {  // rows past the last repeat it and are not written
+  for (int r = 0; r < ROWS; ++r) {  // rows past the last repeat it and are not written
     const half_t *row = q + (int64_t)(r < rows ? r : rows - 1) * q_stride;
 #pragma unroll
     for (int c = 0; c < kDim / kWave; ++c) {
@@ -54,9 +54,9 @@ __device__ __forceinline__ void attend_rows(uint32_t lds, const half_t *q, int64
     }
   }
   lds_fence();
-  float m[kRows], den[kRows], acc[kRows][kDim / kWave];
+  float m[ROWS], den[ROWS], acc[ROWS][kDim / kWave];
 #pragma unroll
-  for (int r = 0; r < kRows; ++r) {
+  for (int r = 0; r < ROWS; ++r) {
     m[r] = -INFINITY;
     den[r] = 0.f;
 #pragma unroll
@@ -66,19 +66,19 @@ __device__ __forceinline__ void attend_rows(uint32_t lds, const half_t *q, int64
   for (int t0 = 0; t0 < n_keys; t0 += kWave) {
     const int tok = t0 + lane;  // this lane's key
     const void *k_row = kv_row(tok < n_keys ? tok : n_keys - 1, false);
-    float s[kRows];
+    float s[ROWS];
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) s[r] = 0.f;
+    for (int r = 0; r < ROWS; ++r) s[r] = 0.f;
     for (int d8 = 0; d8 < kDim / 8; ++d8) {
       const half8_t k8 = load8(k_row, d8);
 #pragma unroll
-      for (int r = 0; r < kRows; ++r) {
+      for (int r = 0; r < ROWS; ++r) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) s[r] += qs[r * kDim + 8 * d8 + e] * (float)k8[e];
       }
     }
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) {
+    for (int r = 0; r < ROWS; ++r) {
       // key 0 is in every row's first step: the running maximum is the maximum of real scores
       const float sv = tok < keys0 + (r < rows ? r : rows - 1) ? s[r] * k_scale : -INFINITY;
       float mx = sv;
@@ -94,7 +94,7 @@ __device__ __forceinline__ void attend_rows(uint32_t lds, const half_t *q, int64
       m[r] = m_new;
 #pragma unroll
       for (int c = 0; c < kDim / kWave; ++c) acc[r][c] *= alpha;
-      ps[lane * (kRows + 1) + r] = p;
+      ps[lane * (ROWS + 1) + r] = p;
     }
     lds_fence();
     const int n_here = n_keys - t0 < kWave ? n_keys - t0 : kWave;
@@ -107,10 +107,10 @@ __device__ __forceinline__ void attend_rows(uint32_t lds, const half_t *q, int64
         v[c] = (float)load8(v_row, d / 8)[d % 8];
       }
 #pragma unroll
-      for (int r = 0; r < kRows; ++r) {
+      for (int r = 0; r < ROWS; ++r) {
         // (a probability of 0 does not keep an infinite value out: 0 * inf is NaN)
         const bool sees = t0 + j < keys0 + (r < rows ? r : rows - 1);
-        const float p = ps[j * (kRows + 1) + r];
+        const float p = ps[j * (ROWS + 1) + r];
 #pragma unroll
         for (int c = 0; c < kDim / kWave; ++c) acc[r][c] += sees ? p * v[c] : 0.f;
       }
@@ -118,7 +118,7 @@ __device__ __forceinline__ void attend_rows(uint32_t lds, const half_t *q, int64
     lds_fence();
   }
 #pragma unroll
-  for (int r = 0; r < kRows; ++r) {
+  for (int r = 0; r < ROWS; ++r) {
     if (r < rows) {
       const float inv = v_scale / den[r];
 #pragma unroll

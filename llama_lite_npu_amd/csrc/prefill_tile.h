@@ -143,7 +143,7 @@ struct PackedSource {
 
 constexpr int kKvTile = 64;
 constexpr int kColTiles = 2;      // 16-column tiles per wavefront
-constexpr int kTiledWaves = 4;    // wavefronts of a prefill workgroup
+constexpr int kTiledWaves = 4;    // wavefronts of a prefill workgroup (see prefill_waves)
 constexpr int kWideWaves = 8;     // a shared prefix: twice the columns on every staged K/V tile (prefill: 2 to 5 % slower)
 constexpr int kWgColTiles = kColTiles * kTiledWaves;
 constexpr int kTileHalfs = kKvTile * kHD;  // one staged tile: 64 rows of 2 * kHD bytes
@@ -169,9 +169,22 @@ constexpr int kPagedPrefill = 0, kPackedPrefill = 1, kSharedPrefix = 2, kPagedPr
 // each; a slice leaves a normalised fp32 partial row + log-sum-exp per (query row, head), and a
 // merge launch folds the slices of a row (prefill_split_merge_kernel in paged_prefill.hip).
 
+// Column tiles per wavefront and wavefronts per workgroup of a prefill of 128 columns. Head dim 256 leaves one
+// workgroup per CU (LDS), which as four wavefronts of two column tiles is a lone wavefront per SIMD: its
+// softmax, LDS latencies and barrier waits stand in the open (MFMA busy 45 %). Eight wavefronts of one column tile
+// are two per SIMD at 256 registers; every K and V fragment then feeds one column tile instead of two, and the
+// 512 KiB a tile of keys reads from LDS (128 bytes a cycle) bound it: 2.3 us a tile, 2.5 before. Kernel time, 16 / 4
+// heads, four to eight wavefronts: 4 prompts of 459 to 1951 tokens 82 -> 76 us; passes with the epilogue, 300 tokens
+// 26.3 -> 21.9, 16 x 500..700 153 -> 132, 64 rows over 2000 cached tokens 54.5 -> 48.3. Codes keep four: their conversion
+// needs the registers (eight spill, and take 0.98 to 1.02 of the time).
+constexpr int prefill_ct(int mode) {
+  return kHD == 256 && (mode == kPagedPrefill || mode == kPackedPrefill) ? 1 : kColTiles;
+}
+constexpr int prefill_waves(int mode) { return kWgColTiles / prefill_ct(mode); }
+
 // Head dim 256: the 16 query rows of column tile t of a block (see prefill_tile_body, whose names these
 // are), in fp32 (prefill_rows.h); `lds` as there.
-template <int KV, bool PAGED>
+template <int KV, bool PAGED, int ROWS>
 __device__ __forceinline__ void tile_by_rows(uint32_t lds, const half_t *q, int64_t q_stride, half_t *out,
                                              int64_t out_stride, const PagedSource &paged,
                                              const PackedSource &packed, int b, int q_start, int q_len, int ctx,
@@ -198,10 +211,15 @@ __device__ __forceinline__ void tile_by_rows(uint32_t lds, const half_t *q, int6
     }
   };
   const int64_t at = (int64_t)hq * kHD;
-  prefill_rows::attend_rows<KV>(lds, q + (int64_t)(q_start + row0) * q_stride + at, q_stride,
-                                out + (int64_t)(q_start + row0) * out_stride + at, out_stride,
-                                q_len - row0 < 16 ? q_len - row0 : 16, ctx + row0 + 1, kv_row, scale_log2,
-                                CODES ? paged.scales[h] : 1.0f, CODES ? paged.scales[paged.num_kv_heads + h] : 1.0f);
+  const int rows = q_len - row0 < 16 ? q_len - row0 : 16;
+#pragma unroll 1
+  for (int r = 0; r < rows; r += ROWS) {
+    prefill_rows::attend_rows<KV, ROWS>(lds, q + (int64_t)(q_start + row0 + r) * q_stride + at, q_stride,
+                                  out + (int64_t)(q_start + row0 + r) * out_stride + at, out_stride,
+                                  rows - r < ROWS ? rows - r : ROWS, ctx + row0 + r + 1,
+                                  kv_row, scale_log2, CODES ? paged.scales[h] : 1.0f,
+                                  CODES ? paged.scales[paged.num_kv_heads + h] : 1.0f);
+  }
 }
 
 // The body of the kernel, run by a workgroup of W wavefronts that stands at (block_x, block_y,
@@ -209,7 +227,7 @@ __device__ __forceinline__ void tile_by_rows(uint32_t lds, const half_t *q, int6
 // staging area (tile_lds_bytes<W>() bytes, 1 KiB aligned). A function, so that the decode step
 // with a shared prefix can run it as one role of its launch (paged_decode.hip).
 template <int W>
-constexpr int tile_lds_bytes() { return (W == kWideWaves ? 6 : 4) * kTileHalfs * 2; }
+constexpr int tile_lds_bytes() { return (W == kWideWaves && kHD != 256 ? 6 : 4) * kTileHalfs * 2; }
 
 template <int MODE, int W, int KG = 1, int CT = kColTiles>
 __device__ __forceinline__ void prefill_tile_body(
@@ -237,12 +255,12 @@ __device__ __forceinline__ void prefill_tile_body(
   // (rows of 64 codes staged by 8 wavefronts would leave a lane 8 codes, half a 16-byte load)
   static_assert(W == kTiledWaves || (W == kWideWaves && (!FP8 || kHD == 128)),
                 "eight wavefronts: fp16 K/V, or 8-bit codes at head dim 128");
-  static_assert(kHD != 256 || (W == kTiledWaves && !KSPLIT && !SHARED), "256: plain prefill only");
+  static_assert(kHD != 256 || (W == prefill_waves(MODE) && CT == prefill_ct(MODE) && !KSPLIT && !SHARED), "256: plain prefill only");
   // Rows of a 64-key tile one wavefront stages (a page, or half of one), and the direct-load
   // instructions that takes per operand.
   constexpr int kRowsPerWave = kKvTile / W;
   constexpr int kLoads = kRowsPerWave / kRowsPerLoad;
-  static_assert(CT == kColTiles || (CT == 1 && KG == 1 && W == kTiledWaves && !SHARED && kHD != 256),
+  static_assert(CT == kColTiles || (CT == 1 && KG == 1 && W == (kHD == 256 ? kWideWaves : kTiledWaves) && !SHARED),
                 "one column tile a wavefront: a prefill");
   static_assert(KG == 1 || (KG == 2 && W == kTiledWaves && !KSPLIT && !SHARED && kHD != 256), "two key groups: a prefill");
   const int wave_in_wg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -357,11 +375,12 @@ __device__ __forceinline__ void prefill_tile_body(
 
   // a wavefront's own quarter of the staging area, for what it does before and after the tiles
   constexpr uint32_t kOwnLds = (uint32_t)tile_lds_bytes<W>() / W;
-  static_assert(kHD != 256 || prefill_rows::kLdsBytes <= kOwnLds, "a tile by rows fits a wavefront's part");
+  constexpr int kByRows = W == kWideWaves ? 8 : 16;  // rows of a tile attended together where it goes by rows
+  static_assert(kHD != 256 || prefill_rows::lds_bytes(kByRows) <= kOwnLds, "rows attended together fit a wavefront's part");
   if constexpr (kHD == 256 && FP8) {
     if (!tile_scale(k_mul)) {  // the K scale's doing: the launch looked at softmax_scale itself
       for (int t = wave * CT; t < (wave + 1) * CT; ++t) {
-        tile_by_rows<KV, PAGED>(k_lds + wave * kOwnLds, q, q_stride, out, out_stride, paged, packed, b, q_start, q_len,
+        tile_by_rows<KV, PAGED, kByRows>(k_lds + wave * kOwnLds, q, q_stride, out, out_stride, paged, packed, b, q_start, q_len,
                                 ctx, m0, t, row_tiles, head0, heads_here, group, h, scale_log2);
       }
       return;
@@ -483,8 +502,9 @@ __device__ __forceinline__ void prefill_tile_body(
   // the fragments are read back from there. Requested before tile 0: vmcnt counts in order.
   uint32_t q_lds = 0;
   if constexpr (!SHARED) {
-    static_assert(SHARED || W == kTiledWaves, "the q rows of four wavefronts fit a tile half of K and of V");
-    q_lds = ((wave & 2) ? v_lds : k_lds) + (uint32_t)(kTileHalfs * 2 + (wave & 1) * (64 * kHD));
+    static_assert(16 * CT * W <= 2 * kKvTile, "the q rows of the wavefronts fit a tile half of K and of V");
+    q_lds = ((wave & (W / 2)) ? v_lds : k_lds) +
+            (uint32_t)(kTileHalfs * 2 + (wave & (W / 2 - 1)) * (kTileHalfs * 4 / W));
 #pragma unroll
     for (int u = 0; u < CT; ++u) {
       const int t = wave * CT + u;
@@ -580,26 +600,31 @@ __device__ __forceinline__ void prefill_tile_body(
   // Swizzled read addresses (LDS bytes) for the tile half in use; they flip between the halves
   // once per tile.
   // K, A operand of S^T: row 16m + n, chunk (4kk + g) ^ n.
-  uint32_t k_addr[kKSteps];
+  // (Rows of 512 bytes: the swizzle stays inside a 256-byte half, so the second half's addresses are
+  // the first's plus a constant.)
+  constexpr int kKAddrs = kHD == 256 ? kKSteps / 2 : kKSteps, kVAddrs = kHD == 256 ? kJTiles / 2 : kJTiles;
+  uint32_t k_addr[kKAddrs];
 #pragma unroll
-  for (int kk = 0; kk < kKSteps; ++kk) {
+  for (int kk = 0; kk < kKAddrs; ++kk) {
     k_addr[kk] = k_lds + 2u * (uint32_t)(n * kHD + 8 * ((4 * kk + g) ^ k_swz(n)));
   }
   // V^T, A operand of O^T: row 32 s2 + 4g + n/4 (+16), halfs 16j + 4(n%4); chunk pair j ^ (r%8).
   const int v_row = 4 * g + (n >> 2);
-  uint32_t v_addr[kJTiles];
+  uint32_t v_addr[kVAddrs];
 #pragma unroll
-  for (int j = 0; j < kJTiles; ++j) {
+  for (int j = 0; j < kVAddrs; ++j) {
     v_addr[j] = v_lds + 2u * (uint32_t)(v_row * kHD + 8 * ((2 * j) ^ v_swz(v_row)) + 4 * (n & 3));
   }
   int flip = kTileHalfs * 2;  // bytes to the other half
   auto flip_halves = [&]() {
 #pragma unroll
-    for (int kk = 0; kk < kKSteps; ++kk) k_addr[kk] += flip;
+    for (int kk = 0; kk < kKAddrs; ++kk) k_addr[kk] += flip;
 #pragma unroll
-    for (int j = 0; j < kJTiles; ++j) v_addr[j] += flip;
+    for (int j = 0; j < kVAddrs; ++j) v_addr[j] += flip;
     flip = -flip;
   };
+  auto k_at = [&](int kk) -> uint32_t { return k_addr[kk % kKAddrs] + 256u * (uint32_t)(kk / kKAddrs); };
+  auto v_at = [&](int j) -> uint32_t { return v_addr[j % kVAddrs] + 256u * (uint32_t)(j / kVAddrs); };
 
   float4_t st[2][CT];
   half8_t pk[CT];
@@ -615,7 +640,7 @@ __device__ __forceinline__ void prefill_tile_body(
 #pragma unroll
       for (int kk = 0; kk < kKSteps; ++kk) {
         const half8_t a =
-            *(const lds_half8_t *)(uintptr_t)(k_addr[kk] + 2u * (32 * s2 + 16 * m) * kHD);
+            *(const lds_half8_t *)(uintptr_t)(k_at(kk) + 2u * (32 * s2 + 16 * m) * kHD);
 #pragma unroll
         for (int u = 0; u < CT; ++u) st[m][u] = mfma_16x16x32(a, qf[u][kk], st[m][u]);
       }
@@ -707,7 +732,7 @@ __device__ __forceinline__ void prefill_tile_body(
     for (int u = 0; u < CT; ++u) dsum[u] = mfma_p(ones, pk[u], pk_lo[u], dsum[u]);
 #pragma unroll
     for (int j = 0; j < kJTiles; ++j) {
-      const uint32_t at = v_addr[j] + 2u * 32 * s2 * kHD;
+      const uint32_t at = v_at(j) + 2u * 32 * s2 * kHD;
       const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t *)(uintptr_t)at);
       const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
           (lds_short4_t *)(uintptr_t)(at + 2u * 16 * kHD));
@@ -719,7 +744,7 @@ __device__ __forceinline__ void prefill_tile_body(
   };
   // V^T fragment j (A operand: d rows 16j.., keys 32 s2 + {4g..4g+3, 16+4g..}) of the staged tile.
   auto load_vfrag = [&](int j, int s2) -> half8_t {
-    const uint32_t at = v_addr[j] + 2u * 32 * s2 * kHD;
+    const uint32_t at = v_at(j) + 2u * 32 * s2 * kHD;
     const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t *)(uintptr_t)at);
     const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
         (lds_short4_t *)(uintptr_t)(at + 2u * 16 * kHD));
@@ -868,7 +893,7 @@ __device__ __forceinline__ void prefill_tile_body(
       // MFMAs, and the first half's V fragments requested before the block ends.
       // Region 1: all eight K fragments of the first half are requested at once.
       auto load_kfrag = [&](int s2, int i) -> half8_t {   // fragment i = (kk = i / 2, m = i % 2)
-        return *(const lds_half8_t *)(uintptr_t)(k_addr[i >> 1] + 2u * (32 * s2 + 16 * (i & 1)) * kHD);
+        return *(const lds_half8_t *)(uintptr_t)(k_at(i >> 1) + 2u * (32 * s2 + 16 * (i & 1)) * kHD);
       };
       half8_t kf[kJTiles];
 #pragma unroll
@@ -1094,7 +1119,7 @@ __device__ __forceinline__ void prefill_tile_body(
         __builtin_amdgcn_s_waitcnt(wait_vm(0));  // the rows' first stores come first
 #pragma unroll 1
         for (int u = 0; u < CT; ++u) {
-          tile_by_rows<FP8 ? KV : kKvF16, PAGED>(mine, q, q_stride, out, out_stride, paged, packed, b, q_start, q_len, ctx,
+          tile_by_rows<FP8 ? KV : kKvF16, PAGED, kByRows>(mine, q, q_stride, out, out_stride, paged, packed, b, q_start, q_len, ctx,
                                                  m0, wave * CT + u, row_tiles, head0, heads_here, group, h, scale_log2);
         }
       }
@@ -1166,25 +1191,25 @@ __device__ __forceinline__ void prefill_tile_body(
 
 // CT: column tiles per wavefront. One instead of two, 64 score columns a workgroup, for launches that would
 // leave most of the device idle (see narrow_fits in paged_prefill.hip). Bound by the chain of its few key tiles.
-template <int MODE, int CT = kColTiles>
-__global__ __launch_bounds__(kTiledWaves *kWave, kWgPerCu) void varlen_prefill_tiled_kernel(
+template <int MODE, int CT = prefill_ct(MODE)>
+__global__ __launch_bounds__(prefill_waves(MODE) * kWave, kWgPerCu *prefill_waves(MODE) / kTiledWaves) void varlen_prefill_tiled_kernel(
     const half_t *__restrict__ q, int64_t q_stride, half_t *__restrict__ out, int64_t out_stride,
     PagedSource paged, PackedSource packed, PrefixTask prefix,
     const int32_t *__restrict__ q_starts_or_cu, const int32_t *__restrict__ q_lens_or_null,
     const int32_t *__restrict__ context_lens, int32_t group, int32_t head_splits,
     int32_t heads_per_wg, int32_t row_tiles, float scale_log2, int32_t key_slices) {
-  __shared__ __attribute__((aligned(1024))) half_t lds_all[tile_lds_bytes<kTiledWaves>() / 2];
+  __shared__ __attribute__((aligned(1024))) half_t lds_all[tile_lds_bytes<prefill_waves(MODE)>() / 2];
   if constexpr (MODE == kPagedPrefillSplit || MODE == kPagedPrefillSplitFp8 ||
                 MODE == kPagedPrefillSplitInt8) {
     // blockIdx.y = row block * key_slices + slice: the slices of a block are neighbours
     const int by = (int)blockIdx.y / key_slices;
-    prefill_tile_body<MODE, kTiledWaves, 1, CT>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, by,
+    prefill_tile_body<MODE, prefill_waves(MODE), 1, CT>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, by,
                                (int)blockIdx.z, (int)gridDim.y / key_slices, q, q_stride, out, out_stride,
                                paged, packed, prefix, q_starts_or_cu, q_lens_or_null, context_lens, group,
                                head_splits, heads_per_wg, row_tiles, scale_log2,
                                (int)blockIdx.y - by * key_slices, key_slices);
   } else {
-    prefill_tile_body<MODE, kTiledWaves, 1, CT>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, (int)blockIdx.y,
+    prefill_tile_body<MODE, prefill_waves(MODE), 1, CT>((uint32_t)(uintptr_t)(lds_half_t *)lds_all, (int)blockIdx.x, (int)blockIdx.y,
                                (int)blockIdx.z, (int)gridDim.y, q, q_stride, out, out_stride, paged, packed,
                                prefix, q_starts_or_cu, q_lens_or_null, context_lens, group, head_splits,
                                heads_per_wg, row_tiles, scale_log2);

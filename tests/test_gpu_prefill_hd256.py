@@ -50,6 +50,21 @@ def test_tiled_prefill_256(hq, hkv, lens, ctx, page_size):
         assert torch.equal(outs[0], packed)
 
 
+@pytest.mark.parametrize("hq,hkv", [(1, 1), (6, 2), (8, 2), (8, 1)])
+def test_row_blocks_of_every_fill_256(hq, hkv):
+    """One column tile per wavefront: blocks of 128, 32 and 16 rows, filled from one row to all, and a
+    prompt whose rows end a tile of keys early, on it and behind it. Bound as above."""
+    lens = [1, 15, 16, 17, 32, 33, 63, 64, 65, 127, 128, 129, 193]
+    print(f"prefill 256 {hq}/{hkv}, every fill of a block", flush=True)
+    case = workloads.make_prefill_case("p256", 5250 + hq + hkv, lens, hq, hkv, device=DEV, head_dim=D)
+    ops.kv_append(case.k, case.v, case.slot_mapping, case.kv_pool)
+    out = ops.paged_prefill(case.q, case.kv_pool, case.block_table, case.cu_q_lens, None, case.max_q_len,
+                            case.softmax_scale)
+    torch.cuda.synchronize()
+    ref = torch.from_numpy(_oracle(case, to_np16(case.kv_pool)))
+    assert bool(((out.float().cpu() - ref).abs() <= 2.0 ** -11 * ref.abs() + 2e-5).all())
+
+
 @pytest.mark.parametrize("fmt", ["fp8", "int8"])
 @pytest.mark.parametrize("lens,ctx,page_size", [([200, 1, 64], [300, 47, 0], 16), ([129], [640], 64)])
 def test_tiled_chunk_prefill_256_of_codes(fmt, lens, ctx, page_size):

@@ -83,7 +83,8 @@ def _rows_with_values(out, ref, key, element, want, group):
 
 
 @pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
-@pytest.mark.parametrize("hq,length,key", [(16, 200, 40), (16, 200, 130), (8, 190, 0), (28, 70, 69), (4, 150, 127)])
+@pytest.mark.parametrize("hq,length,key", [(16, 200, 40), (16, 200, 130), (8, 190, 0), (28, 70, 69), (4, 150, 127),
+                                               (16, 161, 3), (8, 169, 168)])
 def test_an_infinite_value_reaches_the_rows_that_see_it(hq, length, key, value):
     """V of one key, one element: rows from that key on get it (a weight is above 0 at these scores), no
     earlier row and no other element does, wherever the key stands in its tile."""
