@@ -78,17 +78,25 @@ __host__ __device__ __forceinline__ int splits_for_pages(int pages, int max_spli
   return n < max_splits ? n : max_splits;
 }
 
-// One page of an fp16 pool as this lane requested it.
+// One page of an fp16 pool as this lane requested it. A V row is 16 columns of 16 bytes at head dim 128, so a load of
+// the wavefront covers four rows; at 64 it is 8 columns, and a load covers eight (over codes: all sixteen). With
+// the lanes of 128, the upper half re-reading the lower half's columns, every V byte was loaded, converted and
+// staged twice. 32 / 8 heads of 64, a layer's decode, us before and now: fp16, 12 sequences of 100 to 3000 tokens 15.2,
+// 14.7, 64 of 2k to 8k 108.9, 106.7; int8, 64 of 2k to 8k 82.1, 72.9, 128 of 4k to 16k 313, 273.
+constexpr int kVLoads = kHD == 64 ? 2 : 4;
+constexpr int kVStep = kPageSize / kVLoads;  // rows between a lane's loads
+__device__ __forceinline__ int v_row_of(int n, int g) { return kHD == 64 ? 2 * g + (n >> 3) : g; }
+__device__ __forceinline__ int v_col_of(int n) { return 8 * (n & (kVCols - 1)); }  // in elements
 struct PageRegs {
-  half8_t k[4];  // A-operand fragments of K: token n, d = 32*kk + 8*g .. +7
-  half8_t v[4];  // V rows 4*i + g, 16-byte column n
+  half8_t k[4];        // A-operand fragments of K: token n, d = 32*kk + 8*g .. +7
+  half8_t v[kVLoads];  // V rows kVStep*i + v_row_of, columns v_col_of ..
 };
 
 // One page of a pool of 8-bit codes (fp8 or int8): the same bytes per lane in half as many loads. The sum over d of a
 // dot product may run in any order as long as K and q agree, so a lane takes 16 consecutive
 // codes per load and MFMA step kk uses its lower or upper 8:
 //   k[j]: token n, d = 16*(g + 4*j) .. +15      step kk = 2*j + (0: lower, 1: upper 8 codes)
-//   v[i]: V row 8*i + 2*g + n%2, d = 16*(n/2) .. +15
+//   v[i]: V row 8*i + 2*g + n%2, d = 16*(n/2) .. +15    (head dim 64: one load, row 4*g + n/4, d = 16*(n%4) ..)
 // Neighbouring lanes hold the same column of two neighbouring rows: the 32 bytes a lane stages per
 // row (16 codes as fp16) then fall on different LDS banks for the eight lanes a 16-byte store
 // serves per cycle. (With eight neighbouring lanes on one row, 32 bytes apart, every such store
@@ -96,12 +104,14 @@ struct PageRegs {
 template <int KV>
 struct PageRegsQ8 {
   uint4_t k[2];
-  uint4_t v[2];
+  uint4_t v[kHD == 64 ? 1 : 2];
 };
+constexpr int kQ8VLoads = kHD == 64 ? 1 : 2;
+constexpr int kQ8VStep = kPageSize / kQ8VLoads;
 
 // Storage of the pool a kernel reads: fp16, or the codes of format KV (kKvFp8, kKvInt8).
-__device__ __forceinline__ int q8_v_row(int n, int g) { return 2 * g + (n & 1); }  // inside its block of 8 rows
-__device__ __forceinline__ int q8_v_col(int n) { return n >> 1; }                 // in units of 16 codes
+__device__ __forceinline__ int q8_v_row(int n, int g) { return kHD == 64 ? 4 * g + (n >> 2) : 2 * g + (n & 1); }
+__device__ __forceinline__ int q8_v_col(int n) { return kHD == 64 ? n & 3 : n >> 1; }  // in units of 16 codes
 template <int KV> struct KvStore { typedef uint8_t elem; typedef PageRegsQ8<KV> page; };
 template <> struct KvStore<kKvF16> { typedef half_t elem; typedef PageRegs page; };
 
@@ -164,9 +174,9 @@ __device__ __forceinline__ void request_page(PageRegs &r, const half_t *k_lane,
 #pragma unroll
   for (int kk = 0; kk < kKSteps; ++kk) r.k[kk] = __builtin_nontemporal_load((const half8_t *)(kr + kk * k_step));
   const half_t *vr = dummy ? pool + page_off : v_lane + page_off;
-  const int64_t v_step = dummy ? 0 : 4 * row_stride;
+  const int64_t v_step = dummy ? 0 : kVStep * row_stride;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) r.v[i] = __builtin_nontemporal_load((const half8_t *)(vr + i * v_step));
+  for (int i = 0; i < kVLoads; ++i) r.v[i] = __builtin_nontemporal_load((const half8_t *)(vr + i * v_step));
 }
 
 // 8-bit pool: k_lane points at token n, code 16*g; v_lane at row q8_v_row, code 16*q8_v_col.
@@ -180,9 +190,9 @@ __device__ __forceinline__ void request_page(PageRegsQ8<KV> &r, const uint8_t *k
 #pragma unroll
   for (int j = 0; j < kHD / 64; ++j) r.k[j] = __builtin_nontemporal_load((const uint4_t *)(kr + j * k_step));
   const uint8_t *vr = dummy ? pool + page_off : v_lane + page_off;
-  const int64_t v_step = dummy ? 0 : 8 * row_stride;
+  const int64_t v_step = dummy ? 0 : kQ8VStep * row_stride;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) r.v[i] = __builtin_nontemporal_load((const uint4_t *)(vr + i * v_step));
+  for (int i = 0; i < kQ8VLoads; ++i) r.v[i] = __builtin_nontemporal_load((const uint4_t *)(vr + i * v_step));
 }
 
 // Folds page `p` (tokens 16p .. 16p+15 of a sequence of `len` tokens) into the state. `kf` are
@@ -255,11 +265,12 @@ __device__ __forceinline__ void attend_page(HeadState &st, const PageRegs &r,
                                             float scale_log2) {
   attend_core(st, r.k, qf, vt_lane, p, len, n, g, scale_log2, [&](bool tail) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < kVLoads; ++i) {
       half8_t x = r.v[i];
+      const int row = kVStep * i + v_row_of(n, g);
       // Slots past the sequence end hold arbitrary bits: keep them out of the MFMA.
-      if (tail && p * kPageSize + 4 * i + g >= len) x = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-      *(half8_t *)(&vstage[(4 * i + g) * kVPitch + 8 * n]) = x;
+      if (tail && p * kPageSize + row >= len) x = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      *(half8_t *)(&vstage[row * kVPitch + v_col_of(n)]) = x;
     }
   });
 }
@@ -276,8 +287,8 @@ __device__ __forceinline__ void attend_page(HeadState &st, const PageRegsQ8<KV> 
                          codes_to_half<KV>(uint2_t{r.k[1][2], r.k[1][3]})};
   attend_core(st, kf, qf, vt_lane, p, len, n, g, scale_log2, [&](bool tail) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = 8 * i + q8_v_row(n, g);
+    for (int i = 0; i < kQ8VLoads; ++i) {
+      const int row = kQ8VStep * i + q8_v_row(n, g);
       half8_t lo = codes_to_half<KV>(uint2_t{r.v[i][0], r.v[i][1]});
       half8_t hi = codes_to_half<KV>(uint2_t{r.v[i][2], r.v[i][3]});
       if (tail && p * kPageSize + row >= len) {
@@ -395,12 +406,12 @@ __device__ __forceinline__ void attend_pair(HeadState &st, const PageRegs &r0, c
     for (int kk = 0; kk < kKSteps; ++kk) kf[kk] = u == 0 ? r0.k[kk] : r1.k[kk];
   }, [&](int u, bool tail) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < kVLoads; ++i) {
       half8_t x = u == 0 ? r0.v[i] : r1.v[i];
-      const int row = u * kPageSize + 4 * i + g;
+      const int row = u * kPageSize + kVStep * i + v_row_of(n, g);
       // Slots past the end hold arbitrary bits: keep them out of the MFMA.
       if (tail && p * kPageSize + row >= end) x = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-      *(half8_t *)(&vstage[row * kVPitch + 8 * n]) = x;
+      *(half8_t *)(&vstage[row * kVPitch + v_col_of(n)]) = x;
     }
   }, refill);
 }
@@ -417,8 +428,8 @@ __device__ __forceinline__ void attend_pair(HeadState &st, const PageRegsQ8<KV> 
     }
   }, [&](int u, bool tail) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = u * kPageSize + 8 * i + q8_v_row(n, g);
+    for (int i = 0; i < kQ8VLoads; ++i) {
+      const int row = u * kPageSize + kQ8VStep * i + q8_v_row(n, g);
       const uint4_t v = u == 0 ? r0.v[i] : r1.v[i];
       half8_t lo = codes_to_half<KV>(uint2_t{v[0], v[1]});
       half8_t hi = codes_to_half<KV>(uint2_t{v[2], v[3]});
@@ -550,12 +561,12 @@ __device__ __forceinline__ void load_new_rows(uint4_t (&kr)[4], uint4_t (&vr)[2]
       kr[2 * j] = *(const uint4_t *)(kn + 64 * j + 16 * g);
       kr[2 * j + 1] = *(const uint4_t *)(kn + 64 * j + 16 * g + 8);
     }
-    vr[0] = *(const uint4_t *)(vn + 16 * (q8_v_col(n) & (kHD / 16 - 1)));
-    vr[1] = *(const uint4_t *)(vn + 16 * (q8_v_col(n) & (kHD / 16 - 1)) + 8);
+    vr[0] = *(const uint4_t *)(vn + 16 * q8_v_col(n));
+    vr[1] = *(const uint4_t *)(vn + 16 * q8_v_col(n) + 8);
   } else {
 #pragma unroll
     for (int kk = 0; kk < kKSteps; ++kk) kr[kk] = *(const uint4_t *)(kn + 32 * kk + 8 * g);
-    vr[0] = *(const uint4_t *)(vn + 8 * (n & (kVCols - 1)));
+    vr[0] = *(const uint4_t *)(vn + v_col_of(n));
     vr[1] = uint4_t{0, 0, 0, 0};  // fp8 only
   }
 }
@@ -782,9 +793,9 @@ paged_decode_split_kernel(
   const int64_t row_stride = (int64_t)2 * num_kv_heads * kHD;  // elements per slot
   // this lane's row and column inside page 0 (see PageRegs / PageRegsFp8)
   Elem *k_lane = kv + (int64_t)h * kHD + (FP8 ? 16 : 8) * g + n * row_stride;
-  Elem *v_lane = FP8 ? kv + (int64_t)(num_kv_heads + h) * kHD + 16 * (q8_v_col(n) & (kHD / 16 - 1)) +
+  Elem *v_lane = FP8 ? kv + (int64_t)(num_kv_heads + h) * kHD + 16 * q8_v_col(n) +
                            q8_v_row(n, g) * row_stride
-                     : kv + (int64_t)(num_kv_heads + h) * kHD + 8 * (n & (kVCols - 1)) + g * row_stride;
+                     : kv + (int64_t)(num_kv_heads + h) * kHD + v_col_of(n) + v_row_of(n, g) * row_stride;
   const half_t *vt_lane = &vstage[(4 * g + (n >> 2)) * kVPitch + 4 * (n & 3)];
   const int32_t *table = row_of_table();
 
@@ -857,14 +868,14 @@ paged_decode_split_kernel(
               *(uint4_t *)(dst + 64 * j) = x;
             }
           }
-          if (q8_v_row(n, g) == (t_new & 7)) {
+          if (q8_v_row(n, g) == (t_new & (kQ8VStep - 1))) {
             const uint2_t lo = half_to_codes<KV>(__builtin_bit_cast(half8_t, v_row[0]), v_inv);
             const uint2_t hi = half_to_codes<KV>(__builtin_bit_cast(half8_t, v_row[1]), v_inv);
             const uint4_t x = uint4_t{lo[0], lo[1], hi[0], hi[1]};
-            *(uint4_t *)(kv + slot_off + (int64_t)(num_kv_heads + h) * kHD + 16 * (q8_v_col(n) & (kHD / 16 - 1))) = x;
+            *(uint4_t *)(kv + slot_off + (int64_t)(num_kv_heads + h) * kHD + 16 * q8_v_col(n)) = x;
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-              r.v[i] = i == (t_new >> 3) ? x : r.v[i];
+            for (int i = 0; i < kQ8VLoads; ++i) {
+              r.v[i] = i == t_new / kQ8VStep ? x : r.v[i];
             }
           }
         } else {
@@ -877,12 +888,12 @@ paged_decode_split_kernel(
               *(half8_t *)(dst + 32 * kk) = x;
             }
           }
-          if (g == (t_new & 3)) {
+          if (v_row_of(n, g) == (t_new & (kVStep - 1))) {
             const half8_t x = __builtin_bit_cast(half8_t, v_row[0]);
-            *(half8_t *)(kv + slot_off + (int64_t)(num_kv_heads + h) * kHD + 8 * (n & (kVCols - 1))) = x;
+            *(half8_t *)(kv + slot_off + (int64_t)(num_kv_heads + h) * kHD + v_col_of(n)) = x;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              r.v[i] = i == (t_new >> 2) ? x : r.v[i];
+            for (int i = 0; i < kVLoads; ++i) {
+              r.v[i] = i == t_new / kVStep ? x : r.v[i];
             }
           }
         }
