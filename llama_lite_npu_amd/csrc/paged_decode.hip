@@ -2195,10 +2195,26 @@ static int launch_balanced(const char *what, const void *q, int64_t q_batch_stri
                             num_q_heads, num_kv_heads, group, slices, s.heads_per_wg, s.replicas,
                             chunks, 0, softmax_scale * kLog2e);
     };
+    // A page of codes of 64 is 2 KiB of K and V to a wavefront, so two in flight leave the chunk waiting for memory
+    // where a page of fp16 rows or of 128 codes does not: four then, where the block table has 13 pages a chunk
+    // or more (a chunk of a few pages is not long enough to gain: 32 fp8 sequences of 100 to 1500 tokens, 11.7 a chunk
+    // by the table, 15.4 us a layer with two, 15.5 with four). 32 / 8 heads, us a layer: int8, 64 sequences of 2k to 8k
+    // tokens 73.0, 67.7, 128 of 100 to 1500 37.4, 35.8, 128 of 4k to 16k 273, 253; fp8, 48 of 300 to 2200 21.7, 21.3, 4
+    // of 8k to 16k (14 a chunk) 18.1, 17.6. Three or four pages of fp16 rows or of 128 codes: 0.79 to 1.01 of the speed.
+    constexpr int kManyPages = kHD == 64 ? 4 : LITEKV_DECODE_DEPTH;
+    const bool deep = kHD == 64 && (int64_t)batch * sub_stride >= (int64_t)13 * chunks;
+    auto by_depth = [&](auto format_tag) {
+      constexpr int KV = decltype(format_tag)::value;
+      if (deep) {
+        launch(paged_decode_balanced_kernel<kManyPages, KV>, static_cast<uint8_t *>(kv_pool));
+      } else {
+        launch(paged_decode_balanced_kernel<LITEKV_DECODE_DEPTH, KV>, static_cast<uint8_t *>(kv_pool));
+      }
+    };
     if (fp8_scales != nullptr && format == kKvInt8) {
-      launch(paged_decode_balanced_kernel<LITEKV_DECODE_DEPTH, kKvInt8>, static_cast<uint8_t *>(kv_pool));
+      by_depth(std::integral_constant<int, kKvInt8>{});
     } else if (fp8_scales != nullptr) {
-      launch(paged_decode_balanced_kernel<LITEKV_DECODE_DEPTH, kKvFp8>, static_cast<uint8_t *>(kv_pool));
+      by_depth(std::integral_constant<int, kKvFp8>{});
     } else {
       launch(paged_decode_balanced_kernel<LITEKV_DECODE_DEPTH, kKvF16>, static_cast<half_t *>(kv_pool));
     }

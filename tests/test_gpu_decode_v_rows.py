@@ -55,3 +55,46 @@ def test_the_new_token_at_every_place_of_a_page(fmt, head_dim, schedule):
             p = torch.softmax(full[at, h // 3] @ q[b, h] * case.softmax_scale, 0)
             ref[b, h] = p @ full[at, hkv + h // 3]
     assert_attention_close(out, ref.numpy(), f"{fmt} {head_dim} schedule {schedule}")
+
+
+@pytest.mark.parametrize("per_chunk", [1, 3, 4, 5, 8, 13, 17])
+@pytest.mark.parametrize("fmt", ["fp8", "int8"])
+def test_codes_of_64_with_two_and_four_pages_in_flight(fmt, per_chunk):
+    """Four from 13 pages a chunk by the block table's width on: chunks of up to as many pages, cut anywhere in
+    ragged sequences and empty ones, with a table of their own width and with one wide enough for four. The pages are
+    attended one after the other in both: the same bits, and close to float64."""
+    hq, hkv, d = 6, 2, 64
+    lens = [700, 1, -1, 16, 333, 17, -1, 1024, 96, 15]     # tokens before the step's own; -1: an empty row
+    print(f"pages in flight: {fmt}, {per_chunk} pages a chunk", flush=True)
+    case = workloads.make_decode_case("flight", 86, [max(n, 0) for n in lens], hq, hkv, device=DEV, head_dim=d)
+    dtype = torch.uint8 if fmt == "fp8" else torch.int8
+    scales = torch.tensor([0.031, 0.043, 0.027, 0.039], device=DEV)
+    slots = torch.arange(case.kv_pool.shape[0], dtype=torch.int32, device=DEV)
+    pool = torch.empty(case.kv_pool.shape, dtype=dtype, device=DEV)
+    ops.kv_append_quantised(case.kv_pool[:, :hkv], case.kv_pool[:, hkv:], slots, pool, scales)
+    seq = torch.tensor([n + 1 for n in lens], dtype=torch.int32, device=DEV)
+    pages = sum(-(-(n + 1) // 16) for n in lens)
+    chunks = -(-pages // per_chunk)
+    outs, pools = [], []
+    width = case.block_table.shape[1]
+    for w in (width, max(width, -(-13 * chunks // len(lens)))):
+        table = torch.zeros((len(lens), w), dtype=torch.int32, device=DEV)
+        table[:, :width] = case.block_table
+        plan = ops.DecodePlan(table, seq, hq, hkv, case.num_pages, chunks=chunks, kv_dtype=dtype, token_bytes=4 * d)
+        mine = pool.clone()
+        outs.append(ops.decode_step(case.q, mine, plan, case.k_new, case.v_new, case.softmax_scale, kv_scales=scales))
+        pools.append(mine)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(pools[0].view(torch.uint8), pools[1].view(torch.uint8))
+    rows = pools[0].double() if fmt == "int8" else pools[0].view(torch.float8_e4m3fn).double()
+    full = (rows * scales.double()[None, :, None]).cpu()
+    q = case.q.double().cpu()
+    ref = torch.zeros_like(q)
+    for b, n in enumerate(lens):
+        if n < 0:
+            continue
+        at = torch.tensor([int(case.block_table[b, t // 16]) * 16 + t % 16 for t in range(n + 1)])
+        for h in range(hq):
+            p = torch.softmax(full[at, h // 3] @ q[b, h] * case.softmax_scale, 0)
+            ref[b, h] = p @ full[at, hkv + h // 3]
+    assert_attention_close(outs[0], ref.numpy(), f"{fmt} {per_chunk}")
