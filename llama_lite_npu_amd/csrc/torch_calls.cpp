@@ -1,7 +1,8 @@
 // The per-layer calls of a prefill from PyTorch tensors: the checks of ops.py's wrappers and the
 // conversion of their arguments, in native code. A short prompt is bound by the host (two calls per
 // layer against 12 us of kernels), and there most of a call was Python: some sixty attribute reads
-// on tensors and twenty conversions by ctypes. One prompt of 203 tokens, 28 layers, 16 / 8 heads: 543 -> 359 us.
+// on tensors and twenty conversions by ctypes. One prompt of 203 tokens, 28 layers, 16 / 8 heads: 543 -> 359 us. Two
+// chunks of 64 rows over up to 1500 cached tokens, 32 / 8 heads of 64, cut along their keys: 638 -> 426 us.
 //
 // A function takes what it recognises as a plain, well-formed call; anything else (another dtype, a
 // shape that does not fit, a tensor subclass) it leaves alone and answers None, and the wrapper goes
@@ -160,7 +161,8 @@ PyObject *qk_norm_rope_append(PyObject *, PyObject *const *a, Py_ssize_t n) {
 
 // (q, kv_pool, block_table, cu_q_lens, context_lens, max_q_len, softmax_scale, page_size, kv_scales,
 //  max_kv_len or None, stream) -> the output, or the library's status if that is not 0, or None. A launch
-// that is to be cut along its keys is left to the wrapper as well.
+// that is to be cut along its keys (one request's chunk over a long history) gets the workspace of its partial rows
+// here, which like the wrapper's goes back to the allocator of the current stream behind the launches.
 PyObject *paged_prefill(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 11) Py_RETURN_NONE;
   try {
@@ -192,11 +194,18 @@ PyObject *paged_prefill(PyObject *, PyObject *const *a, Py_ssize_t n) {
         hq > INT32_MAX || pool.hkv > INT32_MAX || d > INT32_MAX || table->stride(0) > INT32_MAX) {
       Py_RETURN_NONE;
     }
-    if (a[9] != Py_None && t * hq > 0 && t * hq <= 128 * 512 &&
-        litekv_paged_prefill_key_slices((int32_t)b, (int32_t)hq, (int32_t)pool.hkv, (int32_t)d, (int32_t)max_q, max_kv) > 1) {
-      Py_RETURN_NONE;
+    // (the count's rule and the rows it looks at as in the wrapper)
+    int32_t slices = 1;
+    if (a[9] != Py_None && t * hq > 0 && t * hq <= 128 * 512) {
+      slices = litekv_paged_prefill_key_slices((int32_t)b, (int32_t)hq, (int32_t)pool.hkv, (int32_t)d, (int32_t)max_q, max_kv);
     }
     at::Tensor out = at::empty({t, hq, d}, q->options());
+    at::Tensor partials;
+    size_t partial_bytes = 0;
+    if (slices > 1) {
+      partial_bytes = litekv_paged_prefill_split_workspace_bytes(t, (int32_t)hq, (int32_t)d, slices);
+      partials = at::empty({(int64_t)(partial_bytes / sizeof(float))}, q->options().dtype(at::kFloat));
+    }
     const void *qp = address(q), *pp = address(pool.t);
     const int32_t *tp = static_cast<const int32_t *>(address(table)), *cup = static_cast<const int32_t *>(address(cu));
     const int32_t *ctxp = static_cast<const int32_t *>(address(ctx));
@@ -205,7 +214,18 @@ PyObject *paged_prefill(PyObject *, PyObject *const *a, Py_ssize_t n) {
     PyObject *result = THPVariable_Wrap(std::move(out));  // (before the launch: it may throw)
     const int32_t ts = (int32_t)table->stride(0);
     const int64_t pages = pool.slots / page;
+    void *wp = slices > 1 ? partials.data_ptr() : nullptr;
     const int rc = unlocked([&] {
+      if (slices > 1 && pool.format == kF16) {
+        return litekv_paged_prefill_split(qp, qs, pp, tp, ts, cup, ctxp, op, hq * d, (int32_t)b, (int32_t)hq, (int32_t)pool.hkv,
+                                          (int32_t)d, (int32_t)page, pages, (int32_t)max_q, t, slices, wp, partial_bytes,
+                                          (float)scale, stream);
+      }
+      if (slices > 1) {
+        return litekv_paged_prefill_split_q8(qp, qs, pp, scales, pool.format == kInt8, tp, ts, cup, ctxp, op, hq * d, (int32_t)b,
+                                             (int32_t)hq, (int32_t)pool.hkv, (int32_t)d, (int32_t)page, pages, (int32_t)max_q, t,
+                                             slices, wp, partial_bytes, (float)scale, stream);
+      }
       return litekv_paged_prefill_bounded(qp, qs, pp, scales, pool.format == kInt8, tp, ts, cup, ctxp, op, hq * d, (int32_t)b,
                                           (int32_t)hq, (int32_t)pool.hkv, (int32_t)d, (int32_t)page, pages, (int32_t)max_q,
                                           max_kv < 0 ? 0 : max_kv, (float)scale, stream);

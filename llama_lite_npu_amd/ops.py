@@ -878,7 +878,7 @@ def paged_prefill(q: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Ten
             if type(done) is int:
                 _lib.check(done)
             return done
-    # (not a plain call, or one that is cut along its keys)
+    # (not a plain call)
     _dev_half("q", q)
     fp8 = is_quantised_pool(kv_pool)
     if not fp8:
