@@ -474,7 +474,9 @@ __device__ __forceinline__ void prefill_tile_body(
       vbase = (const char *)packed.v + (int64_t)(q_start + first) * v_pitch;
       src0 = first;
     }
-    const uint32_t dst = (uint32_t)((kt & 1) * kTileHalfs + kRowsPerWave * wave * kHD) * 2u;
+    // (uniform, which the compiler does not see everywhere)
+    const uint32_t dst =
+        __builtin_amdgcn_readfirstlane((uint32_t)((kt & 1) * kTileHalfs + kRowsPerWave * wave * kHD) * 2u);
     auto load_rows = [&](uint32_t i, uint32_t ko, uint32_t vo) {
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                    :
@@ -754,8 +756,8 @@ __device__ __forceinline__ void prefill_tile_body(
     }
   };
   // V^T fragment j (A operand: d rows 16j.., keys 32 s2 + {4g..4g+3, 16+4g..}) of the staged tile.
-  auto load_vfrag = [&](int j, int s2) -> half8_t {
-    const uint32_t at = v_at(j) + 2u * 32 * s2 * kHD;
+  auto load_vfrag = [&](int j, int s2, uint32_t half) -> half8_t {
+    const uint32_t at = v_at(j) + half + 2u * 32 * s2 * kHD;
     const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t *)(uintptr_t)at);
     const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
         (lds_short4_t *)(uintptr_t)(at + 2u * 16 * kHD));
@@ -795,27 +797,26 @@ __device__ __forceinline__ void prefill_tile_body(
   // tile_bases() reads the page id (scalar), issue_rows(i) requests row group i of K and of V.
   const char *next_kbase = nullptr, *next_vbase = nullptr;
   uint32_t next_dst = 0;
-  // The page ids of a tile's four pages, one per lane (lane l: page l % 4 of the tile), requested a
-  // whole tile before tile_bases() needs them: as a scalar value read on the spot the id cost
+  // The page ids of two tiles' eight pages, one per lane (lane l: page l % 8 of tiles kt, kt + 1), requested
+  // whole tiles before tile_bases() needs them: as a scalar value read on the spot the id cost
   // every tile a round trip to memory in front of its first MFMA.
-  auto page_ids_of_tile = [&](int kt) -> int {
+  auto page_ids_of_tiles = [&](int kt) -> int {
     if constexpr (!PAGED) return 0;
-    int pidx = (tile0 + kt) * 4 + (lane & 3);
+    int pidx = (tile0 + kt) * 4 + (lane & 7);
     pidx = pidx < last_page ? pidx : last_page;
     return page_of(pidx);
   };
-  int ids_ahead = 0;  // of the tile after the one being staged
-  auto tile_bases = [&](int kt) {
+  auto tile_bases = [&](int kt, int half, int ids, int first) {  // half: kt % 2; ids: lanes first .. first + 3 those of tile kt
     const int row0 = (tile0 + kt) * kKvTile + kRowsPerWave * wave;
     if (PAGED) {
-      const int pid = __builtin_amdgcn_readlane(ids_ahead, (kRowsPerWave * wave) / 16);
+      const int pid = __builtin_amdgcn_readlane(ids, first + (kRowsPerWave * wave) / 16);
       next_kbase = (const char *)paged.kv + (int64_t)pid * ((int64_t)kPageSize * k_pitch);
       next_vbase = next_kbase;
     } else {
       next_kbase = (const char *)packed.k + (int64_t)(q_start + row0) * k_pitch;
       next_vbase = (const char *)packed.v + (int64_t)(q_start + row0) * v_pitch;
     }
-    next_dst = (uint32_t)((kt & 1) * kTileHalfs + kRowsPerWave * wave * kHD) * 2u;
+    next_dst = (uint32_t)(half * kTileHalfs + kRowsPerWave * wave * kHD) * 2u;
   };
   auto issue_rows = [&](int i) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
@@ -889,116 +890,134 @@ __device__ __forceinline__ void prefill_tile_body(
   // beside the vector ALU work of the other. Returns like fast_tiles (a grown tile is redone
   // from its first half).
   constexpr int kIssueEvery = kJTiles / kLoads;  // MFMA pairs between two row groups of the next tile
-  auto fast_plain_tiles = [&](int kt_end) -> int {
-    if constexpr (!FP8) {
-      if (kt < kt_end) ids_ahead = page_ids_of_tile(kt + 1);
+  // Two tiles an iteration, tile 2i + 1 in the second half of the staging area and tile 2i + 2 in the first: the halves
+  // are offsets of the LDS reads, and neither the addresses nor the page ids cost vector instructions in each tile (14 fewer;
+  // passes as above, 2825 -> 2802 us, 516 -> 509 the chunk over 7601 tokens, 592 -> 584 over int8, 324 -> 320 at 64). Taken
+  // up at an odd tile; taken up and left with the addresses on the half of tile kt - 1, like fast_tiles, or where tile
+  // kt is to be redone on its own.
+  auto plain_tile = [&](auto half_tag, int ids, int first) -> int {
+    constexpr uint32_t kAt = decltype(half_tag)::value ? 2u * kTileHalfs : 0u;
+    sync_and_prefetch(kt, FP8);
+    if constexpr (!FP8) tile_bases(kt + 1, decltype(half_tag)::value ? 0 : 1, ids, first);
+    // Block 1: scores of both halves, the first half's exponentials beside the second half's
+    // MFMAs, and the first half's V fragments requested before the block ends.
+    // Region 1: all eight K fragments of the first half are requested at once.
+    auto load_kfrag = [&](int s2, int i) -> half8_t {   // fragment i = (kk = i / 2, m = i % 2)
+      return *(const lds_half8_t *)(uintptr_t)(k_at(i >> 1) + kAt + 2u * (32 * s2 + 16 * (i & 1)) * kHD);
+    };
+    half8_t kf[kJTiles];
+#pragma unroll
+    for (int i = 0; i < kJTiles; ++i) kf[i] = load_kfrag(0, i);
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+#pragma unroll
+      for (int u = 0; u < CT; ++u) st[m][u] = st1[m][u] = seed[u];
     }
-    for (; kt < kt_end; ++kt) {
-      sync_and_prefetch(kt, FP8);
-      flip_halves();
+    __builtin_amdgcn_sched_barrier(0);
+    // Region 2: the first half's MFMAs; each fragment register takes the second half's
+    // fragment once its pair is issued. Four accumulators in rotation: no MFMA waits for
+    // the one before it.
+    half8_t kf1[kJTiles];
+#pragma unroll
+    for (int i = 0; i < kJTiles; ++i) {
+#pragma unroll
+      for (int u = 0; u < CT; ++u) st[i & 1][u] = mfma_16x16x32(kf[i], qf[u][i >> 1], st[i & 1][u]);
+      kf1[i] = load_kfrag(1, i);
       if constexpr (!FP8) {
-        tile_bases(kt + 1);
-        ids_ahead = page_ids_of_tile(kt + 2);
+        if (i % kIssueEvery == kIssueEvery - 1) issue_rows(i / kIssueEvery);
       }
-      // Block 1: scores of both halves, the first half's exponentials beside the second half's
-      // MFMAs, and the first half's V fragments requested before the block ends.
-      // Region 1: all eight K fragments of the first half are requested at once.
-      auto load_kfrag = [&](int s2, int i) -> half8_t {   // fragment i = (kk = i / 2, m = i % 2)
-        return *(const lds_half8_t *)(uintptr_t)(k_at(i >> 1) + 2u * (32 * s2 + 16 * (i & 1)) * kHD);
-      };
-      half8_t kf[kJTiles];
+    }
 #pragma unroll
-      for (int i = 0; i < kJTiles; ++i) kf[i] = load_kfrag(0, i);
+    for (int i = 0; i < kJTiles; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, CT, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (!FP8 && i % kIssueEvery == kIssueEvery - 1) __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // Region 3: the second half's MFMAs beside the first half's exponentials; the first
+    // half's V fragments are requested on the way.
+    // (Head dim 256: the exponentials stand in front of the MFMAs in the source here and below; behind
+    // them, the scheduler started them late and a tile took 3 % longer.)
+    half8_t vf[kJTiles];
+    if constexpr (kHD == 256) {
 #pragma unroll
-      for (int m = 0; m < 2; ++m) {
+      for (int u = 0; u < CT; ++u) exponentials_seeded(st, pk, pk_lo, u);
+    }
 #pragma unroll
-        for (int u = 0; u < CT; ++u) st[m][u] = st1[m][u] = seed[u];
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      // Region 2: the first half's MFMAs; each fragment register takes the second half's
-      // fragment once its pair is issued. Four accumulators in rotation: no MFMA waits for
-      // the one before it.
-      half8_t kf1[kJTiles];
+    for (int i = 0; i < kJTiles; ++i) {
 #pragma unroll
-      for (int i = 0; i < kJTiles; ++i) {
+      for (int u = 0; u < CT; ++u) st1[i & 1][u] = mfma_16x16x32(kf1[i], qf[u][i >> 1], st1[i & 1][u]);
+      vf[i] = load_vfrag(i, 0, kAt);
+    }
+    if constexpr (kHD != 256) {
 #pragma unroll
-        for (int u = 0; u < CT; ++u) st[i & 1][u] = mfma_16x16x32(kf[i], qf[u][i >> 1], st[i & 1][u]);
-        kf1[i] = load_kfrag(1, i);
-        if constexpr (!FP8) {
-          if (i % kIssueEvery == kIssueEvery - 1) issue_rows(i / kIssueEvery);
-        }
-      }
+      for (int u = 0; u < CT; ++u) exponentials_seeded(st, pk, pk_lo, u);
+    }
+    const bool over_a = overflowed(pk);
 #pragma unroll
-      for (int i = 0; i < kJTiles; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, CT, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        if (!FP8 && i % kIssueEvery == kIssueEvery - 1) __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      // Region 3: the second half's MFMAs beside the first half's exponentials; the first
-      // half's V fragments are requested on the way.
-      // (Head dim 256: the exponentials stand in front of the MFMAs in the source here and below; behind
-      // them, the scheduler started them late and a tile took 3 % longer.)
-      half8_t vf[kJTiles];
-      if constexpr (kHD == 256) {
+    for (int i = 0; i < kJTiles; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, CT, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+    }
+    if (over_a) return 1;
+    // Block 2: second product of the first half beside the second half's exponentials; each
+    // fragment register takes the second half's fragment as soon as its MFMAs are issued.
+    half8_t vf2[kJTiles];
+    if constexpr (kHD == 256) {
 #pragma unroll
-        for (int u = 0; u < CT; ++u) exponentials_seeded(st, pk, pk_lo, u);
-      }
+      for (int u = 0; u < CT; ++u) exponentials_seeded(st1, pk1, pk1_lo, u);
+    }
 #pragma unroll
-      for (int i = 0; i < kJTiles; ++i) {
+    for (int u = 0; u < CT; ++u) dsum[u] = mfma_p(ones, pk[u], pk_lo[u], dsum[u]);
 #pragma unroll
-        for (int u = 0; u < CT; ++u) st1[i & 1][u] = mfma_16x16x32(kf1[i], qf[u][i >> 1], st1[i & 1][u]);
-        vf[i] = load_vfrag(i, 0);
-      }
-      if constexpr (kHD != 256) {
+    for (int j = 0; j < kJTiles; ++j) {
 #pragma unroll
-        for (int u = 0; u < CT; ++u) exponentials_seeded(st, pk, pk_lo, u);
-      }
-      const bool over_a = overflowed(pk);
+      for (int u = 0; u < CT; ++u) acc[j][u] = mfma_p(vf[j], pk[u], pk_lo[u], acc[j][u]);
+      vf2[j] = load_vfrag(j, 1, kAt);
+    }
+    if constexpr (kHD != 256) {
 #pragma unroll
-      for (int i = 0; i < kJTiles; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, CT, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
-      }
-      if (over_a) return 1;
-      // Block 2: second product of the first half beside the second half's exponentials; each
-      // fragment register takes the second half's fragment as soon as its MFMAs are issued.
-      half8_t vf2[kJTiles];
-      if constexpr (kHD == 256) {
+      for (int u = 0; u < CT; ++u) exponentials_seeded(st1, pk1, pk1_lo, u);
+    }
+    const bool over_b = overflowed(pk1);
 #pragma unroll
-        for (int u = 0; u < CT; ++u) exponentials_seeded(st1, pk1, pk1_lo, u);
-      }
-#pragma unroll
-      for (int u = 0; u < CT; ++u) dsum[u] = mfma_p(ones, pk[u], pk_lo[u], dsum[u]);
-#pragma unroll
-      for (int j = 0; j < kJTiles; ++j) {
-#pragma unroll
-        for (int u = 0; u < CT; ++u) acc[j][u] = mfma_p(vf[j], pk[u], pk_lo[u], acc[j][u]);
-        vf2[j] = load_vfrag(j, 1);
-      }
-      if constexpr (kHD != 256) {
-#pragma unroll
-        for (int u = 0; u < CT; ++u) exponentials_seeded(st1, pk1, pk1_lo, u);
-      }
-      const bool over_b = overflowed(pk1);
-#pragma unroll
-      for (int i = 0; i < kJTiles; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, kTwoPartP ? 2 * CT : CT, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
-      }
+    for (int i = 0; i < kJTiles; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, kTwoPartP ? 2 * CT : CT, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
-      if (over_b) return 2;
-      // Block 3: second product of the second half.
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, kTwoPartP ? 2 * CT : CT, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+    if (over_b) return 2;
+    // Block 3: second product of the second half.
 #pragma unroll
-      for (int u = 0; u < CT; ++u) dsum[u] = mfma_p(ones, pk1[u], pk1_lo[u], dsum[u]);
+    for (int u = 0; u < CT; ++u) dsum[u] = mfma_p(ones, pk1[u], pk1_lo[u], dsum[u]);
 #pragma unroll
-      for (int j = 0; j < kJTiles; ++j) {
+    for (int j = 0; j < kJTiles; ++j) {
 #pragma unroll
-        for (int u = 0; u < CT; ++u) acc[j][u] = mfma_p(vf2[j], pk1[u], pk1_lo[u], acc[j][u]);
+      for (int u = 0; u < CT; ++u) acc[j][u] = mfma_p(vf2[j], pk1[u], pk1_lo[u], acc[j][u]);
+    }
+    return 0;
+  };
+  auto fast_plain_tiles = [&](int kt_end) -> int {
+    int ids = 0;  // of tiles kt + 1, kt + 2
+    if constexpr (!FP8) {
+      if (kt < kt_end) ids = page_ids_of_tiles(kt + 1);
+    }
+    while (kt < kt_end) {
+      int ids_next = 0;
+      int grew = plain_tile(std::true_type{}, ids, 0);
+      if (grew == 0) ++kt;
+      if (grew != 0 || kt >= kt_end) {
+        flip_halves();
+        return grew;
       }
+      if constexpr (!FP8) ids_next = page_ids_of_tiles(kt + 2);
+      grew = plain_tile(std::false_type{}, ids, 4);
+      if (grew != 0) return grew;
+      ++kt;
+      ids = ids_next;
     }
     return 0;
   };
@@ -1013,8 +1032,9 @@ __device__ __forceinline__ void prefill_tile_body(
       int n_spread = (last_key + 1) / kKvTile - 1 - tile0;   // tiles kt < n_spread: tile kt + 1 is full
       n_spread = n_spread < n_tiles - 1 ? n_spread : n_tiles - 1;
       n_spread = n_spread < n_plain ? n_spread : n_plain;
-      int grew = fast_plain_tiles(n_spread);
-      if (grew == 0) grew = fast_tiles(n_tiles, std::true_type{});
+      // (an even tile, behind one that was redone, goes the other way too)
+      int grew = kt & 1 ? fast_plain_tiles(n_spread) : 0;
+      if (grew == 0) grew = fast_tiles((kt & 1) == 0 && kt < n_spread ? kt + 1 : n_tiles, std::true_type{});
       if (grew != 0) {
         general_tile(kt, grew - 1);
         ++kt;
