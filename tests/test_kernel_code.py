@@ -7,6 +7,7 @@ import shutil
 import struct
 import subprocess
 
+import msgpack
 import pytest
 
 from llama_lite_npu_amd import _lib
@@ -42,6 +43,36 @@ def listings(code_objects, tmp_path_factory):
             if name:
                 out[name[1]] = [line.split("//")[0].strip() for line in body.splitlines()[1:]]
     return out
+
+
+@pytest.fixture(scope="module")
+def metadata(code_objects):
+    """The compiler's notes per kernel (section type 7, AMDGPU metadata: note type 32)."""
+    out = {}
+    for code in code_objects:
+        sections, = struct.unpack_from("<Q", code, 40)
+        size, count = struct.unpack_from("<HH", code, 58)
+        for at in range(sections, sections + size * count, size):
+            if struct.unpack_from("<I", code, at + 4)[0] != 7:
+                continue
+            note, = struct.unpack_from("<Q", code, at + 24)
+            name_bytes, bytes_, kind = struct.unpack_from("<III", code, note)
+            if kind == 32:
+                first = note + 12 + (name_bytes + 3) // 4 * 4
+                notes = msgpack.unpackb(code[first:first + bytes_], strict_map_key=False)
+                out.update({k[".name"]: k for k in notes["amdhsa.kernels"]})
+    return out
+
+
+def test_decode_kernels_of_narrow_heads_leave_room_for_three_workgroups(metadata):
+    """Head dim 64: three wavefronts per SIMD, which 168 registers (of 512, in steps of 8) and a third of the LDS allow,
+    and nothing spilled for it."""
+    kernels = {name: k for name, k in metadata.items()
+               if "hd64" in name and ("prefix_step_kernel" in name or "paged_decode_balanced_kernel" in name)}
+    assert len(kernels) >= 9
+    for name, k in kernels.items():
+        assert k[".vgpr_count"] <= 168 and k[".vgpr_spill_count"] == 0, (name, k[".vgpr_count"], k[".vgpr_spill_count"])
+        assert 3 * k[".group_segment_fixed_size"] <= 160 * 1024, name
 
 
 def test_page_ids_are_requested_behind_the_barrier(listings):
