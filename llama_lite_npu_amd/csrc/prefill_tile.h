@@ -117,6 +117,14 @@ constexpr float kLog2eP = 1.4426950408889634f;
 // lies outside goes another way there.
 __host__ __device__ constexpr bool tile_scale(float k_mul) { return k_mul >= 0x1p-100f && k_mul <= 0x1p100f; }
 
+// The entry of a block-table row, `bt_stride` (at least 1) of them, that holds page pidx of 16 tokens. A length beyond the row
+// re-reads its last entry, and so does a page in front of the row, which a sequence without a key (a context length of
+// minus its rows or less) asks for: the caller's 32-bit byte offset would take -1 to be 4 GiB past the row.
+__host__ __device__ __forceinline__ uint32_t table_entry(int pidx, int page_shift, int bt_stride) {
+  const uint32_t at = (uint32_t)(pidx >> page_shift), last = (uint32_t)bt_stride - 1u;
+  return at < last ? at : last;
+}
+
 // Where the keys of a sequence live.
 struct PagedSource {
   const half_t *kv;             // pool [slots][2*Hkv][128], fp16 (or E4M3 codes, one byte each)
@@ -421,9 +429,8 @@ __device__ __forceinline__ void prefill_tile_body(
   // The kernel works on 16-token pages: page j of them is part j % (1 << page_shift) of the
   // sequence's page j >> page_shift, whose tokens are contiguous in the pool.
   auto page_of = [&](int pidx) {
-    int at = pidx >> paged.page_shift;
-    at = at < paged.bt_stride ? at : paged.bt_stride - 1;  // a length beyond the row re-reads its last entry
-    int pid = *(const int32_t *)((const char *)table + 4u * (uint32_t)at);  // (a 32-bit offset from a scalar base)
+    const uint32_t at = table_entry(pidx, paged.page_shift, paged.bt_stride);
+    int pid = *(const int32_t *)((const char *)table + 4u * at);  // (a 32-bit offset from a scalar base)
     pid = pid < 0 ? 0 : (pid >= paged.num_pages ? paged.num_pages - 1 : pid);
     return (pid << paged.page_shift) + (pidx & ((1 << paged.page_shift) - 1));
   };
