@@ -1506,9 +1506,10 @@ __global__ __launch_bounds__(kMaxWavesPerWg * kWave) void paged_decode_balanced_
 // joins between hardware queues than they overlapped. Prefix workgroups come first in the grid:
 // they are the long ones, and x = kv head keeps a head's slices on one XCD. Registers are those
 // of the prefix role (two wavefronts per SIMD), so a compute unit holds one workgroup of either
-// role; at head dim 64 three workgroups of four wavefronts, as the LDS allows (51 KB), and the launch bound keeps the registers to
-// that: with 170 for int8, two past it, 64 sequences of 64 to 512 tokens behind 2048 shared ones, 32 / 8 heads, took 24.4 us
-// a layer instead of 19.9, 96 of 100 to 1000 behind 1024 33.8 instead of 29.0.
+// role. At head dim 64 it is three wavefronts per SIMD, and the launch bound keeps it at that: beside a prefix workgroup over codes,
+// four of whose eight wavefronts have left, there is then room for one of the other role. With 170 registers for int8,
+// two too many, 64 sequences of 64 to 512 tokens behind 2048 shared ones, 32 / 8 heads, took 24.4 us a layer instead of
+// 19.9, 96 of 100 to 1000 behind 1024 33.8 instead of 29.0.
 // ---------------------------------------------------------------------------------------------
 template <int KV> struct PrefixMode { static constexpr int value = prefill_tile::kSharedPrefix; };
 template <> struct PrefixMode<kKvFp8> { static constexpr int value = prefill_tile::kSharedPrefixFp8; };
