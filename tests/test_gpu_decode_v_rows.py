@@ -57,15 +57,18 @@ def test_the_new_token_at_every_place_of_a_page(fmt, head_dim, schedule):
     assert_attention_close(out, ref.numpy(), f"{fmt} {head_dim} schedule {schedule}")
 
 
-@pytest.mark.parametrize("per_chunk", [1, 3, 4, 5, 8, 13, 17])
+RAGGED = [700, 1, -1, 16, 333, 17, -1, 1024, 96, 15]        # tokens before the step's own; -1: an empty row
+FULL = [319, 303, 318, 190, 319, -1, 304, 317, 311, 288]    # ... that all but fill a table of 20 pages
+
+
 @pytest.mark.parametrize("fmt", ["fp8", "int8"])
-def test_codes_of_64_with_two_and_four_pages_in_flight(fmt, per_chunk):
-    """Four from 13 pages a chunk by the block table's width on: chunks of up to as many pages, cut anywhere in
-    ragged sequences and empty ones, with a table of their own width and with one wide enough for four. The pages are
-    attended one after the other in both: the same bits, and close to float64."""
+@pytest.mark.parametrize("lens,per_chunk", [(FULL, n) for n in (1, 2, 3, 4, 5, 7, 11)] + [(RAGGED, n) for n in (5, 13, 17, 40)])
+def test_codes_of_64_with_two_and_four_pages_in_flight(fmt, lens, per_chunk):
+    """Four from 13 pages a chunk by the block table's width on. Chunks of up to ``per_chunk`` pages, cut anywhere in the
+    sequences, with a table of their own width, which the full one keeps at two, and with one wide enough for four.
+    The pages are attended one after the other in both: the same bits, and close to float64."""
     hq, hkv, d = 6, 2, 64
-    lens = [700, 1, -1, 16, 333, 17, -1, 1024, 96, 15]     # tokens before the step's own; -1: an empty row
-    print(f"pages in flight: {fmt}, {per_chunk} pages a chunk", flush=True)
+    print(f"pages in flight: {fmt}, {per_chunk} pages a chunk, up to {max(lens)} tokens", flush=True)
     case = workloads.make_decode_case("flight", 86, [max(n, 0) for n in lens], hq, hkv, device=DEV, head_dim=d)
     dtype = torch.uint8 if fmt == "fp8" else torch.int8
     scales = torch.tensor([0.031, 0.043, 0.027, 0.039], device=DEV)
@@ -75,12 +78,17 @@ def test_codes_of_64_with_two_and_four_pages_in_flight(fmt, per_chunk):
     seq = torch.tensor([n + 1 for n in lens], dtype=torch.int32, device=DEV)
     pages = sum(-(-(n + 1) // 16) for n in lens)
     chunks = -(-pages // per_chunk)
-    outs, pools = [], []
     width = case.block_table.shape[1]
-    for w in (width, max(width, -(-13 * chunks // len(lens)))):
+    widths = [width, max(width, -(-13 * chunks // len(lens)))]
+    assert len(lens) * widths[1] >= 13 * chunks                     # four pages in flight
+    if lens is FULL:
+        assert len(lens) * widths[0] < 13 * chunks                  # two
+    outs, pools = [], []
+    for w in widths:
         table = torch.zeros((len(lens), w), dtype=torch.int32, device=DEV)
         table[:, :width] = case.block_table
         plan = ops.DecodePlan(table, seq, hq, hkv, case.num_pages, chunks=chunks, kv_dtype=dtype, token_bytes=4 * d)
+        assert plan.schedule == 0
         mine = pool.clone()
         outs.append(ops.decode_step(case.q, mine, plan, case.k_new, case.v_new, case.softmax_scale, kv_scales=scales))
         pools.append(mine)
