@@ -2205,7 +2205,9 @@ static int launch_balanced(const char *what, const void *q, int64_t q_batch_stri
     // or more (a chunk of a few pages is not long enough to gain: 32 fp8 sequences of 100 to 1500 tokens, 11.7 a chunk
     // by the table, 15.4 us a layer with two, 15.5 with four). 32 / 8 heads, us a layer: int8, 64 sequences of 2k to 8k
     // tokens 73.0, 67.7, 128 of 100 to 1500 37.4, 35.8, 128 of 4k to 16k 273, 253; fp8, 48 of 300 to 2200 21.7, 21.3, 4
-    // of 8k to 16k (14 a chunk) 18.1, 17.6. Three or four pages of fp16 rows or of 128 codes: 0.79 to 1.01 of the speed.
+    // of 8k to 16k (14 a chunk) 18.1, 17.6. A launch is not told the lengths, so short chunks in a table that is wide for them
+    // have four too: in one for 16k tokens 32 of 100 to 1500 took 15.8, 16.2 (int8; fp8 15.3, 15.5), 64 of them 23.2, 23.5,
+    // other batches of 8 to 256 sequences within 1 %. Three or four pages of fp16 rows or of 128 codes: 0.79 to 1.01 of the speed.
     constexpr int kManyPages = kHD == 64 ? 4 : LITEKV_DECODE_DEPTH;
     const bool deep = kHD == 64 && (int64_t)batch * sub_stride >= (int64_t)13 * chunks;
     auto by_depth = [&](auto format_tag) {

@@ -4,8 +4,8 @@
 // whole wavefront in the place of its tile.
 //
 // Bound by LDS reads and fp32 arithmetic: four prompts of 300 to 2048 tokens, 16 / 4 heads, every tile by
-// rows 5.2 ms (the general kernel 9.2, the matrix pipeline 0.08). It stands here so that the launch
-// needs no second kernel and no look at device data from the host.
+// rows, 8 at a time by eight wavefronts, 2.9 ms (16 by four 5.2, the general kernel 9.2, the matrix pipeline 0.08). It
+// stands here so that the launch needs no second kernel and no look at device data from the host.
 #pragma once
 
 #include "common.h"
@@ -15,7 +15,7 @@ namespace litekv {
 namespace prefill_rows {
 
 constexpr int kDim = 256;
-// Per wavefront: 20.6 KiB for 16 rows attended together, 10.3 for 8. (A row's result does not depend on it.)
+// Per wavefront: 20.25 KiB for 16 rows attended together, 10.25 for 8. (A row's result does not depend on it.)
 constexpr int lds_bytes(int rows) { return (rows * kDim + kWave * (rows + 1)) * 4; }
 
 typedef __attribute__((address_space(3))) float lds_float_t;

@@ -104,7 +104,8 @@ constexpr bool kTwoPartP = kHD == 256;
 constexpr int kMaxBias = kTwoPartP ? 9 : 0;
 constexpr int kMaxP = kTwoPartP ? 15 : 8;
 // Workgroups per compute unit: bounded by registers at 64 and 128 (about 150 and 235 per lane), by
-// LDS at 256 (two tiles of K and of V are 128 KiB), where a lane may then use all 512 registers.
+// LDS at 256 (two tiles of K and of V are 128 KiB), where a lane may then use all 512 registers (codes: four wavefronts)
+// or 256 (fp16 rows: eight).
 constexpr int kWgPerCu = kHD == 64 ? 3 : kHD == 128 ? 2 : 1;
 // Immediate of s_waitcnt that waits for all but the n youngest vector memory requests.
 constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
@@ -187,11 +188,12 @@ constexpr int kPagedPrefill = 0, kPackedPrefill = 1, kSharedPrefix = 2, kPagedPr
 // Column tiles per wavefront and wavefronts per workgroup of a prefill of 128 columns. Head dim 256 leaves one
 // workgroup per CU (LDS), which as four wavefronts of two column tiles is a lone wavefront per SIMD: its
 // softmax, LDS latencies and barrier waits stand in the open (MFMA busy 45 %). Eight wavefronts of one column tile
-// are two per SIMD at 256 registers; every K and V fragment then feeds one column tile instead of two, and the
-// 512 KiB a tile of keys reads from LDS (128 bytes a cycle) bound it: 2.3 us a tile, 2.5 before. Kernel time, 16 / 4
-// heads, four to eight wavefronts: 4 prompts of 459 to 1951 tokens 82 -> 76 us; passes with the epilogue, 300 tokens
-// 26.3 -> 21.9, 16 x 500..700 153 -> 132, 64 rows over 2000 cached tokens 54.5 -> 48.3. Codes keep four: their conversion
-// needs the registers (eight spill, and take 0.98 to 1.02 of the time).
+// are two per SIMD at 256 registers (MFMA busy 53 %). Every K and V fragment then feeds one column tile instead of two,
+// and LDS, read twice as much, is busy 36 % instead of 16: 2.3 us a tile of keys, 2.5 before. A launch of few workgroups
+// ends with its longest chain of tiles: 31 x 2.3 of the 76 us below. Kernel time, 16 / 4 heads, four to eight
+// wavefronts: 4 prompts of 459 to 1951 tokens 82 -> 76 us; passes with the epilogue, 300 tokens 26.3 -> 21.9, 16 x 500..700
+// 153 -> 132, 64 rows over 2000 cached tokens 54.5 -> 48.3. Codes keep four: their conversion needs the registers (eight
+// spill, and take 0.98 to 1.02 of the time).
 constexpr int prefill_ct(int mode) {
   return kHD == 256 && (mode == kPagedPrefill || mode == kPackedPrefill) ? 1 : kColTiles;
 }
@@ -388,7 +390,7 @@ __device__ __forceinline__ void prefill_tile_body(
   }
   const int n_tiles = (kv_end + kKvTile - 1) / kKvTile - tile0;
 
-  // a wavefront's own quarter of the staging area, for what it does before and after the tiles
+  // a wavefront's own part of the staging area, for what it does before and after the tiles
   constexpr uint32_t kOwnLds = (uint32_t)tile_lds_bytes<W>() / W;
   constexpr int kByRows = W == kWideWaves ? 8 : 16;  // rows of a tile attended together where it goes by rows
   static_assert(kHD != 256 || prefill_rows::lds_bytes(kByRows) <= kOwnLds, "rows attended together fit a wavefront's part");
@@ -615,7 +617,7 @@ __device__ __forceinline__ void prefill_tile_body(
   asm volatile("" : "+v"(ones));  // in registers: left alone, the constant is moved into them again in every tile
 
   // Swizzled read addresses (LDS bytes) for the tile half in use; they flip between the halves
-  // once per tile.
+  // once per tile (the loop below the diagonal takes two tiles at offsets of its own instead).
   // K, A operand of S^T: row 16m + n, chunk (4kk + g) ^ n.
   // (Rows of 512 bytes: the swizzle stays inside a 256-byte half, so the second half's addresses are
   // the first's plus a constant.)
